@@ -23,6 +23,7 @@
 #include <climits>
 #include <cstdint>
 #include <mutex>
+#include <type_traits>
 
 #include "pdmd_device.h"
 #include "pdmd_engine.h"
@@ -336,14 +337,18 @@ __device__ void set_code(const SysDev&, int row, int col, int code, int& status)
 struct Geo {
     double rx, ry, rz, b, r2, v2;
 };
+// x - round(x) (round: halves away from zero), from the half-to-even
+// rounding instruction: the two differ only where the remainder is exactly
+// one half, whose sign is then the opposite of x's
+__device__ inline double min_image(double x) {
+    const double d = x - __builtin_rint(x);
+    return fabs(d) == 0.5 ? copysign(0.5, -x) : d;
+}
 __device__ inline void geo(const Rec& a, const Rec& c, double tf, Geo& g) {
     const double vx = a.vx - c.vx, vy = a.vy - c.vy, vz = a.vz - c.vz;
-    double rx = a.x - c.x + vx * tf;
-    double ry = a.y - c.y + vy * tf;
-    double rz = a.z - c.z + vz * tf;
-    rx = rx - round(rx);
-    ry = ry - round(ry);
-    rz = rz - round(rz);
+    const double rx = min_image(a.x - c.x + vx * tf);
+    const double ry = min_image(a.y - c.y + vy * tf);
+    const double rz = min_image(a.z - c.z + vz * tf);
     g.rx = rx;
     g.ry = ry;
     g.rz = rz;
@@ -360,93 +365,71 @@ __device__ inline void bond_window(const DevTables& T, int code, double2 bw, dou
         blmax = T.ev_param[3][code];
     }
 }
-// collision time of pair (a, c) with ev_code `code` at false time tf; tij
-// keeps its preset (1e9) and type its value when no event is predicted.
+// collision time of a pair with ev_code `code` from its geometry g at the
+// current false time (ia, ic: identities, the lower bead's first; bonded:
+// the two are H-bonded; bwa: the lower bead's own bond window); tij keeps
+// its preset (1e9) and type its value when no event is predicted.
 // Every predictor of core.f, bond.f, sqwel.f, sqshlder.f and nc_sqwel.f has
 // the same shape: an inner radius^2 A and an outer radius^2 B with
 //   dA = b^2 - v^2 (r^2 - A),  dB = b^2 - v^2 (r^2 - B)
 // and one of four roots: approach to A, (-b - sqrt dA)/v^2; exit through B,
 // (-b + sqrt dB)/v^2; entry through B, (-b - sqrt dB)/v^2; and the stable
 // exit form of bond.f:63, -(r^2 - B)/(sqrt dB + b).  The per-class rules
-// below only choose A, B, the root and the type, so lanes of different
-// classes share one square root and one division, evaluated exactly as
-// each reference routine writes them.
-__device__ void predict(const DevTables& T, int code, const Rec& a, const Rec& c, bool bonded, double2 bwa,
-                        double tf, double& tij, int& type) {
-    const int ia = dyn_ident(a.dyn), ic = dyn_ident(c.dyn);
-    Geo g;
-    geo(a, c, tf, g);
+// below only choose A, B, the root and the type, by selects without a
+// branch: the lanes of a batch hold pairs of different classes, and every
+// class a divergent branch would run on its own.
+__device__ inline void predict_geo(const DevTables& T, int code, int ia, int ic, bool bonded, double2 bwa,
+                                   const Geo& g, double& tij, int& type) {
     const double b = g.b, r2 = g.r2, v2 = g.v2;
+    const bool sqz = code >= 22 && code <= 26;
     const bool is_core = code <= 3 || (code >= 17 && code <= 26);
     const bool is_bond = code >= 4 && code <= 12;
     const bool is_nc = code == 15, is_well = code == 16, is_shl = code >= 40;
-    if (!(is_core || is_bond || is_nc || is_well || is_shl)) {
-        type = -99;  // codes 13, 14, 27..39: error in ev_code matrix
-        return;
-    }
+    const int cc = min((unsigned)code, 50u);
     // inner and outer radii squared
     const double ssq = T.sigma_sq[ia][ic];
-    double A, B = 0.0;
-    if (is_core) {  // core.f:27-31
-        const double pe = T.ev_param[1][code];
-        A = ssq * (pe * pe);
-        if (code >= 22) {
-            const double q = T.sqz610[code - 21][ia > ic ? ia : ic];
-            A = A * (q * q);
-        }
-    } else if (is_bond) {  // bond.f:19-31,70-81
-        double blmin, blmax;
-        bond_window(T, code, bwa, blmin, blmax);
-        A = blmin * blmin;
-        B = blmax * blmax;
-    } else {
-        // nc_sqwel.f / sqwel.f / sqshlder.f: hard core unscaled, except the
-        // bonded N-C pair (core scaled by ev_param(1,15) twice)
-        A = (is_nc && ia + ic != 5 && bonded) ? ssq * T.ev_param[1][15] * T.ev_param[1][15] : ssq;
-        B = is_shl ? T.shlddia_sq[ia][ic] : T.welldia_sq[ia][ic];
-    }
+    const double pe = T.ev_param[1][cc];
+    const double q = T.sqz610[sqz ? code - 21 : 0][ia > ic ? ia : ic];
+    const double wsq = *(is_shl ? &T.shlddia_sq[ia][ic] : &T.welldia_sq[ia][ic]);
+    const double blmin = code >= 10 ? bwa.x : T.ev_param[2][cc], blmax = code >= 10 ? bwa.y : T.ev_param[3][cc];
+    // the bonded N-C pair: core scaled by ev_param(1,15) twice, inside the
+    // well by construction (nc_sqwel.f:76-101)
+    const bool nc_own = is_nc && ia + ic != 5;
+    const bool ncb = nc_own && bonded, ncu = nc_own && !bonded;
+    const bool wl = (is_nc && !nc_own) || is_well || is_shl;
+    double A = ssq * (pe * pe);         // core.f:27-31
+    A = sqz ? A * (q * q) : A;
+    A = wl || ncu ? ssq : A;            // sqwel.f, sqshlder.f, nc_sqwel.f: hard core unscaled
+    A = ncb ? ssq * pe * pe : A;
+    A = is_bond ? blmin * blmin : A;    // bond.f:19-31,70-81
+    const double B = is_bond ? blmax * blmax : wsq;
     const double dA = b * b - v2 * (r2 - A);
     const double diff = r2 - B;
     const double dB = b * b - v2 * diff;
-    // root: 0 none, 1 approach A, 2 exit B, 3 enter B, 4 stable exit B
-    int root = 0, ty = 0;
-    const bool in = b < 0.0;
-    if (is_core) {
-        if (in && dA > 0.0) { root = 1; ty = 1; }
-    } else if (is_bond) {
-        if (in) {
-            if (dA > 0.0) { root = 1; ty = 2; }
-            else if (dB > 0.0) { root = 2; ty = 3; }
-        } else if (dB > 0.0) { root = 4; ty = 3; }
-    } else if (is_nc && ia + ic != 5) {
-        if (bonded) {  // nc_sqwel.f:76-101: inside the well by construction
-            if (in && dA > 0.0) { root = 1; ty = 1; }
-            else { root = 2; ty = 8; }
-        } else if (in && dB > 0.0) { root = 3; ty = 9; }
-    } else {
-        // H-bond N-C well (types 1/16/7), side-chain well (1/8/4), shoulder (1/10/12)
-        const int ex = is_nc ? 16 : (is_well ? 8 : 10);
-        const int en = is_nc ? 7 : (is_well ? 4 : 12);
-        if (in) {
-            if (diff < 0.0) {
-                if (dA > 0.0) { root = 1; ty = 1; }
-                else { root = 2; ty = ex; }
-            } else if (dB > 0.0) { root = 3; ty = en; }
-        } else if (diff < 0.0) { root = 2; ty = ex; }
-    }
-    if (root == 0) return;
-    const double sq = sqrt(root == 1 ? dA : dB);
-    double num, den = v2;
-    if (root == 1 || root == 3)
-        num = -b - sq;
-    else if (root == 2)
-        num = -b + sq;
-    else {
-        num = -diff;
-        den = sq + b;
-    }
-    tij = num / den;
-    type = ty;
+    const bool in = b < 0.0, pA = dA > 0.0, pB = dB > 0.0, inside = diff < 0.0;
+    // root: r1 approach A, r2_ exit B, r3 enter B, r4 stable exit B
+    const bool r1 = in && pA && (is_core || is_bond || ncb || (wl && inside));
+    const bool r2_ = !r1 && ((is_bond && in && pB) || ncb || (wl && inside));
+    const bool r3 = in && pB && (ncu || (wl && !inside));
+    const bool r4 = is_bond && !in && pB;
+    // types: N-C H-bond well 1/16/7, side-chain well 1/8/4, shoulder 1/10/12
+    const int ex = is_bond ? 3 : (ncb || is_well ? 8 : (is_nc ? 16 : 10));
+    const int en = ncu ? 9 : (is_nc ? 7 : (is_well ? 4 : 12));
+    const int ty = r1 ? (is_bond ? 2 : 1) : (r2_ ? ex : (r4 ? 3 : en));
+    const double sq = sqrt(r1 ? dA : dB);
+    const double num = r4 ? -diff : (r2_ ? -b + sq : -b - sq);
+    const double den = r4 ? sq + b : v2;
+    const double t = num / den;
+    const bool any = r1 || r2_ || r3 || r4;
+    tij = any ? t : tij;
+    type = any ? ty : type;
+    if (!(is_core || is_bond || is_nc || is_well || is_shl)) type = -99;  // codes 13, 14, 27..39: error in ev_code matrix
+}
+__device__ inline void predict(const DevTables& T, int code, const Rec& a, const Rec& c, bool bonded, double2 bwa,
+                               double tf, double& tij, int& type) {
+    Geo g;
+    geo(a, c, tf, g);
+    predict_geo(T, code, dyn_ident(a.dyn), dyn_ident(c.dyn), bonded, bwa, g, tij, type);
 }
 
 // ------------------------------------------------------------------------
@@ -487,6 +470,14 @@ __device__ inline void wg_sync(int nw) {
         __syncthreads();
     else
         wave_sync_mem();
+}
+
+// scalar-register copies of wave-uniform values: what depends on them
+// branches and addresses on the scalar unit instead of masking lanes
+__device__ inline int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ inline int4 uni(int4 v) { return make_int4(uni(v.x), uni(v.y), uni(v.z), uni(v.w)); }
+__device__ inline double uni(double v) {
+    return __hiloint2double(uni(__double2hiint(v)), uni(__double2loint(v)));
 }
 
 // DPP lane moves: CTRL row_shr:n = 0x110+n, row_bcast:15 = 0x142,
@@ -655,6 +646,17 @@ __device__ inline int calc_bin(const Sc& c, double tim, bool uncond, int& status
     return j < c.nbin ? -1 : j;
 }
 
+__device__ inline int bin_of(double interval_max, double tbin_off, double sortsize, int nbin, double tim, int& status) {
+    if (!(tim < interval_max)) return -1;
+    int j = (int)((tim + tbin_off) / sortsize) + 1;
+    if (j > kNumbin) j = kNumbin;
+    if (j < 0) {
+        if (!status) status = kErrBin;
+        return -1;
+    }
+    return j < nbin ? -1 : j;
+}
+
 // flags: kPairReadsSp = the outcome resolution read the shoulder set or an
 // H-bond partner; kPairWroteSp = the event rewrote them
 constexpr int kPairReadsSp = 1, kPairWroteSp = 2;
@@ -704,68 +706,101 @@ struct Batch {
     int nbl[kMaxWaves];   // blocks to rescan, in each wavefront's list
     int st[kMaxWaves];    // status after each event
     int wdone[kMaxWaves]; // the wavefront's committed entries are written
+    int st_rep[kMaxWaves];  // status of its replayed updates
     int K;                // entries popped this round (0: stop)
     int cut;              // first wavefront whose event is not committed
     int rebuild;          // the round's sync event rebuilds the lists
+    unsigned long long touched;  // superblocks with a changed block minimum (bit s)
     int gbead;            // the bead of a ghost event leading the round
     long long t0;         // start of a budgeted launch (wall_clock64)
 };
-// Order proxy of a calendar key: the bin in the top 12 bits, then the top
-// 52 bits of the ordered time.  Proxies order keys as key_less does except
-// that distinct keys may share one; the reductions below take the minimum
-// proxy with 64-bit lane moves and settle shared proxies with key_less.
-__device__ inline unsigned long long key_proxy(const Key& k) {
-    return k.bc == kEmptyBc ? ~0ull
-                            : (((unsigned long long)(unsigned)(k.bc >> 8) << 52) | (t_order(k.t) >> 12));
+// Order proxy of a calendar key: a positive double with the bin in its
+// exponent field (bins 1 to kNumbin = 2000 of 2046 values) and the top 52
+// bits below the sign of the time in its mantissa (negative times as 0);
+// +infinity for no entry.  Proxies order keys as key_less does except that
+// distinct keys may share one; the reductions below take the minimum proxy
+// and settle shared proxies with key_less.  As doubles they need one
+// instruction per step for the minimum where 64-bit integers need a compare
+// and two selects, and no proxy is a NaN or a denormal (bins start at 1).
+__device__ inline double key_proxy(const Key& k) {
+    const long long b = __double_as_longlong(k.t);
+    const int hi = (int)(b >> 32);
+    const unsigned h = (unsigned)max(hi, 0), l = hi < 0 ? 0u : (unsigned)b;
+    const unsigned ph = ((unsigned)(k.bc >> 8) << 20) | (h >> 11), pl = (h << 21) | (l >> 11);
+    const bool none = k.bc == kEmptyBc;
+    return __hiloint2double(none ? 0x7FF00000 : (int)ph, none ? 0 : (int)pl);
 }
-template <int CTRL, int RM>
-__device__ inline unsigned long long dpp_u64(unsigned long long v) {
-    const int lo = dpp_i<CTRL, RM>((int)v), hi = dpp_i<CTRL, RM>((int)(v >> 32));
-    return (unsigned long long)(unsigned)lo | ((unsigned long long)(unsigned)hi << 32);
+constexpr int kInfHi = 0x7FF00000;
+__device__ inline bool proxy_none(double p) { return __double2hiint(p) == kInfHi; }
+// v_min_f64 without the quieting of its operands that the compiler puts
+// before it; the wait states that a lane move of the result needs follow
+__device__ inline double min_raw(double a, double b) {
+    double r;
+    asm("v_min_f64 %0, %1, %2\n\ts_nop 1" : "=v"(r) : "v"(a), "v"(b));
+    return r;
 }
-template <int CTRL, int RM>
-__device__ inline void umin_step(unsigned long long& v) {
-    const unsigned long long o = dpp_u64<CTRL, RM>(v);
-    v = o < v ? o : v;
+// a lane move in which every lane has a source (row_ror:n = 0x120 + n)
+template <int CTRL>
+__device__ inline double ror_d(double v) {
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
 }
-// minimum over the wave, returned to every lane
-__device__ inline Key key_min_wave(Key k) {
-    const unsigned long long p = key_proxy(k);
-    unsigned long long m = p;
-    umin_step<0x111, 0xf>(m);
-    umin_step<0x112, 0xf>(m);
-    umin_step<0x114, 0xf>(m);
-    umin_step<0x118, 0xf>(m);
-    umin_step<0x142, 0xa>(m);
-    umin_step<0x143, 0xc>(m);
-    const unsigned long long mn = (unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)m, 63) |
-                                  ((unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(m >> 32), 63) << 32);
-    if (mn == ~0ull) return empty_key();
-    const unsigned long long tie = __ballot(p == mn);
-    Key r = readlane_key(k, __ffsll((long long)tie) - 1);
+// minimum over each row of 16 lanes, in all of its lanes
+__device__ inline double row_min(double v) {
+    v = min_raw(v, ror_d<0x121>(v));
+    v = min_raw(v, ror_d<0x122>(v));
+    v = min_raw(v, ror_d<0x124>(v));
+    return min_raw(v, ror_d<0x128>(v));
+}
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+// minimum over the wave, in every lane
+__device__ inline double wave_min(double v) {
+    v = row_min(v);
+    {
+        const unsigned lo = (unsigned)__double2loint(v), hi = (unsigned)__double2hiint(v);
+        const u32x2 l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+        const u32x2 h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+        v = min_raw(__hiloint2double((int)h.x, (int)l.x), __hiloint2double((int)h.y, (int)l.y));
+    }
+    {
+        const unsigned lo = (unsigned)__double2loint(v), hi = (unsigned)__double2hiint(v);
+        const u32x2 l = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+        const u32x2 h = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+        v = min_raw(__hiloint2double((int)h.x, (int)l.x), __hiloint2double((int)h.y, (int)l.y));
+    }
+    return v;
+}
+// the least key among the lanes of `tie` (not empty), which share a proxy;
+// src becomes its lane
+__device__ inline Key key_of_ties(const Key& k, unsigned long long tie, int& src) {
+    src = __ffsll((long long)tie) - 1;
+    Key r = readlane_key(k, src);
     unsigned long long rest = tie & (tie - 1);
     while (rest) {
-        const Key o = readlane_key(k, __ffsll((long long)rest) - 1);
+        const int o_src = __ffsll((long long)rest) - 1;
+        const Key o = readlane_key(k, o_src);
         rest &= rest - 1;
-        if (key_less(o, r)) r = o;
+        if (key_less(o, r)) {
+            r = o;
+            src = o_src;
+        }
     }
     return r;
 }
+// minimum over the wave, returned to every lane
+__device__ inline Key key_min_wave(const Key& k) {
+    const double p = key_proxy(k), m = wave_min(p);
+    if (proxy_none(readlane_d(m, 0))) return empty_key();
+    int src;
+    return key_of_ties(k, __ballot(p == m), src);
+}
 // minimum over the wave of keys with their add stamps given per lane (new
 // entries, not yet written), returned to every lane with its stamp
-__device__ inline Key key_min_wave_st(Key k, unsigned long long st, unsigned long long& out_st) {
-    const unsigned long long p = key_proxy(k);
-    unsigned long long m = p;
-    umin_step<0x111, 0xf>(m);
-    umin_step<0x112, 0xf>(m);
-    umin_step<0x114, 0xf>(m);
-    umin_step<0x118, 0xf>(m);
-    umin_step<0x142, 0xa>(m);
-    umin_step<0x143, 0xc>(m);
-    const unsigned long long mn = (unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)m, 63) |
-                                  ((unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(m >> 32), 63) << 32);
+__device__ inline Key key_min_wave_st(const Key& k, unsigned long long st, unsigned long long& out_st) {
+    const double p = key_proxy(k), mn = wave_min(p);
     out_st = 0;
-    if (mn == ~0ull) return empty_key();
+    if (proxy_none(readlane_d(mn, 0))) return empty_key();
     const unsigned long long tie = __ballot(p == mn);
     int src = __ffsll((long long)tie) - 1;
     Key r = readlane_key(k, src);
@@ -791,31 +826,21 @@ __device__ inline Key key_min_wave_st(Key k, unsigned long long st, unsigned lon
 // empty or when shared proxies need the exact scan).
 __device__ inline bool key_min_rows(Key& k) {
     const int lane = lane_id();
-    const unsigned long long p = key_proxy(k);
-    unsigned long long m = p;
-    umin_step<0x111, 0xf>(m);
-    umin_step<0x112, 0xf>(m);
-    umin_step<0x114, 0xf>(m);
-    umin_step<0x118, 0xf>(m);
-    const unsigned long long rm = dpp_u64<0x15F, 0xf>(m);  // the row's last lane, to the whole row
-    const unsigned long long tie = __ballot(p == rm && rm != ~0ull);
+    const double p = key_proxy(k), rm = row_min(p);
+    const unsigned long long tie = __ballot(p == rm && !proxy_none(rm));
     const unsigned rb = (unsigned)(tie >> (lane & 48)) & 0xFFFFu;
-    if (__ballot(__popc(rb) > 1)) {
+    if (__ballot((rb & (rb - 1u)) != 0u)) {
         key_min_rows_exact(k);
         return (lane & 15) == 15;
     }
-    if (rm == ~0ull) {
-        k = empty_key();
-        return (lane & 15) == 15;
-    }
-    return p == rm;
+    return proxy_none(rm) ? (lane & 15) == 15 : p == rm;
 }
 
 // LDS views, one set per wavefront: the calendar tree, the master scalars
 // and the round record are shared, the work lists are the wavefront's own
 struct Lds {
     int o_blk, o_sup, o_wm, o_wx, o_blist, o_pair, o_sc, o_leaf, o_wd, o_wt, o_wy, o_slot, o_spec, o_down;
-    int o_msc, o_batch;
+    int o_msc, o_batch, o_mark;
     Leaf* gleaf;  // calendar leaves in HBM when they do not fit in LDS
     // the round's footprint marks: a flat pointer into LDS (behind the
     // leaves, when both fit there) or to SysDev::mark
@@ -843,6 +868,12 @@ struct Lds {
 constexpr int kLdOff = kSdOff + (int)((sizeof(SysDev) + 15) / 16 * 16);
 constexpr int kLdStride = (int)((sizeof(Lds) + 15) / 16 * 16);
 __device__ inline const Lds& ldsv() { return *reinterpret_cast<const Lds*>(smem + kLdOff + wave_id() * kLdStride); }
+// the shared blocks that make_lds lays out after the views
+constexpr int kSupOff = kLdOff + kLdStride * kMaxWaves;
+constexpr int kMscOff = kSupOff + (int)(sizeof(Key) * kSup);
+constexpr int kBatchOff = kMscOff + (int)((sizeof(Sc) + 15) / 16 * 16);
+__device__ inline Sc& master() { return *reinterpret_cast<Sc*>(smem + kMscOff); }
+__device__ inline Batch& round_rec() { return *reinterpret_cast<Batch*>(smem + kBatchOff); }
 template <class T>
 __device__ inline T* sgpr_ptr(T* p) {
     const unsigned long long v = (unsigned long long)p;
@@ -871,6 +902,7 @@ __device__ inline Lds lds_regs() {
     r.o_down = __builtin_amdgcn_readfirstlane(m.o_down);
     r.o_msc = __builtin_amdgcn_readfirstlane(m.o_msc);
     r.o_batch = __builtin_amdgcn_readfirstlane(m.o_batch);
+    r.o_mark = __builtin_amdgcn_readfirstlane(m.o_mark);
     r.gleaf = sgpr_ptr(m.gleaf);
     r.nblk = __builtin_amdgcn_readfirstlane(m.nblk);
     r.nsup = __builtin_amdgcn_readfirstlane(m.nsup);
@@ -900,6 +932,158 @@ __device__ inline void leaf_set(const Lds& L, int k, const Leaf& v) {
         L.lleaf()[k] = v;
     else
         gst(L.gleaf + k, v);
+}
+
+// What the event loop reads of its system and of the LDS plan, as values
+// that stay in scalar registers for the whole launch.
+struct Hot {
+    Rec* rec;
+    double2* bw;
+    int4* extra;
+    int4* ovr;
+    int* nb_up;
+    int* nb_dn;
+    int* nup;
+    int* ndn;
+    Leaf* leaf;
+    unsigned* mark;
+    unsigned long long* stamp;
+    int N, cap, nblk, nsup, o_blk, o_leaf, o_mark, o_w, o_blist;
+    bool leaf_lds, mark_lds;
+};
+__device__ inline Hot load_hot(const SysDev& S, const Lds& L) {
+    Hot H;
+    H.rec = sgpr_ptr(S.rec);
+    H.bw = sgpr_ptr(S.bw);
+    H.extra = sgpr_ptr(S.extra);
+    H.ovr = sgpr_ptr(S.ovr);
+    H.nb_up = sgpr_ptr(S.nb_up);
+    H.nb_dn = sgpr_ptr(S.nb_dn);
+    H.nup = sgpr_ptr(S.nup);
+    H.ndn = sgpr_ptr(S.ndn);
+    H.leaf = sgpr_ptr(S.leaf);
+    H.mark = sgpr_ptr(S.mark);
+    H.stamp = sgpr_ptr(S.stamp);
+    H.N = uni(S.N);
+    H.cap = uni(S.cap);
+    H.nblk = uni(L.nblk);
+    H.nsup = uni(L.nsup);
+    H.o_blk = uni(L.o_blk);
+    H.o_leaf = uni(L.o_leaf);
+    H.o_mark = uni(L.o_mark);
+    H.o_w = uni(L.o_wm);
+    H.o_blist = uni(L.o_blist);
+    H.leaf_lds = uni(L.leaf_lds ? 1 : 0) != 0;
+    H.mark_lds = uni(L.mark_lds ? 1 : 0) != 0;
+    return H;
+}
+// element i of a buffer: scalar base, 32-bit byte offset
+template <class T>
+__device__ inline T ld_at(const T* base, int i) {
+    const GLB char* q = (const GLB char*)base + (unsigned)i * (unsigned)sizeof(T);
+    if constexpr (sizeof(T) % 16 == 0) {
+        u32x4 t[sizeof(T) / 16];
+#pragma unroll
+        for (int k = 0; k < (int)(sizeof(T) / 16); ++k) t[k] = ((const GLB u32x4*)q)[k];
+        T r;
+        __builtin_memcpy(&r, t, sizeof(T));
+        return r;
+    } else
+        return *(const GLB T*)q;
+}
+template <class T>
+__device__ inline void st_at(T* base, int i, const T& v) {
+    GLB char* q = (GLB char*)base + (unsigned)i * (unsigned)sizeof(T);
+    u32x4 t[sizeof(T) / 16];
+    __builtin_memcpy(t, &v, sizeof(T));
+#pragma unroll
+    for (int k = 0; k < (int)(sizeof(T) / 16); ++k) ((GLB u32x4*)q)[k] = t[k];
+}
+__device__ inline Leaf leaf_ld(const Hot& H, int k) {
+    return H.leaf_lds ? reinterpret_cast<const Leaf*>(smem + H.o_leaf)[k] : ld_at(H.leaf, k);
+}
+__device__ inline void leaf_st(const Hot& H, int k, const Leaf& v) {
+    if (H.leaf_lds)
+        reinterpret_cast<Leaf*>(smem + H.o_leaf)[k] = v;
+    else
+        st_at(H.leaf, k, v);
+}
+__device__ inline void stamp_st(const Hot& H, int k, unsigned long long v) {
+    __hip_atomic_store((GLB unsigned long long*)((GLB char*)H.stamp + (unsigned)k * 8u), v, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Block minima of the listed blocks after a round, one row of 16 lanes per
+// block, 16 blocks per step so that four independent reductions overlap.  A
+// block whose minimum came out as it was is not written and leaves its
+// superblock alone; the others mark theirs in Batch::touched.
+__device__ inline void rescan_round(const Hot& H, const int* list, int nb) {
+    const int lane = lane_id(), N3 = H.N + 3;
+    Key* const blk = reinterpret_cast<Key*>(smem + H.o_blk);
+    for (int base = 0; base < nb; base += 16) {
+        Key e[4], old[4];
+        double p[4], m[4];
+        int bq[4];
+        bool dup = false;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int q = base + 4 * u + (lane >> 4);
+            bq[u] = q < nb ? list[q] : -1;
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int idx = bq[u] * kBlk + (lane & 15);
+            e[u] = empty_key();
+            if (bq[u] >= 0) {
+                old[u] = blk[bq[u]];
+                if (idx < N3) e[u] = leaf_key(leaf_ld(H, idx), idx);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) p[u] = key_proxy(e[u]);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) m[u] = row_min(p[u]);
+        bool win[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const unsigned long long tie = __ballot(p[u] == m[u] && !proxy_none(m[u]));
+            const unsigned rb = (unsigned)(tie >> (lane & 48)) & 0xFFFFu;
+            win[u] = proxy_none(m[u]) ? (lane & 15) == 15 : p[u] == m[u];
+            dup |= (rb & (rb - 1u)) != 0u;
+        }
+        if (__ballot(dup)) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) win[u] = key_min_rows(e[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (win[u] && bq[u] >= 0 && (e[u].t != old[u].t || e[u].bc != old[u].bc || e[u].ip != old[u].ip)) {
+                blk[bq[u]] = e[u];
+                if (H.nsup > 1)
+                    __hip_atomic_fetch_or(&round_rec().touched, 1ull << (bq[u] / kSup), __ATOMIC_RELAXED,
+                                          __HIP_MEMORY_SCOPE_WORKGROUP);
+            }
+    }
+}
+// Superblock minima of the round's touched superblocks, shared out over the
+// nw wavefronts.
+__device__ inline void rescan_touched(const Hot& H, int wave, int nw) {
+    const int lane = lane_id();
+    const Key* const blk = reinterpret_cast<const Key*>(smem + H.o_blk);
+    Key* const sup = reinterpret_cast<Key*>(smem + kSupOff);
+    const unsigned long long tv = round_rec().touched;
+    unsigned long long touched = (unsigned long long)(unsigned)uni((int)tv) | ((unsigned long long)(unsigned)uni((int)(tv >> 32)) << 32);
+    int turn = 0;
+    while (touched) {
+        const int s = __ffsll((long long)touched) - 1;
+        touched &= touched - 1;
+        const bool mine = turn == wave;
+        turn = turn + 1 == nw ? 0 : turn + 1;
+        if (!mine) continue;
+        const int b = s * kSup + lane;
+        const Key e = key_min_wave(b < H.nblk ? blk[b] : empty_key());
+        if (lane == 0) sup[s] = e;
+    }
 }
 
 // block minima of the listed blocks (4 blocks per pass, one row of 16 lanes
@@ -1042,6 +1226,11 @@ __device__ inline int spec_abort(const Lds& L, int bk, int& nb) {
     return -1;
 }
 
+__device__ inline void spec_abort_at(int bk, int& nb) {
+    if (lane_id() == 0) atomicMin(&round_rec().cut, bk);
+    bar_to(nb, kRoundBars);
+}
+
 __device__ inline void round_clear_marks(const Lds& L, const SysDev& S, int dent, int i, int j, int sp) {
     const int lane = lane_id();
     if (dent >= 0) mark_clear(L, S, dent);
@@ -1069,6 +1258,35 @@ __device__ inline int batch_accepted(const Batch& B) {
             lo_st = B.knew_st[k];
         }
     }
+    return A;
+}
+
+// The same, one round entry per lane: an exclusive prefix minimum of the new
+// keys' proxies against the popped keys' proxies; a shared proxy goes to the
+// exact form above.  Uniform over the wavefront.
+__device__ inline int accepted(const Batch& B) {
+    const int lane = lane_id();
+    const int top = uni(min(B.K, B.cut));
+    const int q = lane & (kMaxWaves - 1);
+    const bool in = lane < top;
+    const double pk = key_proxy(B.key[q]);
+    const double pn = in ? key_proxy(B.knew[q]) : __hiloint2double(kInfHi, 0);
+    const int st = in ? B.st[q] : 0;
+    auto shr = [](double v, auto ctrl) {
+        constexpr int C = decltype(ctrl)::value;
+        return __hiloint2double(__builtin_amdgcn_update_dpp(kInfHi, __double2hiint(v), C, 0xf, 0xf, false),
+                                __builtin_amdgcn_update_dpp(0, __double2loint(v), C, 0xf, 0xf, false));
+    };
+    double lo = shr(pn, std::integral_constant<int, 0x111>{});
+    lo = min_raw(lo, shr(lo, std::integral_constant<int, 0x111>{}));
+    lo = min_raw(lo, shr(lo, std::integral_constant<int, 0x112>{}));
+    lo = min_raw(lo, shr(lo, std::integral_constant<int, 0x114>{}));
+    const bool live = in && lane >= 1;
+    if (__ballot(live && pk == lo)) return uni(batch_accepted(B));
+    const unsigned long long fail = __ballot(live && pk > lo), sm = __ballot(st != 0);
+    int A = top;
+    if (fail) A = min(A, __ffsll((long long)fail) - 1);
+    if (sm) A = min(A, (int)__ffsll((long long)sm));
     return A;
 }
 
@@ -1485,8 +1703,8 @@ __device__ void reschedule_generic(const SysDev&, const DevTables&, const Lds&, 
 // the partners of the batched beads.  Down sets above one wavefront take
 // the generic path.  extra_blk: a further calendar block to rescan (the
 // ghost entry), or -1
-__device__ void reschedule(const SysDev&, const DevTables&, const Lds&, Sc&, const Pair&, int extra_blk,
-                           bool xpulse_del, int bk, const Rows& rw) {
+__device__ __noinline__ void reschedule(const SysDev&, const DevTables&, const Lds&, Sc&, const Pair&, int extra_blk,
+                           bool xpulse_del, int bk) {
     const Lds L = lds_regs();
 
     const SysDev& S = sdev();
@@ -1518,6 +1736,7 @@ __device__ void reschedule(const SysDev&, const DevTables&, const Lds&, Sc&, con
     int status = 0, nb = 0;
     PH_BEGIN(tph);
     // ---- first loads: list rows of i and j, whole rows with their lengths
+    const Rows rw = load_rows(S, i, j);
     const int nui = rw.nui, ndi = rw.ndi, nuj = rw.nuj, ndj = rw.ndj;
     const int eui = rw.eui, edi = rw.edi, euj = rw.euj, edj = rw.edj;
     const int xi0 = P.xi.x, xi1 = P.xi.y, xi2 = P.xi.z;
@@ -2188,7 +2407,7 @@ __device__ inline void nudge(Rec& bi, Rec& bj, double bd, const Geo& g, int sign
     }
 }
 
-__device__ void eventdyn(const DevTables& T, Rec& bi, Rec& bj, double2 bwi, bool bonded_ij, int evcode, double tf,
+__device__ __forceinline__ void eventdyn(const DevTables& T, Rec& bi, Rec& bj, double2 bwi, bool bonded_ij, int evcode, double tf,
                          int& ct, int& status) {
     const int a = dyn_ident(bi.dyn), c = dyn_ident(bj.dyn);
     Geo g;
@@ -2315,36 +2534,41 @@ __device__ inline double dist_rec(const Rec& a, const Rec& b, double tf) {
     geo(a, b, tf, g);
     return sqrt(g.rx * g.rx + g.ry * g.ry + g.rz * g.rz);
 }
-// repuls_check.f:16-81 (n = the N bead, cb = the C bead)
-__device__ double repuls_check(const SysDev&, const DevTables& T, const Pair& P, int n, int cb, double tf) {
-    const SysDev& S = sdev();
-
-    const Rec rn = load_rec(S, P, n), rc = load_rec(S, P, cb);
+// a bead's record as the event sees it: the colliding pair's own from the
+// wavefront's Pair in LDS, any other from memory
+__device__ inline Rec pair_rec(int m) {
+    const Pair& P = *ldsv().pair();
+    return load_rec(sdev(), P, m);
+}
+// repuls_check.f:16-81 (n = the N bead, cb = the C bead), the colliding pair
+// read from LDS; these run in few events and stay out of line, so that the
+// event's own registers and code stay small
+__device__ __noinline__ bool shoulders_far(int n, int cb, double tf) {
+    const DevTables& T = tabs();
+    const Rec rn = pair_rec(n), rc = pair_rec(cb);
     int ncim1, ncai, ncaj, nnjp1;
     shoulder_idx(n, topo_len(rn.topo), cb, topo_len(rc.topo), ncim1, ncai, ncaj, nnjp1);
-    const double d1 = dist_rec(rn, load_rec(S, P, ncaj), tf), d2 = dist_rec(rn, load_rec(S, P, nnjp1), tf);
-    const double d3 = dist_rec(rc, load_rec(S, P, ncai), tf), d4 = dist_rec(rc, load_rec(S, P, ncim1), tf);
-    if (d1 > T.shder[1] && d2 > T.shder[2] && d3 > T.shder[3] && d4 > T.shder[4]) return 10.0;
-    return 11.0;
+    const double d1 = dist_rec(rn, pair_rec(ncaj), tf), d2 = dist_rec(rn, pair_rec(nnjp1), tf);
+    const double d3 = dist_rec(rc, pair_rec(ncai), tf), d4 = dist_rec(rc, pair_rec(ncim1), tf);
+    return d1 > T.shder[1] && d2 > T.shder[2] && d3 > T.shder[3] && d4 > T.shder[4];
 }
-// repuls_check_3.f:16-102
-__device__ double repuls_check_3(const SysDev&, const DevTables& T, const Pair& P, int n, int cb, int k,
-                                 double tf) {
-    const SysDev& S = sdev();
-
-    const Rec rn = load_rec(S, P, n), rc = load_rec(S, P, cb);
+// repuls_check_3.f:16-102: the three shoulders other than k
+__device__ __noinline__ bool shoulders_far_3(int n, int cb, int k, double tf) {
+    const DevTables& T = tabs();
+    const Rec rn = pair_rec(n), rc = pair_rec(cb);
     int ncim1, ncai, ncaj, nnjp1;
     shoulder_idx(n, topo_len(rn.topo), cb, topo_len(rc.topo), ncim1, ncai, ncaj, nnjp1);
     int m = 0;
-    if (ncaj != k && dist_rec(rn, load_rec(S, P, ncaj), tf) > T.shder[1]) ++m;
-    if (nnjp1 != k && dist_rec(rn, load_rec(S, P, nnjp1), tf) > T.shder[2]) ++m;
-    if (ncai != k && dist_rec(rc, load_rec(S, P, ncai), tf) > T.shder[3]) ++m;
-    if (ncim1 != k && dist_rec(rc, load_rec(S, P, ncim1), tf) > T.shder[4]) ++m;
-    return m == 3 ? 10.0 : 11.0;
+    if (ncaj != k && dist_rec(rn, pair_rec(ncaj), tf) > T.shder[1]) ++m;
+    if (nnjp1 != k && dist_rec(rn, pair_rec(nnjp1), tf) > T.shder[2]) ++m;
+    if (ncai != k && dist_rec(rc, pair_rec(ncai), tf) > T.shder[3]) ++m;
+    if (ncim1 != k && dist_rec(rc, pair_rec(ncim1), tf) > T.shder[4]) ++m;
+    return m == 3;
 }
 // repuls_add.f:14-47 / repuls_del_a.f:14-37 (single lane; n = N bead, cb = C bead)
-__device__ void repuls_add(const SysDev&, int n, int Ln, int cb, int Lc, int& status) {
+__device__ __noinline__ int repuls_add(int n, int Ln, int cb, int Lc) {
     const SysDev& S = sdev();
+    int status = 0;
 
     int ncim1, ncai, ncaj, nnjp1;
     shoulder_idx(n, Ln, cb, Lc, ncim1, ncai, ncaj, nnjp1);
@@ -2369,9 +2593,11 @@ __device__ void repuls_add(const SysDev&, int n, int Ln, int cb, int Lc, int& st
     gs1(&S.extra[nnjp1].z, n);
     gs1(&S.extra[ncai].z, cb);
     gs1(&S.extra[ncim1].z, cb);
+    return status;
 }
-__device__ void repuls_del_a(const SysDev&, int n, int Ln, int cb, int Lc, int& status) {
+__device__ __noinline__ int repuls_del_a(int n, int Ln, int cb, int Lc) {
     const SysDev& S = sdev();
+    int status = 0;
 
     int ncim1, ncai, ncaj, nnjp1;
     shoulder_idx(n, Ln, cb, Lc, ncim1, ncai, ncaj, nnjp1);
@@ -2383,274 +2609,887 @@ __device__ void repuls_del_a(const SysDev&, int n, int Ln, int cb, int Lc, int& 
     set_code(S, cb, ncai, 1, status);
     set_code(S, ncim1, cb, 1, status);
     set_code(S, cb, ncim1, 1, status);
+    return status;
 }
 __device__ inline bool terminal_t(int t) {
     const int k = topo_kind(t), r = topo_res(t), L = topo_len(t);
     return (k == 1 && r == 1) || (k == 2 && r == L);
 }
 
-// One pair event: outcome resolution (main.F90:1487-1634), dynamics, H-bond
-// and shoulder bookkeeping (main.F90:641-921), then partial_events.
-__device__ int pair_event(const SysDev&, const DevTables&, const Lds&, Sc&, int i, int j, int ct, int bk) {
-    const Lds L = lds_regs();
+// The wavefront's work area while an event is rescheduled in one pass.
+struct __attribute__((aligned(16))) BaseRec {
+    Rec r;
+    double2 bw;
+    int idx, pad[3];
+};
+constexpr int kOwners = 2 + kMaxSpec;
+struct OnePass {
+    BaseRec base[kOwners];  // 0: bead i, 1: bead j, then the beads recomputed in full
+    double wt[kW];
+    unsigned long long tkey[kOwners];
+    int wy[kW];
+    int lst[kW];
+};
+static_assert(sizeof(OnePass) <= 4 * 768, "the one-pass work area exceeds a wavefront's work list");
+// result lanes of beads i and j: entries take the lanes below
+constexpr int kLaneI = kW - 2, kLaneJ = kW - 1;
 
-    const SysDev& S = sdev();
-
-    const DevTables& T = tabs();
-    Sc& c = *L.sc();
-
-    const int lane = lane_id();
-    const double tf = c.tfalse;
-    PH_BEGIN(tpe);
-    Pair P;
-    P.i = i;
-    P.j = j;
-    P.flags = 0;
-    P.pad = 0;
-    P.ri = gld(S.rec + (i));
-    P.rj = gld(S.rec + (j));
-    P.bwi = gld(S.bw + (i));
-    P.bwj = gld(S.bw + (j));
-    P.xi = gld(S.extra + (i));
-    P.xj = gld(S.extra + (j));
-    const int4 oi = gld(S.ovr + (i));
-    const Rows rows = load_rows(S, i, j);  // in flight while the outcome is resolved
-    const int evcode = dyn_code(oi, j, static_t(P.ri.topo, P.rj.topo));  // ev_code(i, j)
-    const bool ok = !terminal_t(P.ri.topo) && !terminal_t(P.rj.topo);
-    const int idi = dyn_ident(P.ri.dyn), idj = dyn_ident(P.rj.dyn);
-    int status = 0;
-    bool xpulse = false, fence = false;
-    if (ct == 7 || ct == 10 || ct == 12) P.flags |= kPairReadsSp;
-    if (ct == 7) {
-        if (P.xi.w < 0 && P.xj.w < 0) {
-            if (ok) {
-                const double rating = idi < idj ? repuls_check(S, T, P, i, j, tf) : repuls_check(S, T, P, j, i, tf);
-                ct = rating <= 10.0 ? 4 : 14;
-            } else {
-                // a random draw: its counter value is known only in order
-                int nb = 0;
-                if (bk >= 1) return spec_abort(L, bk, nb);
-                const double ran_non = rng_u01(S.seed, 1, c.rc1++);
-                ct = ran_non <= 0.2 ? 4 : 9;
-            }
-        } else
-            ct = 9;
-    } else if (ct == 10) {
-        double rating;
-        if (evcode < 45) {
-            const int hbp = P.xi.w;
-            const int idh = dyn_ident(load_rec(S, P, hbp).dyn);
-            rating = idi < idh ? repuls_check_3(S, T, P, i, hbp, j, tf) : repuls_check_3(S, T, P, hbp, i, j, tf);
-        } else {
-            const int hbp = P.xj.w;
-            const int idh = dyn_ident(load_rec(S, P, hbp).dyn);
-            rating = idj < idh ? repuls_check_3(S, T, P, j, hbp, i, tf) : repuls_check_3(S, T, P, hbp, j, i, tf);
-        }
-        ct = rating <= 10.0 ? 5 : 15;
-    } else if (ct == 12) {
-        const bool xi_ = evcode < 45;
-        const Rec rx = xi_ ? P.ri : P.rj;
-        const int hbp = xi_ ? P.xi.w : P.xj.w;
-        if (dyn_bptnr(rx.dyn) == hbp) {
-            Geo g;
-            const Rec rh = load_rec(S, P, hbp);
-            geo(rx, rh, tf, g);
-            const double d2 = g.rx * g.rx + g.ry * g.ry + g.rz * g.rz;
-            const double rating = (d2 - T.sigma_sq[dyn_ident(rx.dyn)][dyn_ident(rh.dyn)]) < 0.0 ? 10.0 : 11.0;
-            ct = rating > 10.0 ? 6 : 13;
-        } else
-            ct = 15;
-    }
-    if (ct < 14) eventdyn(T, P.ri, P.rj, P.bwi, dyn_bptnr(P.ri.dyn) == j, evcode, tf, ct, status);
-    const int Li = topo_len(P.ri.topo), Lj = topo_len(P.rj.topo);
-    if (ct == 20) {
-        if (idi + idj == 5) {
-            P.ri.dyn = make_dyn(idi + 4, j);
-            P.rj.dyn = make_dyn(idj + 4, i);
-            if (ok) {
-                int nb = 0;
-                if (bk >= 1) return spec_abort(L, bk, nb);
-                if (lane == 0) {
-                    if (idi < idj) repuls_add(S, i, Li, j, Lj, status);
-                    else repuls_add(S, j, Lj, i, Li, status);
-                }
-                fence = true;
-            }
-        }
-    } else if (ct == 21) {
-        if (idi <= 8) {
-            if (ok) {
-                int nb = 0;
-                if (bk >= 1) return spec_abort(L, bk, nb);
-                if (lane == 0) {
-                    if (idi < idj) repuls_del_a(S, i, Li, j, Lj, status);
-                    else repuls_del_a(S, j, Lj, i, Li, status);
-                }
-                xpulse = true;
-                fence = true;
-            }
-            if (dyn_bptnr(P.ri.dyn) == j) {
-                P.ri.dyn = make_dyn(idi - 4, -1);
-                P.rj.dyn = make_dyn(idj - 4, -1);
-            }
-        }
-    } else if (ct == 24 || ct == 25) {
-        P.flags |= kPairReadsSp;
-        const bool xi_ = evcode < 45;
-        const int hbp = xi_ ? P.xi.w : P.xj.w;
-        const int x = xi_ ? i : j;
-        int xdyn = xi_ ? P.ri.dyn : P.rj.dyn;
-        int hdyn = load_rec(S, P, hbp).dyn;
-        const int idx = dyn_ident(xdyn), idh = dyn_ident(hdyn);
-        bool changed = false;
-        if (ct == 24 && idx + idh == 5) {
-            xdyn = make_dyn(idx + 4, hbp);
-            hdyn = make_dyn(idh + 4, x);
-            changed = true;
-        } else if (ct == 25 && idx >= 5) {
-            xdyn = make_dyn(idx - 4, -1);
-            hdyn = make_dyn(idh - 4, -1);
-            changed = true;
-        }
-        if (changed) {
-            if (xi_) P.ri.dyn = xdyn;
-            else P.rj.dyn = xdyn;
-            if (hbp == i) P.ri.dyn = hdyn;
-            else if (hbp == j) P.rj.dyn = hdyn;
-            else {
-                int nb = 0;
-                if (bk >= 1) return spec_abort(L, bk, nb);
-                if (lane == 0) gs1(&S.rec[hbp].dyn, hdyn);
-                fence = true;
-            }
-        }
-    } else if (ct == 14 || ct == 15 || ct == 16) {
-        // bumped.f: push the pair off the discontinuity
-        Geo g;
-        geo(P.ri, P.rj, tf, g);
-        const double bd = evcode >= 40 ? kSm * sqrt(T.shlddia_sq[idi][idj]) : kSm * sqrt(T.welldia_sq[idi][idj]);
-        nudge(P.ri, P.rj, bd, g, g.b < 0.0 ? -1 : +1);
-        if ((ct == 14 || ct == 16) && ok && bk >= 1) {
-            int nb = 0;
-            return spec_abort(L, bk, nb);
-        }
-        if (ct == 14 && ok) {
-            if (lane == 0) {
-                if (idi < idj) repuls_add(S, i, Li, j, Lj, status);
-                else repuls_add(S, j, Lj, i, Li, status);
-            }
-            fence = true;
-        } else if (ct == 16 && ok) {
-            if (lane == 0) {
-                if (idi < idj) repuls_del_a(S, i, Li, j, Lj, status);
-                else repuls_del_a(S, j, Lj, i, Li, status);
-            }
-            xpulse = true;
-            fence = true;
-        }
-    }
-    if (lane == 0 && bk < 1) {  // a speculative event writes its pair once committed
-        gst(S.rec + (i), P.ri);
-        gst(S.rec + (j), P.rj);
-    }
-    if (lane == 0 && bk >= 0) L.batch()->ty[bk] = ct;
-    if (fence) P.flags |= kPairWroteSp;
-    if (fence) {
-        // shoulder tables changed: make them visible before the predictions
-        wave_sync_mem();
-        P.xi = gld(S.extra + (i));
-        P.xj = gld(S.extra + (j));
-    }
-    status = wave_status(status);
-    if (status && !c.status) c.status = status;
-    if (lane == 0) *L.pair() = P;
-    wave_sync();
-    PH_END(S, kPhPair, tpe);
-    reschedule(S, T, L, c, *L.pair(), -1, xpulse, bk, rows);
-    return ct;
+__device__ inline Rec uni_words(Rec r) {
+    r.topo = uni(r.topo);
+    r.dyn = uni(r.dyn);
+    return r;
+}
+__device__ inline unsigned* lds_words(int off) { return (unsigned*)__builtin_assume_aligned(smem + off, 16); }
+// footprint marks, in LDS (ds operations) or in HBM at the device's L2
+__device__ inline void fp_or(const Hot& H, int b, unsigned bits) {
+    if (H.mark_lds)
+        __hip_atomic_fetch_or(lds_words(H.o_mark) + b, bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    else
+        __hip_atomic_fetch_or((GLB unsigned*)((GLB char*)H.mark + (unsigned)b * 4u), bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline unsigned fp_get(const Hot& H, int b) {
+    if (H.mark_lds)
+        return __hip_atomic_load(lds_words(H.o_mark) + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    return __hip_atomic_load((GLB unsigned*)((GLB char*)H.mark + (unsigned)b * 4u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline void fp_clear(const Hot& H, int b) {
+    if (H.mark_lds)
+        __hip_atomic_store(lds_words(H.o_mark) + b, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    else
+        __hip_atomic_store((GLB unsigned*)((GLB char*)H.mark + (unsigned)b * 4u), 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Andersen ghost collision, main.F90:997-1049
-__device__ int ghost_event(const SysDev&, const DevTables&, const Lds&, Sc&, int bk) {
-    const Lds& L = ldsv();
-
-    const SysDev& S = sdev();
-
-    const DevTables& T = tabs();
-    Sc& c = *L.sc();
-
+// One event of a round on one wavefront: a bead-pair event (outcome
+// resolution main.F90:1487-1634, dynamics, H-bond and shoulder bookkeeping
+// main.F90:641-921) or an Andersen ghost collision (main.F90:997-1049),
+// then partial_events.f:16-201 for it.
+// e: the calendar entry; jp, ct: its partner and type; tf, nbin, coll: the
+// false time, bin and number of the event; bk: its place in the round (-1:
+// the round's only entry).  Returns the round's accepted events if this one
+// is committed (1 alone), else 0.
+//
+// The rescheduling takes one pass of 64 lanes: a lane per candidate of i
+// and j (tags 0 and 1), per down-set entry (tags 2 and 3: its op partner i
+// or j), and per candidate of a down bead that may be recomputed in full
+// (tag 4 + s).  Each lane gathers its own entry's bead and predicts it
+// against its base bead (i, j or the recomputed bead, staged in LDS), so
+// every prediction costs one gather and the event three dependent rounds of
+// loads: the pair and its rows; the entries' beads and the rows of the
+// beads recomputed; those rows' beads.  An event of more than 62 entries (two lanes
+// take the results of i and j) or of more than kMaxSpec full recomputes
+// runs the multi-pass form, which holds any number.  What bounds an event
+// is the length of its dependent chain, so the code keeps wave-uniform
+// values in scalar registers and replaces divergent branches by selects.
+__device__ __forceinline__ int run_event(const Hot& H, int e, int jp, int ct, double tf, int nbin, long long coll, int bk) {
     const int lane = lane_id();
-    const int N = S.N;
-    PH_BEGIN(tg0);
-    int i = 0, guard = 0;
-    do {
-        i = (int)(rng_u01(S.seed, 0, c.rc0++) * N);
-    } while (i == N && ++guard < 1000);
-    c.numghosts++;
-    Pair P;
-    P.i = i;
-    P.j = -1;
-    P.flags = 0;
-    P.pad = 0;
-    P.ri = gld(S.rec + (i));
-    P.bwi = gld(S.bw + (i));
-    P.xi = gld(S.extra + (i));
-    P.rj = P.ri;
-    P.bwj = P.bwi;
-    P.xj = make_int4(-1, -1, -1, -1);
-    Rec b = P.ri;
-    const double tf = c.tfalse, bm = b.bm;
-    b.x = b.x + b.vx * tf;
-    b.y = b.y + b.vy * tf;
-    b.z = b.z + b.vz * tf;
-    double v1, v2, r, fact;
-    do {
-        v1 = 2.0 * rng_u01(S.seed, 0, c.rc0++) - 1.0;
-        v2 = 2.0 * rng_u01(S.seed, 0, c.rc0++) - 1.0;
-        r = v1 * v1 + v2 * v2;
-    } while ((r == 0.0 || r >= 1.0) && ++guard < 1000);
-    fact = sqrt(-2.0 * S.setemp * bm * dlog(r) / r);
-    b.vx = v1 * fact / bm;
-    b.vy = v2 * fact / bm;
-    do {
-        v1 = 2.0 * rng_u01(S.seed, 0, c.rc0++) - 1.0;
-        v2 = 2.0 * rng_u01(S.seed, 0, c.rc0++) - 1.0;
-        r = v1 * v1 + v2 * v2;
-    } while ((r == 0.0 || r >= 1.0) && ++guard < 2000);
-    fact = sqrt(-2.0 * S.setemp * bm * dlog(r) / r);
-    b.vz = v1 * fact / bm;
-    b.x = b.x - b.vx * tf;
-    b.y = b.y - b.vy * tf;
-    b.z = b.z - b.vz * tf;
-    double tgho;
-    do {
-        tgho = rng_u01(S.seed, 0, c.rc0++);
-    } while ((tgho < 1.e-18 || tgho == 1.0) && ++guard < 3000);
-    if (guard >= 1000) c.status = kErrRng;
-    const double tg = -1.0 * dlog(tgho) * S.avegtime + tf;
-    int status = 0;
-    P.ri = b;
-    P.rj = b;
-    if (lane == 0) {
-        gst(S.rec + (i), b);
+    const DevTables& T = tabs();
+    Sc& mc = master();
+    Batch& B = round_rec();
+    const double interval_max = mc.interval_max, tbin_off = mc.tbin_off, sortsize = mc.sortsize;
+    const bool batch = bk >= 0;
+    int i = e, j = -1, flags = 0, st0 = 0, nb = 0, extra_blk = -1;
+    bool xdel = false;
+    Rec ri, rj;
+    double2 bwi, bwj = make_double2(0.0, 0.0);
+    int4 xi, xj = make_int4(-1, -1, -1, -1);
+    int eui, edi, euj = 0, edj = 0, nui, ndi, nuj = 0, ndj = 0;
+    const int cap = H.cap;
+    PH_BEGIN(tph);
+    if (e < H.N) {
+        j = jp;
+        ri = ld_at(H.rec, i);
+        rj = ld_at(H.rec, j);
+        const int4 oi_ = ld_at(H.ovr, i), xi_ = ld_at(H.extra, i), xj_ = ld_at(H.extra, j);
+        bwi = ld_at(H.bw, i);
+        bwj = ld_at(H.bw, j);
+        // the list rows, in flight while the outcome is resolved
+        const int nui_ = ld_at(H.nup, i), ndi_ = ld_at(H.ndn, i), nuj_ = ld_at(H.nup, j), ndj_ = ld_at(H.ndn, j);
+        const int sl = min(lane, cap - 1);
+        eui = ld_at(H.nb_up, i * cap + sl);
+        edi = ld_at(H.nb_dn, i * cap + sl);
+        euj = ld_at(H.nb_up, j * cap + sl);
+        edj = ld_at(H.nb_dn, j * cap + sl);
+        ri = uni_words(ri);
+        rj = uni_words(rj);
+        xi = uni(xi_);
+        xj = uni(xj_);
+        const int evcode = dyn_code(uni(oi_), j, static_t(ri.topo, rj.topo));  // ev_code(i, j)
+        const bool ok = !terminal_t(ri.topo) && !terminal_t(rj.topo);
+        const int idi = dyn_ident(ri.dyn), idj = dyn_ident(rj.dyn);
+        const int Li = topo_len(ri.topo), Lj = topo_len(rj.topo);
+        bool fence = false;
+        auto rec_of = [&](int m) { return m == i ? ri : (m == j ? rj : uni_words(ld_at(H.rec, m))); };
+        auto stage_pair = [&]() {
+            if (lane == 0) {
+                Pair& P = *ldsv().pair();
+                P.i = i;
+                P.j = j;
+                P.ri = ri;
+                P.rj = rj;
+            }
+            wave_sync();
+        };
+        if (ct == 7 || ct == 10 || ct == 12) flags |= kPairReadsSp;
+        if (ct == 7) {
+            if (xi.w < 0 && xj.w < 0) {
+                if (ok) {
+                    stage_pair();
+                    ct = (idi < idj ? shoulders_far(i, j, tf) : shoulders_far(j, i, tf)) ? 4 : 14;
+                } else {
+                    // a random draw: its counter value is known only in order
+                    if (bk >= 1) {
+                        spec_abort_at(bk, nb);
+                        return 0;
+                    }
+                    ct = rng_u01(sdev().seed, 1, mc.rc1++) <= 0.2 ? 4 : 9;
+                    ct = uni(ct);
+                }
+            } else
+                ct = 9;
+        } else if (ct == 10) {
+            const bool own = evcode < 45;
+            const int hbp = own ? xi.w : xj.w, idh = dyn_ident(rec_of(hbp).dyn);
+            stage_pair();
+            bool far;
+            if (own)
+                far = idi < idh ? shoulders_far_3(i, hbp, j, tf) : shoulders_far_3(hbp, i, j, tf);
+            else
+                far = idj < idh ? shoulders_far_3(j, hbp, i, tf) : shoulders_far_3(hbp, j, i, tf);
+            ct = far ? 5 : 15;
+        } else if (ct == 12) {
+            const bool own = evcode < 45;
+            const Rec rx = own ? ri : rj;
+            const int hbp = own ? xi.w : xj.w;
+            if (dyn_bptnr(rx.dyn) == hbp) {
+                Geo g;
+                const Rec rh = rec_of(hbp);
+                geo(rx, rh, tf, g);
+                const double d2 = g.rx * g.rx + g.ry * g.ry + g.rz * g.rz;
+                ct = (d2 - T.sigma_sq[dyn_ident(rx.dyn)][dyn_ident(rh.dyn)]) < 0.0 ? 13 : 6;
+            } else
+                ct = 15;
+        }
+        ct = uni(ct);
+        int status = 0;
+        if (ct < 14) {
+            eventdyn(T, ri, rj, bwi, dyn_bptnr(ri.dyn) == j, evcode, tf, ct, status);
+            ct = uni(ct);
+        }
+        if (ct == 20) {
+            if (idi + idj == 5) {
+                ri.dyn = make_dyn(idi + 4, j);
+                rj.dyn = make_dyn(idj + 4, i);
+                if (ok) {
+                    if (bk >= 1) {
+                        spec_abort_at(bk, nb);
+                        return 0;
+                    }
+                    if (lane == 0) status |= idi < idj ? repuls_add(i, Li, j, Lj) : repuls_add(j, Lj, i, Li);
+                    fence = true;
+                }
+            }
+        } else if (ct == 21) {
+            if (idi <= 8) {
+                if (ok) {
+                    if (bk >= 1) {
+                        spec_abort_at(bk, nb);
+                        return 0;
+                    }
+                    if (lane == 0) status |= idi < idj ? repuls_del_a(i, Li, j, Lj) : repuls_del_a(j, Lj, i, Li);
+                    xdel = true;
+                    fence = true;
+                }
+                if (dyn_bptnr(ri.dyn) == j) {
+                    ri.dyn = make_dyn(idi - 4, -1);
+                    rj.dyn = make_dyn(idj - 4, -1);
+                }
+            }
+        } else if (ct == 24 || ct == 25) {
+            flags |= kPairReadsSp;
+            const bool own = evcode < 45;
+            const int hbp = own ? xi.w : xj.w, x = own ? i : j;
+            int xdyn = own ? ri.dyn : rj.dyn, hdyn = rec_of(hbp).dyn;
+            const int idx = dyn_ident(xdyn), idh = dyn_ident(hdyn);
+            bool changed = false;
+            if (ct == 24 && idx + idh == 5) {
+                xdyn = make_dyn(idx + 4, hbp);
+                hdyn = make_dyn(idh + 4, x);
+                changed = true;
+            } else if (ct == 25 && idx >= 5) {
+                xdyn = make_dyn(idx - 4, -1);
+                hdyn = make_dyn(idh - 4, -1);
+                changed = true;
+            }
+            if (changed) {
+                if (own) ri.dyn = xdyn;
+                else rj.dyn = xdyn;
+                if (hbp == i) ri.dyn = hdyn;
+                else if (hbp == j) rj.dyn = hdyn;
+                else {
+                    if (bk >= 1) {
+                        spec_abort_at(bk, nb);
+                        return 0;
+                    }
+                    if (lane == 0) gs1(&H.rec[hbp].dyn, hdyn);
+                    fence = true;
+                }
+            }
+        } else if (ct == 14 || ct == 15 || ct == 16) {
+            // bumped.f: push the pair off the discontinuity
+            Geo g;
+            geo(ri, rj, tf, g);
+            const double bd = evcode >= 40 ? kSm * sqrt(T.shlddia_sq[idi][idj]) : kSm * sqrt(T.welldia_sq[idi][idj]);
+            nudge(ri, rj, bd, g, g.b < 0.0 ? -1 : +1);
+            if ((ct == 14 || ct == 16) && ok) {
+                if (bk >= 1) {
+                    spec_abort_at(bk, nb);
+                    return 0;
+                }
+                if (lane == 0) {
+                    if (ct == 14)
+                        status |= idi < idj ? repuls_add(i, Li, j, Lj) : repuls_add(j, Lj, i, Li);
+                    else
+                        status |= idi < idj ? repuls_del_a(i, Li, j, Lj) : repuls_del_a(j, Lj, i, Li);
+                }
+                xdel = ct == 16;
+                fence = true;
+            }
+        }
+        if (bk < 1) {  // a speculative event writes its pair once committed
+            if (lane == 0) st_at(H.rec, i, ri);
+            if (lane == 1) st_at(H.rec, j, rj);
+        }
+        if (fence) {
+            flags |= kPairWroteSp;
+            // shoulder tables changed: make them visible before the predictions
+            wave_sync_mem();
+            xi = uni(ld_at(H.extra, i));
+            xj = uni(ld_at(H.extra, j));
+        }
+        st0 = wave_status(status);
+        nui = uni(nui_);
+        ndi = uni(ndi_);
+        nuj = uni(nuj_);
+        ndj = uni(ndj_);
+        PH_END(sdev(), kPhPair, tph);
+    } else {
+        const SysDev& S = sdev();
+        const unsigned long long seed = S.seed;
+        const int N = H.N;
+        unsigned long long rc = mc.rc0;
+        int guard = 0;
+        do {
+            i = (int)(rng_u01(seed, 0, rc++) * N);
+        } while (i == N && ++guard < 1000);
+        i = uni(i);
+        ri = ld_at(H.rec, i);
+        bwi = ld_at(H.bw, i);
+        const int4 xi_ = ld_at(H.extra, i);
+        const int nui_ = ld_at(H.nup, i), ndi_ = ld_at(H.ndn, i), sl = min(lane, cap - 1);
+        eui = ld_at(H.nb_up, i * cap + sl);
+        edi = ld_at(H.nb_dn, i * cap + sl);
+        ri = uni_words(ri);
+        const double bm = ri.bm;
+        ri.x = ri.x + ri.vx * tf;
+        ri.y = ri.y + ri.vy * tf;
+        ri.z = ri.z + ri.vz * tf;
+        double v1, v2, r, fact;
+        do {
+            v1 = 2.0 * rng_u01(seed, 0, rc++) - 1.0;
+            v2 = 2.0 * rng_u01(seed, 0, rc++) - 1.0;
+            r = v1 * v1 + v2 * v2;
+        } while ((r == 0.0 || r >= 1.0) && ++guard < 1000);
+        fact = sqrt(-2.0 * S.setemp * bm * dlog(r) / r);
+        ri.vx = v1 * fact / bm;
+        ri.vy = v2 * fact / bm;
+        do {
+            v1 = 2.0 * rng_u01(seed, 0, rc++) - 1.0;
+            v2 = 2.0 * rng_u01(seed, 0, rc++) - 1.0;
+            r = v1 * v1 + v2 * v2;
+        } while ((r == 0.0 || r >= 1.0) && ++guard < 2000);
+        fact = sqrt(-2.0 * S.setemp * bm * dlog(r) / r);
+        ri.vz = v1 * fact / bm;
+        ri.x = ri.x - ri.vx * tf;
+        ri.y = ri.y - ri.vy * tf;
+        ri.z = ri.z - ri.vz * tf;
+        double tgho;
+        do {
+            tgho = rng_u01(seed, 0, rc++);
+        } while ((tgho < 1.e-18 || tgho == 1.0) && ++guard < 3000);
+        if (guard >= 1000) st0 = kErrRng;
+        const double tg = -1.0 * dlog(tgho) * S.avegtime + tf;
+        int status = 0;
         Leaf g;
         g.tim = tg;
         g.nptnr = -2;
-        g.meta = make_meta(calc_bin(c, tg, false, status), -2);
-        leaf_set(L, N, g);
-        stamp_set(N, mk_stamp(c.coll, 1));  // added before partial_events' adds (main.F90:1041-1049)
+        g.meta = make_meta(bin_of(interval_max, tbin_off, sortsize, nbin, tg, status), -2);
+        if (lane == 0) {
+            st_at(H.rec, i, ri);
+            leaf_st(H, N, g);
+            stamp_st(H, N, mk_stamp(coll, 1));  // added before partial_events' adds (main.F90:1041-1049)
+            mc.rc0 = rc;
+            mc.numghosts++;
+            B.gbead = i;
+        }
+        if (status && !st0) st0 = status;
+        if (tf < mc.old_tfalse) {
+            tf = mc.old_tfalse;
+            if (lane == 0) mc.tfalse = tf;
+        }
+        rj = ri;
+        xi = uni(xi_);
+        nui = uni(nui_);
+        ndi = uni(ndi_);
+        extra_blk = N / kBlk;
+        ct = 0;
+        wave_sync();
+        PH_END(sdev(), kPhGhost, tph);
     }
-    if (status && !c.status) c.status = status;
-    if (c.tfalse < c.old_tfalse) c.tfalse = c.old_tfalse;
-    if (lane == 0) *L.pair() = P;
-    if (lane == 0 && bk >= 0) {
-        L.batch()->ty[bk] = 0;
-        L.batch()->gbead = i;
+    if (lane == 0 && batch) B.ty[bk] = ct;
+    if (lane == 0 && !batch) B.ty[0] = ct;
+
+    OnePass& W = *reinterpret_cast<OnePass*>(smem + H.o_w);
+    const unsigned long long below = (1ull << lane) - 1ull;
+    // place of i's add among this event's calendar adds (a ghost event adds
+    // its own entry first); j follows, then the down set in list order
+    const int sub0 = j >= 0 ? 1 : 2;
+    const double T0 = interval_max + kLt - tf;
+    const int kNoStat = 0xFF << 24;
+    const bool has_x = (xi.x & xi.y & xi.z & xj.x & xj.y & xj.z) != -1;  // any shoulder partner
+    bool multi = nui + ndi + nuj + ndj + (has_x ? 12 : 0) > kLaneI;
+    int ncand = 0, nDi = 0, n0 = 0, ntot = 0, m = 0, tag = 0, stat = 0, nspec = 0, myslot = -1;
+    int cI = 0, cJ = 0, pI = lane, pJ = lane;
+    bool first = false, is_i = false, spec = false, dn = false, act = false;
+    unsigned long long dups = 0;
+    Rec mine;
+    int4 om = make_int4(-1, -1, -1, -1);
+    double2 bwm = make_double2(0.0, 0.0);
+    Leaf lf0;
+    lf0.tim = 0.0;
+    lf0.nptnr = -1;
+    lf0.meta = 0;
+    unsigned long long specm = 0;
+    if (!multi) {
+        // ---- the entry list: candidates of i, candidates of j, the down set
+        //      in reference order (i's down list and lower shoulder partners, then j's)
+        int w = nui;
+        if (lane < nui) W.lst[lane] = eui;
+        auto one = [&](int b, int tg) {
+            if (lane == 0) W.lst[w] = b | (tg << 16) | kNoStat;
+            ++w;
+        };
+        if (has_x) {
+            if (xi.x > i) one(xi.x, 0);
+            if (xi.y > i) one(xi.y, 0);
+            if (xi.z > i) one(xi.z, 0);
+        }
+        if (lane < nuj) W.lst[w + lane] = euj | (1 << 16);
+        w += nuj;
+        if (has_x && j >= 0) {
+            if (xj.x > j) one(xj.x, 1);
+            if (xj.y > j) one(xj.y, 1);
+            if (xj.z > j) one(xj.z, 1);
+        }
+        ncand = w;
+        if (lane < ndi) W.lst[w + lane] = edi | (2 << 16);
+        w += ndi;
+        if (has_x) {
+            if (xi.x >= 0 && xi.x < i) one(xi.x, 2);
+            if (xi.y >= 0 && xi.y < i) one(xi.y, 2);
+            if (xi.z >= 0 && xi.z < i) one(xi.z, 2);
+        }
+        nDi = w - ncand;
+        if (j >= 0) {
+            const bool keep = lane < ndj && (edj & 0xFFFF) != i;
+            const unsigned long long bal = __ballot(keep);
+            if (keep) W.lst[w + __popcll(bal & below)] = edj | (3 << 16);
+            w += __popcll(bal);
+            if (has_x) {
+                if (xj.x >= 0 && xj.x < j) one(xj.x, 3);
+                if (xj.y >= 0 && xj.y < j) one(xj.y, 3);
+                if (xj.z >= 0 && xj.z < j) one(xj.z, 3);
+            }
+        }
+        n0 = w;
+        if (lane < 2) {
+            BaseRec& b = W.base[lane];
+            b.r = lane == 0 ? ri : rj;
+            b.bw = lane == 0 ? bwi : bwj;
+            b.idx = lane == 0 ? i : j;
+        }
+        if (lane < kOwners) W.tkey[lane] = ~0ull;
+        wave_sync();
+        PH_END(sdev(), kPhRows, tph);
+        // ---- every entry's bead; a down entry's own calendar entry, bond
+        //      window, shoulder partners and row length
+        act = lane < n0;
+        const int ent = act ? W.lst[lane] : 0;
+        m = ent & 0xFFFF;
+        tag = (ent >> 16) & 0xFF;
+        stat = (ent >> 24) & 0xFF;
+        dn = act && lane >= ncand;
+        int nul = 0;
+        int4 xl = make_int4(-1, -1, -1, -1);
+        if (act) {
+            mine = ld_at(H.rec, m);
+            om = ld_at(H.ovr, m);
+        }
+        if (dn) {
+            lf0 = leaf_ld(H, m);
+            nul = ld_at(H.nup, m);
+            xl = ld_at(H.extra, m);
+            bwm = ld_at(H.bw, m);
+        }
+        // ---- down entries of one bead: its ops with i and with j, and the
+        //      lane of an op of each kind (equal predictions)
+        {
+            const int key = dn ? m : -1 - lane;
+            int r = ncand;
+            const int rj0 = ncand + nDi;
+            unsigned long long above = ~((2ull << r) - 1ull);
+            for (; r < rj0; ++r, above <<= 1) {
+                const bool eq = key == __builtin_amdgcn_readlane(key, r);
+                cI += eq ? 1 : 0;
+                pI = eq ? r : pI;
+                dups |= __ballot(eq) & above;
+            }
+            for (; r < n0; ++r, above <<= 1) {
+                const bool eq = key == __builtin_amdgcn_readlane(key, r);
+                cJ += eq ? 1 : 0;
+                pJ = eq ? r : pJ;
+                dups |= __ballot(eq) & above;
+            }
+        }
+        first = dn && !((dups >> lane) & 1ull);
+        is_i = first && m == i;
+        // a bead whose updates may take a full recompute
+        spec = first && !is_i && ((lf0.nptnr == i && cI > 0) || (lf0.nptnr == j && cJ > 0) || cI >= 2 || cJ >= 2);
+        specm = __ballot(spec);
+        nspec = __popcll(specm);
+        multi = nspec > kMaxSpec;
+        if (!multi) {
+            myslot = __popcll(specm & below);
+            // rows of the beads recomputed, all in flight together
+            int sent[kMaxSpec];
+            const int sl = min(lane, cap - 1);
+            {
+                unsigned long long sm = specm;
+#pragma unroll
+                for (int q = 0; q < kMaxSpec; ++q) {
+                    if (q < nspec) {
+                        const int l = __builtin_amdgcn_readlane(m, __ffsll((long long)sm) - 1);
+                        sm &= sm - 1;
+                        sent[q] = ld_at(H.nb_up, l * cap + sl);
+                    }
+                }
+            }
+            PH_END(sdev(), kPhScan, tph);
+            // the pair's own beads take their new states
+            if (act && (m == i || m == j)) mine = W.base[m == i ? 0 : 1].r;
+            if (spec) {
+                BaseRec& b = W.base[2 + myslot];
+                b.r = mine;
+                b.bw = bwm;
+                b.idx = m;
+            }
+            const unsigned long long xm = __ballot(spec && (xl.x > m || xl.y > m || xl.z > m));
+            unsigned long long sm = specm;
+            int w2 = n0;
+#pragma unroll
+            for (int q = 0; q < kMaxSpec; ++q) {
+                if (q < nspec) {
+                    const int src = __ffsll((long long)sm) - 1;
+                    sm &= sm - 1;
+                    const int nu = __builtin_amdgcn_readlane(nul, src);
+                    const bool sx = (xm >> src) & 1ull;
+                    if (w2 + nu + (sx ? 3 : 0) > kLaneI) {
+                        multi = true;
+                    } else {
+                        if (lane < nu) W.lst[w2 + lane] = sent[q] | ((4 + q) << 16);
+                        w2 += nu;
+                        if (sx) {
+                            const int l = __builtin_amdgcn_readlane(m, src);
+                            const int x0 = __builtin_amdgcn_readlane(xl.x, src), x1 = __builtin_amdgcn_readlane(xl.y, src),
+                                      x2 = __builtin_amdgcn_readlane(xl.z, src);
+                            const int tg = ((4 + q) << 16) | kNoStat;
+                            if (x0 > l) { if (lane == 0) W.lst[w2] = x0 | tg; ++w2; }
+                            if (x1 > l) { if (lane == 0) W.lst[w2] = x1 | tg; ++w2; }
+                            if (x2 > l) { if (lane == 0) W.lst[w2] = x2 | tg; ++w2; }
+                        }
+                    }
+                }
+            }
+            ntot = w2;
+        }
+    }
+    if (multi) {
+        // the pair and this event's scalars to LDS for the multi-pass form
+        const Lds& L = ldsv();
+        if (lane == 0) {
+            Pair& P = *L.pair();
+            P.i = i;
+            P.j = j;
+            P.flags = flags;
+            P.pad = 0;
+            P.ri = ri;
+            P.rj = rj;
+            P.bwi = bwi;
+            P.bwj = j >= 0 ? bwj : bwi;
+            P.xi = xi;
+            P.xj = xj;
+        }
+        if (bk >= 1) {
+            if (lane < (int)(sizeof(Sc) / 8))
+                reinterpret_cast<long long*>(L.sc())[lane] = reinterpret_cast<const long long*>(&mc)[lane];
+            wave_sync();
+            if (lane == 0) {
+                Sc& c = *L.sc();
+                c.tfalse = tf;
+                c.nbin = nbin;
+                c.coll = coll;
+                c.status = st0;
+            }
+        } else if (lane == 0 && st0 && !mc.status)
+            mc.status = st0;
+        wave_sync();
+        reschedule(sdev(), T, L, *L.sc(), *L.pair(), extra_blk, xdel, bk);
+        if (!batch) {
+            if (lane == 0) {
+                B.nbl[0] = 0;
+                B.st[0] = 0;
+                B.st_rep[0] = 0;
+            }
+            return 1;
+        }
+        if (lane == 0) B.st_rep[bk] = 0;
+        if (bk >= uni(B.cut)) return 0;
+        const int A = accepted(B);
+        return bk < A ? A : 0;
     }
     wave_sync();
-    PH_END(S, kPhGhost, tg0);
-    reschedule(S, T, L, c, *L.pair(), N / kBlk, false, bk, load_rows(S, i, -1));
-    return i;
+    const bool late = lane >= n0 && lane < ntot;
+    if (late) {
+        const int ent = W.lst[lane];
+        m = ent & 0xFFFF;
+        tag = (ent >> 16) & 0xFF;
+        stat = (ent >> 24) & 0xFF;
+        mine = ld_at(H.rec, m);
+        om = ld_at(H.ovr, m);
+    }
+    PH_END(sdev(), kPhLoads, tph);
+    const int own = lane == kLaneI ? i : (lane == kLaneJ ? j : -1);  // the result lanes' beads
+    int rep = -1;   // earlier event whose calendar-entry write this bead's updates replay on
+    int sp = -1;    // the lane's bead of the shoulder set
+    const bool sp_w = (flags & kPairWroteSp) != 0, sp_r = (flags & kPairReadsSp) != 0;
+    // ---- a round's footprint check.  Marks per bead: bit k = wavefront k
+    //      rewrites the bead's state, bit 8+k = it rewrites the bead's
+    //      calendar entry, bit 16+k = that rewrite may be a full recompute.
+    //      Event k commits only if no earlier event of the round rewrites a
+    //      state it reads or an entry it rewrites; a later event reads the
+    //      state before this one's writes (they wait for the round's last
+    //      barrier), as in the serial order.  One exception: a down bead
+    //      whose entry exactly one earlier event rewrote by single-pair
+    //      updates only, and whose own updates here are single-pair ones,
+    //      replays those updates on that event's entry once it is written.
+    auto clear_marks = [&]() {
+        if (dn) fp_clear(H, m);
+        if (own >= 0) fp_clear(H, own);
+        if (bk == 0 && sp_w && sp >= 0) fp_clear(H, sp);
+    };
+    if (batch) {
+        const unsigned sbit = 1u << bk, lbit = 1u << (8 + bk), fbit = 1u << (16 + bk);
+        if ((bk == 0 && sp_w) || (bk >= 1 && sp_r)) {
+            if (lane == 0) {
+                Pair& P = *ldsv().pair();
+                P.i = i;
+                P.j = j;
+                P.ri = ri;
+                P.rj = rj;
+                P.xi = xi;
+                P.xj = xj;
+            }
+            wave_sync();
+            sp = shoulder_bead(sdev(), *ldsv().pair(), lane);
+        }
+        if (lane == 0) B.wdone[bk] = 0;
+        if (dn || own >= 0) fp_or(H, dn ? m : own, dn ? lbit | (spec ? fbit : 0u) : sbit | lbit | fbit);
+        if (bk == 0 && sp_w && sp >= 0) fp_or(H, sp, sbit);
+        bar_to(nb, 1);
+        PH_END(sdev(), kPhBMark, tph);
+        if (bk >= 1) {
+            const unsigned lowS = sbit - 1u, lowL = lowS << 8;
+            const bool look = lane < ntot || own >= 0;
+            bool bad = false;
+            if (look) {
+                const unsigned mk = fp_get(H, own >= 0 ? own : m);
+                bad = (mk & lowS) != 0u;
+                if (own >= 0) bad = (mk & (lowS | lowL)) != 0u;
+                if (!bad && first && (mk & lowL)) {
+                    // (other lanes of the same bead leave it to its first)
+                    const unsigned wl = (mk & lowL) >> 8;
+                    const int q = __ffs(wl) - 1;
+                    if (!is_i && (wl & (wl - 1u)) == 0u && !(mk & (1u << (16 + q))) && !spec)
+                        rep = q;
+                    else
+                        bad = true;
+                }
+            }
+            if (sp_r && sp >= 0 && (fp_get(H, sp) & lowS)) bad = true;
+            if (__ballot(bad) && lane == 0) atomicMin(&B.cut, bk);
+            PH_END(sdev(), kPhBCheck, tph);
+            // the cut only moves down: a wavefront already past it stops here
+            // (the others learn theirs at the next barrier)
+            wave_sync();
+            if (bk >= uni(B.cut)) {
+                bar_to(nb, kRoundBars);
+                clear_marks();
+                return 0;
+            }
+        }
+    }
+    // ---- the predictions: the entry's bead against its base bead
+    PH_ADDN(sdev(), kPhNPred, ntot);
+    PH_ADDN(sdev(), kPhNPredPass, 1);
+    act = lane < ntot;
+    double tij = 1000000000.0;
+    int ty = 0, status = 0;
+    const int slot = tag < 4 ? (tag & 1) : tag - 2;
+    if (act) {
+        const BaseRec& b = W.base[slot];
+        const Rec rb = b.r;
+        const int bidx = b.idx;
+        const double2 bwb = b.bw;
+        if (late && (m == i || m == j)) mine = W.base[m == i ? 0 : 1].r;
+        Geo g;
+        geo(rb, mine, tf, g);  // the order of the two only flips the signs of vectors
+        if (stat == 0xFF) stat = static_t(mine.topo, rb.topo);  // symmetric in its beads
+        const int code = dyn_code(om, bidx, stat);  // ev_code(m, x) of a candidate, ev_code(l, p) of a down bead
+        const int adyn = dn ? mine.dyn : rb.dyn, cdyn = dn ? rb.dyn : mine.dyn;  // the lower bead's first
+        const double2 bwa = make_double2(dn ? bwm.x : bwb.x, dn ? bwm.y : bwb.y);
+        predict_geo(T, code, dyn_ident(adyn), dyn_ident(cdyn), dyn_bptnr(adyn) == (dn ? bidx : m), bwa, g, tij, ty);
+    }
+    // a down bead's prediction is checked where its op uses it
+    const bool err_c = ty == -99, err_t = tij < 0.0 && fabs(tij) > 1.0e-10;
+    if (act && !dn) status = err_t ? kErrNegativeTime : (err_c ? kErrBadCode : 0);
+    // ---- each owner's least (time, list position)
+    const unsigned long long tk = t_order(tij);
+    const bool cnd = act && !dn;
+    if (cnd) atomicMin(&W.tkey[slot], tk);
+    if (dups) {
+        W.wt[lane] = tij;
+        W.wy[lane] = ty;
+    }
+    wave_sync();
+    const unsigned long long win = __ballot(cnd && tk == W.tkey[slot]);
+    PH_END(sdev(), kPhPred, tph);
+    // owner results (full recompute rule: an event only below T0)
+    double ti = T0 + tf, tj = T0 + tf;
+    int pi = -1, ci = -1, pj = -1, cj = -1;
+    auto owner_min = [&](unsigned long long seg, double& t, int& p, int& c) {
+        const unsigned long long w = win & seg;
+        if (w) {
+            const int src = __ffsll((long long)w) - 1;
+            const double bt = readlane_d(tij, src);
+            if (bt < T0) {
+                t = bt + tf;
+                p = __builtin_amdgcn_readlane(m, src);
+                c = __builtin_amdgcn_readlane(ty, src);
+            }
+        }
+    };
+    const unsigned long long tag1 = __ballot(act && tag == 1), tag0 = __ballot(act && tag == 0);
+    owner_min(tag0, ti, pi, ci);
+    owner_min(tag1, tj, pj, cj);
+    double ft = T0 + tf;  // the bead's own full recompute
+    int fp = -1, fc = -1;
+    {
+        unsigned long long sm = specm;
+        for (int q = 0; q < nspec; ++q) {
+            const int src = __ffsll((long long)sm) - 1;
+            sm &= sm - 1;
+            double t = T0 + tf;
+            int p = -1, c = -1;
+            owner_min(__ballot(act && tag == 4 + q), t, p, c);
+            ft = lane == src ? t : ft;
+            fp = lane == src ? p : fp;
+            fc = lane == src ? c : fc;
+        }
+    }
+    // ---- each down bead's ops, those with i first
+    double st_t = is_i ? ti : lf0.tim;
+    int st_p = is_i ? pi : lf0.nptnr, st_c = is_i ? ci : leaf_ct(lf0.meta);
+    bool modified = false;
+    double sI = tij, sJ = tij;
+    int yI = ty, yJ = ty;
+    if (dups) {
+        sI = W.wt[pI];
+        yI = W.wy[pI];
+        sJ = W.wt[pJ];
+        yJ = W.wy[pJ];
+    }
+    if (is_i) {
+        ft = ti;
+        fp = pi;
+        fc = ci;
+    }
+    auto op = [&](bool on, int p, double t, int y) {
+        const bool full = on && st_p == p;
+        const bool single = on && !full;
+        if (single && y == -99) status = kErrBadCode;
+        if (single && t < 0.0 && fabs(t) > 1.0e-10) status = kErrNegativeTime;
+        const double tt = t + tf;
+        const bool less = single && tt < st_t;
+        st_t = full ? ft : (less ? tt : st_t);
+        st_p = full ? fp : (less ? p : st_p);
+        st_c = full ? fc : (less ? y : st_c);
+        modified |= full || less;
+    };
+    op(first && cI >= 1, i, sI, yI);
+    if (__ballot(first && cI >= 2)) {
+        for (int k = 2; k <= 4; ++k) op(first && cI >= k, i, sI, yI);
+    }
+    if (j >= 0) {
+        op(first && cJ >= 1, j, sJ, yJ);
+        if (__ballot(first && cJ >= 2)) {
+            for (int k = 2; k <= 4; ++k) op(first && cJ >= k, j, sJ, yJ);
+        }
+    }
+    // bead i's state lives in (ti, pi, ci) and is written with i's entry
+    const unsigned long long im = __ballot(is_i);
+    if (im) {
+        const int src = __ffsll((long long)im) - 1;
+        ti = readlane_d(st_t, src);
+        pi = __builtin_amdgcn_readlane(st_p, src);
+        ci = __builtin_amdgcn_readlane(st_c, src);
+    }
+    // ---- the new calendar entries, one per lane: the modified down beads',
+    //      i's and j's
+    bool wr = modified && !is_i;
+    if (own >= 0) {
+        st_t = lane == kLaneI ? ti : tj;
+        st_p = lane == kLaneI ? pi : pj;
+        st_c = lane == kLaneI ? ci : cj;
+        wr = true;
+    }
+    const int rb = own >= 0 ? own : m;
+    const unsigned long long stp = mk_stamp(coll, own >= 0 ? sub0 + (lane - kLaneI) : sub0 + 2 + (lane - ncand));
+    Leaf lf;
+    lf.tim = st_t;
+    lf.nptnr = st_p;
+    lf.meta = 0;
+    if (wr) lf.meta = make_meta(bin_of(interval_max, tbin_off, sortsize, nbin, st_t, status), st_c);
+    status = wave_status(status);
+    if (status && !st0) st0 = status;
+    PH_END(sdev(), kPhDown, tph);
+    int A = 1;
+    if (batch) {
+        // report the least new calendar key and the status, then commit
+        // only within the round's accepted prefix
+        Key kn = wr ? leaf_key(lf, rb) : empty_key();
+        unsigned long long ks = stp;
+        if (j < 0 && lane == kLaneJ) {
+            // a ghost event leading the round: its next ghost time
+            kn = leaf_key(leaf_ld(H, H.N), H.N);
+            ks = mk_stamp(coll, 1);  // re-added by this ghost event
+        }
+        unsigned long long kns = 0;
+        kn = key_min_wave_st(kn, ks, kns);
+        if (lane == 0) {
+            B.knew[bk] = kn;
+            B.knew_st[bk] = kns;
+            B.st[bk] = st0;
+            B.st_rep[bk] = 0;
+        }
+        bar_to(nb, kRoundBars);
+        PH_END(sdev(), kPhBKeys, tph);
+        // every wavefront has checked: clear this one's marks
+        clear_marks();
+        A = accepted(B);
+        if (bk >= A) return 0;
+        if (bk >= 1) {
+            if (lane == 0) st_at(H.rec, i, ri);
+            if (lane == 1) st_at(H.rec, j, rj);
+        }
+        if (bk == 0 && st0 && lane == 0 && !mc.status) mc.status = st0;
+    } else if (lane == 0) {
+        B.st[0] = 0;
+        B.st_rep[0] = 0;
+        if (st0 && !mc.status) mc.status = st0;
+    }
+    bool wb = wr;  // the lane's bead takes a new entry (its block is rescanned)
+    if (__ballot(rep >= 0)) {
+        int st2 = 0;
+        if (rep >= 0) {
+            // the earlier event's entry first, then this event's single-pair
+            // updates on it (i before j, eventredo_down.f), as the serial order
+            // would have applied them
+            while (__hip_atomic_load(&B.wdone[rep], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) == 0)
+                __builtin_amdgcn_s_sleep(1);
+            const Leaf cur = leaf_get_fresh(ldsv(), m);
+            lf = cur;
+            int rc = leaf_ct(cur.meta);
+            wb = false;
+            if (cI > 0 && sI + tf < lf.tim) {
+                lf.tim = sI + tf;
+                lf.nptnr = i;
+                rc = yI;
+                wb = true;
+            }
+            if (cJ > 0 && sJ + tf < lf.tim) {
+                lf.tim = sJ + tf;
+                lf.nptnr = j;
+                rc = yJ;
+                wb = true;
+            }
+            if (wb) lf.meta = make_meta(bin_of(interval_max, tbin_off, sortsize, nbin, lf.tim, st2), rc);
+        }
+        st2 = wave_status(st2);
+        if (st2 && lane == 0) B.st_rep[bk] = st2;
+    }
+    if (wb) {
+        leaf_st(H, rb, lf);
+        stamp_st(H, rb, stp);
+    }
+    {
+        int* const bl = reinterpret_cast<int*>(smem + H.o_blist);
+        const unsigned long long mm = __ballot(wb);
+        int n = __popcll(mm);
+        if (wb) bl[__popcll(mm & below)] = rb / kBlk;
+        if (extra_blk >= 0) {
+            if (lane == 0) bl[n] = extra_blk;
+            ++n;
+        }
+        if (lane == 0) B.nbl[batch ? bk : 0] = n;
+    }
+    // repuls_del_b.f once the rescheduling is done
+    if (xdel && lane == 0) {
+        const bool iN = dyn_ident(ri.dyn) < dyn_ident(rj.dyn);
+        const int a = iN ? i : j, b = iN ? j : i;
+        const int La = topo_len(iN ? ri.topo : rj.topo), Lb = topo_len(iN ? rj.topo : ri.topo);
+        const int ncim1 = a + La - 1, ncai = a - La, ncaj = b - 2 * Lb, nnjp1 = b - Lb + 1;
+        int4 ea = gld(H.extra + (a)), eb = gld(H.extra + (b));
+        ea.x = -1;
+        ea.y = -1;
+        ea.w = -1;
+        eb.x = -1;
+        eb.y = -1;
+        eb.w = -1;
+        gst(H.extra + (a), ea);
+        gst(H.extra + (b), eb);
+        gs1(&H.extra[ncaj].z, -1);
+        gs1(&H.extra[nnjp1].z, -1);
+        gs1(&H.extra[ncai].z, -1);
+        gs1(&H.extra[ncim1].z, -1);
+    }
+    if (batch) {
+        // the round's block rescans run after every committed event's
+        // writes; a later event that replays on these entries waits for
+        // the flag
+        wave_sync_mem();
+        if (lane == 0) __hip_atomic_store(&B.wdone[bk], 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    PH_END(sdev(), kPhLeaf, tph);
+    return A;
 }
 
 // ------------------------------------------------------------------------
@@ -3453,6 +4292,7 @@ __device__ Lds make_lds(const SysDev&, int maxw, int lds_bytes, int nw, int wave
     // footprint marks behind the leaves, when both fit
     const int o_mark = (p + N3 * (int)sizeof(Leaf) + 15) / 16 * 16;
     L.mark_lds = L.leaf_lds && o_mark + 4 * S.N <= lds_bytes;
+    L.o_mark = o_mark;
     L.mark = L.mark_lds ? reinterpret_cast<unsigned*>(smem + o_mark) : S.mark;
     return L;
 }
@@ -3632,89 +4472,100 @@ __global__ __launch_bounds__(64 * kSetupWaves) void k_rebuild_events(const SysDe
 
 // Pop up to kmax calendar entries in key order (wavefront 0): pair events
 // only after the first, since a pseudo-event runs alone.  Each popped entry
-// but the last is taken out of the min tree until the round's rescans.
-// Every speculative wavefront k gets a copy of the master scalars (which it
-// sets to its event's time and bin after the round's first barrier); the
-// master takes the first event.  Returns the number popped (0: stop, or an
-// empty calendar).
-__device__ int select_batch(const Lds&, Sc& c, int N, int N3, int kmax) {
-    const Lds& L = ldsv();
-    const SysDev& S = sdev();
-    (void)S;
+// but the last is taken out of the min tree until the round's rescans.  The
+// master takes the first event's bin, time and number.  Returns the number
+// popped (0: stop, or an empty calendar).
+//
+// A pop is a dependent chain (wave minimum, the popped entry's block minimum
+// without it, for larger calendars its superblock's), so the top level and
+// its proxies stay in lane registers and only the popped entry's block is
+// read from LDS.
+__device__ __forceinline__ int select_batch(const Hot& H, Sc& c, int kmax) {
     PH_BEGIN(tsp);
-
-    Batch& B = *L.batch();
-    const int lane = lane_id();
-    // the views this loop uses, read once (wave fences below would make the
-    // compiler read them from LDS again)
-    Key* const blk = L.blk();
-    Key* const sup = L.sup();
-    const int nsup = L.nsup, nblk = L.nblk;
-    const bool leaf_lds = L.leaf_lds;
-    const Leaf* const lleaf = L.lleaf();
-    const Leaf* const gleaf = L.gleaf;
-    int K = 0;
-    unsigned pip = 0xFFFFFFFFu;  // lane m: index << 16 | partner of popped entry m
-    // one superblock (up to 1024 entries): the block minima stay in lane
-    // registers (lane b: block b) and an exclusion replaces one of them; the
-    // tree in LDS keeps its values, which the round's rescans of the popped
-    // blocks confirm or replace
-    const bool one_sup = nsup == 1;
-    Key bmin = empty_key();
-    if (one_sup && lane < nblk) bmin = blk[lane];
+    Batch& B = round_rec();
+    const int lane = lane_id(), N = H.N, N3 = N + 3;
+    Key* const blk = reinterpret_cast<Key*>(smem + H.o_blk);
+    Key* const sup = reinterpret_cast<Key*>(smem + kSupOff);
+    const bool one_sup = H.nsup == 1;
+    // one superblock (up to 1024 entries): lane b holds block b's minimum; an
+    // exclusion replaces one of them, and the tree in LDS keeps its values,
+    // which the round's rescans confirm or replace.  Else lane s holds
+    // superblock s's, and the LDS tree takes the exclusions.
+    Key top = empty_key();
+    if (lane < (one_sup ? H.nblk : H.nsup)) top = one_sup ? blk[lane] : sup[lane];
+    double pr = key_proxy(top);
+    int K = 0, k0bin = 0;
+    double k0t = 0.0;
+    int pidx = -1;        // lane m: index of popped entry m
+    unsigned gone = 0;    // lane b: popped entries of block b (one superblock)
     while (true) {
-        const Key k = one_sup ? key_min_wave(bmin) : key_min_wave(lane < nsup ? sup[lane] : empty_key());
-        if (k.bc == kEmptyBc) {
+        const double mn = wave_min(pr);
+        if (uni(__double2hiint(mn)) == kInfHi) {
             if (K == 0) c.status = kErrBin;
             break;
         }
+        int src;
+        const Key k = key_of_ties(top, __ballot(pr == mn), src);
         const int e = key_idx(k);
         if (K > 0 && e >= N) break;
         if (lane == 0) B.key[K] = k;
-        if (lane == K) pip = k.ip;
+        if (K == 0) {
+            k0bin = key_bin(k);
+            k0t = k.t;
+        }
+        if (lane == K) pidx = e;
         ++K;
         // a ghost event may lead a round (its draws come first in the
         // serial order); sync and output events run alone
         if (e > N || K >= kmax) break;
         // take e out of the tree: its block without the popped entries, then
         // its superblock
-        const int b = e / kBlk, sp = b / kSup;
-        Key x = empty_key();
+        const int b = e / kBlk;
+        Key x = empty_key(), y = empty_key();
         const int idx = b * kBlk + (lane & 15);
-        if (lane < kBlk && idx < N3) {
-            bool popped = false;
-            for (int m = 0; m < K; ++m) popped |= (int)(__builtin_amdgcn_readlane((int)pip, m) >> 16) == idx;
-            if (!popped) x = leaf_key(leaf_lds ? lleaf[idx] : gld(gleaf + idx), idx);
-        }
-        const bool win = key_min_rows(x);
+        bool out = lane >= kBlk || idx >= N3;
         if (one_sup) {
-            const unsigned long long wm = __ballot(win && lane < kBlk);
-            const Key nb = readlane_key(x, __ffsll((long long)wm) - 1);
-            if (lane == b) bmin = nb;
-            continue;
+            if (lane == b) gone |= 1u << (e & (kBlk - 1));
+            out |= ((unsigned)__builtin_amdgcn_readlane((int)gone, b) >> (lane & 15)) & 1u;
+        } else {
+            for (int q = 0; q < K; ++q) out |= __builtin_amdgcn_readlane(pidx, q) == idx;
+            const int bb = src * kSup + lane;
+            if (bb < H.nblk) y = blk[bb];
         }
-        if (win && lane < kBlk) blk[b] = x;
-        wave_sync();
-        const int bb = sp * kSup + lane;
-        const Key y = key_min_wave(bb < nblk ? blk[bb] : empty_key());
-        if (lane == 0) sup[sp] = y;
-        wave_sync();
+        if (!out) x = leaf_key(leaf_ld(H, idx), idx);
+        const double px = key_proxy(x), rm = row_min(px);
+        Key nb = empty_key();
+        if (__builtin_amdgcn_readlane(__double2hiint(rm), 0) != kInfHi) {
+            int s2;
+            nb = key_of_ties(x, __ballot(px == rm) & 0xFFFFull, s2);
+        }
+        if (!one_sup) {
+            if (lane == 0) blk[b] = nb;
+            if (lane == (b & (kSup - 1))) y = nb;
+            const double py = key_proxy(y), ym = wave_min(py);
+            nb = empty_key();
+            if (uni(__double2hiint(ym)) != kInfHi) {
+                int s2;
+                nb = key_of_ties(y, __ballot(py == ym), s2);
+            }
+            if (lane == 0) sup[src] = nb;
+        }
+        if (lane == src) {
+            top = nb;
+            pr = key_proxy(nb);
+        }
     }
-    PH_END(S, kPhSelPop, tsp);
-    wave_sync();
+    PH_END(sdev(), kPhSelPop, tsp);
     if (K == 0) return 0;
-    const long long cw = lane < (int)(sizeof(Sc) / 8) ? reinterpret_cast<const long long*>(&c)[lane] : 0;
-    for (int k = 1; k < K; ++k) {
-        const Lds& Lk = *reinterpret_cast<const Lds*>(smem + kLdOff + k * kLdStride);
-        if (lane < (int)(sizeof(Sc) / 8)) reinterpret_cast<long long*>(Lk.sc())[lane] = cw;
+    if (lane == 0) {
+        c.old_tfalse = c.tfalse;
+        c.nbin = k0bin;
+        c.tfalse = k0t;
+        c.coll++;
+        B.touched = 0;
     }
     wave_sync();
-    const Key k0 = B.key[0];
-    c.old_tfalse = c.tfalse;
-    c.nbin = key_bin(k0);
-    c.tfalse = k0.t;
-    c.coll++;
-    PH_END(S, kPhSelCopy, tsp);
+    PH_END(sdev(), kPhSelCopy, tsp);
     return K;
 }
 
@@ -3789,13 +4640,15 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_run(const SysDev* __restrict
         w0 = B.t0;
     }
     bool stop_out = false;
+    const Hot H = load_hot(S, L);
     while (true) {
         if (wave == 0) {
             PH_BEGIN(tsel);
             int K = 0;
-            if (c.coll < c.target && c.status == 0 && !stop_out && !(budget > 0 && wall_clock64() - w0 > budget)) {
-                long long left = c.target - c.coll;
-                K = select_batch(L, c, N, N3, (int)min((long long)kcap, left));
+            if (uni(c.status) == 0 && !stop_out && !(budget > 0 && wall_clock64() - w0 > budget)) {
+                const long long left = c.target - c.coll;
+                const int room = uni((int)min((long long)kcap, left));
+                if (room > 0) K = select_batch(H, c, room);
             }
             if (lane == 0) {
                 B.K = K;
@@ -3807,11 +4660,11 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_run(const SysDev* __restrict
             __syncthreads();
         else
             wave_sync();
-        const int K = B.K;
+        const int K = uni(B.K);
         if (K == 0) break;
-        if (K == 1) {
-            const Key k = B.key[0];
-            const int e = key_idx(k);
+        const Key k = B.key[wave < K ? wave : 0];
+        const int e = uni(key_idx(k));
+        if (K == 1 && e > N) {
             if (e == N + 1) {
                 // the sync event; every wavefront takes part in a list rebuild
                 if (wave == 0) {
@@ -3828,92 +4681,70 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_run(const SysDev* __restrict
                     t_rebuild += wall_clock64() - tr;
                     ++n_rebuild;
                 }
-                if (wave == 0) {
-                    sync_finish(S, L, c);
-                    log_event(S, log_count, c.coll, e, -1, 0, k.t);
-                }
+                if (wave == 0) sync_finish(S, L, c);
             } else if (wave == 0) {
-                int jj = -1, ty = 0;
-                if (e < N) {
-                    jj = key_p(k);
-                    ty = pair_event(S, T, L, c, e, jj, key_ct(k), -1);
-                    if (ty >= 1 && ty <= 30 && lane == 0) c.nev[ty]++;
-                } else if (e == N) {
-                    jj = ghost_event(S, T, L, c, -1);
-                } else {
-                    output_event(S, L, c);
-                    stop_out = (flags & kStopAtOutput) != 0;
-                }
-                log_event(S, log_count, c.coll, e, jj, ty, k.t);
+                output_event(S, L, c);
+                stop_out = (flags & kStopAtOutput) != 0;
             }
+            if (wave == 0) log_event(S, log_count, c.coll, e, -1, 0, k.t);
             if (nw > 1) __syncthreads();
             continue;
         }
-        // a round of K >= 2 pair events, one per wavefront; a speculative
-        // wavefront's scalars are the master's as its event comes up
-        if (wave >= 1 && wave < K && lane == 0) {
-            // the copy was taken before the master counted the round's first
-            // event: the event number comes from the master, so that every
-            // event of the round stamps its adds with its own number (equal
-            // stamps would order tied entries by index, not last-added first)
-            Sc& ck = *L.sc();
-            ck.old_tfalse = B.key[wave - 1].t;
-            ck.tfalse = B.key[wave].t;
-            ck.nbin = key_bin(B.key[wave]);
-            ck.coll = L.msc()->coll + wave;
-            ck.status = 0;
-        }
-        wave_sync();
+        // pair events (a ghost event may lead them), one per wavefront; event
+        // k of a round is numbered and stamped as the master will count it
+        int A = 0;
         if (wave < K) {
-            const Key k = B.key[wave];
-            if (key_idx(k) == N)
-                ghost_event(S, T, L, c, 0);
-            else
-                pair_event(S, T, L, *L.sc(), key_idx(k), key_p(k), key_ct(k), wave);
-        } else {
+            const int bk = K == 1 ? -1 : wave;
+            A = run_event(H, e, uni(key_p(k)), uni(key_ct(k)), k.t, uni(key_bin(k)), master().coll + wave, bk);
+            if (A > 0 && lane == 0) {
+                const int ty = B.ty[wave];
+                if (ty >= 1 && ty <= 30)
+                    __hip_atomic_fetch_add((unsigned long long*)&master().nev[ty], 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            }
+        } else if (K > 1) {
             int nb = 0;
             bar_to(nb, kRoundBars);
         }
         PH_BEGIN(ttail);
-        const int A = batch_accepted(B);
-        if (wave == 0) {
+        if (wave == 0 && K > 1) {
             PH_COUNT(S, kPhNRound);
             PH_ADDN(S, kPhNPopped, K);
             PH_ADDN(S, kPhNCommit, A);
             PH_ADDN(S, kPhNCutMark, min(K, B.cut) < K ? 1 : 0);
             PH_ADDN(S, kPhNCutKey, A < min(K, B.cut) ? 1 : 0);
         }
-        __syncthreads();
+        wg_sync(nw);
         // block minima of every committed event's blocks and of the popped
         // entries that were not committed, then the superblock minima
-        if (wave == 0) {
-            int nbl = B.nbl[0];
-            for (int k = A; k < K; ++k) {
-                if (lane == 0) L.blist()[nbl] = key_idx(B.key[k]) / kBlk;
-                ++nbl;
+        if (A > 0) {
+            int* const bl = reinterpret_cast<int*>(smem + H.o_blist);
+            int nbl = uni(B.nbl[wave]);
+            if (wave == 0 && A < K) {
+                if (lane < K - A) bl[nbl + lane] = key_idx(B.key[A + lane]) / kBlk;
+                nbl += K - A;
+                wave_sync();
             }
-            if (lane == 0) B.nbl[0] = nbl;
-            wave_sync();
+            rescan_round(H, bl, nbl);
         }
-        if (wave < A) rescan_blocks(L, N3, L.blist(), B.nbl[wave]);
         // a single superblock is never read: selection pops from the block
         // minima (its value is recomputed by the single-event paths)
-        if (L.nsup > 1) {
-            __syncthreads();
-            if (wave < A) rescan_sups(L, L.blist(), B.nbl[wave]);
+        if (H.nsup > 1) {
+            wg_sync(nw);
+            rescan_touched(H, wave, nw);
         }
         if (wave == 0) {
             // the master takes the committed events in order
-            for (int k = 0; k < A; ++k) {
-                const Key kk = B.key[k];
-                const int ty = B.ty[k];
-                if (ty >= 1 && ty <= 30 && lane == 0) c.nev[ty]++;
-                log_event(S, log_count, c.coll + k, key_idx(kk), key_idx(kk) == N ? B.gbead : key_p(kk), ty, kk.t);
-            }
-            if (A >= 2) {
-                if (lane == 0) {
-                    for (int k = 1; k < A; ++k)
-                        if (B.st[k] != 0 && c.status == 0) c.status = B.st[k];
+            if (S.log)
+                for (int q = 0; q < A; ++q) {
+                    const Key kk = B.key[q];
+                    log_event(S, log_count, c.coll + q, key_idx(kk), key_idx(kk) == N ? B.gbead : key_p(kk), B.ty[q], kk.t);
+                }
+            if (lane == 0) {
+                for (int q = 0; q < A; ++q) {
+                    const int st = q > 0 && B.st[q] != 0 ? B.st[q] : B.st_rep[q];
+                    if (st != 0 && c.status == 0) c.status = st;
+                }
+                if (A >= 2) {
                     c.coll += A - 1;
                     c.old_tfalse = B.key[A - 2].t;
                     c.tfalse = B.key[A - 1].t;
@@ -3921,7 +4752,10 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_run(const SysDev* __restrict
                 }
             }
         }
-        __syncthreads();
+        if (nw > 1)
+            __syncthreads();
+        else
+            wave_sync();
         PH_END(S, kPhBTail, ttail);
     }
     __syncthreads();
