@@ -20,6 +20,7 @@
 // Many systems in one launch run concurrently, one workgroup each.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <climits>
 #include <cstdint>
 #include <mutex>
@@ -35,7 +36,7 @@ constexpr int kW = 64;
 constexpr int kBlk = 16;
 constexpr int kSup = 64;
 constexpr int kNumbin = 2000;
-constexpr int kMaxBlist = 256;
+constexpr int kMaxBlist = 160;
 constexpr double kLt = 1e-10;
 constexpr double kSm = 5e-12;
 constexpr int kMaxWaves = 8;  // most wavefronts in one system's workgroup
@@ -713,6 +714,7 @@ struct Batch {
     unsigned long long touched;  // superblocks with a changed block minimum (bit s)
     int gbead;            // the bead of a ghost event leading the round
     long long t0;         // start of a budgeted launch (wall_clock64)
+    Leaf pseudo[3];       // the ghost, sync and output entries across a list rebuild
 };
 // Order proxy of a calendar key: a positive double with the bin in its
 // exponent field (bins 1 to kNumbin = 2000 of 2046 values) and the top 52
@@ -840,7 +842,8 @@ __device__ inline bool key_min_rows(Key& k) {
 // and the round record are shared, the work lists are the wavefront's own
 struct Lds {
     int o_blk, o_sup, o_wm, o_wx, o_blist, o_pair, o_sc, o_leaf, o_wd, o_wt, o_wy, o_slot, o_spec, o_down;
-    int o_msc, o_batch, o_mark;
+    int o_msc, o_batch, o_mark, o_one, o_pool;
+    int nwr;  // wavefronts of a list rebuild that have scratch in the pool
     Leaf* gleaf;  // calendar leaves in HBM when they do not fit in LDS
     // the round's footprint marks: a flat pointer into LDS (behind the
     // leaves, when both fit there) or to SysDev::mark
@@ -903,6 +906,9 @@ __device__ inline Lds lds_regs() {
     r.o_msc = __builtin_amdgcn_readfirstlane(m.o_msc);
     r.o_batch = __builtin_amdgcn_readfirstlane(m.o_batch);
     r.o_mark = __builtin_amdgcn_readfirstlane(m.o_mark);
+    r.o_one = __builtin_amdgcn_readfirstlane(m.o_one);
+    r.o_pool = __builtin_amdgcn_readfirstlane(m.o_pool);
+    r.nwr = __builtin_amdgcn_readfirstlane(m.nwr);
     r.gleaf = sgpr_ptr(m.gleaf);
     r.nblk = __builtin_amdgcn_readfirstlane(m.nblk);
     r.nsup = __builtin_amdgcn_readfirstlane(m.nsup);
@@ -971,7 +977,7 @@ __device__ inline Hot load_hot(const SysDev& S, const Lds& L) {
     H.o_blk = uni(L.o_blk);
     H.o_leaf = uni(L.o_leaf);
     H.o_mark = uni(L.o_mark);
-    H.o_w = uni(L.o_wm);
+    H.o_w = uni(L.o_one);
     H.o_blist = uni(L.o_blist);
     H.leaf_lds = uni(L.leaf_lds ? 1 : 0) != 0;
     H.mark_lds = uni(L.mark_lds ? 1 : 0) != 0;
@@ -1220,12 +1226,6 @@ __device__ inline void bar_to(int& nb, int n) {
         ++nb;
     }
 }
-__device__ inline int spec_abort(const Lds& L, int bk, int& nb) {
-    if (lane_id() == 0) atomicMin(&L.batch()->cut, bk);
-    bar_to(nb, kRoundBars);
-    return -1;
-}
-
 __device__ inline void spec_abort_at(int bk, int& nb) {
     if (lane_id() == 0) atomicMin(&round_rec().cut, bk);
     bar_to(nb, kRoundBars);
@@ -1687,9 +1687,8 @@ __device__ void reschedule_generic(const SysDev&, const DevTables&, const Lds&, 
         wave_sync_mem();
     else
         wave_sync();
+    if (lane == 0) L.batch()->nbl[0] = nbl;
     PH_END(S, kPhLeaf, tph);
-    rescan_block_list(L, N3, nbl);
-    PH_END(S, kPhRescan, tph);
 }
 
 // partial_events.f:16-201 after an event of pair (i, j) (j < 0: ghost of i).
@@ -1790,20 +1789,13 @@ __device__ __noinline__ void reschedule(const SysDev&, const DevTables&, const L
     }
     const int nD = d;
     if (nD > kW) {
-        // the generic form writes as it goes: it runs only as a round's
-        // first event, and no other event of the round is committed
-        if (bk >= 1) {
-            spec_abort(L, bk, nb);
-            return;
-        }
+        // the generic form writes as it goes: no other event of the round
+        // is committed
         if (batch && lane == 0) atomicMin(&L.batch()->cut, 1);
         wave_sync_mem();
         PH_COUNT(S, kPhNGeneric);
         reschedule_generic(S, T, L, c, P, extra_blk, xpulse_del);
-        if (batch) {
-            if (lane == 0) L.batch()->nbl[bk] = 0;
-            bar_to(nb, kRoundBars);
-        }
+        if (batch) bar_to(nb, kRoundBars);
         return;
     }
     if (lane < 2 + kMaxSpec) {
@@ -1932,7 +1924,6 @@ __device__ __noinline__ void reschedule(const SysDev&, const DevTables&, const L
     }
     int sp = -1;  // the wavefront's bead of the shoulder set, marked in a round
     bool sp_w = false;
-    int rep = -1;  // earlier event whose calendar-entry write this bead's updates replay on
     // the down bead's updates may take a full recompute (a pending op)
     const bool mfull = first && !is_i && ((lf0.nptnr == i && cI > 0) || (lf0.nptnr == j && cJ > 0) || cI >= 2 || cJ >= 2);
     // single-pair predictions of the down beads (placed after the pairs)
@@ -1940,70 +1931,21 @@ __device__ __noinline__ void reschedule(const SysDev&, const DevTables&, const L
     const unsigned long long mI = __ballot(wantI), mJ = __ballot(wantJ);
     const int nI = __popcll(mI), nsing = nI + __popcll(mJ);
     const bool sing_fit = npairs + nsing <= maxw;
-    // ---- a round's footprint check.  Marks per bead: bit k = wavefront k
-    //      rewrites the bead's state, bit 8+k = it rewrites the bead's
-    //      calendar entry, bit 16+k = that rewrite may be a full recompute.
-    //      Event k commits only if no earlier event of the round rewrites a
-    //      state it reads or an entry it rewrites; a later event reads the
-    //      state before this one's writes (they wait for the round's last
-    //      barrier), as in the serial order.  One exception: a down bead
-    //      whose entry exactly one earlier event rewrote by single-pair
-    //      updates only, and whose own updates here are single-pair ones,
-    //      replays those updates on that event's entry once it is written.
+    // ---- the round's footprint marks (run_event): this event leads the
+    //      round, so it checks nothing and is always committed
     if (batch) {
         PH_RESET(tph);
         Batch& B = *L.batch();
-        const unsigned sbit = 1u << bk, lbit = 1u << (8 + bk), fbit = 1u << (16 + bk);
+        const unsigned sbit = 1u, lbit = 1u << 8, fbit = 1u << 16;
         sp = shoulder_bead(S, P, lane);
-        if (lane == 0) B.wdone[bk] = 0;
+        if (lane == 0) B.wdone[0] = 0;
         if (dent >= 0) mark_or(L, S, dent, lbit | (mfull ? fbit : 0u));
         if (lane == 0) mark_or(L, S, i, sbit | lbit | fbit);
         if (lane == 1 && j >= 0) mark_or(L, S, j, sbit | lbit | fbit);
         sp_w = (P.flags & kPairWroteSp) != 0;
-        const bool sp_r = (P.flags & kPairReadsSp) != 0;
-        if (bk == 0 && sp_w && sp >= 0) mark_or(L, S, sp, sbit);
+        if (sp_w && sp >= 0) mark_or(L, S, sp, sbit);
         bar_to(nb, 1);
         PH_END(S, kPhBMark, tph);
-        if (bk >= 1) {
-            const unsigned lowS = sbit - 1u, lowL = lowS << 8;
-            bool bad = false;
-            for (int base = 0; base < npairs; base += kW) {
-                const int q = base + lane;
-                if (q < npairs) {
-                    const int m = (base == 0 && q < ncand ? cent : v_wm[q]) & 0xFFFFFF;
-                    if (mark_get(L, S, m) & lowS) bad = true;
-                }
-            }
-            if (dent >= 0) {
-                const unsigned mk = mark_get(L, S, dent);
-                if (mk & lowS) {
-                    bad = true;
-                } else if ((mk & lowL) && first) {
-                    // (other lanes of the same bead leave it to its first)
-                    const unsigned wl = (mk & lowL) >> 8;
-                    const int m = __ffs(wl) - 1;
-                    if (!is_i && __popc(wl) == 1 && !(mk & (1u << (16 + m))) && !mfull && sing_fit)
-                        rep = m;
-                    else
-                        bad = true;
-                }
-            }
-            if (lane == 0 && (mark_get(L, S, i) & (lowS | lowL))) bad = true;
-            if (lane == 1 && j >= 0 && (mark_get(L, S, j) & (lowS | lowL))) bad = true;
-            if (sp_r && sp >= 0 && (mark_get(L, S, sp) & lowS)) bad = true;
-            // a down bead whose full recompute is not in the batch would
-            // read rows that were not checked
-            if (mfull && !(spec && v_spec[myslot].off >= 0)) bad = true;
-            if (__ballot(bad) && lane == 0) atomicMin(&B.cut, bk);
-        }
-        PH_END(S, kPhBCheck, tph);
-        // the cut only moves down: a wavefront already past it stops here
-        // (the others learn theirs at the next barrier)
-        if (bk >= B.cut) {
-            bar_to(nb, kRoundBars);
-            round_clear_marks(L, S, dent, i, j, bk == 0 && sp_w ? sp : -1);
-            return;
-        }
     }
     // ---- the single-pair predictions (l, i) and (l, j) of each down bead,
     //      after the pair entries: each is the same for every op of l with
@@ -2269,62 +2211,16 @@ __device__ __noinline__ void reschedule(const SysDev&, const DevTables&, const L
         unsigned long long kns = 0;
         kn = key_min_wave_st(kn, ks, kns);
         if (lane == 0) {
-            B.knew[bk] = kn;
-            B.knew_st[bk] = kns;
-            B.st[bk] = c.status;
+            B.knew[0] = kn;
+            B.knew_st[0] = kns;
+            B.st[0] = c.status;
         }
         bar_to(nb, kRoundBars);
         PH_END(S, kPhBKeys, tph);
         // every wavefront has checked: clear this one's marks
-        round_clear_marks(L, S, dent, i, j, bk == 0 && sp_w ? sp : -1);
-        if (bk >= batch_accepted(B)) return;
-        if (bk >= 1 && lane == 0) {
-            gst(S.rec + (i), P.ri);
-            gst(S.rec + (j), P.rj);
-        }
+        round_clear_marks(L, S, dent, i, j, sp_w ? sp : -1);
     }
-    bool wb = wr;  // the lane's bead takes a new entry (its block is rescanned)
-    if (rep >= 0) {
-        // the earlier event's entry first, then this event's single-pair
-        // updates on it (i before j, eventredo_down.f), as the serial order
-        // would have applied them
-        Batch& B = *L.batch();
-        while (__hip_atomic_load(&B.wdone[rep], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) == 0)
-            __builtin_amdgcn_s_sleep(1);
-        const Leaf cur = leaf_get_fresh(L, l);
-        double rt = cur.tim;
-        int rp = cur.nptnr, rc = leaf_ct(cur.meta), st2 = 0;
-        bool mod = false;
-        if (cI > 0) {
-            const double t = v_wt[sqI] + tf;
-            if (t < rt) {
-                rt = t;
-                rp = i;
-                rc = v_wy[sqI];
-                mod = true;
-            }
-        }
-        if (cJ > 0) {
-            const double t = v_wt[sqJ] + tf;
-            if (t < rt) {
-                rt = t;
-                rp = j;
-                rc = v_wy[sqJ];
-                mod = true;
-            }
-        }
-        if (mod) {
-            Leaf nl;
-            nl.tim = rt;
-            nl.nptnr = rp;
-            nl.meta = make_meta(calc_bin(c, rt, false, st2), rc);
-            leaf_set(L, l, nl);
-            stamp_set(l, mk_stamp(c.coll, sub0 + 2 + lane));
-        }
-        st2 = wave_status(st2);
-        if (st2 && lane == 0 && B.st[bk] == 0) B.st[bk] = st2;
-        wb = mod;
-    } else if (wr) {
+    if (wr) {
         leaf_set(L, l, lf);
         stamp_set(l, mk_stamp(c.coll, sub0 + 2 + lane));
     }
@@ -2333,9 +2229,9 @@ __device__ __noinline__ void reschedule(const SysDev&, const DevTables&, const L
         L.blist()[1] = j >= 0 ? j / kBlk : i / kBlk;
         L.blist()[2] = extra_blk >= 0 ? extra_blk : i / kBlk;
     }
-    const unsigned long long mm = __ballot(wb);
+    const unsigned long long mm = __ballot(wr);
     const int pre = __popcll(mm & ((1ull << lane) - 1ull));
-    if (wb) L.blist()[3 + pre] = l / kBlk;
+    if (wr) L.blist()[3 + pre] = l / kBlk;
     const int nbl = 3 + __popcll(mm);
     PH_END(S, kPhDown, tph);
     if (lane == 0) {
@@ -2372,8 +2268,8 @@ __device__ __noinline__ void reschedule(const SysDev&, const DevTables&, const L
         // the flag
         wave_sync_mem();
         if (lane == 0) {
-            L.batch()->nbl[bk] = nbl;
-            __hip_atomic_store(&L.batch()->wdone[bk], 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+            L.batch()->nbl[0] = nbl;
+            __hip_atomic_store(&L.batch()->wdone[0], 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
         }
         return;
     }
@@ -2381,9 +2277,8 @@ __device__ __noinline__ void reschedule(const SysDev&, const DevTables&, const L
         wave_sync_mem();
     } else
         wave_sync();
+    if (lane == 0) L.batch()->nbl[0] = nbl;
     PH_END(S, kPhLeaf, tph);
-    rescan_block_list(L, N3, nbl);
-    PH_END(S, kPhRescan, tph);
 }
 
 // ------------------------------------------------------------------------
@@ -2630,7 +2525,6 @@ struct OnePass {
     int wy[kW];
     int lst[kW];
 };
-static_assert(sizeof(OnePass) <= 4 * 768, "the one-pass work area exceeds a wavefront's work list");
 // result lanes of beads i and j: entries take the lanes below
 constexpr int kLaneI = kW - 2, kLaneJ = kW - 1;
 
@@ -3123,7 +3017,12 @@ __device__ __forceinline__ int run_event(const Hot& H, int e, int jp, int ct, do
         }
     }
     if (multi) {
-        // the pair and this event's scalars to LDS for the multi-pass form
+        // only the first wavefront has the multi-pass form's work lists: a
+        // speculative event that needs them waits to lead a round
+        if (bk >= 1) {
+            spec_abort_at(bk, nb);
+            return 0;
+        }
         const Lds& L = ldsv();
         if (lane == 0) {
             Pair& P = *L.pair();
@@ -3138,33 +3037,11 @@ __device__ __forceinline__ int run_event(const Hot& H, int e, int jp, int ct, do
             P.xi = xi;
             P.xj = xj;
         }
-        if (bk >= 1) {
-            if (lane < (int)(sizeof(Sc) / 8))
-                reinterpret_cast<long long*>(L.sc())[lane] = reinterpret_cast<const long long*>(&mc)[lane];
-            wave_sync();
-            if (lane == 0) {
-                Sc& c = *L.sc();
-                c.tfalse = tf;
-                c.nbin = nbin;
-                c.coll = coll;
-                c.status = st0;
-            }
-        } else if (lane == 0 && st0 && !mc.status)
-            mc.status = st0;
+        if (lane == 0 && st0 && !mc.status) mc.status = st0;
         wave_sync();
         reschedule(sdev(), T, L, *L.sc(), *L.pair(), extra_blk, xdel, bk);
-        if (!batch) {
-            if (lane == 0) {
-                B.nbl[0] = 0;
-                B.st[0] = 0;
-                B.st_rep[0] = 0;
-            }
-            return 1;
-        }
-        if (lane == 0) B.st_rep[bk] = 0;
-        if (bk >= uni(B.cut)) return 0;
-        const int A = accepted(B);
-        return bk < A ? A : 0;
+        if (lane == 0) B.st_rep[0] = 0;
+        return batch ? accepted(B) : 1;
     }
     wave_sync();
     const bool late = lane >= n0 && lane < ntot;
@@ -3504,6 +3381,11 @@ __device__ __forceinline__ int run_event(const Hot& H, int e, int jp, int ct, do
 // cells, all cell ranges requested before the candidates, each candidate
 // read with two independent loads.  Candidates come in a fixed cell order
 // and ascending bead index within a cell, so the lists are deterministic.
+// A wavefront's LDS scratch of a list rebuild: the search's cell ranges (27
+// per lane) or the row sort's keys and entries.  It lies over the work
+// areas, block minima and leaves, which a rebuild leaves free.
+constexpr int kScratch = 15872;
+static_assert(27 * kW * (int)sizeof(int2) <= kScratch, "cell ranges exceed the rebuild scratch");
 // v mod m for v in [-1, m]
 __device__ inline int wrap1(int v, int m) { return v < 0 ? v + m : (v >= m ? v - m : v); }
 __device__ void rebuild_lists(const SysDev&, const Lds&, Sc& c) {
@@ -3606,12 +3488,12 @@ __device__ void rebuild_lists(const SysDev&, const Lds&, Sc& c) {
     int mx = 0, status = 0;
     const int noff = Mq > 2 ? 3 : Mq;  // distinct coarse offsets {0, +1, -1}
     // per lane, its bead's non-empty neighbour cell ranges, [t][lane] in the
-    // wavefront's own work area; wavefronts take 64-bead chunks in turn
-    int2* rng = reinterpret_cast<int2*>(smem + L.o_wm);
+    // wavefront's scratch; wavefronts take 64-bead chunks in turn
+    int2* rng = reinterpret_cast<int2*>(smem + L.o_pool + wave * kScratch);
     // beads are taken in cell order (64 consecutive sorted places per
     // chunk): the lanes of a chunk sit in the same or adjacent cells, so
     // their candidate reads fall on shared cache lines
-    for (int i0 = wave * kW; i0 < N; i0 += nw * kW) {
+    for (int i0 = wave * kW; wave < L.nwr && i0 < N; i0 += L.nwr * kW) {
         const int ps = i0 + lane;
         const bool act = ps < N;
         const int4 si = act ? gld(S.sinfo + (ps)) : make_int4(-1, 0, 0, 0);
@@ -3732,20 +3614,17 @@ __device__ void rebuild_lists(const SysDev&, const Lds&, Sc& c) {
 
 // Neighbour lists of a small system (N <= kDenseN) without the cell sort.
 // Positions, topology words, override slots and fine cells are staged in
-// LDS (wavefront 0's work area is free during a rebuild); each wavefront
+// LDS (wavefront 0's rebuild scratch); each wavefront
 // takes beads in turn, tests the fine-cell stencil of all candidates one per
 // lane, and queues the (bead, candidate) pairs that pass; full 64-lane
 // batches of the queue then take the pair-code and cutoff test.  Membership
 // is rebuild_lists' own (the n_wrap = 2 stencil, then the bonded/local codes
 // or the cutoff, nbor.f:63-128); rows come in bead-index order.
-// Wavefront 0's area holds at least 24 * maxw bytes (its work lists, maxw >=
-// kMinMaxw); the staging takes 60 bytes per bead and its queue 512 bytes
-// after it.
-constexpr int kMinMaxw = 768;
+// The staging takes 60 bytes per bead of wavefront 0's scratch and its queue
+// 512 bytes after it.
 constexpr int kDenseN = 256;
 constexpr int kDenseQ = 128;  // queue ring: under 64 entries + one pass of 64
-static_assert(60 * kDenseN + 4 * kDenseQ <= 24 * kMinMaxw, "dense list staging exceeds wavefront 0's work area");
-static_assert(4 * kDenseQ <= 4 * kMinMaxw, "dense list queue exceeds a wavefront's work list");
+static_assert(60 * kDenseN + 4 * kDenseQ <= kScratch, "dense list staging exceeds wavefront 0's scratch");
 struct __attribute__((aligned(16))) Stage {
     double x, y, z;
     int topo, pad;
@@ -3760,12 +3639,13 @@ __device__ void rebuild_lists_dense(const SysDev&, const Lds&, Sc& c) {
     const int tid = (int)threadIdx.x, nthr = kW * nw;
     const int N = S.N, M = S.M, cap = S.cap;
     PH_BEGIN(trl);
-    unsigned char* const w0 = smem + reinterpret_cast<const Lds*>(smem + kLdOff)->o_wm;
+    const int nr = L.nwr;
+    unsigned char* const w0 = smem + L.o_pool;
     Stage* const stg = reinterpret_cast<Stage*>(w0);
     int4* const sovr = reinterpret_cast<int4*>(w0 + 32 * N);
     int2* const cnt = reinterpret_cast<int2*>(w0 + 48 * N);
     int* const sfine = reinterpret_cast<int*>(w0 + 56 * N);
-    int* const q = wave == 0 ? reinterpret_cast<int*>(w0 + 60 * N) : reinterpret_cast<int*>(smem + L.o_wm);
+    int* const q = wave == 0 ? reinterpret_cast<int*>(w0 + 60 * N) : reinterpret_cast<int*>(w0 + wave * kScratch);
     for (int k = tid; k < N; k += nthr) {
         const Rec b = gld(S.rec + (k));
         int cx = (int)((b.x + S.half) / S.width);
@@ -3784,7 +3664,7 @@ __device__ void rebuild_lists_dense(const SysDev&, const Lds&, Sc& c) {
         sovr[k] = gld(S.ovr + (k));
         sfine[k] = cx | (cy << 10) | (cz << 20);
     }
-    for (int i = wave + nw * lane; i < N; i += nw * kW) cnt[i] = make_int2(0, 0);
+    for (int i = tid; i < N; i += nthr) cnt[i] = make_int2(0, 0);
     wg_sync(nw);
     // fine cells and each bead's place in its fine cell's list (cell_add.f:
     // head first, the highest index at 1), for the rows' nbor.f order: lane
@@ -3859,7 +3739,7 @@ __device__ void rebuild_lists_dense(const SysDev&, const Lds&, Sc& c) {
         qh = (qh + nb) & (kDenseQ - 1);
         qn -= nb;
     };
-    for (int i = wave; i < N; i += nw) {
+    for (int i = wave; wave < nr && i < N; i += nr) {
         const int fi = sfine[i];
         const int ix = fi & 1023, iy = (fi >> 10) & 1023, iz = fi >> 20;
         for (int base = 0; base < N; base += kW) {
@@ -3882,7 +3762,7 @@ __device__ void rebuild_lists_dense(const SysDev&, const Lds&, Sc& c) {
     }
     while (qn > 0) drain();
     int mx = 0, status = 0;
-    for (int i = wave + nw * lane; i < N; i += nw * kW) {
+    for (int i = wave + nr * lane; wave < nr && i < N; i += nr * kW) {
         const int2 n2 = cnt[i];
         gs1(S.nup + (i), min(n2.x, cap));
         gs1(S.ndn + (i), min(n2.y, cap));
@@ -3898,7 +3778,7 @@ __device__ void rebuild_lists_dense(const SysDev&, const Lds&, Sc& c) {
 }
 
 // events.f:11-127 with tfalse = 0: every bead's next event, then the
-// calendar; all wavefronts of the system take part (the master scalars'
+// calendar (the pseudo-events' entries from Batch::pseudo); all wavefronts of the system take part (the master scalars'
 // scan position is at bin 1 already)
 __device__ void events_all(const SysDev&, const DevTables&, const Lds&, Sc&) {
     const Lds& L = ldsv();
@@ -3959,7 +3839,7 @@ __device__ void events_all(const SysDev&, const DevTables&, const Lds&, Sc&) {
         stamp_set(i, mk_stamp(c.coll, i + 1));  // events.f:111-122 adds in index order
     }
     for (int e = N + tid; e < N + 3; e += nthr) {
-        Leaf lf = leaf_get(L, e);
+        Leaf lf = L.batch()->pseudo[e - N];
         lf.meta = make_meta(calc_bin(c, lf.tim, false, status), -2);
         leaf_set(L, e, lf);
         stamp_set(e, mk_stamp(c.coll, e + 1));
@@ -3975,21 +3855,21 @@ __device__ void events_all(const SysDev&, const DevTables&, const Lds&, Sc&) {
 // is the one eventredo_up.f's strict < takes in nbor.f's row, and down
 // rows are walked in partial_events.f's order.  One lane per row (row r:
 // bead r / 2, its up row for even r, its down row for odd r): the row's
-// entries and keys in the wavefront's work area (kSortMax each per lane,
+// entries and keys in the wavefront's scratch (kSortMax each per lane,
 // [slot][lane]), the row in up to five 16-byte loads and all its partner
 // loads in flight, then every entry written at its rank; a longer row is
 // sorted by the whole wavefront, one lane per entry.
 constexpr int kSortMax = 20;
-static_assert(12 * kSortMax * kW <= 20 * kMinMaxw, "row sort staging exceeds a wavefront's work area");
+static_assert(12 * kSortMax * kW <= kScratch, "row sort staging exceeds the rebuild scratch");
 __device__ void sort_rows(const SysDev&, const DevTables&, const Lds&) {
     const Lds& L = ldsv();
     const SysDev& S = sdev();
     const DevTables& T = tabs();
     const int lane = lane_id(), wave = wave_id(), nw = L.nw, N = S.N, cap = S.cap, M = S.M;
-    unsigned long long* const keys = reinterpret_cast<unsigned long long*>(smem + L.o_wm);  // [kSortMax][kW]
+    unsigned long long* const keys = reinterpret_cast<unsigned long long*>(smem + L.o_pool + wave * kScratch);  // [kSortMax][kW]
     int* const ents = reinterpret_cast<int*>(keys + kSortMax * kW);                        // [kSortMax][kW]
     const bool vec = (cap & 3) == 0;  // rows of whole int4s (row bases are 16-byte aligned)
-    for (int r0 = wave * kW; r0 < 2 * N; r0 += nw * kW) {
+    for (int r0 = wave * kW; wave < L.nwr && r0 < 2 * N; r0 += L.nwr * kW) {
         const int r = r0 + lane;
         const bool act = r < 2 * N;
         const int x = act ? r >> 1 : 0;
@@ -4069,6 +3949,7 @@ __device__ void wrap_and_lists(const SysDev&, const Lds&, Sc&) {
 
     const int tid = (int)threadIdx.x, nthr = kW * L.nw;
     if (tid == 0) c.nbin = 1;
+    if (tid < 3) L.batch()->pseudo[tid] = leaf_get(L, S.N + tid);
     for (int k = tid; k < S.N; k += nthr) {
         Rec b = gld(S.rec + (k));
         b.x = b.x - round(b.x);
@@ -4095,6 +3976,9 @@ __device__ void rebuild(const SysDev&, const DevTables&, const Lds&, Sc&) {
     wrap_and_lists(S, L, c);
     PH_END(S, kPhLists, trb);
     events_all(S, T, L, c);
+    // the scratch lay over the round's footprint marks too
+    if (L.mark_lds)
+        for (int b = (int)threadIdx.x; b < S.N; b += kW * L.nw) L.mark[b] = 0u;
     PH_END(S, kPhEvents, trb);
     PH_COUNT(S, kPhNRebuild);
 }
@@ -4232,12 +4116,26 @@ __device__ void output_event(const SysDev&, const Lds&, Sc&) {
 }
 
 // LDS plan: tables, SysDev, the views, the superblock minima, master
-// scalars and round record, then each wavefront's work area (wavefront 0's
-// is the larger: the list rebuild and the generic rescheduling use it as
-// scratch; its scalars are the master copy), then this system's block
-// minima, then as many calendar leaves as the workgroup's lds_bytes hold:
-// a small system in a launch sized for a large one keeps all its leaves in
-// LDS
+// scalars and round record; each wavefront's one-pass work area, block list
+// and pair, wavefront 0's with the multi-pass form's work lists after them;
+// then this system's block minima, then as many calendar leaves as the
+// workgroup's lds_bytes hold: a small system in a launch sized for a large
+// one keeps all its leaves in LDS.  Everything from the work areas on is
+// also the scratch pool of a list rebuild.  One set of work lists (15 KB)
+// instead of one per wavefront (25 KB each) leaves room for eight
+// wavefronts at every size: only an event of more than 62 predictions needs
+// them, and such an event runs as the first of its round.
+__device__ __host__ inline int lds_wave_bytes() {
+    return (int)((sizeof(OnePass) + 15) / 16 * 16 + sizeof(int) * kMaxBlist + (sizeof(Pair) + 15) / 16 * 16);
+}
+__device__ __host__ inline int lds_multi_bytes(int maxw) {
+    return (4 * maxw + 15) / 16 * 16 * 3 + (8 * maxw + 15) / 16 * 16 + 64 +
+           (int)(sizeof(MinSlot) * (2 + kMaxSpec) + sizeof(SpecInfo) * kMaxSpec + sizeof(DownInfo) * kW);
+}
+constexpr int kPoolOff = kBatchOff + (int)((sizeof(Batch) + 15) / 16 * 16);
+static_assert(sizeof(MinSlot) % 16 == 0 && sizeof(SpecInfo) % 16 == 0 && sizeof(DownInfo) % 16 == 0 &&
+                  sizeof(int) * kMaxBlist % 16 == 0,
+              "work areas are whole 16-byte units");
 __device__ Lds make_lds(const SysDev&, int maxw, int lds_bytes, int nw, int wave) {
     const SysDev& S = sdev();
 
@@ -4247,44 +4145,29 @@ __device__ Lds make_lds(const SysDev&, int maxw, int lds_bytes, int nw, int wave
     L.nsup = (L.nblk + kSup - 1) / kSup;
     L.maxw = maxw;
     L.nw = nw;
-    int p = 0;
+    L.o_sup = kSupOff;
+    L.o_msc = kMscOff;
+    L.o_batch = kBatchOff;
+    L.o_pool = kPoolOff;
+    int p = kPoolOff + wave * lds_wave_bytes();
     auto take = [&](int bytes) {
         const int o = p;
         p = (p + bytes + 15) / 16 * 16;
         return o;
     };
-    take((int)sizeof(DevTables));        // the tables, at offset 0
-    take((int)sizeof(SysDev));           // the system's SysDev, at kSdOff
-    take(kLdStride * kMaxWaves);         // these views, at kLdOff
-    L.o_sup = take((int)sizeof(Key) * kSup);
-    L.o_msc = take((int)sizeof(Sc));
-    L.o_batch = take((int)sizeof(Batch));
-    for (int w = 0; w <= wave; ++w) {
-        L.o_wm = take((int)sizeof(int) * maxw);
-        L.o_wx = take((int)sizeof(int) * maxw);
-        L.o_blist = take((int)sizeof(int) * kMaxBlist);
-        L.o_wd = take((int)sizeof(int) * (w == 0 ? maxw : 16));
-        L.o_wy = take((int)sizeof(int) * maxw);
-        L.o_wt = take((int)sizeof(double) * maxw);
-        L.o_slot = take((int)sizeof(MinSlot) * (2 + kMaxSpec));
-        L.o_spec = take((int)sizeof(SpecInfo) * kMaxSpec);
-        L.o_down = take((int)sizeof(DownInfo) * kW);
-        L.o_pair = take((int)sizeof(Pair));
-        L.o_sc = w == 0 ? L.o_msc : take((int)sizeof(Sc));
-    }
-    for (int w = wave + 1; w < nw; ++w) {
-        take((int)sizeof(int) * maxw);
-        take((int)sizeof(int) * maxw);
-        take((int)sizeof(int) * kMaxBlist);
-        take((int)sizeof(int) * 16);
-        take((int)sizeof(int) * maxw);
-        take((int)sizeof(double) * maxw);
-        take((int)sizeof(MinSlot) * (2 + kMaxSpec));
-        take((int)sizeof(SpecInfo) * kMaxSpec);
-        take((int)sizeof(DownInfo) * kW);
-        take((int)sizeof(Pair));
-        take((int)sizeof(Sc));
-    }
+    L.o_one = take((int)sizeof(OnePass));
+    L.o_blist = take((int)sizeof(int) * kMaxBlist);
+    L.o_pair = take((int)sizeof(Pair));
+    p = kPoolOff + nw * lds_wave_bytes();
+    L.o_wm = take((int)sizeof(int) * maxw);
+    L.o_wx = take((int)sizeof(int) * maxw);
+    L.o_wy = take((int)sizeof(int) * maxw);
+    L.o_wt = take((int)sizeof(double) * maxw);
+    L.o_wd = take(64);
+    L.o_slot = take((int)sizeof(MinSlot) * (2 + kMaxSpec));
+    L.o_spec = take((int)sizeof(SpecInfo) * kMaxSpec);
+    L.o_down = take((int)sizeof(DownInfo) * kW);
+    L.o_sc = kMscOff;
     L.o_blk = take((int)sizeof(Key) * L.nblk);
     L.o_leaf = p;
     L.leaf_lds = N3 <= (lds_bytes - p) / (int)sizeof(Leaf);
@@ -4294,6 +4177,9 @@ __device__ Lds make_lds(const SysDev&, int maxw, int lds_bytes, int nw, int wave
     L.mark_lds = L.leaf_lds && o_mark + 4 * S.N <= lds_bytes;
     L.o_mark = o_mark;
     L.mark = L.mark_lds ? reinterpret_cast<unsigned*>(smem + o_mark) : S.mark;
+    // the rebuild kernels' launches (lds_bytes 0) hold every wavefront's scratch
+    const int room = lds_bytes > 0 ? (lds_bytes - kPoolOff) / kScratch : nw;
+    L.nwr = room < nw ? room : nw;
     return L;
 }
 
@@ -4465,6 +4351,8 @@ __global__ __launch_bounds__(64 * kSetupWaves) void k_rebuild_events(const SysDe
     const SysDev& S = sdev();
     const Lds& L = ldsv();
     Sc& c = *L.msc();
+    if (threadIdx.x < 3) L.batch()->pseudo[threadIdx.x] = gld(S.leaf + (S.N + (int)threadIdx.x));
+    __syncthreads();
     events_all(S, tabs(), L, c);
     __syncthreads();
     if (threadIdx.x == 0) store_sc(S.st, c);
@@ -5039,40 +4927,39 @@ __global__ void k_predict(const SysDev* sys, int id, int n, const int* pi, const
     type[k] = ty;
 }
 
-// also sized for the list rebuild's per-lane cell ranges (27 x 64 int2 over
-// the work-list arrays)
-int engine_maxw(int cap) { return max((4 + kMaxSpec) * (cap + 3), kMinMaxw); }
+// predictions of i and j in full, their down sets and a share of the beads
+// recomputed (one that finds no room is recomputed on its own)
+int engine_maxw(int cap) { return 6 * (cap + 3); }
 
 static size_t r16(size_t b) { return (b + 15) / 16 * 16; }
-// the bytes make_lds lays out before the leaves, for nw wavefronts
+// the bytes make_lds lays out before the leaves, for nw wavefronts; at
+// least one wavefront's rebuild scratch
 static size_t lds_fixed(int nblk_max, int maxw, int nw) {
-    size_t b = r16(sizeof(DevTables)) + r16(sizeof(SysDev)) + (size_t)kLdStride * kMaxWaves +
-               r16(sizeof(Key) * nblk_max) + r16(sizeof(Key) * kSup) + r16(sizeof(Sc)) + r16(sizeof(Batch));
-    const size_t common = 3 * r16(sizeof(int) * maxw) + r16(sizeof(int) * kMaxBlist) + r16(sizeof(double) * maxw) +
-                          r16(sizeof(MinSlot) * (2 + kMaxSpec)) + r16(sizeof(SpecInfo) * kMaxSpec) +
-                          r16(sizeof(DownInfo) * kW) + r16(sizeof(Pair));
-    b += common + r16(sizeof(int) * maxw);                                          // wavefront 0
-    b += (size_t)(nw - 1) * (common + r16(sizeof(int) * 16) + r16(sizeof(Sc)));   // the others
-    return b;
+    const size_t b = (size_t)kPoolOff + (size_t)nw * lds_wave_bytes() + lds_multi_bytes(maxw) + r16(sizeof(Key) * nblk_max);
+    return std::max(b, (size_t)kPoolOff + kScratch);
 }
 size_t engine_lds_bytes(int nblk_max, int maxw, int leaf_cap, int nw) {
     return lds_fixed(nblk_max, maxw, nw) + sizeof(Leaf) * (size_t)leaf_cap;
+}
+// the rebuild kernels: scratch for every wavefront, no leaves
+static size_t lds_rebuild(int nblk_max, int maxw, int nw) {
+    return std::max(lds_fixed(nblk_max, maxw, nw), (size_t)kPoolOff + (size_t)nw * kScratch);
 }
 static int nblk_for(int n) { return (n + 3 + kBlk - 1) / kBlk; }
 
 hipError_t engine_setup(const SysDev* d_sys, const int* d_ids, int n, int max_n, int maxw, size_t lds_limit,
                         hipStream_t s) {
     int nw = kSetupWaves;
-    while (nw > 1 && engine_lds_bytes(nblk_for(max_n), maxw, 0, nw) > lds_limit) --nw;
-    const size_t lds = engine_lds_bytes(nblk_for(max_n), maxw, 0, nw);
+    while (nw > 1 && lds_rebuild(nblk_for(max_n), maxw, nw) > lds_limit) --nw;
+    const size_t lds = lds_rebuild(nblk_for(max_n), maxw, nw);
     hipLaunchKernelGGL(k_setup, dim3(n), dim3(kW * nw), lds, s, d_sys, d_ids, maxw);
     return hipGetLastError();
 }
 hipError_t engine_rebuild(const SysDev* d_sys, const int* d_ids, int n, int max_n, int maxw, size_t lds_limit,
                           hipStream_t s) {
     int nw = kSetupWaves;
-    while (nw > 1 && engine_lds_bytes(nblk_for(max_n), maxw, 0, nw) > lds_limit) --nw;
-    const size_t lds = engine_lds_bytes(nblk_for(max_n), maxw, 0, nw);
+    while (nw > 1 && lds_rebuild(nblk_for(max_n), maxw, nw) > lds_limit) --nw;
+    const size_t lds = lds_rebuild(nblk_for(max_n), maxw, nw);
     hipLaunchKernelGGL(k_rebuild_lists, dim3(n), dim3(kW * nw), lds, s, d_sys, d_ids, maxw);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
