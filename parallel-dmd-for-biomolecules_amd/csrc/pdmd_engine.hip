@@ -697,6 +697,9 @@ __device__ inline unsigned long long t_order(double t) {
 }
 
 
+// lanes of the selection: candidates from the tree, then the committed
+// events' new entries, then up to 8 popped entries that were not committed
+constexpr int kCandMax = 24, kFreshMax = 32;
 // One round of a multi-wavefront system: the popped calendar entries (in
 // key order, one per wavefront) and what each wavefront reports back.
 struct Batch {
@@ -704,7 +707,7 @@ struct Batch {
     Key knew[kMaxWaves];  // least key among the wavefront's new calendar entries
     unsigned long long knew_st[kMaxWaves];  // its add stamp
     int ty[kMaxWaves];    // resolved type of each event
-    int nbl[kMaxWaves];   // blocks to rescan, in each wavefront's list
+    int nbl;              // blocks to rescan in wavefront 0's list (multi-pass forms)
     int st[kMaxWaves];    // status after each event
     int wdone[kMaxWaves]; // the wavefront's committed entries are written
     int st_rep[kMaxWaves];  // status of its replayed updates
@@ -712,6 +715,22 @@ struct Batch {
     int cut;              // first wavefront whose event is not committed
     int rebuild;          // the round's sync event rebuilds the lists
     unsigned long long touched;  // superblocks with a changed block minimum (bit s)
+    // The pool the next round is selected from: every calendar entry whose
+    // proxy lies below `edge` and that the round in flight has not popped is
+    // in cand (as of the round's start) or, rewritten by a committed event
+    // of the round, in that event's wavefront's share of fresh.
+    double edge;
+    double width;                // time the edge lies ahead of the round's last event
+    int ncand;
+    int full;                    // the pool is not complete: collect it again before selecting
+    int nfresh[kMaxWaves];
+    int order[kMaxWaves];        // lane of the entry of each rank (selection)
+    Key cand[kCandMax];
+    Key fresh[kFreshMax];
+    // blocks with rewritten entries, a bit per block and a word per
+    // superblock, by the round's parity: one is written while the other is
+    // worked off
+    unsigned long long dirty[2][kSup];
     int gbead;            // the bead of a ghost event leading the round
     long long t0;         // start of a budgeted launch (wall_clock64)
     Leaf pseudo[3];       // the ghost, sync and output entries across a list rebuild
@@ -1019,11 +1038,19 @@ __device__ inline void stamp_st(const Hot& H, int k, unsigned long long v) {
                        __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Block minima of the listed blocks after a round, one row of 16 lanes per
-// block, 16 blocks per step so that four independent reductions overlap.  A
-// block whose minimum came out as it was is not written and leaves its
-// superblock alone; the others mark theirs in Batch::touched.
-__device__ inline void rescan_round(const Hot& H, const int* list, int nb) {
+__device__ inline void dirty_or(int par, int blk) {
+    __hip_atomic_fetch_or(&round_rec().dirty[par][blk / kSup], 1ull << (blk & (kSup - 1)), __ATOMIC_RELAXED,
+                          __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ inline unsigned long long readlane_u64(unsigned long long v, int l) {
+    return (unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)v, l) |
+           ((unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(v >> 32), l) << 32);
+}
+// Block minima of the listed blocks, one row of 16 lanes per block, 16
+// blocks per step so that four independent reductions overlap.  A block
+// whose minimum came out as it was is not written and leaves its superblock
+// alone; the others mark theirs in Batch::touched.
+__device__ inline void rescan_listed(const Hot& H, const int* list, int nb) {
     const int lane = lane_id(), N3 = H.N + 3;
     Key* const blk = reinterpret_cast<Key*>(smem + H.o_blk);
     for (int base = 0; base < nb; base += 16) {
@@ -1071,80 +1098,143 @@ __device__ inline void rescan_round(const Hot& H, const int* list, int nb) {
             }
     }
 }
-// Superblock minima of the round's touched superblocks, shared out over the
-// nw wavefronts.
-__device__ inline void rescan_touched(const Hot& H, int wave, int nw) {
+constexpr int kListMax = 512;  // blocks of a work list (one wavefront's one-pass area)
+// Adds the blocks of superblock s in mask to the list.
+__device__ inline int list_blocks(int* list, int n, int s, unsigned long long mask) {
     const int lane = lane_id();
+    if ((mask >> lane) & 1ull) list[n + __popcll(mask & ((1ull << lane) - 1ull))] = s * kSup + lane;
+    return n + __popcll(mask);
+}
+// The min tree after the entries of the blocks in Batch::dirty[par] changed
+// (one wavefront; the mask is cleared).
+__device__ inline void tree_update(const Hot& H, int par, int* list) {
+    const int lane = lane_id();
+    Batch& B = round_rec();
+    unsigned long long d = 0;
+    if (lane < H.nsup) {
+        d = B.dirty[par][lane];
+        B.dirty[par][lane] = 0;
+    }
+    unsigned long long sm = __ballot(d != 0);
+    if (!sm) return;
+    if (lane == 0) B.touched = 0;
+    int n = 0;
+    while (sm) {
+        const int s = __ffsll((long long)sm) - 1;
+        sm &= sm - 1;
+        n = list_blocks(list, n, s, readlane_u64(d, s));
+        if (n > kListMax - kSup || !sm) {
+            wave_sync();
+            rescan_listed(H, list, n);
+            wave_sync();
+            n = 0;
+        }
+    }
+    if (H.nsup == 1) return;  // a single superblock is never read: the block minima fit one wavefront
     const Key* const blk = reinterpret_cast<const Key*>(smem + H.o_blk);
     Key* const sup = reinterpret_cast<Key*>(smem + kSupOff);
-    const unsigned long long tv = round_rec().touched;
+    const unsigned long long tv = B.touched;
     unsigned long long touched = (unsigned long long)(unsigned)uni((int)tv) | ((unsigned long long)(unsigned)uni((int)(tv >> 32)) << 32);
-    int turn = 0;
     while (touched) {
         const int s = __ffsll((long long)touched) - 1;
         touched &= touched - 1;
-        const bool mine = turn == wave;
-        turn = turn + 1 == nw ? 0 : turn + 1;
-        if (!mine) continue;
         const int b = s * kSup + lane;
         const Key e = key_min_wave(b < H.nblk ? blk[b] : empty_key());
         if (lane == 0) sup[s] = e;
     }
+    wave_sync();
 }
-
-// block minima of the listed blocks (4 blocks per pass, one row of 16 lanes
-// each); a block listed twice gets the same value twice
-__device__ void rescan_blocks(const Lds&, int N3, const int* list, int nb) {
-    const Lds L = lds_regs();
-
-    const int lane = lane_id(), k = lane & 15;
-    // 16 blocks per step: the leaf loads of four passes are in flight together
-    for (int base = 0; base < nb; base += 16) {
-        Key e[4];
-        int bq[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int q = base + 4 * u + (lane >> 4);
-            bq[u] = q < nb ? list[q] : -1;
-            const int idx = bq[u] * kBlk + k;
-            e[u] = empty_key();
-            if (bq[u] >= 0 && idx < N3) e[u] = leaf_key(leaf_get(L, idx), idx);
+// The pool of the next selection from the up-to-date min tree (one
+// wavefront): every entry whose proxy lies below an edge, the K entries
+// popped by the round in flight left out.  The edge lies Batch::width after
+// t0; the width follows the density of events so that the pool holds a few
+// more entries than a round takes (`want`), tried again up to `tries` times.
+// Left with too many entries for the pool, it is empty (edge 0: nothing lies
+// below it).
+__device__ inline void collect_pool(const Hot& H, int K, double t0, int want, int tries, int* list) {
+    const int lane = lane_id(), N3 = H.N + 3;
+    Batch& B = round_rec();
+    const Sc& c = master();
+    const Key* const blk = reinterpret_cast<const Key*>(smem + H.o_blk);
+    const Key* const sup = reinterpret_cast<const Key*>(smem + kSupOff);
+    const double off = c.tbin_off, sortsize = c.sortsize, imax = c.interval_max;
+    double w = B.width;
+    const int pidx = lane < K ? key_idx(B.key[lane & (kMaxWaves - 1)]) : -1;
+    int count = 0;
+    double edge = 0.0;
+    for (int tr = 0; tr < tries; ++tr) {
+        Key ek;
+        ek.t = t0 + w;
+        const int bin = (int)min((ek.t + off) / sortsize, (double)kNumbin) + 1;
+        ek.bc = min(max(bin, 1), kNumbin) << 8;
+        ek.ip = 0;
+        edge = key_proxy(ek);
+        // blocks with a minimum below the edge
+        int n = 0;
+        bool many = false;
+        if (H.nsup == 1) {
+            n = list_blocks(list, 0, 0, __ballot(lane < H.nblk && key_proxy(blk[lane]) < edge));
+        } else {
+            unsigned long long sm = __ballot(lane < H.nsup && key_proxy(sup[lane]) < edge);
+            while (sm && !many) {
+                const int s = __ffsll((long long)sm) - 1;
+                sm &= sm - 1;
+                const int b = s * kSup + lane;
+                n = list_blocks(list, n, s, __ballot(b < H.nblk && key_proxy(blk[b]) < edge));
+                many = n > kListMax - kSup;
+            }
         }
+        wave_sync();
+        // their entries below it
+        count = 0;
+        for (int base = 0; base < n && !many; base += 16) {
+            Key e[4];
+            double p[4];
+            int idx[4];
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
-            if (base + 4 * u < nb && key_min_rows(e[u]) && bq[u] >= 0) L.blk()[bq[u]] = e[u];
+            for (int u = 0; u < 4; ++u) {
+                const int q = base + 4 * u + (lane >> 4);
+                idx[u] = (q < n ? list[q] : H.nblk) * kBlk + (lane & 15);
+                e[u] = empty_key();
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (idx[u] < N3) e[u] = leaf_key(leaf_ld(H, idx[u]), idx[u]);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) p[u] = key_proxy(e[u]);
+            for (int q = 0; q < K; ++q) {
+                const int pq = __builtin_amdgcn_readlane(pidx, q);
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    if (idx[u] == pq) p[u] = __hiloint2double(kInfHi, 0);
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const unsigned long long m = __ballot(p[u] < edge);
+                const int pos = count + __popcll(m & ((1ull << lane) - 1ull));
+                if (p[u] < edge && pos < kCandMax) B.cand[pos] = e[u];
+                count += __popcll(m);
+            }
+            many = count > kCandMax;
+        }
+        if (many) {
+            w *= 0.5;
+            count = kCandMax + 1;
+        } else if (count < want && ek.t < imax) {
+            w *= count == 0 ? 4.0 : 1.6;
+        } else {
+            if (count > want + 6) w *= 0.9;
+            break;
+        }
     }
-}
-// superblock minima over the superblocks of the listed blocks (at most 64),
-// each reduced once
-__device__ void rescan_sups(const Lds&, const int* list, int nb) {
-    const Lds L = lds_regs();
-
-    const int lane = lane_id();
-    unsigned long long touched = 0;
-    for (int base = 0; base < nb; base += kW) {
-        const int q = base + lane;
-        const int sq = q < nb ? list[q] / kSup : 0;
-        const int nr = min(nb - base, kW);
-        for (int r = 0; r < nr; ++r) touched |= 1ull << __builtin_amdgcn_readlane(sq, r);
+    if (lane == 0) {
+        B.width = w;
+        B.ncand = count > kCandMax ? 0 : count;
+        B.edge = count > kCandMax ? 0.0 : edge;
     }
-    while (touched) {
-        const int s = __ffsll((long long)touched) - 1;
-        touched &= touched - 1;
-        const int b = s * kSup + lane;
-        const Key e = key_min_wave(b < L.nblk ? L.blk()[b] : empty_key());
-        if (lane == 0) L.sup()[s] = e;
-    }
-}
-// both levels for the wavefront's block list
-__device__ void rescan_block_list(const Lds&, int N3, int nb) {
-    const Lds& L = ldsv();
-
-    rescan_blocks(L, N3, L.blist(), nb);
     wave_sync();
-    rescan_sups(L, L.blist(), nb);
-    wave_sync();
 }
+
 // every block and superblock minimum; all wavefronts of the system take part
 __device__ void rescan_all(const Lds&, int N3) {
     const Lds& L = ldsv();
@@ -1687,7 +1777,7 @@ __device__ void reschedule_generic(const SysDev&, const DevTables&, const Lds&, 
         wave_sync_mem();
     else
         wave_sync();
-    if (lane == 0) L.batch()->nbl[0] = nbl;
+    if (lane == 0) L.batch()->nbl = nbl;
     PH_END(S, kPhLeaf, tph);
 }
 
@@ -2268,7 +2358,7 @@ __device__ __noinline__ void reschedule(const SysDev&, const DevTables&, const L
         // the flag
         wave_sync_mem();
         if (lane == 0) {
-            L.batch()->nbl[0] = nbl;
+            L.batch()->nbl = nbl;
             __hip_atomic_store(&L.batch()->wdone[0], 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
         }
         return;
@@ -2277,7 +2367,7 @@ __device__ __noinline__ void reschedule(const SysDev&, const DevTables&, const L
         wave_sync_mem();
     } else
         wave_sync();
-    if (lane == 0) L.batch()->nbl[0] = nbl;
+    if (lane == 0) L.batch()->nbl = nbl;
     PH_END(S, kPhLeaf, tph);
 }
 
@@ -2558,9 +2648,13 @@ __device__ inline void fp_clear(const Hot& H, int b) {
 // main.F90:641-921) or an Andersen ghost collision (main.F90:997-1049),
 // then partial_events.f:16-201 for it.
 // e: the calendar entry; jp, ct: its partner and type; tf, nbin, coll: the
-// false time, bin and number of the event; bk: its place in the round (-1:
-// the round's only entry).  Returns the round's accepted events if this one
-// is committed (1 alone), else 0.
+// false time, bin and number of the event; bk: its place in the round.
+// Returns the round's accepted events if this one is committed, else 0.
+//
+// solo: the round's only event, which needs no footprint marks and no
+// acceptance.  The new calendar entries below the pool's edge go to the
+// wavefront's share of Batch::fresh and the rewritten blocks to
+// Batch::dirty[par].
 //
 // The rescheduling takes one pass of 64 lanes: a lane per candidate of i
 // and j (tags 0 and 1), per down-set entry (tags 2 and 3: its op partner i
@@ -2574,13 +2668,14 @@ __device__ inline void fp_clear(const Hot& H, int b) {
 // runs the multi-pass form, which holds any number.  What bounds an event
 // is the length of its dependent chain, so the code keeps wave-uniform
 // values in scalar registers and replaces divergent branches by selects.
-__device__ __forceinline__ int run_event(const Hot& H, int e, int jp, int ct, double tf, int nbin, long long coll, int bk) {
+__device__ __forceinline__ int run_event(const Hot& H, int e, int jp, int ct, double tf, int nbin, long long coll, int bk,
+                                         bool solo, int par, int fsh) {
     const int lane = lane_id();
     const DevTables& T = tabs();
     Sc& mc = master();
     Batch& B = round_rec();
     const double interval_max = mc.interval_max, tbin_off = mc.tbin_off, sortsize = mc.sortsize;
-    const bool batch = bk >= 0;
+    const bool batch = !solo;
     int i = e, j = -1, flags = 0, st0 = 0, nb = 0, extra_blk = -1;
     bool xdel = false;
     Rec ri, rj;
@@ -2839,8 +2934,7 @@ __device__ __forceinline__ int run_event(const Hot& H, int e, int jp, int ct, do
         wave_sync();
         PH_END(sdev(), kPhGhost, tph);
     }
-    if (lane == 0 && batch) B.ty[bk] = ct;
-    if (lane == 0 && !batch) B.ty[0] = ct;
+    if (lane == 0) B.ty[bk] = ct;
 
     OnePass& W = *reinterpret_cast<OnePass*>(smem + H.o_w);
     const unsigned long long below = (1ull << lane) - 1ull;
@@ -3039,8 +3133,15 @@ __device__ __forceinline__ int run_event(const Hot& H, int e, int jp, int ct, do
         }
         if (lane == 0 && st0 && !mc.status) mc.status = st0;
         wave_sync();
-        reschedule(sdev(), T, L, *L.sc(), *L.pair(), extra_blk, xdel, bk);
-        if (lane == 0) B.st_rep[0] = 0;
+        reschedule(sdev(), T, L, *L.sc(), *L.pair(), extra_blk, xdel, batch ? 0 : -1);
+        if (solo) bar_to(nb, 1);
+        // its new entries are not offered to the pool
+        for (int q = lane; q < B.nbl; q += kW) dirty_or(par, L.blist()[q]);
+        if (lane == 0) {
+            B.full = 1;
+            if (solo) B.st[0] = 0;
+            B.st_rep[0] = 0;
+        }
         return batch ? accepted(B) : 1;
     }
     wave_sync();
@@ -3288,10 +3389,13 @@ __device__ __forceinline__ int run_event(const Hot& H, int e, int jp, int ct, do
             if (lane == 1) st_at(H.rec, j, rj);
         }
         if (bk == 0 && st0 && lane == 0 && !mc.status) mc.status = st0;
-    } else if (lane == 0) {
-        B.st[0] = 0;
-        B.st_rep[0] = 0;
-        if (st0 && !mc.status) mc.status = st0;
+    } else {
+        if (lane == 0) {
+            B.st[0] = 0;
+            B.st_rep[0] = 0;
+            if (st0 && !mc.status) mc.status = st0;
+        }
+        bar_to(nb, 1);  // the pool's edge is known
     }
     bool wb = wr;  // the lane's bead takes a new entry (its block is rescanned)
     if (__ballot(rep >= 0)) {
@@ -3328,15 +3432,23 @@ __device__ __forceinline__ int run_event(const Hot& H, int e, int jp, int ct, do
         stamp_st(H, rb, stp);
     }
     {
-        int* const bl = reinterpret_cast<int*>(smem + H.o_blist);
-        const unsigned long long mm = __ballot(wb);
-        int n = __popcll(mm);
-        if (wb) bl[__popcll(mm & below)] = rb / kBlk;
-        if (extra_blk >= 0) {
-            if (lane == 0) bl[n] = extra_blk;
-            ++n;
+        Key kx = wb ? leaf_key(lf, rb) : empty_key();
+        bool put = wb;
+        int blk_ = rb / kBlk;
+        if (extra_blk >= 0 && lane == kLaneJ) {  // the ghost entry
+            kx = leaf_key(leaf_ld(H, H.N), H.N);
+            put = true;
+            blk_ = extra_blk;
         }
-        if (lane == 0) B.nbl[batch ? bk : 0] = n;
+        if (put) dirty_or(par, blk_);
+        const bool near = key_proxy(kx) < B.edge;
+        const unsigned long long nm = __ballot(near);
+        const int n = __popcll(nm), cap_f = 1 << fsh, pos = __popcll(nm & below);
+        if (near && pos < cap_f) B.fresh[(bk << fsh) + pos] = kx;
+        if (lane == 0) {
+            B.nfresh[bk] = min(n, cap_f);
+            if (n > cap_f) B.full = 1;
+        }
     }
     // repuls_del_b.f once the rescheduling is done
     if (xdel && lane == 0) {
@@ -4076,14 +4188,9 @@ __device__ void sync_finish(const SysDev&, const Lds&, Sc&) {
         lf.meta = make_meta(calc_bin(c, t2, true, status), -2);
         leaf_set(L, N + 1, lf);
         stamp_set(N + 1, mk_stamp(c.coll, N + 4));  // after a rebuild's events() adds
-        L.blist()[0] = (N + 1) / kBlk;
     }
     if (status && !c.status) c.status = status;
-    if (!L.leaf_lds)
-        wave_sync_mem();
-    else
-        wave_sync();
-    rescan_block_list(L, N + 3, 1);
+    wave_sync_mem();
     PH_END(S, kPhSync, tsy);
 }
 
@@ -4105,14 +4212,9 @@ __device__ void output_event(const SysDev&, const Lds&, Sc&) {
         lf.meta = make_meta(calc_bin(c, t3, false, status), -2);
         leaf_set(L, N + 2, lf);
         stamp_set(N + 2, mk_stamp(c.coll, 1));
-        L.blist()[0] = (N + 2) / kBlk;
     }
     if (status && !c.status) c.status = status;
-    if (!L.leaf_lds)
-        wave_sync_mem();
-    else
-        wave_sync();
-    rescan_block_list(L, N + 3, 1);
+    wave_sync_mem();
 }
 
 // LDS plan: tables, SysDev, the views, the superblock minima, master
@@ -4358,102 +4460,131 @@ __global__ __launch_bounds__(64 * kSetupWaves) void k_rebuild_events(const SysDe
     if (threadIdx.x == 0) store_sc(S.st, c);
 }
 
-// Pop up to kmax calendar entries in key order (wavefront 0): pair events
-// only after the first, since a pseudo-event runs alone.  Each popped entry
-// but the last is taken out of the min tree until the round's rescans.  The
-// master takes the first event's bin, time and number.  Returns the number
-// popped (0: stop, or an empty calendar).
+// Takes up to kmax entries from the pool in key order (wavefront 0): the
+// tree's candidates, the new entries of the last round's committed events
+// and its popped entries that were not committed (B.key[A] to B.key[Kp - 1]).
+// An entry whose key is no longer its leaf's was rewritten meanwhile and is
+// dropped.  Pair events only after the first, since a pseudo-event runs
+// alone; a ghost event may lead a round (its draws come first in the serial
+// order).  Returns the number taken, 0 if the pool is empty.
 //
-// A pop is a dependent chain (wave minimum, the popped entry's block minimum
-// without it, for larger calendars its superblock's), so the top level and
-// its proxies stay in lane registers and only the popped entry's block is
-// read from LDS.
-__device__ __forceinline__ int select_batch(const Hot& H, Sc& c, int kmax) {
+// Every lane counts the proxies below its own, so one sweep over the
+// entries (about a dozen) orders all of them; popping a round's entries one
+// by one from the min tree took 2 200 cycles each.
+__device__ __forceinline__ int select_pool(const Hot& H, int kmax, int A, int Kp, int ne, int fsh) {
+    Batch& B = round_rec();
+    const int lane = lane_id(), N = H.N;
+    Key k = empty_key();
+    bool have = false;
+    const int f = lane - kCandMax, q = A + lane - (kCandMax + kFreshMax);
+    if (lane < kCandMax) {
+        have = lane < B.ncand;
+        k = B.cand[lane];
+    } else if (f < kFreshMax) {
+        const int w = f >> fsh;
+        have = w < ne && (f & ((1 << fsh) - 1)) < B.nfresh[min(w, kMaxWaves - 1)];
+        k = B.fresh[f];
+    } else {
+        have = q < Kp;
+        k = B.key[min(q, kMaxWaves - 1)];
+    }
+    const int idx = key_idx(k);
+    const double pk = key_proxy(k);
+    have = have && pk < B.edge;
+    if (have) {
+        const Key now = leaf_key(leaf_ld(H, idx), idx);
+        have = now.t == k.t && now.bc == k.bc && now.ip == k.ip;
+    }
+    // an entry rewritten with an equal key stands in fresh and elsewhere
+    const bool isf = lane >= kCandMax && lane < kCandMax + kFreshMax;
+    unsigned long long fm = __ballot(have && isf);
+    while (fm) {
+        const int s = __ffsll((long long)fm) - 1;
+        fm &= fm - 1;
+        if (idx == __builtin_amdgcn_readlane(idx, s) && lane != s) have = have && isf && lane < s;
+    }
+    const double p = have ? pk : __hiloint2double(kInfHi, 0);
+    const unsigned long long vm = __ballot(have);
+    const int n = __popcll(vm);
+    if (n == 0) return 0;
+    int rank = 0;
+    unsigned long long sm = vm;
+    while (sm) {
+        const int s = __ffsll((long long)sm) - 1;
+        sm &= sm - 1;
+        rank += readlane_d(p, s) < p ? 1 : 0;
+    }
+    const int last = kmax < kMaxWaves ? kmax : kMaxWaves - 1;
+    if (have && rank <= last) B.order[rank] = lane;
+    wave_sync();
+    if (__ballot(have && rank <= last && B.order[rank] != lane)) {
+        // shared proxies: the exact order
+        rank = 0;
+        sm = vm;
+        while (sm) {
+            const int s = __ffsll((long long)sm) - 1;
+            sm &= sm - 1;
+            rank += s != lane && key_less(readlane_key(k, s), k) ? 1 : 0;
+        }
+    }
+    int K = min(kmax, n);
+    unsigned long long special = __ballot(have && idx >= N);
+    while (special) {
+        const int s = __ffsll((long long)special) - 1;
+        special &= special - 1;
+        const int r = __builtin_amdgcn_readlane(rank, s), e = __builtin_amdgcn_readlane(idx, s);
+        if (r > 0)
+            K = min(K, r);
+        else if (e > N)
+            K = 1;
+    }
+    if (have && rank < K) B.key[rank] = k;
+    wave_sync();
+    return K;
+}
+
+// The round's entries (wavefront 0): from the pool, after collecting it
+// again where it is incomplete or empty; the least entry of the tree alone
+// where no edge gives a pool (many entries of one time).  The master takes
+// the first event's bin, time and number.  Returns 0 for an empty calendar.
+__device__ __forceinline__ int select_round(const Hot& H, Sc& c, int kmax, int A, int Kp, int ne, int fsh, int want, int par) {
     PH_BEGIN(tsp);
     Batch& B = round_rec();
-    const int lane = lane_id(), N = H.N, N3 = N + 3;
-    Key* const blk = reinterpret_cast<Key*>(smem + H.o_blk);
-    Key* const sup = reinterpret_cast<Key*>(smem + kSupOff);
-    const bool one_sup = H.nsup == 1;
-    // one superblock (up to 1024 entries): lane b holds block b's minimum; an
-    // exclusion replaces one of them, and the tree in LDS keeps its values,
-    // which the round's rescans confirm or replace.  Else lane s holds
-    // superblock s's, and the LDS tree takes the exclusions.
-    Key top = empty_key();
-    if (lane < (one_sup ? H.nblk : H.nsup)) top = one_sup ? blk[lane] : sup[lane];
-    double pr = key_proxy(top);
-    int K = 0, k0bin = 0;
-    double k0t = 0.0;
-    int pidx = -1;        // lane m: index of popped entry m
-    unsigned gone = 0;    // lane b: popped entries of block b (one superblock)
-    while (true) {
-        const double mn = wave_min(pr);
-        if (uni(__double2hiint(mn)) == kInfHi) {
-            if (K == 0) c.status = kErrBin;
-            break;
-        }
-        int src;
-        const Key k = key_of_ties(top, __ballot(pr == mn), src);
-        const int e = key_idx(k);
-        if (K > 0 && e >= N) break;
-        if (lane == 0) B.key[K] = k;
-        if (K == 0) {
-            k0bin = key_bin(k);
-            k0t = k.t;
-        }
-        if (lane == K) pidx = e;
-        ++K;
-        // a ghost event may lead a round (its draws come first in the
-        // serial order); sync and output events run alone
-        if (e > N || K >= kmax) break;
-        // take e out of the tree: its block without the popped entries, then
-        // its superblock
-        const int b = e / kBlk;
-        Key x = empty_key(), y = empty_key();
-        const int idx = b * kBlk + (lane & 15);
-        bool out = lane >= kBlk || idx >= N3;
-        if (one_sup) {
-            if (lane == b) gone |= 1u << (e & (kBlk - 1));
-            out |= ((unsigned)__builtin_amdgcn_readlane((int)gone, b) >> (lane & 15)) & 1u;
-        } else {
-            for (int q = 0; q < K; ++q) out |= __builtin_amdgcn_readlane(pidx, q) == idx;
-            const int bb = src * kSup + lane;
-            if (bb < H.nblk) y = blk[bb];
-        }
-        if (!out) x = leaf_key(leaf_ld(H, idx), idx);
-        const double px = key_proxy(x), rm = row_min(px);
-        Key nb = empty_key();
-        if (__builtin_amdgcn_readlane(__double2hiint(rm), 0) != kInfHi) {
-            int s2;
-            nb = key_of_ties(x, __ballot(px == rm) & 0xFFFFull, s2);
-        }
-        if (!one_sup) {
-            if (lane == 0) blk[b] = nb;
-            if (lane == (b & (kSup - 1))) y = nb;
-            const double py = key_proxy(y), ym = wave_min(py);
-            nb = empty_key();
-            if (uni(__double2hiint(ym)) != kInfHi) {
-                int s2;
-                nb = key_of_ties(y, __ballot(py == ym), s2);
-            }
-            if (lane == 0) sup[src] = nb;
-        }
-        if (lane == src) {
-            top = nb;
-            pr = key_proxy(nb);
-        }
+    const int lane = lane_id();
+    int K = 0;
+    for (int att = 0; att < 2; ++att) {
+        if (att == 1 || !uni(B.full)) K = select_pool(H, kmax, A, Kp, ne, fsh);
+        if (K > 0 || att == 1) break;
+        PH_END(sdev(), kPhSelPop, tsp);
+        int* const list = reinterpret_cast<int*>(smem + H.o_w);
+        tree_update(H, par, list);
+        collect_pool(H, 0, uni(c.tfalse), want, 24, list);
+        if (lane < kMaxWaves) B.nfresh[lane] = 0;
+        if (lane == 0) B.full = 0;
+        wave_sync();
+        A = Kp = 0;
+        PH_END(sdev(), kPhSelCopy, tsp);
     }
     PH_END(sdev(), kPhSelPop, tsp);
-    if (K == 0) return 0;
+    if (K == 0) {
+        const Key* const top = H.nsup == 1 ? reinterpret_cast<const Key*>(smem + H.o_blk) : reinterpret_cast<const Key*>(smem + kSupOff);
+        const Key k = key_min_wave(lane < (H.nsup == 1 ? H.nblk : H.nsup) ? top[lane] : empty_key());
+        if (k.bc == kEmptyBc) {
+            c.status = kErrBin;
+            return 0;
+        }
+        if (lane == 0) B.key[0] = k;
+        wave_sync();
+        K = 1;
+    }
     if (lane == 0) {
+        const Key k0 = B.key[0];
         c.old_tfalse = c.tfalse;
-        c.nbin = k0bin;
-        c.tfalse = k0t;
+        c.nbin = key_bin(k0);
+        c.tfalse = k0.t;
         c.coll++;
-        B.touched = 0;
     }
     wave_sync();
-    PH_END(sdev(), kPhSelCopy, tsp);
     return K;
 }
 
@@ -4486,7 +4617,8 @@ __device__ inline void log_event(const SysDev& S, int& log_count, long long coll
 __global__ __launch_bounds__(64 * kMaxWaves) void k_run(const SysDev* __restrict__ sys, const int* ids, const long long* inc,
                                                        int maxw, int lds_bytes, long long budget, int flags,
                                                        unsigned long long* launch_t0) {
-    const int nw = (int)(blockDim.x >> 6), wave = wave_id(), lane = lane_id();
+    // event wavefronts 0 to ne - 1, then the calendar wavefront
+    const int nw = (int)(blockDim.x >> 6), ne = nw - 1, wave = wave_id(), lane = lane_id();
     if (threadIdx.x == 0) *reinterpret_cast<SysDev*>(smem + kSdOff) = sys[ids[blockIdx.x]];
     __syncthreads();
     const SysDev& S = sdev();
@@ -4518,7 +4650,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_run(const SysDev* __restrict
     const long long t_begin = w0;
     long long t_rebuild = 0, n_rebuild = 0;
     // the system's own limit on pair events per round (its tuned wavefronts)
-    const int kcap = S.waves_cap > 0 && S.waves_cap < nw ? S.waves_cap : nw;
+    const int kcap = S.waves_cap > 0 && S.waves_cap < ne ? S.waves_cap : ne;
     if (budget > 0) {
         if (threadIdx.x == 0) {
             atomicMin(launch_t0, (unsigned long long)w0);
@@ -4529,6 +4661,16 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_run(const SysDev* __restrict
     }
     bool stop_out = false;
     const Hot H = load_hot(S, L);
+    // the pool holds a few entries more than a round takes; each event
+    // wavefront has an equal share of the fresh entries' places
+    const int want = kcap + 2, fsh = ne <= 1 ? 5 : (ne <= 2 ? 4 : (ne <= 4 ? 3 : 2));
+    int par = 0, A = 0, Kp = 0;
+    if (threadIdx.x < kSup) B.dirty[0][threadIdx.x] = B.dirty[1][threadIdx.x] = 0;
+    if (threadIdx.x == 0) {
+        B.full = 1;
+        B.width = c.interval / 64.0;
+    }
+    __syncthreads();
     while (true) {
         if (wave == 0) {
             PH_BEGIN(tsel);
@@ -4536,7 +4678,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_run(const SysDev* __restrict
             if (uni(c.status) == 0 && !stop_out && !(budget > 0 && wall_clock64() - w0 > budget)) {
                 const long long left = c.target - c.coll;
                 const int room = uni((int)min((long long)kcap, left));
-                if (room > 0) K = select_batch(H, c, room);
+                if (room > 0) K = select_round(H, c, room, A, Kp, ne, fsh, want, par ^ 1);
             }
             if (lane == 0) {
                 B.K = K;
@@ -4544,25 +4686,23 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_run(const SysDev* __restrict
             }
             PH_END(S, kPhSelect, tsel);
         }
-        if (nw > 1)
-            __syncthreads();
-        else
-            wave_sync();
+        __syncthreads();
         const int K = uni(B.K);
         if (K == 0) break;
         const Key k = B.key[wave < K ? wave : 0];
         const int e = uni(key_idx(k));
+        int* const list = reinterpret_cast<int*>(smem + H.o_w);
         if (K == 1 && e > N) {
+            // the sync or output event, on the tree as of now
+            if (wave == ne) tree_update(H, par ^ 1, list);
+            __syncthreads();
             if (e == N + 1) {
-                // the sync event; every wavefront takes part in a list rebuild
+                // every wavefront takes part in a list rebuild
                 if (wave == 0) {
                     const bool rb = sync_begin(S, T, L, c);
                     if (lane == 0) B.rebuild = rb ? 1 : 0;
                 }
-                if (nw > 1)
-                    __syncthreads();
-                else
-                    wave_sync();
+                __syncthreads();
                 if (B.rebuild) {
                     const long long tr = wall_clock64();
                     rebuild(S, T, L, c);
@@ -4574,25 +4714,46 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_run(const SysDev* __restrict
                 output_event(S, L, c);
                 stop_out = (flags & kStopAtOutput) != 0;
             }
-            if (wave == 0) log_event(S, log_count, c.coll, e, -1, 0, k.t);
-            if (nw > 1) __syncthreads();
+            if (wave == 0) {
+                log_event(S, log_count, c.coll, e, -1, 0, k.t);
+                if (lane == 0) {
+                    dirty_or(par ^ 1, e / kBlk);
+                    B.full = 1;
+                }
+            }
+            A = Kp = 0;
+            __syncthreads();
             continue;
         }
-        // pair events (a ghost event may lead them), one per wavefront; event
-        // k of a round is numbered and stamped as the master will count it
-        int A = 0;
-        if (wave < K) {
-            const int bk = K == 1 ? -1 : wave;
-            A = run_event(H, e, uni(key_p(k)), uni(key_ct(k)), k.t, uni(key_bin(k)), master().coll + wave, bk);
-            if (A > 0 && lane == 0) {
-                const int ty = B.ty[wave];
-                if (ty >= 1 && ty <= 30)
-                    __hip_atomic_fetch_add((unsigned long long*)&master().nev[ty], 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        A = 0;
+        Kp = K;
+        if (wave == ne) {
+            // the calendar wavefront: the tree after the last round's
+            // events, then the pool the next round is taken from, while
+            // this round's events run
+            tree_update(H, par ^ 1, list);
+            if (K > 1) __syncthreads();
+            collect_pool(H, K, uni(B.key[K - 1].t), want, 2, list);
+            __syncthreads();
+        } else {
+            if (lane == 0) B.nfresh[wave] = 0;
+            if (wave < K) {
+                // pair events (a ghost event may lead them), one per
+                // wavefront; event k of a round is numbered and stamped as
+                // the master will count it
+                A = run_event(H, e, uni(key_p(k)), uni(key_ct(k)), k.t, uni(key_bin(k)), master().coll + wave, wave, K == 1,
+                              par, fsh);
+                if (A > 0 && lane == 0) {
+                    const int ty = B.ty[wave];
+                    if (ty >= 1 && ty <= 30)
+                        __hip_atomic_fetch_add((unsigned long long*)&master().nev[ty], 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                }
+            } else {
+                int nb = 0;
+                bar_to(nb, K > 1 ? kRoundBars : 1);
             }
-        } else if (K > 1) {
-            int nb = 0;
-            bar_to(nb, kRoundBars);
         }
+        par ^= 1;
         PH_BEGIN(ttail);
         if (wave == 0 && K > 1) {
             PH_COUNT(S, kPhNRound);
@@ -4601,25 +4762,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_run(const SysDev* __restrict
             PH_ADDN(S, kPhNCutMark, min(K, B.cut) < K ? 1 : 0);
             PH_ADDN(S, kPhNCutKey, A < min(K, B.cut) ? 1 : 0);
         }
-        wg_sync(nw);
-        // block minima of every committed event's blocks and of the popped
-        // entries that were not committed, then the superblock minima
-        if (A > 0) {
-            int* const bl = reinterpret_cast<int*>(smem + H.o_blist);
-            int nbl = uni(B.nbl[wave]);
-            if (wave == 0 && A < K) {
-                if (lane < K - A) bl[nbl + lane] = key_idx(B.key[A + lane]) / kBlk;
-                nbl += K - A;
-                wave_sync();
-            }
-            rescan_round(H, bl, nbl);
-        }
-        // a single superblock is never read: selection pops from the block
-        // minima (its value is recomputed by the single-event paths)
-        if (H.nsup > 1) {
-            wg_sync(nw);
-            rescan_touched(H, wave, nw);
-        }
+        __syncthreads();
         if (wave == 0) {
             // the master takes the committed events in order
             if (S.log)
@@ -4639,11 +4782,8 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_run(const SysDev* __restrict
                     c.nbin = key_bin(B.key[A - 1]);
                 }
             }
-        }
-        if (nw > 1)
-            __syncthreads();
-        else
             wave_sync();
+        }
         PH_END(S, kPhBTail, ttail);
     }
     __syncthreads();
@@ -4974,8 +5114,9 @@ hipError_t engine_run(const SysDev* d_sys, const int* d_ids, const long long* d_
                       size_t lds_limit, hipStream_t s, long long budget_ticks, int flags, int waves,
                       unsigned long long* launch_t0) {
     const int nblk = nblk_for(max_n);
-    int nw = waves < 1 ? 1 : (waves > kMaxWaves ? kMaxWaves : waves);
-    while (nw > 1 && engine_lds_bytes(nblk, maxw, 0, nw) > lds_limit) --nw;
+    // the event wavefronts and the calendar wavefront
+    int nw = 1 + (waves < 1 ? 1 : (waves > kMaxWaves - 1 ? kMaxWaves - 1 : waves));
+    while (nw > 2 && engine_lds_bytes(nblk, maxw, 0, nw) > lds_limit) --nw;
     const size_t base = engine_lds_bytes(nblk, maxw, 0, nw);
     // up to one workgroup per compute unit: each takes the whole LDS
     // budget, so every system keeps as many leaves in LDS as fit beside
@@ -5005,8 +5146,8 @@ hipError_t engine_run(const SysDev* d_sys, const int* d_ids, const long long* d_
 }
 int engine_max_waves(int max_n, int maxw, size_t lds_limit) {
     int nw = kMaxWaves;
-    while (nw > 1 && engine_lds_bytes(nblk_for(max_n), maxw, 0, nw) > lds_limit) --nw;
-    return nw;
+    while (nw > 2 && engine_lds_bytes(nblk_for(max_n), maxw, 0, nw) > lds_limit) --nw;
+    return nw - 1;
 }
 hipError_t engine_predict(const SysDev* d_sys, int id, int n, const int* pi, const int* pj, double* tij, int* type,
                           hipStream_t s) {
