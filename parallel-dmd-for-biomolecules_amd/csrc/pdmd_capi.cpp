@@ -404,7 +404,7 @@ int64_t device_bytes(const Prep& pp) {
     const int64_t N = H.N, cap = H.cap, nc = (int64_t)pp.Mq * pp.Mq * pp.Mq;
     const int64_t sizes[] = {(int64_t)sizeof(DevTables), N * (int64_t)sizeof(Rec), N * 16 /*bw*/, N * 16 /*extra*/,
                              N * 16 /*ovr*/, N * 32 /*old_r*/, N * cap * 4 /*nb_up*/, N * cap * 4 /*nb_dn*/,
-                             N * 4 /*nup*/, N * 4 /*ndn*/, (N + 3) * (int64_t)sizeof(Leaf), N * 4 /*cfine*/,
+                             (N + 1) * 4 /*nup*/, (N + 1) * 4 /*ndn*/, (N + 3) * (int64_t)sizeof(Leaf), N * 4 /*cfine*/,
                              N * 4 /*ckey*/, N * 8 /*cfp*/, N * 4 /*csorted*/, N * 32 /*spos*/, N * 16 /*sinfo*/, N * 4 /*mark*/,
                              (nc + 1) * 4 /*cstart*/, nc * 4 /*crun*/, (N + 3) * 8 /*stamp*/,
                              (int64_t)sizeof(SysState)};
@@ -566,8 +566,8 @@ int prepared_add(pdmd_ctx* ctx, PreparedSystem* ps, int32_t* sys_id) {
     HIPCHK(H.old_r.alloc(N));
     HIPCHK(H.nb_up.alloc((size_t)N * H.cap));
     HIPCHK(H.nb_dn.alloc((size_t)N * H.cap));
-    HIPCHK(H.nup.alloc(N));
-    HIPCHK(H.ndn.alloc(N));
+    HIPCHK(H.nup.alloc(N + 1));  // one more: the event loop's pair gather reads 8 bytes
+    HIPCHK(H.ndn.alloc(N + 1));
     HIPCHK(H.leaf.alloc(N + 3));
     HIPCHK(H.cfine.alloc(N));
     HIPCHK(H.ckey.alloc(N));
@@ -1107,11 +1107,12 @@ int pdmd_lists(pdmd_ctx* ctx, int32_t id, int32_t* n_up, int32_t* up, int32_t* n
     const size_t N = (size_t)H->N, cap = (size_t)H->cap;
     if (n_up) HIPCHK(hipMemcpy(n_up, H->nup.p, sizeof(int) * N, hipMemcpyDeviceToHost));
     if (n_dn) HIPCHK(hipMemcpy(n_dn, H->ndn.p, sizeof(int) * N, hipMemcpyDeviceToHost));
-    // rows hold partner | static code << 24; the ABI gives 1-based partners
+    // rows hold partner | (down rows: its up-row length << 16) | static code
+    // << 24; the ABI gives 1-based partners
     auto rows = [&](const int* src, int32_t* dst) -> int {
         std::vector<int> r(N * cap);
         HIPCHK(hipMemcpy(r.data(), src, sizeof(int) * N * cap, hipMemcpyDeviceToHost));
-        for (size_t k = 0; k < N * cap; ++k) dst[k] = (r[k] & 0xFFFFFF) + 1;
+        for (size_t k = 0; k < N * cap; ++k) dst[k] = (r[k] & 0xFFFF) + 1;
         return 0;
     };
     if (up)

@@ -8,7 +8,8 @@
 //   bw[N]       16 B  bond window of the bead's own side-chain bond
 //                     (Calpha: code 10, N: code 11, C: code 12)
 //   ovr/extra   int4  pair-code overrides and H-bond shoulder partners
-//   nb_up/nb_dn int32 [N*cap]: partner | static pair code << 24
+//   nb_up/nb_dn int32 [N*cap]: partner | static pair code << 24; down rows
+//                     also the partner's up-row length << 16
 //   leaf[N+3]   16 B  {tim, nptnr, coltype|bin} per calendar entry: beads,
 //                     then the ghost, sync and output pseudo-events
 // Indices are 0-based on the device; the C ABI converts to the reference's
@@ -123,7 +124,7 @@ struct SysDev {
     Leaf* leaf;
     int* cfine;    // packed fine cell coordinates per bead
     int* ckey;     // coarse cell per bead
-    int2* cfp;     // [N] fine cell and the place in its list as cell_add.f builds it (1 = highest index)
+    int2* cfp;     // [N] fine cell; the place in its list as cell_add.f builds it (1 = highest index) | up-row length << 16
     int* cstart;   // [ncoarse+1]
     int* crun;     // [ncoarse]
     int* csorted;  // [N]

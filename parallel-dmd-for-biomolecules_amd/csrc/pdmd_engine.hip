@@ -282,7 +282,7 @@ __device__ inline int static_t(int ta, int tb) {
 // A bead's neighbour rows in nbor.f's order are its rows sorted by this key.
 // a and b: the beads' fine cells (10 bits per axis) and list places.
 __device__ inline unsigned long long nbor_key(int M, const DevTables& T, int2 a, int2 b) {
-    const int fa = a.x, fb = b.x, pa = a.y, pb = b.y, nc = M + 4;
+    const int fa = a.x, fb = b.x, pa = a.y & 0xFFFF, pb = b.y & 0xFFFF, nc = M + 4;
     int d[3];
     for (int q = 0; q < 3; ++q) {
         // periodic offset in [-(M / 2), M - M / 2), in [-2, 2] for neighbours
@@ -498,6 +498,10 @@ __device__ inline double readlane_d(double v, int l) {
     const int lo = __builtin_amdgcn_readlane((int)b, l), hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
     return __longlong_as_double((long long)(unsigned)lo | ((long long)hi << 32));
 }
+__device__ inline unsigned long long readlane_u64(unsigned long long v, int l) {
+    return (unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)v, l) |
+           ((unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(v >> 32), l) << 32);
+}
 // first non-zero status of the wave (0 if none); wave-uniform
 __device__ inline int wave_status(int v) {
     const unsigned long long m = __ballot(v != 0);
@@ -572,8 +576,10 @@ __device__ inline bool key_less_st(const Key& a, unsigned long long sa, const Ke
     if (a.bc == kEmptyBc || sa == sb) return a.ip < b.ip;
     return sa > sb;
 }
-// a before b, both entries of the calendar (their stamps written)
-__device__ inline bool key_less(const Key& a, const Key& b) {
+// a before b, both entries of the calendar (their stamps written).  Only
+// shared order proxies come here, a few times in a million entries: out of
+// line, so that the event loop's code stays small.
+__device__ __noinline__ bool key_less(Key a, Key b) {
     const int ab = a.bc >> 8, bb = b.bc >> 8;
     if (ab != bb) return ab < bb;
     if (a.t != b.t) return a.t < b.t;
@@ -610,11 +616,12 @@ __device__ inline void key_step(Key& k) {
     if (key_less(o, k)) k = o;
 }
 // exact minimum over each row of 16 lanes, in the row's last lane
-__device__ inline void key_min_rows_exact(Key& k) {
+__device__ __noinline__ Key key_min_rows_exact(Key k) {
     key_step<0x111, 0xf>(k);
     key_step<0x112, 0xf>(k);
     key_step<0x114, 0xf>(k);
     key_step<0x118, 0xf>(k);
+    return k;
 }
 __device__ inline Key readlane_key(const Key& k, int l) {
     Key r;
@@ -792,10 +799,9 @@ __device__ inline double wave_min(double v) {
     }
     return v;
 }
-// the least key among the lanes of `tie` (not empty), which share a proxy;
-// src becomes its lane
-__device__ inline Key key_of_ties(const Key& k, unsigned long long tie, int& src) {
-    src = __ffsll((long long)tie) - 1;
+// the lane of the least key among the lanes of `tie`, which share a proxy
+__device__ __noinline__ int tie_lane(Key k, unsigned long long tie) {
+    int src = __ffsll((long long)tie) - 1;
     Key r = readlane_key(k, src);
     unsigned long long rest = tie & (tie - 1);
     while (rest) {
@@ -807,40 +813,45 @@ __device__ inline Key key_of_ties(const Key& k, unsigned long long tie, int& src
             src = o_src;
         }
     }
-    return r;
+    return src;
 }
 // minimum over the wave, returned to every lane
 __device__ inline Key key_min_wave(const Key& k) {
     const double p = key_proxy(k), m = wave_min(p);
     if (proxy_none(readlane_d(m, 0))) return empty_key();
-    int src;
-    return key_of_ties(k, __ballot(p == m), src);
+    const unsigned long long tie = __ballot(p == m);
+    return readlane_key(k, (tie & (tie - 1)) ? uni(tie_lane(k, tie)) : __ffsll((long long)tie) - 1);
 }
-// minimum over the wave of keys with their add stamps given per lane (new
-// entries, not yet written), returned to every lane with its stamp
+// the lane of the least key among the lanes of `tie`, which share a proxy,
+// with their add stamps given per lane (new entries, not yet written)
+__device__ __noinline__ int tie_lane_st(Key k, unsigned long long st, unsigned long long tie) {
+    int src = __ffsll((long long)tie) - 1;
+    Key r = readlane_key(k, src);
+    unsigned long long rs = readlane_u64(st, src);
+    unsigned long long rest = tie & (tie - 1);
+    while (rest) {
+        const int o_src = __ffsll((long long)rest) - 1;
+        rest &= rest - 1;
+        const Key o = readlane_key(k, o_src);
+        const unsigned long long os = readlane_u64(st, o_src);
+        if (key_less_st(o, os, r, rs)) {
+            r = o;
+            rs = os;
+            src = o_src;
+        }
+    }
+    return src;
+}
+// minimum over the wave of keys with their add stamps, returned to every
+// lane with its stamp
 __device__ inline Key key_min_wave_st(const Key& k, unsigned long long st, unsigned long long& out_st) {
     const double p = key_proxy(k), mn = wave_min(p);
     out_st = 0;
     if (proxy_none(readlane_d(mn, 0))) return empty_key();
     const unsigned long long tie = __ballot(p == mn);
-    int src = __ffsll((long long)tie) - 1;
-    Key r = readlane_key(k, src);
-    unsigned long long rs = (unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)st, src) |
-                            ((unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(st >> 32), src) << 32);
-    unsigned long long rest = tie & (tie - 1);
-    while (rest) {
-        src = __ffsll((long long)rest) - 1;
-        rest &= rest - 1;
-        const Key o = readlane_key(k, src);
-        const unsigned long long os = (unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)st, src) |
-                                      ((unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(st >> 32), src) << 32);
-        if (key_less_st(o, os, r, rs)) {
-            r = o;
-            rs = os;
-        }
-    }
-    out_st = rs;
-    return r;
+    const int src = (tie & (tie - 1)) ? uni(tie_lane_st(k, st, tie)) : __ffsll((long long)tie) - 1;
+    out_st = readlane_u64(st, src);
+    return readlane_key(k, src);
 }
 // Minimum over each row of 16 lanes.  Returns true on the lane that holds
 // its row's minimum in k afterwards (the row's last lane when the row is
@@ -851,7 +862,7 @@ __device__ inline bool key_min_rows(Key& k) {
     const unsigned long long tie = __ballot(p == rm && !proxy_none(rm));
     const unsigned rb = (unsigned)(tie >> (lane & 48)) & 0xFFFFu;
     if (__ballot((rb & (rb - 1u)) != 0u)) {
-        key_min_rows_exact(k);
+        k = key_min_rows_exact(k);
         return (lane & 15) == 15;
     }
     return proxy_none(rm) ? (lane & 15) == 15 : p == rm;
@@ -1041,10 +1052,6 @@ __device__ inline void stamp_st(const Hot& H, int k, unsigned long long v) {
 __device__ inline void dirty_or(int par, int blk) {
     __hip_atomic_fetch_or(&round_rec().dirty[par][blk / kSup], 1ull << (blk & (kSup - 1)), __ATOMIC_RELAXED,
                           __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-__device__ inline unsigned long long readlane_u64(unsigned long long v, int l) {
-    return (unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)v, l) |
-           ((unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(v >> 32), l) << 32);
 }
 // Block minima of the listed blocks, one row of 16 lanes per block, 16
 // blocks per step so that four independent reductions overlap.  A block
@@ -1332,7 +1339,8 @@ __device__ inline void round_clear_marks(const Lds& L, const SysDev& S, int dent
 // before the first event after an error, and before the first event whose
 // key is not below every new calendar key of the events before it (the
 // serial order would have run one of those first).
-__device__ inline int batch_accepted(const Batch& B) {
+__device__ __noinline__ int batch_accepted() {
+    const Batch& B = round_rec();
     int A = min(B.K, B.cut);
     Key lo = B.knew[0];
     unsigned long long lo_st = B.knew_st[0];
@@ -1372,7 +1380,7 @@ __device__ inline int accepted(const Batch& B) {
     lo = min_raw(lo, shr(lo, std::integral_constant<int, 0x112>{}));
     lo = min_raw(lo, shr(lo, std::integral_constant<int, 0x114>{}));
     const bool live = in && lane >= 1;
-    if (__ballot(live && pk == lo)) return uni(batch_accepted(B));
+    if (__ballot(live && pk == lo)) return uni(batch_accepted());
     const unsigned long long fail = __ballot(live && pk > lo), sm = __ballot(st != 0);
     int A = top;
     if (fail) A = min(A, __ffsll((long long)fail) - 1);
@@ -1383,6 +1391,8 @@ __device__ inline int accepted(const Batch& B) {
 // ------------------------------------------------------------------------
 // rescheduling after an event: partial_events.f:16-201
 // ------------------------------------------------------------------------
+__device__ __noinline__ void shoulders_clear(int n, int Ln, int cb, int Lc);
+
 // The list rows of i and j (lane k: slot k) with their lengths; they do not
 // change between list rebuilds, so a pair event loads them before it
 // resolves its outcome
@@ -1552,7 +1562,7 @@ __device__ void reschedule_generic(const SysDev&, const DevTables&, const Lds&, 
     }
     const int ncand = w;
     if (lane < ndi) {
-        L.wm()[w + lane] = edi & 0xFFFFFF;
+        L.wm()[w + lane] = edi & 0xFFFF;
         L.wx()[w + lane] = 2;
     }
     w += ndi;
@@ -1560,7 +1570,7 @@ __device__ void reschedule_generic(const SysDev&, const DevTables&, const Lds&, 
     if (xi1 >= 0 && xi1 < i) { if (lane == 0) { L.wm()[w] = xi1; L.wx()[w] = 2; } ++w; }
     if (xi2 >= 0 && xi2 < i) { if (lane == 0) { L.wm()[w] = xi2; L.wx()[w] = 2; } ++w; }
     if (j >= 0) {
-        const int l = edj & 0xFFFFFF;
+        const int l = edj & 0xFFFF;
         const bool keep = lane < ndj && l != i;
         const unsigned long long bal = __ballot(keep);
         const int pre = __popcll(bal & ((1ull << lane) - 1ull));
@@ -1754,22 +1764,11 @@ __device__ void reschedule_generic(const SysDev&, const DevTables&, const Lds&, 
     // repuls_del_b.f once the rescheduling is done
     if (xpulse_del && lane == 0) {
         const bool iN = dyn_ident(P.ri.dyn) < dyn_ident(P.rj.dyn);
-        const int a = iN ? i : j, b = iN ? j : i;
-        const int La = topo_len(iN ? P.ri.topo : P.rj.topo), Lb = topo_len(iN ? P.rj.topo : P.ri.topo);
-        const int ncim1 = a + La - 1, ncai = a - La, ncaj = b - 2 * Lb, nnjp1 = b - Lb + 1;
-        int4 ea = gld(S.extra + (a)), eb = gld(S.extra + (b));
-        ea.x = -1;
-        ea.y = -1;
-        ea.w = -1;
-        eb.x = -1;
-        eb.y = -1;
-        eb.w = -1;
-        gst(S.extra + (a), ea);
-        gst(S.extra + (b), eb);
-        gs1(&S.extra[ncaj].z, -1);
-        gs1(&S.extra[nnjp1].z, -1);
-        gs1(&S.extra[ncai].z, -1);
-        gs1(&S.extra[ncim1].z, -1);
+        const int Li = topo_len(P.ri.topo), Lj = topo_len(P.rj.topo);
+        if (iN)
+            shoulders_clear(i, Li, j, Lj);
+        else
+            shoulders_clear(j, Lj, i, Li);
     }
     status = wave_status(status);
     if (status && !c.status) c.status = status;
@@ -1856,7 +1855,7 @@ __device__ __noinline__ void reschedule(const SysDev&, const DevTables&, const L
     //      reference order: i's down list and lower shoulder partners, then j's
     int d = 0;
     if (lane < ndi) {
-        v_wm[dbase + lane] = edi & 0xFFFFFF;
+        v_wm[dbase + lane] = edi & 0xFFFF;
         v_wx[dbase + lane] = 2;
     }
     d = ndi;
@@ -1864,7 +1863,7 @@ __device__ __noinline__ void reschedule(const SysDev&, const DevTables&, const L
     if (xi1 >= 0 && xi1 < i) { if (lane == 0) { v_wm[dbase + d] = xi1; v_wx[dbase + d] = 2; } ++d; }
     if (xi2 >= 0 && xi2 < i) { if (lane == 0) { v_wm[dbase + d] = xi2; v_wx[dbase + d] = 2; } ++d; }
     if (j >= 0) {
-        const int l = edj & 0xFFFFFF;
+        const int l = edj & 0xFFFF;
         const bool keep = lane < ndj && l != i;
         const unsigned long long bal = __ballot(keep);
         const int pre = __popcll(bal & ((1ull << lane) - 1ull));
@@ -2335,22 +2334,11 @@ __device__ __noinline__ void reschedule(const SysDev&, const DevTables&, const L
     // repuls_del_b.f once the rescheduling is done
     if (xpulse_del && lane == 0) {
         const bool iN = dyn_ident(P.ri.dyn) < dyn_ident(P.rj.dyn);
-        const int a = iN ? i : j, b = iN ? j : i;
-        const int La = topo_len(iN ? P.ri.topo : P.rj.topo), Lb = topo_len(iN ? P.rj.topo : P.ri.topo);
-        const int ncim1 = a + La - 1, ncai = a - La, ncaj = b - 2 * Lb, nnjp1 = b - Lb + 1;
-        int4 ea = gld(S.extra + (a)), eb = gld(S.extra + (b));
-        ea.x = -1;
-        ea.y = -1;
-        ea.w = -1;
-        eb.x = -1;
-        eb.y = -1;
-        eb.w = -1;
-        gst(S.extra + (a), ea);
-        gst(S.extra + (b), eb);
-        gs1(&S.extra[ncaj].z, -1);
-        gs1(&S.extra[nnjp1].z, -1);
-        gs1(&S.extra[ncai].z, -1);
-        gs1(&S.extra[ncim1].z, -1);
+        const int Li = topo_len(P.ri.topo), Lj = topo_len(P.rj.topo);
+        if (iN)
+            shoulders_clear(i, Li, j, Lj);
+        else
+            shoulders_clear(j, Lj, i, Li);
     }
     if (batch) {
         // the round's block rescans run after every committed event's
@@ -2374,144 +2362,83 @@ __device__ __noinline__ void reschedule(const SysDev&, const DevTables&, const L
 // ------------------------------------------------------------------------
 // event dynamics: eventdyn.f, bumped.f, repuls_*.f (uniform over lanes)
 // ------------------------------------------------------------------------
-__device__ inline void nudge(Rec& bi, Rec& bj, double bd, const Geo& g, int sign) {
-    if (sign > 0) {
-        bi.x = bi.x + bd * g.rx;
-        bi.y = bi.y + bd * g.ry;
-        bi.z = bi.z + bd * g.rz;
-        bj.x = bj.x - bd * g.rx;
-        bj.y = bj.y - bd * g.ry;
-        bj.z = bj.z - bd * g.rz;
-    } else {
-        bi.x = bi.x - bd * g.rx;
-        bi.y = bi.y - bd * g.ry;
-        bi.z = bi.z - bd * g.rz;
-        bj.x = bj.x + bd * g.rx;
-        bj.y = bj.y + bd * g.ry;
-        bj.z = bj.z + bd * g.rz;
-    }
-}
-
-__device__ __forceinline__ void eventdyn(const DevTables& T, Rec& bi, Rec& bj, double2 bwi, bool bonded_ij, int evcode, double tf,
-                         int& ct, int& status) {
-    const int a = dyn_ident(bi.dyn), c = dyn_ident(bj.dyn);
-    Geo g;
-    geo(bi, bj, tf, g);
-    const double bmi = bi.bm, bmj = bj.bm;
+// Outcome of eventdyn.f for event type ct (in: predicted or resolved by the
+// caller, out: resolved): the impulse ratio along the pair vector, and the
+// nudge bumped.f's callers give the pair off the discontinuity, bd along the
+// pair vector (sgn +1: apart, -1: together, 0: none).  g: the pair's
+// geometry; a, c: identities; bwi: bead i's own bond window.
+__device__ __forceinline__ void impulse(const DevTables& T, const Geo& g, double bmi, double bmj, int a, int c, double2 bwi,
+                                        bool bonded_ij, int evcode, int& ct, double& ratio, double& bd, int& sgn,
+                                        int& status) {
     const double rmass = 2 * bmi * bmj / (bmi + bmj);
-    double ratio = 0.0, wellsq, epsave, del_pe, bd;
-    switch (ct) {
-        case 2:
-        case 3: {
-            double blmin, blmax;
-            bond_window(T, evcode, bwi, blmin, blmax);
-            ratio = ct == 2 ? rmass * g.b / (blmin * blmin) : rmass * g.b / (blmax * blmax);
-            break;
-        }
-        case 1: {
-            double sigsq;
-            if (evcode == 15) {
-                if (bonded_ij) {
-                    const double pe = T.ev_param[1][evcode];
-                    sigsq = T.sigma_sq[a][c] * (pe * pe);
-                } else
-                    sigsq = T.sigma_sq[a][c];
-            } else {
-                const double pe = T.ev_param[1][evcode];
-                sigsq = T.sigma_sq[a][c] * (pe * pe);
+    const double b = g.b;
+    ratio = 0.0;
+    sgn = 0;
+    bd = 0.0;
+    if (ct <= 3) {
+        double sq;
+        if (ct == 1) {
+            const double pe = T.ev_param[1][evcode], ssq = T.sigma_sq[a][c];
+            if (evcode == 15 && !bonded_ij)
+                sq = ssq;
+            else {
+                sq = ssq * (pe * pe);
                 if (evcode >= 22 && evcode <= 26) {
                     const double q = T.sqz610[evcode - 21][a > c ? a : c];
-                    sigsq = sigsq * (q * q);
+                    sq = sq * (q * q);
                 }
             }
-            ratio = rmass * g.b / sigsq;
-            break;
+        } else {
+            double blmin, blmax;
+            bond_window(T, evcode, bwi, blmin, blmax);
+            sq = ct == 2 ? blmin * blmin : blmax * blmax;
         }
+        ratio = rmass * b / sq;
+        if (ct < 1) status = kErrDyn;
+        return;
+    }
+    const bool shl = ct == 5 || ct == 6 || ct == 13;
+    if (!shl && ct != 4 && ct != 8 && ct != 9) {
+        status = kErrDyn;
+        return;
+    }
+    const double wellsq = shl ? T.shlddia_sq[a][c] : T.welldia_sq[a][c];
+    const double epsave = shl ? -T.epsilon1 : T.ep_sqrt[a][c];
+    const double del_pe = 4.0 * wellsq * epsave / rmass;
+    bd = kSm * sqrt(wellsq);
+    bool bounce = false;
+    double root = 0.0;
+    switch (ct) {
         case 4:
-            wellsq = T.welldia_sq[a][c];
-            epsave = T.ep_sqrt[a][c];
-            del_pe = 4.0 * wellsq * epsave / rmass;
-            bd = kSm * sqrt(wellsq);
-            if (g.b * g.b + del_pe > 0.0) {
-                ratio = rmass * (sqrt((4.0 * wellsq * epsave / rmass) + g.b * g.b) + g.b) / (2.0 * wellsq);
-                ct = 20;
-                nudge(bi, bj, bd, g, -1);
-            } else {
-                ratio = rmass * g.b / wellsq;
-                ct = 22;
-                nudge(bi, bj, bd, g, +1);
-            }
+            bounce = !(b * b + del_pe > 0.0);
+            root = sqrt(del_pe + b * b);
+            ct = bounce ? 22 : 20;
+            sgn = bounce ? 1 : -1;
             break;
         case 8:
-            wellsq = T.welldia_sq[a][c];
-            epsave = T.ep_sqrt[a][c];
-            del_pe = 4.0 * wellsq * epsave / rmass;
-            bd = kSm * sqrt(wellsq);
-            if (g.b * g.b > del_pe) {
-                ratio = rmass * (-sqrt(-del_pe + g.b * g.b) + g.b) / (2.0 * wellsq);
-                ct = 21;
-                nudge(bi, bj, bd, g, +1);
-            } else {
-                ratio = rmass * g.b / wellsq;
-                ct = 22;
-                nudge(bi, bj, bd, g, -1);
-            }
-            break;
-        case 9:
-            wellsq = T.welldia_sq[a][c];
-            ratio = rmass * g.b / wellsq;
-            ct = 23;
-            bd = kSm * sqrt(wellsq);
-            nudge(bi, bj, bd, g, +1);
+            bounce = !(b * b > del_pe);
+            root = -sqrt(-del_pe + b * b);
+            ct = bounce ? 22 : 21;
+            sgn = bounce ? -1 : 1;
             break;
         case 5:
-            wellsq = T.shlddia_sq[a][c];
-            epsave = -T.epsilon1;
-            del_pe = 4.0 * wellsq * epsave / rmass;
-            bd = kSm * sqrt(wellsq);
-            ratio = rmass * (-sqrt(-del_pe + g.b * g.b) + g.b) / (2.0 * wellsq);
+            root = -sqrt(-del_pe + b * b);
             ct = 24;
-            nudge(bi, bj, bd, g, +1);
+            sgn = 1;
             break;
         case 6:
-            wellsq = T.shlddia_sq[a][c];
-            epsave = -T.epsilon1;
-            del_pe = 4.0 * wellsq * epsave / rmass;
-            bd = kSm * sqrt(wellsq);
-            if (g.b * g.b > -del_pe) {
-                ratio = rmass * (sqrt(del_pe + g.b * g.b) + g.b) / (2.0 * wellsq);
-                ct = 25;
-                nudge(bi, bj, bd, g, -1);
-            } else {
-                ratio = rmass * g.b / wellsq;
-                ct = 26;
-                nudge(bi, bj, bd, g, +1);
-            }
+            bounce = !(b * b > -del_pe);
+            root = sqrt(del_pe + b * b);
+            ct = bounce ? 26 : 25;
+            sgn = bounce ? 1 : -1;
             break;
-        case 13:
-            wellsq = T.shlddia_sq[a][c];
-            ratio = rmass * g.b / wellsq;
-            ct = 27;
-            bd = kSm * sqrt(wellsq);
-            nudge(bi, bj, bd, g, +1);
+        default:  // 9, 13
+            bounce = true;
+            ct = shl ? 27 : 23;
+            sgn = 1;
             break;
-        default:
-            status = kErrDyn;
-            return;
     }
-    const double dvx = ratio * g.rx, dvy = ratio * g.ry, dvz = ratio * g.rz;
-    bi.vx = bi.vx - dvx / bmi;
-    bj.vx = bj.vx + dvx / bmj;
-    bi.vy = bi.vy - dvy / bmi;
-    bj.vy = bj.vy + dvy / bmj;
-    bi.vz = bi.vz - dvz / bmi;
-    bj.vz = bj.vz + dvz / bmj;
-    bi.x = bi.x + dvx * tf / bmi;
-    bi.y = bi.y + dvy * tf / bmi;
-    bi.z = bi.z + dvz * tf / bmi;
-    bj.x = bj.x - dvx * tf / bmj;
-    bj.y = bj.y - dvy * tf / bmj;
-    bj.z = bj.z - dvz * tf / bmj;
+    ratio = bounce ? rmass * b / wellsq : rmass * (root + b) / (2.0 * wellsq);
 }
 
 __device__ inline double dist_rec(const Rec& a, const Rec& b, double tf) {
@@ -2549,6 +2476,31 @@ __device__ __noinline__ bool shoulders_far_3(int n, int cb, int k, double tf) {
     if (ncai != k && dist_rec(rc, pair_rec(ncai), tf) > T.shder[3]) ++m;
     if (ncim1 != k && dist_rec(rc, pair_rec(ncim1), tf) > T.shder[4]) ++m;
     return m == 3;
+}
+// squared distance of two beads, the colliding pair read from LDS
+__device__ __noinline__ double pair_r2(int a, int b, double tf) {
+    Geo g;
+    geo(pair_rec(a), pair_rec(b), tf, g);
+    return g.r2;
+}
+// repuls_del_b.f (single lane; n = N bead, cb = C bead)
+__device__ __noinline__ void shoulders_clear(int n, int Ln, int cb, int Lc) {
+    const SysDev& S = sdev();
+    int ncim1, ncai, ncaj, nnjp1;
+    shoulder_idx(n, Ln, cb, Lc, ncim1, ncai, ncaj, nnjp1);
+    int4 en = gld(S.extra + (n)), ec = gld(S.extra + (cb));
+    en.x = -1;
+    en.y = -1;
+    en.w = -1;
+    ec.x = -1;
+    ec.y = -1;
+    ec.w = -1;
+    gst(S.extra + (n), en);
+    gst(S.extra + (cb), ec);
+    gs1(&S.extra[ncaj].z, -1);
+    gs1(&S.extra[nnjp1].z, -1);
+    gs1(&S.extra[ncai].z, -1);
+    gs1(&S.extra[ncim1].z, -1);
 }
 // repuls_add.f:14-47 / repuls_del_a.f:14-37 (single lane; n = N bead, cb = C bead)
 __device__ __noinline__ int repuls_add(int n, int Ln, int cb, int Lc) {
@@ -2618,11 +2570,6 @@ struct OnePass {
 // result lanes of beads i and j: entries take the lanes below
 constexpr int kLaneI = kW - 2, kLaneJ = kW - 1;
 
-__device__ inline Rec uni_words(Rec r) {
-    r.topo = uni(r.topo);
-    r.dyn = uni(r.dyn);
-    return r;
-}
 __device__ inline unsigned* lds_words(int off) { return (unsigned*)__builtin_assume_aligned(smem + off, 16); }
 // footprint marks, in LDS (ds operations) or in HBM at the device's L2
 __device__ inline void fp_or(const Hot& H, int b, unsigned bits) {
@@ -2643,6 +2590,101 @@ __device__ inline void fp_clear(const Hot& H, int b) {
         __hip_atomic_store((GLB unsigned*)((GLB char*)H.mark + (unsigned)b * 4u), 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// A lane's part of one gather that fetches everything an event needs of its
+// two beads, 8 bytes per lane: lanes 0-7 and 8-15 the records of i and j,
+// 16-17 the overrides of i, 18-21 the shoulder partners, 22-25 the bond
+// windows, 26-29 the list lengths (up and down of i, then of j).  As
+// wave-uniform 16-byte loads the same data took thirteen instructions of
+// 1 KB each through the CU's 64 B/cycle path.
+struct Gather {
+    const GLB char* base;
+    int sh;  // log2 of the buffer's element size
+};
+constexpr unsigned kGatherJ = 0x3330FF00u;  // lanes of bead j
+constexpr int kGatherLanes = 30;
+__device__ inline Gather load_gather(const SysDev& S) {
+    const int lane = lane_id();
+    // (addresses as numbers: a select between pointer fields keeps its
+    // struct in memory)
+    const unsigned long long rec = (unsigned long long)S.rec, ovr = (unsigned long long)S.ovr,
+                             ext = (unsigned long long)S.extra, bw = (unsigned long long)S.bw,
+                             nup = (unsigned long long)S.nup, ndn = (unsigned long long)S.ndn;
+    unsigned long long p = rec + (unsigned)(lane & 7) * 8u;
+    Gather G;
+    G.sh = 6;
+    if (lane >= 16) {
+        p = (lane < 18 ? ovr : (lane < 22 ? ext : bw)) + (unsigned)(lane & 1) * 8u;
+        G.sh = 4;
+    }
+    if (lane >= 26) {
+        p = (lane & 1) == 0 ? nup : ndn;
+        G.sh = 2;
+    }
+    G.base = (const GLB char*)p;
+    return G;
+}
+// lane l takes lane l + 3 of its row of 16
+__device__ inline double up3(double v) {
+    return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), 0x103, 0xf, 0xf, true),
+                            __builtin_amdgcn_mov_dpp(__double2loint(v), 0x103, 0xf, 0xf, true));
+}
+
+// The draws of an Andersen ghost collision (main.F90:1000-1041) from counter
+// rc on: bead, two accepted polar pairs and the next ghost time's uniform.
+struct GhostDraw {
+    int i, guard;
+    double v1, v2, r, w1, wr, tg;
+    unsigned long long rc;
+};
+// one draw after the other, for draws that a single sweep of 64 does not hold
+__device__ __noinline__ GhostDraw ghost_draw_serial(unsigned long long seed, unsigned long long rc, int N) {
+    GhostDraw d;
+    d.guard = 0;
+    do {
+        d.i = (int)(rng_u01(seed, 0, rc++) * N);
+    } while (d.i == N && ++d.guard < 1000);
+    do {
+        d.v1 = 2.0 * rng_u01(seed, 0, rc++) - 1.0;
+        d.v2 = 2.0 * rng_u01(seed, 0, rc++) - 1.0;
+        d.r = d.v1 * d.v1 + d.v2 * d.v2;
+    } while ((d.r == 0.0 || d.r >= 1.0) && ++d.guard < 1000);
+    do {
+        d.w1 = 2.0 * rng_u01(seed, 0, rc++) - 1.0;
+        const double w2 = 2.0 * rng_u01(seed, 0, rc++) - 1.0;
+        d.wr = d.w1 * d.w1 + w2 * w2;
+    } while ((d.wr == 0.0 || d.wr >= 1.0) && ++d.guard < 2000);
+    do {
+        d.tg = rng_u01(seed, 0, rc++);
+    } while ((d.tg < 1.e-18 || d.tg == 1.0) && ++d.guard < 3000);
+    d.rc = rc;
+    return d;
+}
+// the same draws, lane l holding the uniform of counter rc + l
+__device__ inline GhostDraw ghost_draw(unsigned long long seed, unsigned long long rc, int N) {
+    const int lane = lane_id();
+    const double u = rng_u01(seed, 0, rc + (unsigned long long)lane);
+    GhostDraw d;
+    d.guard = 0;
+    d.i = uni((int)(u * N));
+    // polar pairs start at the odd lanes
+    const double v1 = 2.0 * u - 1.0, v2 = 2.0 * __shfl_down(u, 1, kW) - 1.0;
+    const double r = v1 * v1 + v2 * v2;
+    const unsigned long long m = __ballot((lane & 1) && lane < kW - 2 && !(r == 0.0 || r >= 1.0));
+    const unsigned long long m2 = m & (m - 1);
+    if (d.i < N && m2 != 0) {
+        const int p1 = __ffsll((long long)m) - 1, p2 = __ffsll((long long)m2) - 1;
+        d.v1 = readlane_d(v1, p1);
+        d.v2 = readlane_d(v2, p1);
+        d.r = readlane_d(r, p1);
+        d.w1 = readlane_d(v1, p2);
+        d.wr = readlane_d(r, p2);
+        d.tg = readlane_d(u, p2 + 2);
+        d.rc = rc + (unsigned long long)(p2 + 3);
+        if (!(d.tg < 1.e-18 || d.tg == 1.0)) return d;
+    }
+    return ghost_draw_serial(seed, rc, N);
+}
+
 // One event of a round on one wavefront: a bead-pair event (outcome
 // resolution main.F90:1487-1634, dynamics, H-bond and shoulder bookkeeping
 // main.F90:641-921) or an Andersen ghost collision (main.F90:997-1049),
@@ -2650,11 +2692,16 @@ __device__ inline void fp_clear(const Hot& H, int b) {
 // e: the calendar entry; jp, ct: its partner and type; tf, nbin, coll: the
 // false time, bin and number of the event; bk: its place in the round.
 // Returns the round's accepted events if this one is committed, else 0.
-//
 // solo: the round's only event, which needs no footprint marks and no
 // acceptance.  The new calendar entries below the pool's edge go to the
 // wavefront's share of Batch::fresh and the rewritten blocks to
 // Batch::dirty[par].
+//
+// The pair's records stay spread over lanes 0 to 15 as the gather brings
+// them (one component per lane): the impulse, the nudge and the ghost's
+// velocity draw update them with one division for all components, and they
+// go to LDS and back to memory as they lie.  What decides control flow or is
+// shared by all lanes is read from the lanes into scalar registers.
 //
 // The rescheduling takes one pass of 64 lanes: a lane per candidate of i
 // and j (tags 0 and 1), per down-set entry (tags 2 and 3: its op partner i
@@ -2668,186 +2715,233 @@ __device__ inline void fp_clear(const Hot& H, int b) {
 // runs the multi-pass form, which holds any number.  What bounds an event
 // is the length of its dependent chain, so the code keeps wave-uniform
 // values in scalar registers and replaces divergent branches by selects.
-__device__ __forceinline__ int run_event(const Hot& H, int e, int jp, int ct, double tf, int nbin, long long coll, int bk,
-                                         bool solo, int par, int fsh) {
+__device__ __forceinline__ int run_event(const Hot& H, const Gather& G, int e, int jp, int ct, double tf, int nbin,
+                                         long long coll, int bk, bool solo, int par, int fsh) {
     const int lane = lane_id();
     const DevTables& T = tabs();
     Sc& mc = master();
     Batch& B = round_rec();
+    OnePass& W = *reinterpret_cast<OnePass*>(smem + H.o_w);
     const double interval_max = mc.interval_max, tbin_off = mc.tbin_off, sortsize = mc.sortsize;
     const bool batch = !solo;
-    int i = e, j = -1, flags = 0, st0 = 0, nb = 0, extra_blk = -1;
+    int flags = 0, st0 = 0, nb = 0, extra_blk = -1;
     bool xdel = false;
-    Rec ri, rj;
-    double2 bwi, bwj = make_double2(0.0, 0.0);
-    int4 xi, xj = make_int4(-1, -1, -1, -1);
-    int eui, edi, euj = 0, edj = 0, nui, ndi, nuj = 0, ndj = 0;
-    const int cap = H.cap;
+    const int cap = H.cap, sl = min(lane, cap - 1);
+    const bool jside = (lane & 8) != 0;        // lanes 8 to 15: bead j
+    const int comp = lane & 7;                 // component of a record's lane
+    const bool ispos = lane < 16 && comp < 3, isvel = lane < 16 && comp >= 3 && comp < 6;
     PH_BEGIN(tph);
-    if (e < H.N) {
-        j = jp;
-        ri = ld_at(H.rec, i);
-        rj = ld_at(H.rec, j);
-        const int4 oi_ = ld_at(H.ovr, i), xi_ = ld_at(H.extra, i), xj_ = ld_at(H.extra, j);
-        bwi = ld_at(H.bw, i);
-        bwj = ld_at(H.bw, j);
-        // the list rows, in flight while the outcome is resolved
-        const int nui_ = ld_at(H.nup, i), ndi_ = ld_at(H.ndn, i), nuj_ = ld_at(H.nup, j), ndj_ = ld_at(H.ndn, j);
-        const int sl = min(lane, cap - 1);
-        eui = ld_at(H.nb_up, i * cap + sl);
-        edi = ld_at(H.nb_dn, i * cap + sl);
-        euj = ld_at(H.nb_up, j * cap + sl);
-        edj = ld_at(H.nb_dn, j * cap + sl);
-        ri = uni_words(ri);
-        rj = uni_words(rj);
-        xi = uni(xi_);
-        xj = uni(xj_);
-        const int evcode = dyn_code(uni(oi_), j, static_t(ri.topo, rj.topo));  // ev_code(i, j)
-        const bool ok = !terminal_t(ri.topo) && !terminal_t(rj.topo);
-        const int idi = dyn_ident(ri.dyn), idj = dyn_ident(rj.dyn);
-        const int Li = topo_len(ri.topo), Lj = topo_len(rj.topo);
+    GhostDraw gd;
+    const bool ghost = e >= H.N;
+    int bead = e;
+    if (ghost) {
+        gd = ghost_draw(sdev().seed, mc.rc0, H.N);
+        bead = uni(gd.i);
+    }
+    // (selects below take plain values: one between captured variables or
+    // fields would be made on their addresses and keep them in memory)
+    const int i = bead, j = ghost ? -1 : jp;
+    const int lane_bead = jside ? j : i;
+    // ---- the pair's data and its list rows
+    const int jx = ghost ? i : j;
+    double val = 0.0;
+    if (lane < kGatherLanes)
+        val = *(const GLB double*)(G.base + ((unsigned)(((kGatherJ >> (lane & 31)) & 1u) ? jx : i) << G.sh));
+    const int eui = ld_at(H.nb_up, i * cap + sl), edi = ld_at(H.nb_dn, i * cap + sl);
+    const int euj = ld_at(H.nb_up, jx * cap + sl), edj = ld_at(H.nb_dn, jx * cap + sl);
+    auto lane_lo = [&](int l) __attribute__((always_inline)) { return __builtin_amdgcn_readlane(__double2loint(val), l); };
+    auto lane_hi = [&](int l) __attribute__((always_inline)) { return __builtin_amdgcn_readlane(__double2hiint(val), l); };
+    auto lane_int4 = [&](int l) __attribute__((always_inline)) { return make_int4(lane_lo(l), lane_hi(l), lane_lo(l + 1), lane_hi(l + 1)); };
+    const int topoi = lane_lo(7), topoj = lane_lo(15);
+    int dyni = lane_hi(7), dynj = lane_hi(15);
+    int4 xi = lane_int4(18), xj = lane_int4(20);
+    const int nui = lane_lo(26), ndi = lane_lo(27);
+    const int nuj = ghost ? 0 : lane_lo(28), ndj = ghost ? 0 : lane_lo(29);
+    const double bmi = readlane_d(val, 6);
+    auto store_pair = [&]() __attribute__((always_inline)) {  // the records of i and j to memory
+        if (lane < 16 && !(ghost && jside))
+            *(GLB double*)(G.base + ((unsigned)lane_bead << 6)) = val;
+    };
+    auto stage_pair = [&]() __attribute__((always_inline)) {  // ... to the wavefront's Pair in LDS
+        Pair& P = *ldsv().pair();
+        if (lane < 16) reinterpret_cast<double*>(jside ? &P.rj : &P.ri)[comp] = val;
+        if (lane == 0) {
+            P.i = i;
+            P.j = j;
+            P.xi = xi;
+            P.xj = xj;
+        }
+        wave_sync();
+    };
+    if (!ghost) {
+        const int evcode = dyn_code(lane_int4(16), j, static_t(topoi, topoj));  // ev_code(i, j)
+        const bool ok = !terminal_t(topoi) && !terminal_t(topoj);
+        const int idi = dyn_ident(dyni), idj = dyn_ident(dynj);
+        const int Li = topo_len(topoi), Lj = topo_len(topoj);
+        // the pair vectors: lane k < 6 of i minus lane k of j
+        const double df = val - __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(val), 0x128, 0xf, 0xf, true),
+                                                 __builtin_amdgcn_mov_dpp(__double2loint(val), 0x128, 0xf, 0xf, true));
+        Geo g;
+        {
+            const double vx = readlane_d(df, 3), vy = readlane_d(df, 4), vz = readlane_d(df, 5);
+            g.rx = min_image(readlane_d(df, 0) + vx * tf);
+            g.ry = min_image(readlane_d(df, 1) + vy * tf);
+            g.rz = min_image(readlane_d(df, 2) + vz * tf);
+            g.b = g.rx * vx + g.ry * vy + g.rz * vz;
+            g.r2 = 0.0;
+            g.v2 = 0.0;
+        }
         bool fence = false;
-        auto rec_of = [&](int m) { return m == i ? ri : (m == j ? rj : uni_words(ld_at(H.rec, m))); };
-        auto stage_pair = [&]() {
-            if (lane == 0) {
-                Pair& P = *ldsv().pair();
-                P.i = i;
-                P.j = j;
-                P.ri = ri;
-                P.rj = rj;
-            }
-            wave_sync();
-        };
-        if (ct == 7 || ct == 10 || ct == 12) flags |= kPairReadsSp;
+        auto dyn_of = [&](int m) __attribute__((always_inline)) { return m == i ? dyni : (m == j ? dynj : uni(gl1(&H.rec[m].dyn))); };
         if (ct == 7) {
+            flags |= kPairReadsSp;
             if (xi.w < 0 && xj.w < 0) {
                 if (ok) {
                     stage_pair();
-                    ct = (idi < idj ? shoulders_far(i, j, tf) : shoulders_far(j, i, tf)) ? 4 : 14;
+                    ct = uni((idi < idj ? shoulders_far(i, j, tf) : shoulders_far(j, i, tf)) ? 4 : 14);
                 } else {
                     // a random draw: its counter value is known only in order
                     if (bk >= 1) {
                         spec_abort_at(bk, nb);
                         return 0;
                     }
-                    ct = rng_u01(sdev().seed, 1, mc.rc1++) <= 0.2 ? 4 : 9;
-                    ct = uni(ct);
+                    const unsigned long long rc = mc.rc1;
+                    ct = uni(rng_u01(sdev().seed, 1, rc) <= 0.2 ? 4 : 9);
+                    if (lane == 0) mc.rc1 = rc + 1;
                 }
             } else
                 ct = 9;
         } else if (ct == 10) {
+            flags |= kPairReadsSp;
             const bool own = evcode < 45;
-            const int hbp = own ? xi.w : xj.w, idh = dyn_ident(rec_of(hbp).dyn);
+            const int hbp = own ? xi.w : xj.w, idh = dyn_ident(dyn_of(hbp));
             stage_pair();
             bool far;
             if (own)
                 far = idi < idh ? shoulders_far_3(i, hbp, j, tf) : shoulders_far_3(hbp, i, j, tf);
             else
                 far = idj < idh ? shoulders_far_3(j, hbp, i, tf) : shoulders_far_3(hbp, j, i, tf);
-            ct = far ? 5 : 15;
+            ct = uni(far ? 5 : 15);
         } else if (ct == 12) {
+            flags |= kPairReadsSp;
             const bool own = evcode < 45;
-            const Rec rx = own ? ri : rj;
             const int hbp = own ? xi.w : xj.w;
-            if (dyn_bptnr(rx.dyn) == hbp) {
-                Geo g;
-                const Rec rh = rec_of(hbp);
-                geo(rx, rh, tf, g);
-                const double d2 = g.rx * g.rx + g.ry * g.ry + g.rz * g.rz;
-                ct = (d2 - T.sigma_sq[dyn_ident(rx.dyn)][dyn_ident(rh.dyn)]) < 0.0 ? 13 : 6;
+            const int xd = own ? dyni : dynj;
+            if (dyn_bptnr(xd) == hbp) {
+                stage_pair();
+                const double d2 = pair_r2(own ? i : j, hbp, tf);
+                ct = uni((d2 - T.sigma_sq[dyn_ident(xd)][dyn_ident(dyn_of(hbp))]) < 0.0 ? 13 : 6);
             } else
                 ct = 15;
         }
-        ct = uni(ct);
         int status = 0;
-        if (ct < 14) {
-            eventdyn(T, ri, rj, bwi, dyn_bptnr(ri.dyn) == j, evcode, tf, ct, status);
+        double bd = 0.0;
+        int sgn = 0;
+        const double gx = g.rx, gy = g.ry, gz = g.rz;
+        const double rk = comp == 0 || comp == 3 ? gx : (comp == 1 || comp == 4 ? gy : gz);
+        const bool hit = ct < 14;
+        double ratio = 0.0;
+        const double bmj = readlane_d(val, 14);
+        if (hit) {
+            const double2 bwi = make_double2(readlane_d(val, 22), readlane_d(val, 23));
+            impulse(T, g, bmi, bmj, idi, idj, bwi, dyn_bptnr(dyni) == j, evcode, ct, ratio, bd, sgn, status);
             ct = uni(ct);
-        }
-        if (ct == 20) {
-            if (idi + idj == 5) {
-                ri.dyn = make_dyn(idi + 4, j);
-                rj.dyn = make_dyn(idj + 4, i);
-                if (ok) {
-                    if (bk >= 1) {
-                        spec_abort_at(bk, nb);
-                        return 0;
-                    }
-                    if (lane == 0) status |= idi < idj ? repuls_add(i, Li, j, Lj) : repuls_add(j, Lj, i, Li);
-                    fence = true;
-                }
-            }
-        } else if (ct == 21) {
-            if (idi <= 8) {
-                if (ok) {
-                    if (bk >= 1) {
-                        spec_abort_at(bk, nb);
-                        return 0;
-                    }
-                    if (lane == 0) status |= idi < idj ? repuls_del_a(i, Li, j, Lj) : repuls_del_a(j, Lj, i, Li);
-                    xdel = true;
-                    fence = true;
-                }
-                if (dyn_bptnr(ri.dyn) == j) {
-                    ri.dyn = make_dyn(idi - 4, -1);
-                    rj.dyn = make_dyn(idj - 4, -1);
-                }
-            }
-        } else if (ct == 24 || ct == 25) {
-            flags |= kPairReadsSp;
-            const bool own = evcode < 45;
-            const int hbp = own ? xi.w : xj.w, x = own ? i : j;
-            int xdyn = own ? ri.dyn : rj.dyn, hdyn = rec_of(hbp).dyn;
-            const int idx = dyn_ident(xdyn), idh = dyn_ident(hdyn);
-            bool changed = false;
-            if (ct == 24 && idx + idh == 5) {
-                xdyn = make_dyn(idx + 4, hbp);
-                hdyn = make_dyn(idh + 4, x);
-                changed = true;
-            } else if (ct == 25 && idx >= 5) {
-                xdyn = make_dyn(idx - 4, -1);
-                hdyn = make_dyn(idh - 4, -1);
-                changed = true;
-            }
-            if (changed) {
-                if (own) ri.dyn = xdyn;
-                else rj.dyn = xdyn;
-                if (hbp == i) ri.dyn = hdyn;
-                else if (hbp == j) rj.dyn = hdyn;
-                else {
-                    if (bk >= 1) {
-                        spec_abort_at(bk, nb);
-                        return 0;
-                    }
-                    if (lane == 0) gs1(&H.rec[hbp].dyn, hdyn);
-                    fence = true;
-                }
-            }
-        } else if (ct == 14 || ct == 15 || ct == 16) {
+            sgn = uni(sgn);
+        } else {
             // bumped.f: push the pair off the discontinuity
-            Geo g;
-            geo(ri, rj, tf, g);
-            const double bd = evcode >= 40 ? kSm * sqrt(T.shlddia_sq[idi][idj]) : kSm * sqrt(T.welldia_sq[idi][idj]);
-            nudge(ri, rj, bd, g, g.b < 0.0 ? -1 : +1);
-            if ((ct == 14 || ct == 16) && ok) {
-                if (bk >= 1) {
-                    spec_abort_at(bk, nb);
-                    return 0;
+            bd = evcode >= 40 ? kSm * sqrt(T.shlddia_sq[idi][idj]) : kSm * sqrt(T.welldia_sq[idi][idj]);
+            sgn = uni(g.b < 0.0 ? -1 : 1);
+        }
+        if (sgn != 0) {
+            const double nd = bd * rk;
+            val = ispos ? ((sgn < 0) != jside ? val - nd : val + nd) : val;
+        }
+        if (hit) {
+            // v -+ dv / m, x +- dv tf / m: one division per component lane
+            const double dv = ratio * rk;
+            const double q = (ispos ? dv * tf : dv) / (jside ? bmj : bmi);
+            const bool neg = isvel ? !jside : jside;
+            val = ispos || isvel ? (neg ? val - q : val + q) : val;
+        }
+        if (ct >= 20) {
+            if (ct == 20) {
+                if (idi + idj == 5) {
+                    dyni = make_dyn(idi + 4, j);
+                    dynj = make_dyn(idj + 4, i);
+                    if (ok) {
+                        if (bk >= 1) {
+                            spec_abort_at(bk, nb);
+                            return 0;
+                        }
+                        if (lane == 0) status |= idi < idj ? repuls_add(i, Li, j, Lj) : repuls_add(j, Lj, i, Li);
+                        fence = true;
+                    }
                 }
-                if (lane == 0) {
-                    if (ct == 14)
-                        status |= idi < idj ? repuls_add(i, Li, j, Lj) : repuls_add(j, Lj, i, Li);
-                    else
-                        status |= idi < idj ? repuls_del_a(i, Li, j, Lj) : repuls_del_a(j, Lj, i, Li);
+            } else if (ct == 21) {
+                if (idi <= 8) {
+                    if (ok) {
+                        if (bk >= 1) {
+                            spec_abort_at(bk, nb);
+                            return 0;
+                        }
+                        if (lane == 0) status |= idi < idj ? repuls_del_a(i, Li, j, Lj) : repuls_del_a(j, Lj, i, Li);
+                        xdel = true;
+                        fence = true;
+                    }
+                    if (dyn_bptnr(dyni) == j) {
+                        dyni = make_dyn(idi - 4, -1);
+                        dynj = make_dyn(idj - 4, -1);
+                    }
                 }
-                xdel = ct == 16;
-                fence = true;
+            } else if (ct == 24 || ct == 25) {
+                flags |= kPairReadsSp;
+                const bool own = evcode < 45;
+                const int hbp = own ? xi.w : xj.w, x = own ? i : j;
+                int xdyn = own ? dyni : dynj, hdyn = dyn_of(hbp);
+                const int idx = dyn_ident(xdyn), idh = dyn_ident(hdyn);
+                bool changed = false;
+                if (ct == 24 && idx + idh == 5) {
+                    xdyn = make_dyn(idx + 4, hbp);
+                    hdyn = make_dyn(idh + 4, x);
+                    changed = true;
+                } else if (ct == 25 && idx >= 5) {
+                    xdyn = make_dyn(idx - 4, -1);
+                    hdyn = make_dyn(idh - 4, -1);
+                    changed = true;
+                }
+                if (changed) {
+                    if (own) dyni = xdyn;
+                    else dynj = xdyn;
+                    if (hbp == i) dyni = hdyn;
+                    else if (hbp == j) dynj = hdyn;
+                    else {
+                        if (bk >= 1) {
+                            spec_abort_at(bk, nb);
+                            return 0;
+                        }
+                        if (lane == 0) gs1(&H.rec[hbp].dyn, hdyn);
+                        fence = true;
+                    }
+                }
             }
+            const int di = dyni, dj = dynj;
+            const int dd = jside ? dj : di;
+            val = lane < 16 && comp == 7 ? __hiloint2double(dd, __double2loint(val)) : val;
+        } else if ((ct == 14 || ct == 16) && ok) {
+            if (bk >= 1) {
+                spec_abort_at(bk, nb);
+                return 0;
+            }
+            if (lane == 0) {
+                if (ct == 14)
+                    status |= idi < idj ? repuls_add(i, Li, j, Lj) : repuls_add(j, Lj, i, Li);
+                else
+                    status |= idi < idj ? repuls_del_a(i, Li, j, Lj) : repuls_del_a(j, Lj, i, Li);
+            }
+            xdel = ct == 16;
+            fence = true;
         }
-        if (bk < 1) {  // a speculative event writes its pair once committed
-            if (lane == 0) st_at(H.rec, i, ri);
-            if (lane == 1) st_at(H.rec, j, rj);
-        }
+        if (bk < 1) store_pair();  // a speculative event writes its pair once committed
         if (fence) {
             flags |= kPairWroteSp;
             // shoulder tables changed: make them visible before the predictions
@@ -2856,98 +2950,63 @@ __device__ __forceinline__ int run_event(const Hot& H, int e, int jp, int ct, do
             xj = uni(ld_at(H.extra, j));
         }
         st0 = wave_status(status);
-        nui = uni(nui_);
-        ndi = uni(ndi_);
-        nuj = uni(nuj_);
-        ndj = uni(ndj_);
         PH_END(sdev(), kPhPair, tph);
     } else {
         const SysDev& S = sdev();
-        const unsigned long long seed = S.seed;
         const int N = H.N;
-        unsigned long long rc = mc.rc0;
-        int guard = 0;
-        do {
-            i = (int)(rng_u01(seed, 0, rc++) * N);
-        } while (i == N && ++guard < 1000);
-        i = uni(i);
-        ri = ld_at(H.rec, i);
-        bwi = ld_at(H.bw, i);
-        const int4 xi_ = ld_at(H.extra, i);
-        const int nui_ = ld_at(H.nup, i), ndi_ = ld_at(H.ndn, i), sl = min(lane, cap - 1);
-        eui = ld_at(H.nb_up, i * cap + sl);
-        edi = ld_at(H.nb_dn, i * cap + sl);
-        ri = uni_words(ri);
-        const double bm = ri.bm;
-        ri.x = ri.x + ri.vx * tf;
-        ri.y = ri.y + ri.vy * tf;
-        ri.z = ri.z + ri.vz * tf;
-        double v1, v2, r, fact;
-        do {
-            v1 = 2.0 * rng_u01(seed, 0, rc++) - 1.0;
-            v2 = 2.0 * rng_u01(seed, 0, rc++) - 1.0;
-            r = v1 * v1 + v2 * v2;
-        } while ((r == 0.0 || r >= 1.0) && ++guard < 1000);
-        fact = sqrt(-2.0 * S.setemp * bm * dlog(r) / r);
-        ri.vx = v1 * fact / bm;
-        ri.vy = v2 * fact / bm;
-        do {
-            v1 = 2.0 * rng_u01(seed, 0, rc++) - 1.0;
-            v2 = 2.0 * rng_u01(seed, 0, rc++) - 1.0;
-            r = v1 * v1 + v2 * v2;
-        } while ((r == 0.0 || r >= 1.0) && ++guard < 2000);
-        fact = sqrt(-2.0 * S.setemp * bm * dlog(r) / r);
-        ri.vz = v1 * fact / bm;
-        ri.x = ri.x - ri.vx * tf;
-        ri.y = ri.y - ri.vy * tf;
-        ri.z = ri.z - ri.vz * tf;
-        double tgho;
-        do {
-            tgho = rng_u01(seed, 0, rc++);
-        } while ((tgho < 1.e-18 || tgho == 1.0) && ++guard < 3000);
-        if (guard >= 1000) st0 = kErrRng;
-        const double tg = -1.0 * dlog(tgho) * S.avegtime + tf;
+        // the three logarithms in lanes 0 to 2, the velocity scales in lanes 0 and 1
+        const double d1 = gd.r, d2 = gd.wr, d3 = gd.tg, p1 = gd.v1, p2 = gd.v2, p3 = gd.w1;
+        const double lr = lane == 0 ? d1 : (lane == 1 ? d2 : d3);
+        const double lg = dlog(lr);
+        const double fact = sqrt(-2.0 * S.setemp * bmi * lg / lr);
+        const double f0 = readlane_d(fact, 0), f1 = readlane_d(fact, 1);
+        const double v_old = up3(val);  // (lane moves need every lane: not inside a select)
+        val = lane < 3 ? val + v_old * tf : val;
+        const double nv = (lane == 3 ? p1 * f0 : (lane == 4 ? p2 * f0 : p3 * f1)) / bmi;
+        val = lane >= 3 && lane < 6 ? nv : val;
+        const double v_new = up3(val);
+        val = lane < 3 ? val - v_new * tf : val;
+        if (gd.guard >= 1000) st0 = kErrRng;
+        const double tg = -1.0 * readlane_d(lg, 2) * S.avegtime + tf;
         int status = 0;
         Leaf g;
         g.tim = tg;
         g.nptnr = -2;
         g.meta = make_meta(bin_of(interval_max, tbin_off, sortsize, nbin, tg, status), -2);
+        store_pair();
         if (lane == 0) {
-            st_at(H.rec, i, ri);
             leaf_st(H, N, g);
             stamp_st(H, N, mk_stamp(coll, 1));  // added before partial_events' adds (main.F90:1041-1049)
-            mc.rc0 = rc;
+            mc.rc0 = gd.rc;
             mc.numghosts++;
             B.gbead = i;
         }
         if (status && !st0) st0 = status;
-        if (tf < mc.old_tfalse) {
-            tf = mc.old_tfalse;
+        const double tf_old = uni(mc.old_tfalse);
+        if (tf < tf_old) {
+            tf = tf_old;
             if (lane == 0) mc.tfalse = tf;
         }
-        rj = ri;
-        xi = uni(xi_);
-        nui = uni(nui_);
-        ndi = uni(ndi_);
+        xj = make_int4(-1, -1, -1, -1);
         extra_blk = N / kBlk;
         ct = 0;
-        wave_sync();
         PH_END(sdev(), kPhGhost, tph);
     }
     if (lane == 0) B.ty[bk] = ct;
 
-    OnePass& W = *reinterpret_cast<OnePass*>(smem + H.o_w);
     const unsigned long long below = (1ull << lane) - 1ull;
     // place of i's add among this event's calendar adds (a ghost event adds
     // its own entry first); j follows, then the down set in list order
     const int sub0 = j >= 0 ? 1 : 2;
     const double T0 = interval_max + kLt - tf;
-    const int kNoStat = 0xFF << 24;
+    // an entry of the list: bead | up-row length of a down bead << 16 (127:
+    // not known) | static code << 24 (63: not known) | tag << 30
+    const int kNoRow = (0x3F << 24) | (127 << 16);
     const bool has_x = (xi.x & xi.y & xi.z & xj.x & xj.y & xj.z) != -1;  // any shoulder partner
     bool multi = nui + ndi + nuj + ndj + (has_x ? 12 : 0) > kLaneI;
-    int ncand = 0, nDi = 0, n0 = 0, ntot = 0, m = 0, tag = 0, stat = 0, nspec = 0, myslot = -1;
+    int ncand = 0, n0 = 0, ntot = 0, m = 0, tag = 0, stat = 0, nspec = 0;
     int cI = 0, cJ = 0, pI = lane, pJ = lane;
-    bool first = false, is_i = false, spec = false, dn = false, act = false;
+    bool first = false, is_i = false, spec = false, dn = false, act = false, late = false;
     unsigned long long dups = 0;
     Rec mine;
     int4 om = make_int4(-1, -1, -1, -1);
@@ -2960,74 +3019,73 @@ __device__ __forceinline__ int run_event(const Hot& H, int e, int jp, int ct, do
     if (!multi) {
         // ---- the entry list: candidates of i, candidates of j, the down set
         //      in reference order (i's down list and lower shoulder partners, then j's)
-        int w = nui;
-        if (lane < nui) W.lst[lane] = eui;
-        auto one = [&](int b, int tg) {
-            if (lane == 0) W.lst[w] = b | (tg << 16) | kNoStat;
-            ++w;
-        };
-        if (has_x) {
-            if (xi.x > i) one(xi.x, 0);
-            if (xi.y > i) one(xi.y, 0);
-            if (xi.z > i) one(xi.z, 0);
-        }
-        if (lane < nuj) W.lst[w + lane] = euj | (1 << 16);
-        w += nuj;
-        if (has_x && j >= 0) {
-            if (xj.x > j) one(xj.x, 1);
-            if (xj.y > j) one(xj.y, 1);
-            if (xj.z > j) one(xj.z, 1);
-        }
-        ncand = w;
-        if (lane < ndi) W.lst[w + lane] = edi | (2 << 16);
-        w += ndi;
-        if (has_x) {
-            if (xi.x >= 0 && xi.x < i) one(xi.x, 2);
-            if (xi.y >= 0 && xi.y < i) one(xi.y, 2);
-            if (xi.z >= 0 && xi.z < i) one(xi.z, 2);
-        }
-        nDi = w - ncand;
-        if (j >= 0) {
+        const int kDnI = (int)0x80000000u, kDnJ = (int)0xC0000000u, kCaJ = 0x40000000;
+        int nDi;
+        if (!has_x) {
             const bool keep = lane < ndj && (edj & 0xFFFF) != i;
             const unsigned long long bal = __ballot(keep);
-            if (keep) W.lst[w + __popcll(bal & below)] = edj | (3 << 16);
-            w += __popcll(bal);
-            if (has_x) {
-                if (xj.x >= 0 && xj.x < j) one(xj.x, 3);
-                if (xj.y >= 0 && xj.y < j) one(xj.y, 3);
-                if (xj.z >= 0 && xj.z < j) one(xj.z, 3);
+            ncand = nui + nuj;
+            nDi = ndi;
+            n0 = ncand + ndi + __popcll(bal);
+            if (lane < nui) W.lst[lane] = eui;
+            if (lane < nuj) W.lst[nui + lane] = euj | kCaJ;
+            if (lane < ndi) W.lst[ncand + lane] = edi | kDnI;
+            if (keep) W.lst[ncand + ndi + __popcll(bal & below)] = edj | kDnJ;
+        } else {
+            int w = nui;
+            if (lane < nui) W.lst[lane] = eui;
+            auto one = [&](int b, int tg) __attribute__((always_inline)) {
+                if (lane == 0) W.lst[w] = b | tg | kNoRow;
+                ++w;
+            };
+            auto uppers = [&](const int4& x, int b, int tg) __attribute__((always_inline)) {
+                if (x.x > b) one(x.x, tg);
+                if (x.y > b) one(x.y, tg);
+                if (x.z > b) one(x.z, tg);
+            };
+            auto lowers = [&](const int4& x, int b, int tg) __attribute__((always_inline)) {
+                if (x.x >= 0 && x.x < b) one(x.x, tg);
+                if (x.y >= 0 && x.y < b) one(x.y, tg);
+                if (x.z >= 0 && x.z < b) one(x.z, tg);
+            };
+            uppers(xi, i, 0);
+            if (lane < nuj) W.lst[w + lane] = euj | kCaJ;
+            w += nuj;
+            if (j >= 0) uppers(xj, j, kCaJ);
+            ncand = w;
+            if (lane < ndi) W.lst[w + lane] = edi | kDnI;
+            w += ndi;
+            lowers(xi, i, kDnI);
+            nDi = w - ncand;
+            if (j >= 0) {
+                const bool keep = lane < ndj && (edj & 0xFFFF) != i;
+                const unsigned long long bal = __ballot(keep);
+                if (keep) W.lst[w + __popcll(bal & below)] = edj | kDnJ;
+                w += __popcll(bal);
+                lowers(xj, j, kDnJ);
             }
+            n0 = w;
         }
-        n0 = w;
-        if (lane < 2) {
-            BaseRec& b = W.base[lane];
-            b.r = lane == 0 ? ri : rj;
-            b.bw = lane == 0 ? bwi : bwj;
-            b.idx = lane == 0 ? i : j;
-        }
+        // the base beads i and j
+        if (lane < 16) reinterpret_cast<double*>(&W.base[jside ? 1 : 0].r)[comp] = val;
+        if (lane >= 22 && lane < 26) reinterpret_cast<double*>(&W.base[(lane - 22) >> 1].bw)[lane & 1] = val;
+        if (lane < 2) W.base[lane].idx = lane == 0 ? i : j;
         if (lane < kOwners) W.tkey[lane] = ~0ull;
         wave_sync();
         PH_END(sdev(), kPhRows, tph);
-        // ---- every entry's bead; a down entry's own calendar entry, bond
-        //      window, shoulder partners and row length
+        // ---- every entry's bead; a down entry's own calendar entry and bond window
         act = lane < n0;
         const int ent = act ? W.lst[lane] : 0;
         m = ent & 0xFFFF;
-        tag = (ent >> 16) & 0xFF;
-        stat = (ent >> 24) & 0xFF;
+        tag = (int)((unsigned)ent >> 30);
+        stat = (ent >> 24) & 0x3F;
         dn = act && lane >= ncand;
-        int nul = 0;
-        int4 xl = make_int4(-1, -1, -1, -1);
+        if (dn) lf0 = leaf_ld(H, m);
         if (act) {
             mine = ld_at(H.rec, m);
             om = ld_at(H.ovr, m);
         }
-        if (dn) {
-            lf0 = leaf_ld(H, m);
-            nul = ld_at(H.nup, m);
-            xl = ld_at(H.extra, m);
-            bwm = ld_at(H.bw, m);
-        }
+        if (dn) bwm = ld_at(H.bw, m);
         // ---- down entries of one bead: its ops with i and with j, and the
         //      lane of an op of each kind (equal predictions)
         {
@@ -3056,58 +3114,66 @@ __device__ __forceinline__ int run_event(const Hot& H, int e, int jp, int ct, do
         nspec = __popcll(specm);
         multi = nspec > kMaxSpec;
         if (!multi) {
-            myslot = __popcll(specm & below);
-            // rows of the beads recomputed, all in flight together
-            int sent[kMaxSpec];
-            const int sl = min(lane, cap - 1);
-            {
-                unsigned long long sm = specm;
-#pragma unroll
-                for (int q = 0; q < kMaxSpec; ++q) {
-                    if (q < nspec) {
-                        const int l = __builtin_amdgcn_readlane(m, __ffsll((long long)sm) - 1);
-                        sm &= sm - 1;
-                        sent[q] = ld_at(H.nb_up, l * cap + sl);
-                    }
+            // ---- their candidates: up rows (the entry carries the length)
+            //      and upper shoulder partners, a lane each from n0 on
+            int4 xl = make_int4(-1, -1, -1, -1);
+            if (spec) xl = ld_at(H.extra, m);
+            int w2 = n0, rowat = -1, q = 0;
+            for (unsigned long long sm = specm; sm; sm &= sm - 1, ++q) {
+                const int src = __ffsll((long long)sm) - 1;
+                const int l = __builtin_amdgcn_readlane(m, src);
+                int nu = (__builtin_amdgcn_readlane(ent, src) >> 16) & 127;
+                if (nu == 127) nu = uni(gl1(H.nup + l));
+                const int k = lane - w2;
+                if (k >= 0 && k < nu) {
+                    rowat = l * cap + k;
+                    tag = 4 + q;
                 }
+                w2 += nu;
             }
-            PH_END(sdev(), kPhScan, tph);
-            // the pair's own beads take their new states
-            if (act && (m == i || m == j)) mine = W.base[m == i ? 0 : 1].r;
-            if (spec) {
-                BaseRec& b = W.base[2 + myslot];
-                b.r = mine;
-                b.bw = bwm;
-                b.idx = m;
-            }
+            late = lane >= n0 && lane < w2;
+            int ent2 = 0;
+            if (late) ent2 = ld_at(H.nb_up, rowat);
             const unsigned long long xm = __ballot(spec && (xl.x > m || xl.y > m || xl.z > m));
-            unsigned long long sm = specm;
-            int w2 = n0;
-#pragma unroll
-            for (int q = 0; q < kMaxSpec; ++q) {
-                if (q < nspec) {
+            if (xm) {
+                // shoulder partners follow their rows' order within an owner
+                // because the owner's least position wins only among equal times
+                q = 0;
+                for (unsigned long long sm = specm; sm; sm &= sm - 1, ++q) {
                     const int src = __ffsll((long long)sm) - 1;
-                    sm &= sm - 1;
-                    const int nu = __builtin_amdgcn_readlane(nul, src);
-                    const bool sx = (xm >> src) & 1ull;
-                    if (w2 + nu + (sx ? 3 : 0) > kLaneI) {
-                        multi = true;
-                    } else {
-                        if (lane < nu) W.lst[w2 + lane] = sent[q] | ((4 + q) << 16);
-                        w2 += nu;
-                        if (sx) {
-                            const int l = __builtin_amdgcn_readlane(m, src);
-                            const int x0 = __builtin_amdgcn_readlane(xl.x, src), x1 = __builtin_amdgcn_readlane(xl.y, src),
-                                      x2 = __builtin_amdgcn_readlane(xl.z, src);
-                            const int tg = ((4 + q) << 16) | kNoStat;
-                            if (x0 > l) { if (lane == 0) W.lst[w2] = x0 | tg; ++w2; }
-                            if (x1 > l) { if (lane == 0) W.lst[w2] = x1 | tg; ++w2; }
-                            if (x2 > l) { if (lane == 0) W.lst[w2] = x2 | tg; ++w2; }
+                    if (!((xm >> src) & 1ull)) continue;
+                    const int l = __builtin_amdgcn_readlane(m, src);
+#pragma unroll
+                    for (int u = 0; u < 3; ++u) {
+                        const int x = __builtin_amdgcn_readlane(u == 0 ? xl.x : (u == 1 ? xl.y : xl.z), src);
+                        if (x > l) {
+                            if (lane == w2) {
+                                ent2 = x | kNoRow;
+                                tag = 4 + q;
+                                late = true;
+                            }
+                            ++w2;
                         }
                     }
                 }
             }
+            multi = w2 > kLaneI;
             ntot = w2;
+            PH_END(sdev(), kPhScan, tph);
+            // the pair's own beads take their new states
+            if (act && (m == i || m == j)) mine = W.base[m == i ? 0 : 1].r;
+            if (spec) {
+                BaseRec& b = W.base[2 + __popcll(specm & below)];
+                b.r = mine;
+                b.bw = bwm;
+                b.idx = m;
+            }
+            if (late && !multi) {
+                m = ent2 & 0xFFFF;
+                stat = (ent2 >> 24) & 0x3F;
+                mine = ld_at(H.rec, m);
+                om = ld_at(H.ovr, m);
+            }
         }
     }
     if (multi) {
@@ -3118,20 +3184,18 @@ __device__ __forceinline__ int run_event(const Hot& H, int e, int jp, int ct, do
             return 0;
         }
         const Lds& L = ldsv();
-        if (lane == 0) {
+        stage_pair();
+        {
             Pair& P = *L.pair();
-            P.i = i;
-            P.j = j;
-            P.flags = flags;
-            P.pad = 0;
-            P.ri = ri;
-            P.rj = rj;
-            P.bwi = bwi;
-            P.bwj = j >= 0 ? bwj : bwi;
-            P.xi = xi;
-            P.xj = xj;
+            if (lane >= 22 && lane < 26) reinterpret_cast<double*>(lane < 24 || ghost ? &P.bwi : &P.bwj)[lane & 1] = val;
+            if (ghost && lane >= 22 && lane < 24) reinterpret_cast<double*>(&P.bwj)[lane & 1] = val;
+            if (ghost && lane < 8) reinterpret_cast<double*>(&P.rj)[comp] = val;
+            if (lane == 0) {
+                P.flags = flags;
+                P.pad = 0;
+                if (st0 && !mc.status) mc.status = st0;
+            }
         }
-        if (lane == 0 && st0 && !mc.status) mc.status = st0;
         wave_sync();
         reschedule(sdev(), T, L, *L.sc(), *L.pair(), extra_blk, xdel, batch ? 0 : -1);
         if (solo) bar_to(nb, 1);
@@ -3143,16 +3207,6 @@ __device__ __forceinline__ int run_event(const Hot& H, int e, int jp, int ct, do
             B.st_rep[0] = 0;
         }
         return batch ? accepted(B) : 1;
-    }
-    wave_sync();
-    const bool late = lane >= n0 && lane < ntot;
-    if (late) {
-        const int ent = W.lst[lane];
-        m = ent & 0xFFFF;
-        tag = (ent >> 16) & 0xFF;
-        stat = (ent >> 24) & 0xFF;
-        mine = ld_at(H.rec, m);
-        om = ld_at(H.ovr, m);
     }
     PH_END(sdev(), kPhLoads, tph);
     const int own = lane == kLaneI ? i : (lane == kLaneJ ? j : -1);  // the result lanes' beads
@@ -3169,7 +3223,7 @@ __device__ __forceinline__ int run_event(const Hot& H, int e, int jp, int ct, do
     //      whose entry exactly one earlier event rewrote by single-pair
     //      updates only, and whose own updates here are single-pair ones,
     //      replays those updates on that event's entry once it is written.
-    auto clear_marks = [&]() {
+    auto clear_marks = [&]() __attribute__((always_inline)) {
         if (dn) fp_clear(H, m);
         if (own >= 0) fp_clear(H, own);
         if (bk == 0 && sp_w && sp >= 0) fp_clear(H, sp);
@@ -3177,16 +3231,7 @@ __device__ __forceinline__ int run_event(const Hot& H, int e, int jp, int ct, do
     if (batch) {
         const unsigned sbit = 1u << bk, lbit = 1u << (8 + bk), fbit = 1u << (16 + bk);
         if ((bk == 0 && sp_w) || (bk >= 1 && sp_r)) {
-            if (lane == 0) {
-                Pair& P = *ldsv().pair();
-                P.i = i;
-                P.j = j;
-                P.ri = ri;
-                P.rj = rj;
-                P.xi = xi;
-                P.xj = xj;
-            }
-            wave_sync();
+            stage_pair();
             sp = shoulder_bead(sdev(), *ldsv().pair(), lane);
         }
         if (lane == 0) B.wdone[bk] = 0;
@@ -3229,6 +3274,7 @@ __device__ __forceinline__ int run_event(const Hot& H, int e, int jp, int ct, do
     PH_ADDN(sdev(), kPhNPred, ntot);
     PH_ADDN(sdev(), kPhNPredPass, 1);
     act = lane < ntot;
+    wave_sync();
     double tij = 1000000000.0;
     int ty = 0, status = 0;
     const int slot = tag < 4 ? (tag & 1) : tag - 2;
@@ -3240,7 +3286,7 @@ __device__ __forceinline__ int run_event(const Hot& H, int e, int jp, int ct, do
         if (late && (m == i || m == j)) mine = W.base[m == i ? 0 : 1].r;
         Geo g;
         geo(rb, mine, tf, g);  // the order of the two only flips the signs of vectors
-        if (stat == 0xFF) stat = static_t(mine.topo, rb.topo);  // symmetric in its beads
+        if (stat == 0x3F) stat = static_t(mine.topo, rb.topo);  // symmetric in its beads
         const int code = dyn_code(om, bidx, stat);  // ev_code(m, x) of a candidate, ev_code(l, p) of a down bead
         const int adyn = dn ? mine.dyn : rb.dyn, cdyn = dn ? rb.dyn : mine.dyn;  // the lower bead's first
         const double2 bwa = make_double2(dn ? bwm.x : bwb.x, dn ? bwm.y : bwb.y);
@@ -3263,7 +3309,7 @@ __device__ __forceinline__ int run_event(const Hot& H, int e, int jp, int ct, do
     // owner results (full recompute rule: an event only below T0)
     double ti = T0 + tf, tj = T0 + tf;
     int pi = -1, ci = -1, pj = -1, cj = -1;
-    auto owner_min = [&](unsigned long long seg, double& t, int& p, int& c) {
+    auto owner_min = [&](unsigned long long seg, double& t, int& p, int& c) __attribute__((always_inline)) {
         const unsigned long long w = win & seg;
         if (w) {
             const int src = __ffsll((long long)w) - 1;
@@ -3275,16 +3321,15 @@ __device__ __forceinline__ int run_event(const Hot& H, int e, int jp, int ct, do
             }
         }
     };
-    const unsigned long long tag1 = __ballot(act && tag == 1), tag0 = __ballot(act && tag == 0);
+    const unsigned long long tag0 = __ballot(act && tag == 0), tag1 = __ballot(act && tag == 1);
     owner_min(tag0, ti, pi, ci);
     owner_min(tag1, tj, pj, cj);
     double ft = T0 + tf;  // the bead's own full recompute
     int fp = -1, fc = -1;
     {
-        unsigned long long sm = specm;
-        for (int q = 0; q < nspec; ++q) {
+        int q = 0;
+        for (unsigned long long sm = specm; sm; sm &= sm - 1, ++q) {
             const int src = __ffsll((long long)sm) - 1;
-            sm &= sm - 1;
             double t = T0 + tf;
             int p = -1, c = -1;
             owner_min(__ballot(act && tag == 4 + q), t, p, c);
@@ -3310,7 +3355,7 @@ __device__ __forceinline__ int run_event(const Hot& H, int e, int jp, int ct, do
         fp = pi;
         fc = ci;
     }
-    auto op = [&](bool on, int p, double t, int y) {
+    auto op = [&](bool on, int p, double t, int y) __attribute__((always_inline)) {
         const bool full = on && st_p == p;
         const bool single = on && !full;
         if (single && y == -99) status = kErrBadCode;
@@ -3323,14 +3368,12 @@ __device__ __forceinline__ int run_event(const Hot& H, int e, int jp, int ct, do
         modified |= full || less;
     };
     op(first && cI >= 1, i, sI, yI);
-    if (__ballot(first && cI >= 2)) {
+    if (has_x && __ballot(first && cI >= 2)) {
         for (int k = 2; k <= 4; ++k) op(first && cI >= k, i, sI, yI);
     }
-    if (j >= 0) {
-        op(first && cJ >= 1, j, sJ, yJ);
-        if (__ballot(first && cJ >= 2)) {
-            for (int k = 2; k <= 4; ++k) op(first && cJ >= k, j, sJ, yJ);
-        }
+    op(first && cJ >= 1, j, sJ, yJ);
+    if (has_x && __ballot(first && cJ >= 2)) {
+        for (int k = 2; k <= 4; ++k) op(first && cJ >= k, j, sJ, yJ);
     }
     // bead i's state lives in (ti, pi, ci) and is written with i's entry
     const unsigned long long im = __ballot(is_i);
@@ -3358,22 +3401,22 @@ __device__ __forceinline__ int run_event(const Hot& H, int e, int jp, int ct, do
     if (wr) lf.meta = make_meta(bin_of(interval_max, tbin_off, sortsize, nbin, st_t, status), st_c);
     status = wave_status(status);
     if (status && !st0) st0 = status;
+    // the keys they will have; a ghost event's own new entry takes the idle lane of j
+    Key kn = wr ? leaf_key(lf, rb) : empty_key();
+    unsigned long long ks = stp;
+    if (ghost && lane == kLaneJ) {
+        kn = leaf_key(leaf_ld(H, H.N), H.N);
+        ks = mk_stamp(coll, 1);  // re-added by this ghost event
+    }
     PH_END(sdev(), kPhDown, tph);
     int A = 1;
     if (batch) {
         // report the least new calendar key and the status, then commit
         // only within the round's accepted prefix
-        Key kn = wr ? leaf_key(lf, rb) : empty_key();
-        unsigned long long ks = stp;
-        if (j < 0 && lane == kLaneJ) {
-            // a ghost event leading the round: its next ghost time
-            kn = leaf_key(leaf_ld(H, H.N), H.N);
-            ks = mk_stamp(coll, 1);  // re-added by this ghost event
-        }
         unsigned long long kns = 0;
-        kn = key_min_wave_st(kn, ks, kns);
+        const Key kl = key_min_wave_st(kn, ks, kns);
         if (lane == 0) {
-            B.knew[bk] = kn;
+            B.knew[bk] = kl;
             B.knew_st[bk] = kns;
             B.st[bk] = st0;
             B.st_rep[bk] = 0;
@@ -3384,10 +3427,7 @@ __device__ __forceinline__ int run_event(const Hot& H, int e, int jp, int ct, do
         clear_marks();
         A = accepted(B);
         if (bk >= A) return 0;
-        if (bk >= 1) {
-            if (lane == 0) st_at(H.rec, i, ri);
-            if (lane == 1) st_at(H.rec, j, rj);
-        }
+        if (bk >= 1) store_pair();
         if (bk == 0 && st0 && lane == 0 && !mc.status) mc.status = st0;
     } else {
         if (lane == 0) {
@@ -3423,6 +3463,7 @@ __device__ __forceinline__ int run_event(const Hot& H, int e, int jp, int ct, do
                 wb = true;
             }
             if (wb) lf.meta = make_meta(bin_of(interval_max, tbin_off, sortsize, nbin, lf.tim, st2), rc);
+            kn = wb ? leaf_key(lf, rb) : empty_key();
         }
         st2 = wave_status(st2);
         if (st2 && lane == 0) B.st_rep[bk] = st2;
@@ -3432,19 +3473,12 @@ __device__ __forceinline__ int run_event(const Hot& H, int e, int jp, int ct, do
         stamp_st(H, rb, stp);
     }
     {
-        Key kx = wb ? leaf_key(lf, rb) : empty_key();
-        bool put = wb;
-        int blk_ = rb / kBlk;
-        if (extra_blk >= 0 && lane == kLaneJ) {  // the ghost entry
-            kx = leaf_key(leaf_ld(H, H.N), H.N);
-            put = true;
-            blk_ = extra_blk;
-        }
-        if (put) dirty_or(par, blk_);
-        const bool near = key_proxy(kx) < B.edge;
+        const bool gl = ghost && lane == kLaneJ;
+        if (wb || gl) dirty_or(par, gl ? extra_blk : rb / kBlk);
+        const bool near = key_proxy(kn) < B.edge;
         const unsigned long long nm = __ballot(near);
         const int n = __popcll(nm), cap_f = 1 << fsh, pos = __popcll(nm & below);
-        if (near && pos < cap_f) B.fresh[(bk << fsh) + pos] = kx;
+        if (near && pos < cap_f) B.fresh[(bk << fsh) + pos] = kn;
         if (lane == 0) {
             B.nfresh[bk] = min(n, cap_f);
             if (n > cap_f) B.full = 1;
@@ -3452,26 +3486,13 @@ __device__ __forceinline__ int run_event(const Hot& H, int e, int jp, int ct, do
     }
     // repuls_del_b.f once the rescheduling is done
     if (xdel && lane == 0) {
-        const bool iN = dyn_ident(ri.dyn) < dyn_ident(rj.dyn);
+        const bool iN = dyn_ident(dyni) < dyn_ident(dynj);
         const int a = iN ? i : j, b = iN ? j : i;
-        const int La = topo_len(iN ? ri.topo : rj.topo), Lb = topo_len(iN ? rj.topo : ri.topo);
-        const int ncim1 = a + La - 1, ncai = a - La, ncaj = b - 2 * Lb, nnjp1 = b - Lb + 1;
-        int4 ea = gld(H.extra + (a)), eb = gld(H.extra + (b));
-        ea.x = -1;
-        ea.y = -1;
-        ea.w = -1;
-        eb.x = -1;
-        eb.y = -1;
-        eb.w = -1;
-        gst(H.extra + (a), ea);
-        gst(H.extra + (b), eb);
-        gs1(&H.extra[ncaj].z, -1);
-        gs1(&H.extra[nnjp1].z, -1);
-        gs1(&H.extra[ncai].z, -1);
-        gs1(&H.extra[ncim1].z, -1);
+        const int La = topo_len(iN ? topoi : topoj), Lb = topo_len(iN ? topoj : topoi);
+        shoulders_clear(a, La, b, Lb);
     }
     if (batch) {
-        // the round's block rescans run after every committed event's
+        // the round's tree update runs after every committed event's
         // writes; a later event that replays on these entries waits for
         // the flag
         wave_sync_mem();
@@ -3596,6 +3617,7 @@ __device__ void rebuild_lists(const SysDev&, const Lds&, Sc& c) {
         for (int q2 = p2 + 1; q2 < end; ++q2) pos += gl1(&S.sinfo[q2].z) == si.z ? 1 : 0;
         gs2(S.cfp + (si.x), make_int2(si.z, pos));
     }
+    wg_sync(nw);  // every bead's list place is written
     PH_END(S, kPhLCopy, trl);
     int mx = 0, status = 0;
     const int noff = Mq > 2 ? 3 : Mq;  // distinct coarse offsets {0, +1, -1}
@@ -3713,6 +3735,10 @@ __device__ void rebuild_lists(const SysDev&, const Lds&, Sc& c) {
             mx = max(mx, max(nu, nd));
             gs1(S.nup + (i), min(nu, cap));
             gs1(S.ndn + (i), min(nd, cap));
+            // the up-row length rides with the bead's list place, for the
+            // down rows that name the bead (sort_rows)
+            const int2 fp = gl2(S.cfp + (i));
+            gs2(S.cfp + (i), make_int2(fp.x, fp.y | (min(nu, cap) << 16)));
         }
         wave_sync();
     }
@@ -3873,11 +3899,14 @@ __device__ void rebuild_lists_dense(const SysDev&, const Lds&, Sc& c) {
         }
     }
     while (qn > 0) drain();
+    wg_sync(nw);  // every bead's list place is written
     int mx = 0, status = 0;
     for (int i = wave + nr * lane; wave < nr && i < N; i += nr * kW) {
         const int2 n2 = cnt[i];
         gs1(S.nup + (i), min(n2.x, cap));
         gs1(S.ndn + (i), min(n2.y, cap));
+        const int2 fp = gl2(S.cfp + (i));
+        gs2(S.cfp + (i), make_int2(fp.x, fp.y | (min(n2.x, cap) << 16)));
         if (n2.x > cap || n2.y > cap) status = kErrListCapacity;
         mx = max(mx, max(n2.x, n2.y));
     }
@@ -3988,7 +4017,8 @@ __device__ void sort_rows(const SysDev&, const DevTables&, const Lds&) {
         int* const row = ((r & 1) == 0 ? S.nb_up : S.nb_dn) + (size_t)x * cap;
         const int n = act ? min(gl1(((r & 1) == 0 ? S.nup : S.ndn) + (x)), cap) : 0;
         const int2 cx = gl2(S.cfp + (x));
-        if (n >= 2 && n <= kSortMax) {
+        const bool dnr = (r & 1) != 0;  // a down row's entries carry their bead's up-row length in bits 16 to 22
+        if ((n >= 2 || (dnr && n == 1)) && n <= kSortMax) {
             if (vec) {
                 // reads up to the next multiple of 4 (<= kSortMax, <= cap)
                 int4 v[kSortMax / 4];
@@ -4016,7 +4046,10 @@ __device__ void sort_rows(const SysDev&, const DevTables&, const Lds&) {
                     if (u < n) cb[u] = gl2(S.cfp + (e[u]));
 #pragma unroll
                 for (int u = 0; u < kSortMax; ++u)
-                    if (u < n) keys[u * kW + lane] = nbor_key(M, T, cx, cb[u]);
+                    if (u < n) {
+                        keys[u * kW + lane] = nbor_key(M, T, cx, cb[u]);
+                        if (dnr) ents[u * kW + lane] |= (cb[u].y >> 16) << 16;
+                    }
             }
             for (int k = 0; k < n; ++k) {
                 const unsigned long long kk = keys[k * kW + lane];
@@ -4034,9 +4067,10 @@ __device__ void sort_rows(const SysDev&, const DevTables&, const Lds&) {
             const int rb_ = r0 + src, xb = rb_ >> 1, nbig = __shfl(n, src, kW);
             int* const rb = ((rb_ & 1) == 0 ? S.nb_up : S.nb_dn) + (size_t)xb * cap;
             const int2 cxb = gl2(S.cfp + (xb));
-            const int e = lane < nbig ? gl1(rb + (lane)) : 0;
-            const unsigned long long kk =
-                lane < nbig ? nbor_key(M, T, cxb, gl2(S.cfp + (e & 0xFFFFFF))) : ~0ull;
+            int e = lane < nbig ? gl1(rb + (lane)) : 0;
+            const int2 ce = gl2(S.cfp + (e & 0xFFFF));
+            const unsigned long long kk = lane < nbig ? nbor_key(M, T, cxb, ce) : ~0ull;
+            if ((rb_ & 1) != 0) e |= (ce.y >> 16) << 16;
             int rk = 0;
             for (int m = 0; m < nbig; ++m) {
                 const unsigned long long km = (unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)kk, m) |
@@ -4661,6 +4695,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_run(const SysDev* __restrict
     }
     bool stop_out = false;
     const Hot H = load_hot(S, L);
+    const Gather G = load_gather(S);
     // the pool holds a few entries more than a round takes; each event
     // wavefront has an equal share of the fresh entries' places
     const int want = kcap + 2, fsh = ne <= 1 ? 5 : (ne <= 2 ? 4 : (ne <= 4 ? 3 : 2));
@@ -4741,7 +4776,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_run(const SysDev* __restrict
                 // pair events (a ghost event may lead them), one per
                 // wavefront; event k of a round is numbered and stamped as
                 // the master will count it
-                A = run_event(H, e, uni(key_p(k)), uni(key_ct(k)), k.t, uni(key_bin(k)), master().coll + wave, wave, K == 1,
+                A = run_event(H, G, e, uni(key_p(k)), uni(key_ct(k)), k.t, uni(key_bin(k)), master().coll + wave, wave, K == 1,
                               par, fsh);
                 if (A > 0 && lane == 0) {
                     const int ty = B.ty[wave];
