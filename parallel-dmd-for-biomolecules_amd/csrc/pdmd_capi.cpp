@@ -71,7 +71,6 @@ struct HostSys {
     DevBuf<Leaf> leaf;
     DevBuf<double4> old_r, spos;
     DevBuf<int4> sinfo;
-    DevBuf<unsigned> mark;
     DevBuf<unsigned long long> stamp;
     DevBuf<SysState> st;
     DevBuf<LogRec> log;
@@ -405,7 +404,7 @@ int64_t device_bytes(const Prep& pp) {
     const int64_t sizes[] = {(int64_t)sizeof(DevTables), N * (int64_t)sizeof(Rec), N * 16 /*bw*/, N * 16 /*extra*/,
                              N * 16 /*ovr*/, N * 32 /*old_r*/, N * cap * 4 /*nb_up*/, N * cap * 4 /*nb_dn*/,
                              (N + 1) * 4 /*nup*/, (N + 1) * 4 /*ndn*/, (N + 3) * (int64_t)sizeof(Leaf), N * 4 /*cfine*/,
-                             N * 4 /*ckey*/, N * 8 /*cfp*/, N * 4 /*csorted*/, N * 32 /*spos*/, N * 16 /*sinfo*/, N * 4 /*mark*/,
+                             N * 4 /*ckey*/, N * 8 /*cfp*/, N * 4 /*csorted*/, N * 32 /*spos*/, N * 16 /*sinfo*/,
                              (nc + 1) * 4 /*cstart*/, nc * 4 /*crun*/, (N + 3) * 8 /*stamp*/,
                              (int64_t)sizeof(SysState)};
     int64_t b = 0;
@@ -575,8 +574,6 @@ int prepared_add(pdmd_ctx* ctx, PreparedSystem* ps, int32_t* sys_id) {
     HIPCHK(H.csorted.alloc(N));
     HIPCHK(H.spos.alloc(N));
     HIPCHK(H.sinfo.alloc(N));
-    HIPCHK(H.mark.alloc(N));
-    HIPCHK(hipMemsetAsync(H.mark.p, 0, sizeof(unsigned) * (size_t)N, ctx->stream));
     HIPCHK(H.stamp.alloc(N + 3));
     HIPCHK(hipMemsetAsync(H.stamp.p, 0, sizeof(unsigned long long) * (size_t)(N + 3), ctx->stream));
     HIPCHK(H.cstart.alloc((size_t)Mq * Mq * Mq + 1));
@@ -622,7 +619,6 @@ int prepared_add(pdmd_ctx* ctx, PreparedSystem* ps, int32_t* sys_id) {
     D.csorted = H.csorted.p;
     D.spos = H.spos.p;
     D.sinfo = H.sinfo.p;
-    D.mark = H.mark.p;
     D.stamp = H.stamp.p;
     D.st = H.st.p;
     D.log = nullptr;

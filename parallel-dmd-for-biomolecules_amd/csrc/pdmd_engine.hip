@@ -721,7 +721,7 @@ struct Batch {
     int K;                // entries popped this round (0: stop)
     int cut;              // first wavefront whose event is not committed
     int rebuild;          // the round's sync event rebuilds the lists
-    unsigned long long touched;  // superblocks with a changed block minimum (bit s)
+    unsigned long long moved;    // largest displacement of a sync event, as ordered bits
     // The pool the next round is selected from: every calendar entry whose
     // proxy lies below `edge` and that the round in flight has not popped is
     // in cand (as of the round's start) or, rewritten by a committed event
@@ -734,8 +734,8 @@ struct Batch {
     int order[kMaxWaves];        // lane of the entry of each rank (selection)
     Key cand[kCandMax];
     Key fresh[kFreshMax];
-    // blocks with rewritten entries, a bit per block and a word per
-    // superblock, by the round's parity: one is written while the other is
+    // blocks with rewritten entries, a bit per block and a word per 64
+    // blocks, by the round's parity: one is written while the other is
     // worked off
     unsigned long long dirty[2][kSup];
     int gbead;            // the bead of a ghost event leading the round
@@ -871,17 +871,13 @@ __device__ inline bool key_min_rows(Key& k) {
 // LDS views, one set per wavefront: the calendar tree, the master scalars
 // and the round record are shared, the work lists are the wavefront's own
 struct Lds {
-    int o_blk, o_sup, o_wm, o_wx, o_blist, o_pair, o_sc, o_leaf, o_wd, o_wt, o_wy, o_slot, o_spec, o_down;
+    int o_blk, o_wm, o_wx, o_blist, o_pair, o_sc, o_leaf, o_wd, o_wt, o_wy, o_slot, o_spec, o_down;
     int o_msc, o_batch, o_mark, o_one, o_pool;
     int nwr;  // wavefronts of a list rebuild that have scratch in the pool
     Leaf* gleaf;  // calendar leaves in HBM when they do not fit in LDS
-    // the round's footprint marks: a flat pointer into LDS (behind the
-    // leaves, when both fit there) or to SysDev::mark
-    unsigned* mark;
+    unsigned mark_mask;  // footprint mark of bead b: word b & mark_mask
     int nblk, nsup, maxw, nw;
-    bool leaf_lds, mark_lds;
-    __device__ Key* blk() const { return reinterpret_cast<Key*>(smem + o_blk); }
-    __device__ Key* sup() const { return reinterpret_cast<Key*>(smem + o_sup); }
+    bool leaf_lds;
     __device__ int* wm() const { return reinterpret_cast<int*>(smem + o_wm); }  // work list: partner / bead
     __device__ int* wx() const { return reinterpret_cast<int*>(smem + o_wx); }  // work list: owner / op tag
     __device__ int* wd() const { return reinterpret_cast<int*>(smem + o_wd); }
@@ -902,8 +898,7 @@ constexpr int kLdOff = kSdOff + (int)((sizeof(SysDev) + 15) / 16 * 16);
 constexpr int kLdStride = (int)((sizeof(Lds) + 15) / 16 * 16);
 __device__ inline const Lds& ldsv() { return *reinterpret_cast<const Lds*>(smem + kLdOff + wave_id() * kLdStride); }
 // the shared blocks that make_lds lays out after the views
-constexpr int kSupOff = kLdOff + kLdStride * kMaxWaves;
-constexpr int kMscOff = kSupOff + (int)(sizeof(Key) * kSup);
+constexpr int kMscOff = kLdOff + kLdStride * kMaxWaves;
 constexpr int kBatchOff = kMscOff + (int)((sizeof(Sc) + 15) / 16 * 16);
 __device__ inline Sc& master() { return *reinterpret_cast<Sc*>(smem + kMscOff); }
 __device__ inline Batch& round_rec() { return *reinterpret_cast<Batch*>(smem + kBatchOff); }
@@ -920,7 +915,6 @@ __device__ inline Lds lds_regs() {
     const Lds& m = ldsv();
     Lds r;
     r.o_blk = __builtin_amdgcn_readfirstlane(m.o_blk);
-    r.o_sup = __builtin_amdgcn_readfirstlane(m.o_sup);
     r.o_wm = __builtin_amdgcn_readfirstlane(m.o_wm);
     r.o_wx = __builtin_amdgcn_readfirstlane(m.o_wx);
     r.o_blist = __builtin_amdgcn_readfirstlane(m.o_blist);
@@ -945,8 +939,7 @@ __device__ inline Lds lds_regs() {
     r.maxw = __builtin_amdgcn_readfirstlane(m.maxw);
     r.nw = __builtin_amdgcn_readfirstlane(m.nw);
     r.leaf_lds = __builtin_amdgcn_readfirstlane(m.leaf_lds ? 1 : 0) != 0;
-    r.mark = sgpr_ptr(m.mark);
-    r.mark_lds = __builtin_amdgcn_readfirstlane(m.mark_lds ? 1 : 0) != 0;
+    r.mark_mask = (unsigned)__builtin_amdgcn_readfirstlane((int)m.mark_mask);
     return r;
 }
 __device__ inline Leaf leaf_get(const Lds& L, int k) { return L.leaf_lds ? L.lleaf()[k] : gld(L.gleaf + k); }
@@ -970,6 +963,7 @@ __device__ inline void leaf_set(const Lds& L, int k, const Leaf& v) {
         gst(L.gleaf + k, v);
 }
 
+__device__ inline unsigned* lds_words(int off) { return (unsigned*)__builtin_assume_aligned(smem + off, 16); }
 // What the event loop reads of its system and of the LDS plan, as values
 // that stay in scalar registers for the whole launch.
 struct Hot {
@@ -982,10 +976,10 @@ struct Hot {
     int* nup;
     int* ndn;
     Leaf* leaf;
-    unsigned* mark;
     unsigned long long* stamp;
+    unsigned mark_mask;
     int N, cap, nblk, nsup, o_blk, o_leaf, o_mark, o_w, o_blist;
-    bool leaf_lds, mark_lds;
+    bool leaf_lds;
 };
 __device__ inline Hot load_hot(const SysDev& S, const Lds& L) {
     Hot H;
@@ -998,7 +992,7 @@ __device__ inline Hot load_hot(const SysDev& S, const Lds& L) {
     H.nup = sgpr_ptr(S.nup);
     H.ndn = sgpr_ptr(S.ndn);
     H.leaf = sgpr_ptr(S.leaf);
-    H.mark = sgpr_ptr(S.mark);
+    H.mark_mask = (unsigned)uni((int)L.mark_mask);
     H.stamp = sgpr_ptr(S.stamp);
     H.N = uni(S.N);
     H.cap = uni(S.cap);
@@ -1010,7 +1004,6 @@ __device__ inline Hot load_hot(const SysDev& S, const Lds& L) {
     H.o_w = uni(L.o_one);
     H.o_blist = uni(L.o_blist);
     H.leaf_lds = uni(L.leaf_lds ? 1 : 0) != 0;
-    H.mark_lds = uni(L.mark_lds ? 1 : 0) != 0;
     return H;
 }
 // element i of a buffer: scalar base, 32-bit byte offset
@@ -1053,67 +1046,67 @@ __device__ inline void dirty_or(int par, int blk) {
     __hip_atomic_fetch_or(&round_rec().dirty[par][blk / kSup], 1ull << (blk & (kSup - 1)), __ATOMIC_RELAXED,
                           __HIP_MEMORY_SCOPE_WORKGROUP);
 }
-// Block minima of the listed blocks, one row of 16 lanes per block, 16
-// blocks per step so that four independent reductions overlap.  A block
-// whose minimum came out as it was is not written and leaves its superblock
-// alone; the others mark theirs in Batch::touched.
+// A calendar entry's time as the block minima hold it: the bits of the
+// nearest float (negative times as 0), in the order of the times except that
+// near ones may share a value; +infinity for no entry.  The minima only say
+// which blocks can hold an entry below a time, so four bytes per block and
+// one instruction per reduction step do: the exact keys are compared where
+// entries are taken.
+constexpr unsigned kNoTime = 0x7F800000u;
+__device__ inline unsigned leaf_time(const Leaf& lf) {
+    const float f = (float)lf.tim;
+    const unsigned u = (unsigned)max(__float_as_int(f), 0);
+    return leaf_bin(lf.meta) < 0 ? kNoTime : u;
+}
+template <int CTRL>
+__device__ inline unsigned ror_min(unsigned v) {
+    return min(v, (unsigned)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xf, 0xf, true));
+}
+// minima of the blocks in the list: one row of 16 lanes per block, 32 blocks
+// per step so that eight independent reductions overlap
 __device__ inline void rescan_listed(const Hot& H, const int* list, int nb) {
     const int lane = lane_id(), N3 = H.N + 3;
-    Key* const blk = reinterpret_cast<Key*>(smem + H.o_blk);
-    for (int base = 0; base < nb; base += 16) {
-        Key e[4], old[4];
-        double p[4], m[4];
-        int bq[4];
-        bool dup = false;
+    unsigned* const blk = lds_words(H.o_blk);
+    for (int base = 0; base < nb; base += 32) {
+        unsigned v[8];
+        int bq[8];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
+        for (int u = 0; u < 8; ++u) {
             const int q = base + 4 * u + (lane >> 4);
             bq[u] = q < nb ? list[q] : -1;
         }
+        Leaf lf[8];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
+        for (int u = 0; u < 8; ++u) {
             const int idx = bq[u] * kBlk + (lane & 15);
-            e[u] = empty_key();
-            if (bq[u] >= 0) {
-                old[u] = blk[bq[u]];
-                if (idx < N3) e[u] = leaf_key(leaf_ld(H, idx), idx);
-            }
+            lf[u].meta = 0;
+            lf[u].tim = 0.0;
+            if (base + 4 * u < nb && bq[u] >= 0 && idx < N3) lf[u] = leaf_ld(H, idx);
         }
 #pragma unroll
-        for (int u = 0; u < 4; ++u) p[u] = key_proxy(e[u]);
+        for (int u = 0; u < 8; ++u) v[u] = leaf_time(lf[u]);
 #pragma unroll
-        for (int u = 0; u < 4; ++u) m[u] = row_min(p[u]);
-        bool win[4];
+        for (int u = 0; u < 8; ++u) v[u] = ror_min<0x121>(v[u]);
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const unsigned long long tie = __ballot(p[u] == m[u] && !proxy_none(m[u]));
-            const unsigned rb = (unsigned)(tie >> (lane & 48)) & 0xFFFFu;
-            win[u] = proxy_none(m[u]) ? (lane & 15) == 15 : p[u] == m[u];
-            dup |= (rb & (rb - 1u)) != 0u;
-        }
-        if (__ballot(dup)) {
+        for (int u = 0; u < 8; ++u) v[u] = ror_min<0x122>(v[u]);
 #pragma unroll
-            for (int u = 0; u < 4; ++u) win[u] = key_min_rows(e[u]);
-        }
+        for (int u = 0; u < 8; ++u) v[u] = ror_min<0x124>(v[u]);
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
-            if (win[u] && bq[u] >= 0 && (e[u].t != old[u].t || e[u].bc != old[u].bc || e[u].ip != old[u].ip)) {
-                blk[bq[u]] = e[u];
-                if (H.nsup > 1)
-                    __hip_atomic_fetch_or(&round_rec().touched, 1ull << (bq[u] / kSup), __ATOMIC_RELAXED,
-                                          __HIP_MEMORY_SCOPE_WORKGROUP);
-            }
+        for (int u = 0; u < 8; ++u) v[u] = ror_min<0x128>(v[u]);
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            if ((lane & 15) == 0 && bq[u] >= 0) blk[bq[u]] = v[u];
     }
 }
 constexpr int kListMax = 512;  // blocks of a work list (one wavefront's one-pass area)
-// Adds the blocks of superblock s in mask to the list.
+// Adds the blocks 64 s + bit of mask to the list.
 __device__ inline int list_blocks(int* list, int n, int s, unsigned long long mask) {
     const int lane = lane_id();
     if ((mask >> lane) & 1ull) list[n + __popcll(mask & ((1ull << lane) - 1ull))] = s * kSup + lane;
     return n + __popcll(mask);
 }
-// The min tree after the entries of the blocks in Batch::dirty[par] changed
-// (one wavefront; the mask is cleared).
+// The block minima after the entries of the blocks in Batch::dirty[par]
+// changed (one wavefront; the mask is cleared).
 __device__ inline void tree_update(const Hot& H, int par, int* list) {
     const int lane = lane_id();
     Batch& B = round_rec();
@@ -1123,8 +1116,6 @@ __device__ inline void tree_update(const Hot& H, int par, int* list) {
         B.dirty[par][lane] = 0;
     }
     unsigned long long sm = __ballot(d != 0);
-    if (!sm) return;
-    if (lane == 0) B.touched = 0;
     int n = 0;
     while (sm) {
         const int s = __ffsll((long long)sm) - 1;
@@ -1137,21 +1128,8 @@ __device__ inline void tree_update(const Hot& H, int par, int* list) {
             n = 0;
         }
     }
-    if (H.nsup == 1) return;  // a single superblock is never read: the block minima fit one wavefront
-    const Key* const blk = reinterpret_cast<const Key*>(smem + H.o_blk);
-    Key* const sup = reinterpret_cast<Key*>(smem + kSupOff);
-    const unsigned long long tv = B.touched;
-    unsigned long long touched = (unsigned long long)(unsigned)uni((int)tv) | ((unsigned long long)(unsigned)uni((int)(tv >> 32)) << 32);
-    while (touched) {
-        const int s = __ffsll((long long)touched) - 1;
-        touched &= touched - 1;
-        const int b = s * kSup + lane;
-        const Key e = key_min_wave(b < H.nblk ? blk[b] : empty_key());
-        if (lane == 0) sup[s] = e;
-    }
-    wave_sync();
 }
-// The pool of the next selection from the up-to-date min tree (one
+// The pool of the next selection from the up-to-date block minima (one
 // wavefront): every entry whose proxy lies below an edge, the K entries
 // popped by the round in flight left out.  The edge lies Batch::width after
 // t0; the width follows the density of events so that the pool holds a few
@@ -1162,11 +1140,14 @@ __device__ inline void collect_pool(const Hot& H, int K, double t0, int want, in
     const int lane = lane_id(), N3 = H.N + 3;
     Batch& B = round_rec();
     const Sc& c = master();
-    const Key* const blk = reinterpret_cast<const Key*>(smem + H.o_blk);
-    const Key* const sup = reinterpret_cast<const Key*>(smem + kSupOff);
+    const unsigned* const blk = lds_words(H.o_blk);
     const double off = c.tbin_off, sortsize = c.sortsize, imax = c.interval_max;
     double w = B.width;
-    const int pidx = lane < K ? key_idx(B.key[lane & (kMaxWaves - 1)]) : -1;
+    // the popped entries are the calendar's least: all proxies below the
+    // last one's, and those that share its proxy by index
+    const Key kl = B.key[K > 0 ? K - 1 : 0];
+    const double pl = K > 0 ? key_proxy(kl) : -1.0;
+    const int il = K > 0 ? key_idx(kl) : -1;
     int count = 0;
     double edge = 0.0;
     for (int tr = 0; tr < tries; ++tr) {
@@ -1176,50 +1157,54 @@ __device__ inline void collect_pool(const Hot& H, int K, double t0, int want, in
         ek.bc = min(max(bin, 1), kNumbin) << 8;
         ek.ip = 0;
         edge = key_proxy(ek);
-        // blocks with a minimum below the edge
+        // blocks that can hold an entry below the edge (its time rounded up:
+        // bins and times agree to far less than a float's spacing)
+        const unsigned te = (unsigned)max(__float_as_int((float)ek.t), 0) + 2u;
         int n = 0;
         bool many = false;
-        if (H.nsup == 1) {
-            n = list_blocks(list, 0, 0, __ballot(lane < H.nblk && key_proxy(blk[lane]) < edge));
-        } else {
-            unsigned long long sm = __ballot(lane < H.nsup && key_proxy(sup[lane]) < edge);
-            while (sm && !many) {
-                const int s = __ffsll((long long)sm) - 1;
-                sm &= sm - 1;
-                const int b = s * kSup + lane;
-                n = list_blocks(list, n, s, __ballot(b < H.nblk && key_proxy(blk[b]) < edge));
-                many = n > kListMax - kSup;
+        for (int s0 = 0; s0 < H.nsup && !many; s0 += 4) {
+            unsigned v[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int b = (s0 + u) * kSup + lane;
+                v[u] = b < H.nblk ? blk[b] : kNoTime;
             }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const unsigned long long m = __ballot(v[u] < te);
+                if (m) n = list_blocks(list, n, s0 + u, m);
+            }
+            many = n > kListMax - 4 * kSup;
         }
         wave_sync();
         // their entries below it
         count = 0;
-        for (int base = 0; base < n && !many; base += 16) {
-            Key e[4];
-            double p[4];
-            int idx[4];
+        for (int base = 0; base < n && !many; base += 32) {
+            Leaf lf[8];
+            int idx[8];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
+            for (int u = 0; u < 8; ++u) {
                 const int q = base + 4 * u + (lane >> 4);
                 idx[u] = (q < n ? list[q] : H.nblk) * kBlk + (lane & 15);
-                e[u] = empty_key();
+                lf[u].meta = 0;
+                lf[u].tim = 0.0;
+                lf[u].nptnr = 0;
             }
 #pragma unroll
-            for (int u = 0; u < 4; ++u)
-                if (idx[u] < N3) e[u] = leaf_key(leaf_ld(H, idx[u]), idx[u]);
+            for (int u = 0; u < 8; ++u)
+                if (base + 4 * u < n && idx[u] < N3) lf[u] = leaf_ld(H, idx[u]);
 #pragma unroll
-            for (int u = 0; u < 4; ++u) p[u] = key_proxy(e[u]);
-            for (int q = 0; q < K; ++q) {
-                const int pq = __builtin_amdgcn_readlane(pidx, q);
-#pragma unroll
-                for (int u = 0; u < 4; ++u)
-                    if (idx[u] == pq) p[u] = __hiloint2double(kInfHi, 0);
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const unsigned long long m = __ballot(p[u] < edge);
+            for (int u = 0; u < 8; ++u) {
+                if (base + 4 * u >= n) continue;
+                const Key e = leaf_key(lf[u], idx[u]);
+                const double p = key_proxy(e);
+                bool in = p < edge && p >= pl && idx[u] != il;
+                if (__ballot(in && p == pl)) {
+                    for (int q = 0; q < K; ++q) in = in && uni(key_idx(B.key[q])) != idx[u];
+                }
+                const unsigned long long m = __ballot(in);
                 const int pos = count + __popcll(m & ((1ull << lane) - 1ull));
-                if (p[u] < edge && pos < kCandMax) B.cand[pos] = e[u];
+                if (in && pos < kCandMax) B.cand[pos] = e;
                 count += __popcll(m);
             }
             many = count > kCandMax;
@@ -1242,25 +1227,20 @@ __device__ inline void collect_pool(const Hot& H, int K, double t0, int want, in
     wave_sync();
 }
 
-// every block and superblock minimum; all wavefronts of the system take part
-__device__ void rescan_all(const Lds&, int N3) {
-    const Lds& L = ldsv();
-
-    const int lane = lane_id(), wave = wave_id(), nw = L.nw;
-    for (int base = 4 * wave; base < L.nblk; base += 4 * nw) {
-        const int b = base + (lane >> 4), k = lane & 15;
-        Key e = empty_key();
-        const int idx = b * kBlk + k;
-        if (b < L.nblk && idx < N3) e = leaf_key(leaf_get(L, idx), idx);
-        if (key_min_rows(e) && b < L.nblk) L.blk()[b] = e;
+// every block minimum; all wavefronts of the system take part
+__device__ inline void rescan_all(const Hot& H, int wave, int nw) {
+    const int lane = lane_id(), N3 = H.N + 3;
+    unsigned* const blk = lds_words(H.o_blk);
+    for (int base = 4 * wave; base < H.nblk; base += 4 * nw) {
+        const int b = base + (lane >> 4), idx = b * kBlk + (lane & 15);
+        unsigned v = kNoTime;
+        if (idx < N3) v = leaf_time(leaf_ld(H, idx));
+        v = ror_min<0x121>(v);
+        v = ror_min<0x122>(v);
+        v = ror_min<0x124>(v);
+        v = ror_min<0x128>(v);
+        if ((lane & 15) == 0 && b < H.nblk) blk[b] = v;
     }
-    wg_sync(nw);
-    for (int s = wave; s < L.nsup; s += nw) {
-        const int b = s * kSup + lane;
-        const Key e = key_min_wave(b < L.nblk ? L.blk()[b] : empty_key());
-        if (lane == 0) L.sup()[s] = e;
-    }
-    wg_sync(nw);
 }
 
 // ------------------------------------------------------------------------
@@ -1299,17 +1279,14 @@ __device__ inline int shoulder_bead(const SysDev&, const Pair& P, int lane) {
     const int v = q == 0 ? a[0] : (q == 1 ? a[1] : (q == 2 ? a[2] : a[3]));
     return (v >= 0 && v < S.N) ? v : -1;
 }
-// the marks live in HBM and are read and written at the device's L2
-// Footprint marks of bead b through Lds::mark (flat: LDS when the system's
-// leaves and marks fit there, else SysDev::mark in HBM).
-__device__ inline void mark_or(const Lds& L, const SysDev&, int b, unsigned bits) {
-    __hip_atomic_fetch_or(L.mark + b, bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+// Footprint marks of bead b, in LDS.  Where a word per bead does not fit, the
+// words are shared (b & mark_mask): a shared word can only end a round
+// earlier or replay an update on an entry that nobody rewrote.
+__device__ inline void mark_or(const Lds& L, int b, unsigned bits) {
+    __hip_atomic_fetch_or(lds_words(L.o_mark) + ((unsigned)b & L.mark_mask), bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
-__device__ inline unsigned mark_get(const Lds& L, const SysDev&, int b) {
-    return __hip_atomic_load(L.mark + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ inline void mark_clear(const Lds& L, const SysDev&, int b) {
-    __hip_atomic_store(L.mark + b, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+__device__ inline void mark_clear(const Lds& L, int b) {
+    __hip_atomic_store(lds_words(L.o_mark) + ((unsigned)b & L.mark_mask), 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 // A wavefront's place in a multi-wavefront round: -1 alone; 0 the round's
 // first event (always committed, writes as it goes); k >= 1 a speculative
@@ -1330,10 +1307,10 @@ __device__ inline void spec_abort_at(int bk, int& nb) {
 
 __device__ inline void round_clear_marks(const Lds& L, const SysDev& S, int dent, int i, int j, int sp) {
     const int lane = lane_id();
-    if (dent >= 0) mark_clear(L, S, dent);
-    if (lane == 0) mark_clear(L, S, i);
-    if (lane == 1 && j >= 0) mark_clear(L, S, j);
-    if (sp >= 0) mark_clear(L, S, sp);
+    if (dent >= 0) mark_clear(L, dent);
+    if (lane == 0) mark_clear(L, i);
+    if (lane == 1 && j >= 0) mark_clear(L, j);
+    if (sp >= 0) mark_clear(L, sp);
 }
 // Events of a round committed: the prefix before the first cut-off event,
 // before the first event after an error, and before the first event whose
@@ -2028,11 +2005,11 @@ __device__ __noinline__ void reschedule(const SysDev&, const DevTables&, const L
         const unsigned sbit = 1u, lbit = 1u << 8, fbit = 1u << 16;
         sp = shoulder_bead(S, P, lane);
         if (lane == 0) B.wdone[0] = 0;
-        if (dent >= 0) mark_or(L, S, dent, lbit | (mfull ? fbit : 0u));
-        if (lane == 0) mark_or(L, S, i, sbit | lbit | fbit);
-        if (lane == 1 && j >= 0) mark_or(L, S, j, sbit | lbit | fbit);
+        if (dent >= 0) mark_or(L, dent, lbit | (mfull ? fbit : 0u));
+        if (lane == 0) mark_or(L, i, sbit | lbit | fbit);
+        if (lane == 1 && j >= 0) mark_or(L, j, sbit | lbit | fbit);
         sp_w = (P.flags & kPairWroteSp) != 0;
-        if (sp_w && sp >= 0) mark_or(L, S, sp, sbit);
+        if (sp_w && sp >= 0) mark_or(L, sp, sbit);
         bar_to(nb, 1);
         PH_END(S, kPhBMark, tph);
     }
@@ -2570,24 +2547,15 @@ struct OnePass {
 // result lanes of beads i and j: entries take the lanes below
 constexpr int kLaneI = kW - 2, kLaneJ = kW - 1;
 
-__device__ inline unsigned* lds_words(int off) { return (unsigned*)__builtin_assume_aligned(smem + off, 16); }
-// footprint marks, in LDS (ds operations) or in HBM at the device's L2
+// footprint marks in LDS (a word per bead, or shared: mark_or)
 __device__ inline void fp_or(const Hot& H, int b, unsigned bits) {
-    if (H.mark_lds)
-        __hip_atomic_fetch_or(lds_words(H.o_mark) + b, bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    else
-        __hip_atomic_fetch_or((GLB unsigned*)((GLB char*)H.mark + (unsigned)b * 4u), bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_fetch_or(lds_words(H.o_mark) + ((unsigned)b & H.mark_mask), bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 __device__ inline unsigned fp_get(const Hot& H, int b) {
-    if (H.mark_lds)
-        return __hip_atomic_load(lds_words(H.o_mark) + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    return __hip_atomic_load((GLB unsigned*)((GLB char*)H.mark + (unsigned)b * 4u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return __hip_atomic_load(lds_words(H.o_mark) + ((unsigned)b & H.mark_mask), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 __device__ inline void fp_clear(const Hot& H, int b) {
-    if (H.mark_lds)
-        __hip_atomic_store(lds_words(H.o_mark) + b, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    else
-        __hip_atomic_store((GLB unsigned*)((GLB char*)H.mark + (unsigned)b * 4u), 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(lds_words(H.o_mark) + ((unsigned)b & H.mark_mask), 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
 // A lane's part of one gather that fetches everything an event needs of its
@@ -3988,7 +3956,6 @@ __device__ void events_all(const SysDev&, const DevTables&, const Lds&, Sc&) {
     status = wave_status(status);
     if (status && !c.status) c.status = status;
     wg_sync(L.nw);
-    rescan_all(L, N + 3);
 }
 
 // Rows in nbor.f's order: every bead's up and down rows sorted by
@@ -4123,54 +4090,48 @@ __device__ void rebuild(const SysDev&, const DevTables&, const Lds&, Sc&) {
     PH_END(S, kPhLists, trb);
     events_all(S, T, L, c);
     // the scratch lay over the round's footprint marks too
-    if (L.mark_lds)
-        for (int b = (int)threadIdx.x; b < S.N; b += kW * L.nw) L.mark[b] = 0u;
+    if (L.o_mark >= 0) {
+        const int nm = (int)min((unsigned)S.N, L.mark_mask) + 1;
+        for (int b = (int)threadIdx.x; b < nm; b += kW * L.nw) lds_words(L.o_mark)[b] = 0u;
+    }
     PH_END(S, kPhEvents, trb);
     PH_COUNT(S, kPhNRebuild);
 }
 
-// sync pseudo-event, main.F90:1126-1187, in two parts around the list
-// rebuild that all wavefronts run: sync_begin (wavefront 0) advances the
-// free flight, shifts the calendar and returns whether the lists are
-// rebuilt; sync_finish (wavefront 0) schedules the next sync.
-__device__ bool sync_begin(const SysDev&, const DevTables&, const Lds&, Sc&) {
-    const Lds& L = ldsv();
-
-    const SysDev& S = sdev();
-
-    const DevTables& T = tabs();
-    Sc& c = *L.sc();
-
-    const int lane = lane_id();
-    const int N = S.N;
-    const double tf = c.tfalse;
-    PH_BEGIN(tsy);
-    PH_COUNT(S, kPhNSync);
-    c.t = c.t + tf;
-    for (int e = lane; e < N + 3; e += kW) {
-        Leaf lf = leaf_get(L, e);
+// sync pseudo-event, main.F90:1126-1187, on all wavefronts of the system:
+// sync_move advances the free flight, shifts the calendar and takes the
+// displacement test (displ.f); after a barrier sync_decide (one lane) moves
+// the time origin and says whether the lists are rebuilt; sync_finish
+// (wavefront 0) schedules the next sync.
+__device__ inline void sync_move(const Hot& H, const SysDev& S, double tf, int nthr) {
+    const int tid = (int)threadIdx.x, N = H.N;
+    for (int e = tid; e < N + 3; e += nthr) {
+        Leaf lf = leaf_ld(H, e);
         lf.tim = lf.tim - tf;
-        leaf_set(L, e, lf);
+        leaf_st(H, e, lf);
     }
-    c.interval_max = c.interval_max - tf;
-    c.tbin_off = c.tbin_off + tf;
     double moved_far = 0.0;
-    // free flight to real positions and the displacement check (displ.f),
-    // four beads per lane in flight at a time
-#pragma unroll 4
-    for (int k = lane; k < N; k += kW) {
-        Rec b = gld(S.rec + (k));
+#pragma unroll 2
+    for (int k = tid; k < N; k += nthr) {
+        Rec b = ld_at(H.rec, k);
         const double4 o = gld(S.old_r + (k));
         b.x = b.x + b.vx * tf;
         b.y = b.y + b.vy * tf;
         b.z = b.z + b.vz * tf;
-        gst(S.rec + (k), b);
+        st_at(H.rec, k, b);
         const double a = o.x - b.x, bb = o.y - b.y, cc = o.z - b.z;
         const double dis = a * a + bb * bb + cc * cc;
         const double moved = dis / S.hdelr;
         if (moved > moved_far) moved_far = moved;
     }
     moved_far = wave_max(moved_far);
+    if (lane_id() == 0) atomicMax(&round_rec().moved, (unsigned long long)__double_as_longlong(moved_far));
+}
+__device__ inline bool sync_decide(const SysDev& S, Sc& c, double tf) {
+    const double moved_far = __longlong_as_double((long long)round_rec().moved);
+    c.t = c.t + tf;
+    c.interval_max = c.interval_max - tf;
+    c.tbin_off = c.tbin_off + tf;
     c.tfalse = 0.0;
     bool update = false;
     if (moved_far >= 0.1) {  // displ.f:37-46
@@ -4180,28 +4141,16 @@ __device__ bool sync_begin(const SysDev&, const DevTables&, const Lds&, Sc&) {
             c.interval = c.t_fact / sqrt(S.setemp);
         }
     }
-    wave_sync_mem();
-    if (update || c.interval > c.interval_max) {
-        if (!update) {
-            c.nforced++;
-            c.n_forced = c.n_forced * 1.01;
-        }
-        c.interval_max = c.interval * c.n_forced;
-        c.sortsize = c.interval_max / (double)kNumbin;
-        c.tbin_off = 0.0;
-        c.nupdates++;
-        PH_END(S, kPhSync, tsy);
-        return true;
-    } else {
-        // every entry moved by the same -tf: the cached block and superblock
-        // minima are shifted exactly as their leaves were
-        for (int b = lane; b < L.nblk; b += kW)
-            if (L.blk()[b].bc != kEmptyBc) L.blk()[b].t = L.blk()[b].t - tf;
-        if (lane < L.nsup && L.sup()[lane].bc != kEmptyBc) L.sup()[lane].t = L.sup()[lane].t - tf;
-        wave_sync_mem();
+    if (!(update || c.interval > c.interval_max)) return false;
+    if (!update) {
+        c.nforced++;
+        c.n_forced = c.n_forced * 1.01;
     }
-    PH_END(S, kPhSync, tsy);
-    return false;
+    c.interval_max = c.interval * c.n_forced;
+    c.sortsize = c.interval_max / (double)kNumbin;
+    c.tbin_off = 0.0;
+    c.nupdates++;
+    return true;
 }
 __device__ void sync_finish(const SysDev&, const Lds&, Sc&) {
     const Lds& L = ldsv();
@@ -4251,12 +4200,11 @@ __device__ void output_event(const SysDev&, const Lds&, Sc&) {
     wave_sync_mem();
 }
 
-// LDS plan: tables, SysDev, the views, the superblock minima, master
-// scalars and round record; each wavefront's one-pass work area, block list
+// LDS plan: tables, SysDev, the views, master scalars and round record; each wavefront's one-pass work area, block list
 // and pair, wavefront 0's with the multi-pass form's work lists after them;
-// then this system's block minima, then as many calendar leaves as the
-// workgroup's lds_bytes hold: a small system in a launch sized for a large
-// one keeps all its leaves in LDS.  Everything from the work areas on is
+// then this system's block minima, its footprint marks and, if they fit the
+// workgroup's lds_bytes, its calendar leaves: a small system in a launch
+// sized for a large one keeps all its leaves in LDS.  Everything from the work areas on is
 // also the scratch pool of a list rebuild.  One set of work lists (15 KB)
 // instead of one per wavefront (25 KB each) leaves room for eight
 // wavefronts at every size: only an event of more than 62 predictions needs
@@ -4281,7 +4229,6 @@ __device__ Lds make_lds(const SysDev&, int maxw, int lds_bytes, int nw, int wave
     L.nsup = (L.nblk + kSup - 1) / kSup;
     L.maxw = maxw;
     L.nw = nw;
-    L.o_sup = kSupOff;
     L.o_msc = kMscOff;
     L.o_batch = kBatchOff;
     L.o_pool = kPoolOff;
@@ -4304,15 +4251,23 @@ __device__ Lds make_lds(const SysDev&, int maxw, int lds_bytes, int nw, int wave
     L.o_spec = take((int)sizeof(SpecInfo) * kMaxSpec);
     L.o_down = take((int)sizeof(DownInfo) * kW);
     L.o_sc = kMscOff;
-    L.o_blk = take((int)sizeof(Key) * L.nblk);
+    L.o_blk = take((int)sizeof(unsigned) * L.nblk);
+    // a footprint mark per bead, or as large a power of two as fits
+    L.o_mark = -1;
+    L.mark_mask = ~0u;
+    if (lds_bytes > 0) {
+        const int words = (lds_bytes - p) / (int)sizeof(unsigned);
+        int n = S.N + 1;
+        if (n > words) {
+            n = 1024;
+            while (2 * n <= words) n *= 2;
+            L.mark_mask = (unsigned)n - 1u;
+        }
+        L.o_mark = take((int)sizeof(unsigned) * n);
+    }
     L.o_leaf = p;
     L.leaf_lds = N3 <= (lds_bytes - p) / (int)sizeof(Leaf);
     L.gleaf = S.leaf;
-    // footprint marks behind the leaves, when both fit
-    const int o_mark = (p + N3 * (int)sizeof(Leaf) + 15) / 16 * 16;
-    L.mark_lds = L.leaf_lds && o_mark + 4 * S.N <= lds_bytes;
-    L.o_mark = o_mark;
-    L.mark = L.mark_lds ? reinterpret_cast<unsigned*>(smem + o_mark) : S.mark;
     // the rebuild kernels' launches (lds_bytes 0) hold every wavefront's scratch
     const int room = lds_bytes > 0 ? (lds_bytes - kPoolOff) / kScratch : nw;
     L.nwr = room < nw ? room : nw;
@@ -4578,8 +4533,8 @@ __device__ __forceinline__ int select_pool(const Hot& H, int kmax, int A, int Kp
 }
 
 // The round's entries (wavefront 0): from the pool, after collecting it
-// again where it is incomplete or empty; the least entry of the tree alone
-// where no edge gives a pool (many entries of one time).  The master takes
+// again where it is incomplete or empty; the least entry of the calendar
+// alone where no edge gives a pool (many entries of one time).  The master takes
 // the first event's bin, time and number.  Returns 0 for an empty calendar.
 __device__ __forceinline__ int select_round(const Hot& H, Sc& c, int kmax, int A, int Kp, int ne, int fsh, int want, int par) {
     PH_BEGIN(tsp);
@@ -4601,8 +4556,12 @@ __device__ __forceinline__ int select_round(const Hot& H, Sc& c, int kmax, int A
     }
     PH_END(sdev(), kPhSelPop, tsp);
     if (K == 0) {
-        const Key* const top = H.nsup == 1 ? reinterpret_cast<const Key*>(smem + H.o_blk) : reinterpret_cast<const Key*>(smem + kSupOff);
-        const Key k = key_min_wave(lane < (H.nsup == 1 ? H.nblk : H.nsup) ? top[lane] : empty_key());
+        Key least = empty_key();
+        for (int idx = lane; idx < H.N + 3; idx += kW) {
+            const Key q = leaf_key(leaf_ld(H, idx), idx);
+            if (q.bc != kEmptyBc && (least.bc == kEmptyBc || key_less(q, least))) least = q;
+        }
+        const Key k = key_min_wave(least);
         if (k.bc == kEmptyBc) {
             c.status = kErrBin;
             return 0;
@@ -4664,8 +4623,8 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_run(const SysDev* __restrict
     copy_tables(S.tab, const_cast<DevTables*>(&tabs()));
     if (L.leaf_lds)
         for (int e = (int)threadIdx.x; e < N3; e += (int)blockDim.x) L.lleaf()[e] = gld(S.leaf + (e));
-    if (L.mark_lds)
-        for (int b = (int)threadIdx.x; b < N; b += (int)blockDim.x) L.mark[b] = 0u;
+    for (int b = (int)threadIdx.x, nm = (int)min((unsigned)N, L.mark_mask) + 1; b < nm; b += (int)blockDim.x)
+        lds_words(L.o_mark)[b] = 0u;
     __syncthreads();
     const DevTables& T = tabs();
     Sc& c = *L.sc();  // wavefront 0: the master scalars; others: their own copy
@@ -4675,7 +4634,9 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_run(const SysDev* __restrict
         c.target = c.coll + inc[blockIdx.x];
     }
     __syncthreads();
-    rescan_all(L, N3);
+    const Hot H = load_hot(S, L);
+    const Gather G = load_gather(S);
+    rescan_all(H, wave, nw);
     int log_count = S.st->log_count;
     // the budget runs from the launch's start: the earliest start among the
     // workgroups (launch_t0 is reset to all ones before a budgeted launch),
@@ -4694,8 +4655,6 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_run(const SysDev* __restrict
         w0 = B.t0;
     }
     bool stop_out = false;
-    const Hot H = load_hot(S, L);
-    const Gather G = load_gather(S);
     // the pool holds a few entries more than a round takes; each event
     // wavefront has an equal share of the fresh entries' places
     const int want = kcap + 2, fsh = ne <= 1 ? 5 : (ne <= 2 ? 4 : (ne <= 4 ? 3 : 2));
@@ -4728,22 +4687,28 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_run(const SysDev* __restrict
         const int e = uni(key_idx(k));
         int* const list = reinterpret_cast<int*>(smem + H.o_w);
         if (K == 1 && e > N) {
-            // the sync or output event, on the tree as of now
+            // the sync or output event; the pool is collected again after it
             if (wave == ne) tree_update(H, par ^ 1, list);
+            const double tf = uni(master().tfalse);
+            if (threadIdx.x == 0) B.moved = 0;
             __syncthreads();
             if (e == N + 1) {
-                // every wavefront takes part in a list rebuild
-                if (wave == 0) {
-                    const bool rb = sync_begin(S, T, L, c);
-                    if (lane == 0) B.rebuild = rb ? 1 : 0;
-                }
+                PH_BEGIN(tsy);
+                PH_COUNT(S, kPhNSync);
+                sync_move(H, S, tf, kW * nw);
                 __syncthreads();
+                if (threadIdx.x == 0) B.rebuild = sync_decide(S, c, tf) ? 1 : 0;
+                __syncthreads();
+                PH_END(S, kPhSync, tsy);
                 if (B.rebuild) {
                     const long long tr = wall_clock64();
                     rebuild(S, T, L, c);
                     t_rebuild += wall_clock64() - tr;
                     ++n_rebuild;
+                    __syncthreads();
                 }
+                // every entry moved
+                rescan_all(H, wave, nw);
                 if (wave == 0) sync_finish(S, L, c);
             } else if (wave == 0) {
                 output_event(S, L, c);
@@ -4805,17 +4770,19 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_run(const SysDev* __restrict
                     const Key kk = B.key[q];
                     log_event(S, log_count, c.coll + q, key_idx(kk), key_idx(kk) == N ? B.gbead : key_p(kk), B.ty[q], kk.t);
                 }
-            if (lane == 0) {
-                for (int q = 0; q < A; ++q) {
-                    const int st = q > 0 && B.st[q] != 0 ? B.st[q] : B.st_rep[q];
-                    if (st != 0 && c.status == 0) c.status = st;
-                }
-                if (A >= 2) {
-                    c.coll += A - 1;
-                    c.old_tfalse = B.key[A - 2].t;
-                    c.tfalse = B.key[A - 1].t;
-                    c.nbin = key_bin(B.key[A - 1]);
-                }
+            {
+                const int q = lane & (kMaxWaves - 1);
+                int st = q > 0 ? B.st[q] : 0;
+                st = st != 0 ? st : B.st_rep[q];
+                st = wave_status(lane < A ? st : 0);
+                if (st != 0 && lane == 0 && c.status == 0) c.status = st;
+            }
+            if (A >= 2 && lane == 0) {
+                const Key kp = B.key[A - 2], kk = B.key[A - 1];
+                c.coll += A - 1;
+                c.old_tfalse = kp.t;
+                c.tfalse = kk.t;
+                c.nbin = key_bin(kk);
             }
             wave_sync();
         }
@@ -5110,7 +5077,8 @@ static size_t r16(size_t b) { return (b + 15) / 16 * 16; }
 // the bytes make_lds lays out before the leaves, for nw wavefronts; at
 // least one wavefront's rebuild scratch
 static size_t lds_fixed(int nblk_max, int maxw, int nw) {
-    const size_t b = (size_t)kPoolOff + (size_t)nw * lds_wave_bytes() + lds_multi_bytes(maxw) + r16(sizeof(Key) * nblk_max);
+    const size_t b = (size_t)kPoolOff + (size_t)nw * lds_wave_bytes() + lds_multi_bytes(maxw) + r16(sizeof(unsigned) * nblk_max) +
+                     4096;  // the fewest footprint marks
     return std::max(b, (size_t)kPoolOff + kScratch);
 }
 size_t engine_lds_bytes(int nblk_max, int maxw, int leaf_cap, int nw) {
@@ -5167,7 +5135,7 @@ hipError_t engine_run(const SysDev* d_sys, const int* d_ids, const long long* d_
     }
     size_t lds = lds_limit;
     if (n > ncu) {
-        size_t want = base + sizeof(Leaf) * (size_t)(max_n + 3);
+        size_t want = base + (sizeof(Leaf) + sizeof(unsigned)) * (size_t)(max_n + 4);
         lds = want < lds_limit ? want : lds_limit;
     }
     if (lds < base) lds = base;
