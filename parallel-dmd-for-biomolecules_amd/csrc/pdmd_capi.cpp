@@ -65,7 +65,7 @@ struct HostSys {
     DevBuf<DevTables> tab;
     DevBuf<Rec> rec;
     DevBuf<double2> bw;
-    DevBuf<int> nb_up, nup, nb_dn, ndn, cfine, ckey, cstart, crun, csorted;
+    DevBuf<int> nb_up, nup, nb_dn, ndn, ckey, cstart, crank;
     DevBuf<int4> extra, ovr;
     DevBuf<int2> cfp;
     DevBuf<Leaf> leaf;
@@ -361,6 +361,9 @@ int prepare_system(const Params& raw, const pdmd_system_desc* d, Prep& out) {
     for (int k = 0; k < 5; ++k) tab.shder[k] = P.shder_dist[k];
     tab.epsilon1 = P.epsilon[1];
     half_stencil(tab.halfst);
+    for (int ka = 0; ka < 4; ++ka)
+        for (int kb = 0; kb < 4; ++kb)
+            for (int dd = -4; dd <= 4; ++dd) tab.statc[(4 * ka + kb) * 9 + dd + 4] = (signed char)chain_code(ka, kb, dd);
     // per-bead topology/identity words and own side-chain bond windows
     // (inputinfo.f:300-349, bond.f:21-31: Calpha owns code 10, N code 11, C code 12)
     std::vector<double2>& bw = out.bw;
@@ -403,9 +406,9 @@ int64_t device_bytes(const Prep& pp) {
     const int64_t N = H.N, cap = H.cap, nc = (int64_t)pp.Mq * pp.Mq * pp.Mq;
     const int64_t sizes[] = {(int64_t)sizeof(DevTables), N * (int64_t)sizeof(Rec), N * 16 /*bw*/, N * 16 /*extra*/,
                              N * 16 /*ovr*/, N * 32 /*old_r*/, N * cap * 4 /*nb_up*/, N * cap * 4 /*nb_dn*/,
-                             (N + 1) * 4 /*nup*/, (N + 1) * 4 /*ndn*/, (N + 3) * (int64_t)sizeof(Leaf), N * 4 /*cfine*/,
-                             N * 4 /*ckey*/, N * 8 /*cfp*/, N * 4 /*csorted*/, N * 32 /*spos*/, N * 16 /*sinfo*/,
-                             (nc + 1) * 4 /*cstart*/, nc * 4 /*crun*/, (N + 3) * 8 /*stamp*/,
+                             (N + 1) * 4 /*nup*/, (N + 1) * 4 /*ndn*/, (N + 3) * (int64_t)sizeof(Leaf),
+                             N * 4 /*ckey*/, N * 8 /*cfp*/, N * 4 /*crank*/, N * 32 /*spos*/, N * 16 /*sinfo*/,
+                             (nc + 1) * 4 /*cstart*/, (N + 3) * 8 /*stamp*/,
                              (int64_t)sizeof(SysState)};
     int64_t b = 0;
     for (int64_t x : sizes) b += (x + 4095) / 4096 * 4096;
@@ -568,16 +571,14 @@ int prepared_add(pdmd_ctx* ctx, PreparedSystem* ps, int32_t* sys_id) {
     HIPCHK(H.nup.alloc(N + 1));  // one more: the event loop's pair gather reads 8 bytes
     HIPCHK(H.ndn.alloc(N + 1));
     HIPCHK(H.leaf.alloc(N + 3));
-    HIPCHK(H.cfine.alloc(N));
     HIPCHK(H.ckey.alloc(N));
     HIPCHK(H.cfp.alloc(N));
-    HIPCHK(H.csorted.alloc(N));
+    HIPCHK(H.crank.alloc(N));
     HIPCHK(H.spos.alloc(N));
     HIPCHK(H.sinfo.alloc(N));
     HIPCHK(H.stamp.alloc(N + 3));
     HIPCHK(hipMemsetAsync(H.stamp.p, 0, sizeof(unsigned long long) * (size_t)(N + 3), ctx->stream));
     HIPCHK(H.cstart.alloc((size_t)Mq * Mq * Mq + 1));
-    HIPCHK(H.crun.alloc((size_t)Mq * Mq * Mq));
     {
         std::vector<SysState> sv(1, st);
         HIPCHK(upload(H.st, sv));
@@ -611,12 +612,10 @@ int prepared_add(pdmd_ctx* ctx, PreparedSystem* ps, int32_t* sys_id) {
     D.nb_dn = H.nb_dn.p;
     D.ndn = H.ndn.p;
     D.leaf = H.leaf.p;
-    D.cfine = H.cfine.p;
     D.ckey = H.ckey.p;
     D.cfp = H.cfp.p;
     D.cstart = H.cstart.p;
-    D.crun = H.crun.p;
-    D.csorted = H.csorted.p;
+    D.crank = H.crank.p;
     D.spos = H.spos.p;
     D.sinfo = H.sinfo.p;
     D.stamp = H.stamp.p;

@@ -228,52 +228,31 @@ __device__ double dlog(double x) {
 // ------------------------------------------------------------------------
 // pair codes: closed form of make_code.f from two topo words, overrides
 // ------------------------------------------------------------------------
-__device__ inline int static_t0(int ta, int tb) {
-    int ka = topo_kind(ta), ra = topo_res(ta), kb = topo_kind(tb), rb = topo_res(tb);
-    if (topo_chain(ta) == topo_chain(tb)) {
-        // -Dchaptype=2 builds no code inside a second-species chain
-        // (make_code.f:349,366; its side-chain loop finds no firstside2 entry)
-        if (topo_free(ta)) return 1;
-        if (ka > kb || (ka == kb && ra > rb)) {
-            int t = ka;
-            ka = kb;
-            kb = t;
-            t = ra;
-            ra = rb;
-            rb = t;
-        }
-        const int d = rb - ra;
-        switch (ka * 4 + kb) {
-            case 0: return d == 1 ? 9 : 1;
-            case 1: return d == 0 ? 4 : (d == 1 ? 7 : (d == -1 ? 18 : 1));
-            case 2: return d == 0 ? 5 : (d == -1 ? 8 : (d == 1 ? 17 : 1));
-            case 3: return d == 0 ? 10 : (d == 1 ? 24 : (d == -1 ? 25 : 1));
-            case 5: return d == 1 ? 20 : 1;
-            case 6:
-                if (d == -1) return 6;
-                if (d == 0) return 8;
-                if (d == -2) return 19;
-                return (d >= -3 && d <= 3) ? 1 : 15;
-            case 7: return d == 0 ? 11 : (d == -1 ? 23 : 1);
-            case 10: return d == 1 ? 21 : 1;
-            case 11: return d == 0 ? 12 : (d == 1 ? 22 : (d == 2 ? 26 : 1));
-            case 15: return (d >= 4 && topo_hp(ta) && topo_hp(tb)) ? 16 : 1;
-            default: return 1;
-        }
-    }
+// without a branch: the same-chain rules come from a table over the two bead
+// kinds and their residue distance, clamped to 4 either way (DevTables::statc,
+// chain_code).  As a switch, every rule that some lane needed ran on its own.
+__device__ inline int static_t(const DevTables& T, int ta, int tb) {
+    const int ka = topo_kind(ta), ra = topo_res(ta), kb = topo_kind(tb), rb = topo_res(tb);
+    const bool swap = ka > kb || (ka == kb && ra > rb);
+    const int k4 = swap ? kb * 4 + ka : ka * 4 + kb, d = swap ? ra - rb : rb - ra;
+    int same = T.statc[k4 * 9 + min(max(d, -4), 4) + 4];
+    const bool hp = topo_hp(ta) && topo_hp(tb);
+    same = same == 16 && !hp ? 1 : same;
+    // -Dchaptype=2 builds no code inside a second-species chain
+    // (make_code.f:349,366; its side-chain loop finds no firstside2 entry)
+    same = topo_free(ta) ? 1 : same;
     // -Dno_h zeroes hp only where make_code.f:80-104 reads it (different
     // chains); the same-chain loops read hp1/hp2 (make_code.f:174-186)
     // and none between two second-species chains (make_code.f:519-547)
-    if (ka == 3 && kb == 3) return (topo_hp(ta) && topo_hp(tb) && !topo_noh(ta) && !(topo_free(ta) && topo_free(tb))) ? 16 : 1;
-    if (ka == 1 && kb == 2) return (topo_pro(ta) && topo_chain(ta) < topo_chain(tb)) ? 1 : 15;
-    if (ka == 2 && kb == 1) return (topo_pro(tb) && topo_chain(tb) < topo_chain(ta)) ? 1 : 15;
-    return 1;
-}
-// under -Dno_hbs make_code.f skips every code-15 assignment (:114-170,
-// :192-208, :348-365): those pairs keep the hard-core code 1
-__device__ inline int static_t(int ta, int tb) {
-    const int r = static_t0(ta, tb);
-    return (r == 15 && topo_nohbs(ta)) ? 1 : r;
+    const bool rr = ka == 3 && kb == 3, well = rr && hp && !topo_noh(ta) && !(topo_free(ta) && topo_free(tb));
+    const bool nc = (ka == 1 && kb == 2) || (ka == 2 && kb == 1);
+    const int tn = ka == 1 ? ta : tb, tc = ka == 1 ? tb : ta;
+    const bool pro = topo_pro(tn) && topo_chain(tn) < topo_chain(tc);
+    const int other = well ? 16 : (nc && !pro ? 15 : 1);
+    const int r = topo_chain(ta) == topo_chain(tb) ? same : other;
+    // under -Dno_hbs make_code.f skips every code-15 assignment (:114-170,
+    // :192-208, :348-365): those pairs keep the hard-core code 1
+    return r == 15 && topo_nohbs(ta) ? 1 : r;
 }
 // Where nbor.f finds the pair {a, b}, as one 64-bit key: the cell it scans
 // (cell_add.f's linear index, cells in ascending order), the place of that
@@ -281,25 +260,27 @@ __device__ inline int static_t(int ta, int tb) {
 // (cell_link.f's half stencil; 0 for the own cell), the other bead's place.
 // A bead's neighbour rows in nbor.f's order are its rows sorted by this key.
 // a and b: the beads' fine cells (10 bits per axis) and list places.
-__device__ inline unsigned long long nbor_key(int M, const DevTables& T, int2 a, int2 b) {
-    const int fa = a.x, fb = b.x, pa = a.y & 0xFFFF, pb = b.y & 0xFFFF, nc = M + 4;
-    int d[3];
+__device__ inline unsigned fine_lin(int f, int nc) {
+    return 1u + (unsigned)((f & 1023) + 2) + (unsigned)((((f >> 10) & 1023) + 2) + ((f >> 20) + 2) * nc) * (unsigned)nc;
+}
+// la: fine_lin of a's cell
+__device__ inline unsigned long long nbor_key(int M, const DevTables& T, int2 a, unsigned la, int2 b) {
+    const int fa = a.x, fb = b.x, pa = a.y & 0xFFFF, pb = b.y & 0xFFFF;
+    int at = 62;  // (dx + 2) + 5 (dy + 2) + 25 (dz + 2) of the periodic offset, each in [-2, 2]
+    const int mul[3] = {1, 5, 25};
+#pragma unroll
     for (int q = 0; q < 3; ++q) {
         // periodic offset in [-(M / 2), M - M / 2), in [-2, 2] for neighbours
         int t = ((fb >> (10 * q)) & 1023) - ((fa >> (10 * q)) & 1023);
         t += t < 0 ? M : 0;
-        d[q] = t < M - M / 2 ? t : t - M;
+        at += mul[q] * (t < M - M / 2 ? t : t - M);
     }
-    auto lin = [&](int f) {
-        return 1ull + (unsigned long long)((f & 1023) + 2) + (unsigned long long)(((f >> 10) & 1023) + 2) * nc +
-               (unsigned long long)((f >> 20) + 2) * nc * nc;
-    };
-    if (d[0] == 0 && d[1] == 0 && d[2] == 0)
-        return (lin(fa) << 26) | ((unsigned long long)min(pa, pb) << 16) | (unsigned long long)max(pa, pb);
-    const int h = T.halfst[(d[0] + 2) + 5 * (d[1] + 2) + 25 * (d[2] + 2)];
-    if (h > 0) return (lin(fa) << 26) | ((unsigned long long)pa << 16) | ((unsigned long long)h << 10) | (unsigned)pb;
-    const int g = T.halfst[(2 - d[0]) + 5 * (2 - d[1]) + 25 * (2 - d[2])];
-    return (lin(fb) << 26) | ((unsigned long long)pb << 16) | ((unsigned long long)g << 10) | (unsigned)pa;
+    const int h = T.halfst[at], g = T.halfst[124 - at];
+    const bool own = at == 62, by_a = own || h > 0;
+    const unsigned lin = by_a ? la : fine_lin(fb, M + 4);
+    const unsigned first = own ? min(pa, pb) : (by_a ? pa : pb);
+    const unsigned rest = own ? max(pa, pb) : (by_a ? (unsigned)(h << 10 | pb) : (unsigned)(g << 10 | pa));
+    return ((unsigned long long)lin << 26) | (first << 16) | rest;
 }
 
 // ev_code(row, col) with row's override slots o
@@ -316,7 +297,7 @@ __device__ void set_code(const SysDev&, int row, int col, int code, int& status)
     const SysDev& S = sdev();
 
     int4 o = gld(S.ovr + (row));
-    const int stat = static_t(gl1(&S.rec[row].topo), gl1(&S.rec[col].topo));
+    const int stat = static_t(tabs(), gl1(&S.rec[row].topo), gl1(&S.rec[col].topo));
     if (o.x >= 0 && (o.x >> 8) == col) o.x = -1;
     if (o.y >= 0 && (o.y >> 8) == col) o.y = -1;
     if (o.z >= 0 && (o.z >> 8) == col) o.z = -1;
@@ -1443,7 +1424,7 @@ __device__ void full_one(const SysDev&, const Lds&, int l, const Rec& rl, double
             }
             const Rec rm = load_rec(S, P, m);
             const int4 om = gld(S.ovr + (m));
-            if (stat < 0) stat = static_t(rm.topo, rl.topo);
+            if (stat < 0) stat = static_t(T, rm.topo, rl.topo);
             const int code = dyn_code(om, l, stat);  // ev_code(m, l), eventredo_up.f:28
             double tij = 1000000000.0;
             int ty = 0;
@@ -1473,7 +1454,7 @@ __device__ void full_one(const SysDev&, const Lds&, int l, const Rec& rl, double
 // eventredo_down.f: single-pair update of (st_t, st_p, st_c) of bead l
 __device__ inline void single_update(const DevTables& T, const Rec& rl, int4 ol, double2 bwl, int p, const Rec& rp,
                                      double tf, double& st_t, int& st_p, int& st_c, bool& modified, int& status) {
-    const int code = dyn_code(ol, p, static_t(rl.topo, rp.topo));  // ev_code(l, p)
+    const int code = dyn_code(ol, p, static_t(T, rl.topo, rp.topo));  // ev_code(l, p)
     double tij = 1000000000.0;
     int ty = 0;
     predict(T, code, rl, rp, dyn_bptnr(rl.dyn) == p, bwl, tf, tij, ty);
@@ -1580,7 +1561,7 @@ __device__ void reschedule_generic(const SysDev&, const DevTables&, const Lds&, 
             const int x = owner == 0 ? i : j;
             const Rec rm = load_rec(S, P, m);
             const int4 om = gld(S.ovr + (m));
-            if (stat == 0xFF) stat = static_t(rm.topo, rx.topo);
+            if (stat == 0xFF) stat = static_t(T, rm.topo, rx.topo);
             const int code = dyn_code(om, x, stat);  // ev_code(m, x)
             double tij = 1000000000.0;
             int ty = 0;
@@ -2055,7 +2036,7 @@ __device__ __noinline__ void reschedule(const SysDev&, const DevTables&, const L
                 oc = di.o;
                 bwa = di.bw;
                 xc = m;
-                stat = static_t(ra.topo, rb.topo);
+                stat = static_t(T, ra.topo, rb.topo);
             } else {
                 m = ent & 0xFFFFFF;
                 stat = (ent >> 24) & 0xFF;
@@ -2080,7 +2061,7 @@ __device__ __noinline__ void reschedule(const SysDev&, const DevTables&, const L
                     rb = load_rec(S, P, m);
                     oc = gld(S.ovr + (m));
                 }
-                if (stat == 0xFF) stat = static_t(rb.topo, ra.topo);
+                if (stat == 0xFF) stat = static_t(T, rb.topo, ra.topo);
             }
             const int code = dyn_code(oc, xc, stat);  // ev_code(m, x), or ev_code(l, p) for a single
             double tij = 1000000000.0;
@@ -2742,7 +2723,7 @@ __device__ __forceinline__ int run_event(const Hot& H, const Gather& G, int e, i
         wave_sync();
     };
     if (!ghost) {
-        const int evcode = dyn_code(lane_int4(16), j, static_t(topoi, topoj));  // ev_code(i, j)
+        const int evcode = dyn_code(lane_int4(16), j, uni(static_t(T, topoi, topoj)));  // ev_code(i, j)
         const bool ok = !terminal_t(topoi) && !terminal_t(topoj);
         const int idi = dyn_ident(dyni), idj = dyn_ident(dynj);
         const int Li = topo_len(topoi), Lj = topo_len(topoj);
@@ -3254,7 +3235,7 @@ __device__ __forceinline__ int run_event(const Hot& H, const Gather& G, int e, i
         if (late && (m == i || m == j)) mine = W.base[m == i ? 0 : 1].r;
         Geo g;
         geo(rb, mine, tf, g);  // the order of the two only flips the signs of vectors
-        if (stat == 0x3F) stat = static_t(mine.topo, rb.topo);  // symmetric in its beads
+        if (stat == 0x3F) stat = static_t(T, mine.topo, rb.topo);  // symmetric in its beads
         const int code = dyn_code(om, bidx, stat);  // ev_code(m, x) of a candidate, ev_code(l, p) of a down bead
         const int adyn = dn ? mine.dyn : rb.dyn, cdyn = dn ? rb.dyn : mine.dyn;  // the lower bead's first
         const double2 bwa = make_double2(dn ? bwm.x : bwb.x, dn ? bwm.y : bwb.y);
@@ -3476,240 +3457,241 @@ __device__ __forceinline__ int run_event(const Hot& H, const Gather& G, int e, i
 // Pair (i, j) is listed when its fine cells (cell_add.f binning) are within
 // the n_wrap=2 stencil (|d| <= 2 per axis, periodic) and either its code is
 // a bond/local one (4-12, 17-26) or r^2 <= rlsq(code) (nbor.f:63-128).
-// Steps: fine and coarse cell of every bead; stable counting sort of the
-// beads by coarse cell; copies of position, topology and fine cell in that
-// order; then one lane per bead scans the (up to 27) neighbouring coarse
-// cells, all cell ranges requested before the candidates, each candidate
-// read with two independent loads.  Candidates come in a fixed cell order
-// and ascending bead index within a cell, so the lists are deterministic.
-// A wavefront's LDS scratch of a list rebuild: the search's cell ranges (27
-// per lane) or the row sort's keys and entries.  It lies over the work
-// areas, block minima and leaves, which a rebuild leaves free.
+// Steps: the fine and coarse cell of every bead and its place in the coarse
+// cell (the count's atomic returns it; places come in any order, the rows are
+// sorted afterwards); the cells' starts; copies of position, topology and
+// fine cell in cell order; then a wavefront per coarse cell tests the beads
+// of the cells around it (list_search).
+//
+// A wavefront's LDS scratch of a small system's list rebuild (the staged
+// beads).  It lies over the work areas, block minima and leaves, which a
+// rebuild leaves free.
 constexpr int kScratch = 15872;
-static_assert(27 * kW * (int)sizeof(int2) <= kScratch, "cell ranges exceed the rebuild scratch");
 // v mod m for v in [-1, m]
 __device__ inline int wrap1(int v, int m) { return v < 0 ? v + m : (v >= m ? v - m : v); }
+// fine cell of a bead (cell_add.f), 10 bits per axis
+__device__ inline int fine_cell(const SysDev& S, double x, double y, double z) {
+    const int M = S.M;
+    int cx = (int)((x + S.half) / S.width);
+    int cy = (int)((y + S.half) / S.width);
+    int cz = (int)((z + S.half) / S.width);
+    cx = ((cx % M) + M) % M;
+    cy = ((cy % M) + M) % M;
+    cz = ((cz % M) + M) % M;
+    return cx | (cy << 10) | (cz << 20);
+}
+// The coarse cell of a fine one: cq >= 2 fine cells each, the last one takes
+// the remainder, so every fine cell within the n_wrap = 2 stencil of a bead's
+// lies in the 27 coarse cells around the bead's own.
+__device__ inline void coarse_of(int f, int cq, int Mq, int& qx, int& qy, int& qz) {
+    qx = min((f & 1023) / cq, Mq - 1);
+    qy = min(((f >> 10) & 1023) / cq, Mq - 1);
+    qz = min((f >> 20) / cq, Mq - 1);
+}
+// beads [tid, N) by nthr: fine cell (cfp), coarse cell and place in it
+__device__ inline void list_cells(const SysDev& S, int tid, int nthr) {
+    const int N = S.N, cq = S.cq, Mq = S.M / cq;
+#pragma unroll 2
+    for (int k = tid; k < N; k += nthr) {
+        const Rec b = gld(S.rec + (k));
+        const int f = fine_cell(S, b.x, b.y, b.z);
+        int qx, qy, qz;
+        coarse_of(f, cq, Mq, qx, qy, qz);
+        const int key = qx + Mq * (qy + Mq * qz);
+        gs1(&S.cfp[k].x, f);
+        gs1(S.ckey + (k), key);
+        gs1(S.crank + (k), atomicAdd(&S.cstart[key], 1));
+    }
+}
+// wave-inclusive sum
+__device__ inline int wave_scan(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
+    return v;
+}
+// Exclusive scan of the NC cell counts on the workgroup's nw wavefronts, a
+// contiguous part each: its sum, then (after the others' sums) its starts.
+// part: nw words of LDS.  The counts were made by atomics: read at the L2.
+__device__ inline void list_scan(int* cnt, int NC, int* part, int wave, int nw) {
+    const int lane = lane_id();
+    const int seg = ((NC + nw - 1) / nw + 255) / 256 * 256, lo = min(wave * seg, NC), hi = min(lo + seg, NC);
+    auto at = [&](int q) { return q < hi ? __hip_atomic_load((GLB int*)cnt + q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0; };
+    int sum = 0;
+#pragma unroll 4
+    for (int q = lo + lane; q < hi; q += kW) sum += at(q);
+    sum = __builtin_amdgcn_readlane(wave_scan(sum), kW - 1);
+    if (lane == 0) part[wave] = sum;
+    wg_sync(nw);
+    int carry = 0, all = 0;
+    for (int w = 0; w < nw; ++w) {
+        carry += w < wave ? part[w] : 0;
+        all += part[w];
+    }
+    for (int base = lo; base < hi; base += 4 * kW) {
+        int v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] = at(base + u * kW + lane);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int q = base + u * kW + lane, incl = wave_scan(v[u]);
+            if (q < hi) gs1(cnt + q, carry + incl - v[u]);
+            carry += __builtin_amdgcn_readlane(incl, kW - 1);
+        }
+    }
+    if (wave == 0 && lane == 0) gs1(cnt + NC, all);
+}
+// beads [tid, N) by nthr to their sorted places
+__device__ inline void list_copy(const SysDev& S, int tid, int nthr) {
+#pragma unroll 2
+    for (int k = tid; k < S.N; k += nthr) {
+        const Rec b = gld(S.rec + (k));
+        const int p = gl1(S.cstart + (gl1(S.ckey + (k)))) + gl1(S.crank + (k));
+        gst(S.spos + (p), make_double4(b.x, b.y, b.z, 0.0));
+        gst(S.sinfo + (p), make_int4(k, b.topo, gl1(&S.cfp[k].x), 0));
+    }
+}
+// The lists of the coarse cells whose first sorted bead lies in the 64 places
+// from i0 on (one wavefront): rows, their lengths, and each bead's place in
+// its fine cell's list as cell_add.f builds it (head first: the highest index
+// at 1) with the up-row length in cfp.  mx: longest row met.
+// A cell's candidates (the beads of the up to 27 cells around it) are loaded
+// once, one per lane, and tested against each of the cell's beads in turn:
+// lanes stay full, rows are written by ballot, and only the next cell's loads
+// are a dependent chain.  One lane per bead, each with its own cell ranges,
+// waited for the longest range among 64 scattered beads at every step (178 K
+// cycles per 64 beads at 6144 beads).
+__device__ inline void list_search(const SysDev& S, const DevTables& T, int i0, int& mx, int& status) {
+    const int lane = lane_id();
+    const int N = S.N, M = S.M, cq = S.cq, Mq = M / cq, cap = S.cap;
+    const unsigned long long below = (1ull << lane) - 1ull;
+    const int ps = i0 + lane;
+    int c0 = -1, c1 = -1, q = 0;
+    if (ps < N) {
+        const int4 si = gld(S.sinfo + (ps));
+        int qx, qy, qz;
+        coarse_of(si.z, cq, Mq, qx, qy, qz);
+        q = qx | (qy << 10) | (qz << 20);
+        const int key = qx + Mq * (qy + Mq * qz);
+        c0 = gl1(S.cstart + (key));
+        c1 = gl1(S.cstart + (key + 1));
+    }
+    // lane t < 9: the cells of one (y, z) neighbour row, consecutive along x;
+    // lane 9 + t: the one across the box's face where there is one
+    const int noff = Mq > 2 ? 3 : Mq;  // distinct offsets {0, +1, -1}
+    const int t9 = lane < 9 ? lane : lane - 9, oy = t9 / 3, oz = t9 - 3 * oy;
+    const bool rowl = lane < 18 && oy < noff && oz < noff;
+    for (unsigned long long heads = __ballot(c0 == ps && ps < N); heads; heads &= heads - 1) {
+        const int src = __ffsll((long long)heads) - 1;
+        const int b0 = __builtin_amdgcn_readlane(c0, src), b1 = __builtin_amdgcn_readlane(c1, src);
+        const int qq = __builtin_amdgcn_readlane(q, src);
+        const int qx = qq & 1023, qy = (qq >> 10) & 1023, qz = qq >> 20;
+        const bool wrap = Mq > 2 && (qx == 0 || qx == Mq - 1);
+        int r0 = 0, len = 0;
+        if (rowl && (lane < 9 || wrap)) {
+            const int ny = wrap1(qy + (oy == 2 ? -1 : oy), Mq), nz = wrap1(qz + (oz == 2 ? -1 : oz), Mq);
+            const int row = Mq * (ny + Mq * nz), xw = qx == 0 ? Mq - 1 : 0;
+            r0 = gl1(S.cstart + (row + (lane < 9 ? max(qx - 1, 0) : xw)));
+            len = gl1(S.cstart + (row + (lane < 9 ? min(qx + 1, Mq - 1) : xw) + 1)) - r0;
+        }
+        const int incl = wave_scan(len), excl = incl - len;
+        const int C = __builtin_amdgcn_readlane(incl, kW - 1);
+        const unsigned long long rows = __ballot(len > 0);
+        for (int bb = b0; bb < b1; bb += kW) {
+            // the cell's beads, one per lane
+            const int nb = min(b1 - bb, kW);
+            int4 sb = make_int4(0, 0, 0, 0), ob = make_int4(-1, -1, -1, -1);
+            double4 bp = make_double4(0.0, 0.0, 0.0, 0.0);
+            if (lane < nb) {
+                sb = gld(S.sinfo + (bb + lane));
+                bp = gld(S.spos + (bb + lane));
+                ob = gld(S.ovr + (sb.x));
+            }
+            const unsigned long long om = __ballot((ob.x & ob.y & ob.z & ob.w) != -1);
+            int nu = 0, nd = 0, place = 1;
+            for (int cb = 0; cb < C; cb += kW) {
+                const int cpos = cb + lane;
+                int at = 0;
+                for (unsigned long long rm = rows; rm; rm &= rm - 1) {
+                    const int t = __ffsll((long long)rm) - 1;
+                    const int ex = __builtin_amdgcn_readlane(excl, t), st = __builtin_amdgcn_readlane(r0, t);
+                    at = cpos >= ex ? st + (cpos - ex) : at;
+                }
+                const bool cand = cpos < C;
+                at = cand ? at : 0;
+                const int4 inf = gld(S.sinfo + (at));
+                const double4 pj = gld(S.spos + (at));
+                const int jb = inf.x, fj = inf.z;
+                for (int b = 0; b < nb; ++b) {
+                    const int i = __builtin_amdgcn_readlane(sb.x, b), fi = __builtin_amdgcn_readlane(sb.z, b);
+                    const int ti = __builtin_amdgcn_readlane(sb.y, b);
+                    // fine cells lie in [0, M): differences in (-M, M), taken mod M
+                    int dx = (fj & 1023) - (fi & 1023), dy = ((fj >> 10) & 1023) - ((fi >> 10) & 1023), dz = (fj >> 20) - (fi >> 20);
+                    dx += dx < 0 ? M : 0;
+                    dy += dy < 0 ? M : 0;
+                    dz += dz < 0 ? M : 0;
+                    const bool far = (dx > 2 && dx < M - 2) || (dy > 2 && dy < M - 2) || (dz > 2 && dz < M - 2);
+                    const bool in = cand && jb != i && !far;
+                    const int stat = static_t(T, inf.y, ti);
+                    // ev_code(j,i), nbor.f:63: j's overrides exist only towards i's
+                    int code = stat;
+                    if ((om >> b) & 1ull) {
+                        const int ox = __builtin_amdgcn_readlane(ob.x, b), oyv = __builtin_amdgcn_readlane(ob.y, b);
+                        const int ozv = __builtin_amdgcn_readlane(ob.z, b), ow = __builtin_amdgcn_readlane(ob.w, b);
+                        if (in && ((ox >= 0 && (ox >> 8) == jb) || (oyv >= 0 && (oyv >> 8) == jb) ||
+                                   (ozv >= 0 && (ozv >> 8) == jb) || (ow >= 0 && (ow >> 8) == jb)))
+                            code = dyn_code(gld(S.ovr + (jb)), i, stat);
+                    }
+                    const double rx = min_image(readlane_d(bp.x, b) - pj.x), ry = min_image(readlane_d(bp.y, b) - pj.y),
+                                 rz = min_image(readlane_d(bp.z, b) - pj.z);
+                    const double r2 = rx * rx + ry * ry + rz * rz;
+                    const bool local = (code >= 4 && code <= 12) || (code >= 17 && code < 27);
+                    const bool cut = code >= 1 && code <= 50 && r2 <= T.rlsq[min((unsigned)code, 50u)];
+                    const bool take = in && (local || cut), up = jb > i;
+                    const unsigned long long mu = __ballot(take && up), md = __ballot(take && !up);
+                    const unsigned long long mp = __ballot(cand && fj == fi && up);
+                    const int pos = up ? __builtin_amdgcn_readlane(nu, b) + __popcll(mu & below)
+                                       : __builtin_amdgcn_readlane(nd, b) + __popcll(md & below);
+                    if (take && pos < cap) gs1((up ? S.nb_up : S.nb_dn) + ((size_t)i * cap + pos), jb | (stat << 24));
+                    nu += lane == b ? __popcll(mu) : 0;
+                    nd += lane == b ? __popcll(md) : 0;
+                    place += lane == b ? __popcll(mp) : 0;
+                }
+            }
+            if (lane < nb) {
+                if (nu > cap || nd > cap) status = kErrListCapacity;
+                mx = max(mx, max(nu, nd));
+                gs1(S.nup + (sb.x), min(nu, cap));
+                gs1(S.ndn + (sb.x), min(nd, cap));
+                gs2(S.cfp + (sb.x), make_int2(sb.z, place | (min(nu, cap) << 16)));
+            }
+        }
+    }
+}
 __device__ void rebuild_lists(const SysDev&, const Lds&, Sc& c) {
     const Lds& L = ldsv();
-
     const SysDev& S = sdev();
-
     const DevTables& T = tabs();
     const int lane = lane_id(), wave = wave_id(), nw = L.nw;
     const int tid = (int)threadIdx.x, nthr = kW * nw;
-    // coarse cells of cq >= 2 fine cells each (the last one takes the
-    // remainder): every fine cell within the n_wrap = 2 stencil of a bead's
-    // lies in the 27 coarse cells around the bead's own
-    const int N = S.N, M = S.M, cq = S.cq, Mq = M / cq, NC = Mq * Mq * Mq, cap = S.cap;
+    const int Mq = S.M / S.cq, NC = Mq * Mq * Mq;
     PH_BEGIN(trl);
-#pragma unroll 4
-    for (int k = tid; k < N; k += nthr) {
-        const Rec b = gld(S.rec + (k));
-        int cx = (int)((b.x + S.half) / S.width);
-        int cy = (int)((b.y + S.half) / S.width);
-        int cz = (int)((b.z + S.half) / S.width);
-        cx = ((cx % M) + M) % M;
-        cy = ((cy % M) + M) % M;
-        cz = ((cz % M) + M) % M;
-        gs1(S.cfine + (k), cx | (cy << 10) | (cz << 20));
-        const int qx = min(cx / cq, Mq - 1), qy = min(cy / cq, Mq - 1), qz = min(cz / cq, Mq - 1);
-        gs1(S.ckey + (k), qx + Mq * (qy + Mq * qz));
-    }
-    for (int q = tid; q < NC; q += nthr) {
-        gs1(S.cstart + (q), 0);
-        gs1(S.crun + (q), 0);
-    }
+    for (int q = tid; q < NC; q += nthr) gs1(S.cstart + (q), 0);
     wg_sync(nw);
-    for (int k = tid; k < N; k += nthr) atomicAdd(&S.cstart[gl1(S.ckey + k)], 1);
+    list_cells(S, tid, nthr);
     wg_sync(nw);
     PH_END(S, kPhLCells, trl);
-    // exclusive scan of the cell counts (wavefront 0)
-    int carry = 0;
-    for (int base = 0; wave == 0 && base < NC; base += kW) {
-        const int q = base + lane;
-        const int v = q < NC ? gl1(S.cstart + (q)) : 0;
-        int incl = v;
-        incl += __builtin_amdgcn_update_dpp(0, incl, 0x111, 0xf, 0xf, false);
-        incl += __builtin_amdgcn_update_dpp(0, incl, 0x112, 0xf, 0xf, false);
-        incl += __builtin_amdgcn_update_dpp(0, incl, 0x114, 0xf, 0xf, false);
-        incl += __builtin_amdgcn_update_dpp(0, incl, 0x118, 0xf, 0xf, false);
-        incl += __builtin_amdgcn_update_dpp(0, incl, 0x142, 0xa, 0xf, false);
-        incl += __builtin_amdgcn_update_dpp(0, incl, 0x143, 0xc, 0xf, false);
-        if (q < NC) gs1(S.cstart + (q), carry + incl - v);
-        carry += __builtin_amdgcn_readlane(incl, kW - 1);
-    }
-    if (wave == 0 && lane == 0) gs1(S.cstart + (NC), carry);
+    list_scan(S.cstart, NC, reinterpret_cast<int*>(smem + L.o_pool), wave, nw);
     wg_sync(nw);
     PH_END(S, kPhLScan, trl);
-    // stable scatter in bead order (wavefront 0): rank among the lower lanes
-    // of the same cell
-    for (int base = 0; wave == 0 && base < N; base += kW) {
-        const int k = base + lane;
-        const int key = k < N ? gl1(S.ckey + (k)) : -1;
-        int rank = 0, cnt = 0;
-        const int nl = min(N - base, kW);
-        for (int r = 0; r < nl; ++r) {
-            const int o = __builtin_amdgcn_readlane(key, r);
-            if (o == key) {
-                if (r < lane) ++rank;
-                ++cnt;
-            }
-        }
-        const int basepos = k < N ? gl1(S.cstart + (key)) + gl1(S.crun + (key)) : 0;
-        wave_sync_mem();
-        if (k < N) {
-            gs1(S.csorted + (basepos + rank), k);
-            if (rank == cnt - 1) gs1(S.crun + (key), gl1(S.crun + (key)) + cnt);
-        }
-        wave_sync_mem();
-    }
+    list_copy(S, tid, nthr);
     wg_sync(nw);
-    PH_END(S, kPhLScatter, trl);
-    // positions, topology and fine cells in sorted order
-#pragma unroll 4
-    for (int p2 = tid; p2 < N; p2 += nthr) {
-        const int jb = gl1(S.csorted + (p2));
-        const Rec b = gld(S.rec + (jb));
-        gst(S.spos + (p2), make_double4(b.x, b.y, b.z, 0.0));
-        gst(S.sinfo + (p2), make_int4(jb, b.topo, gl1(S.cfine + jb), 0));
-    }
-    wg_sync(nw);
-    // each bead's place in its fine cell's list as cell_add.f builds it
-    // (head first, the highest index at 1): the beads of a fine cell sit
-    // in its coarse cell's sorted run in index order
-    for (int p2 = tid; p2 < N; p2 += nthr) {
-        const int4 si = gld(S.sinfo + (p2));
-        const int end = gl1(S.cstart + (gl1(S.ckey + si.x) + 1));
-        int pos = 1;
-#pragma unroll 4
-        for (int q2 = p2 + 1; q2 < end; ++q2) pos += gl1(&S.sinfo[q2].z) == si.z ? 1 : 0;
-        gs2(S.cfp + (si.x), make_int2(si.z, pos));
-    }
-    wg_sync(nw);  // every bead's list place is written
     PH_END(S, kPhLCopy, trl);
     int mx = 0, status = 0;
-    const int noff = Mq > 2 ? 3 : Mq;  // distinct coarse offsets {0, +1, -1}
-    // per lane, its bead's non-empty neighbour cell ranges, [t][lane] in the
-    // wavefront's scratch; wavefronts take 64-bead chunks in turn
-    int2* rng = reinterpret_cast<int2*>(smem + L.o_pool + wave * kScratch);
-    // beads are taken in cell order (64 consecutive sorted places per
-    // chunk): the lanes of a chunk sit in the same or adjacent cells, so
-    // their candidate reads fall on shared cache lines
-    for (int i0 = wave * kW; wave < L.nwr && i0 < N; i0 += L.nwr * kW) {
-        const int ps = i0 + lane;
-        const bool act = ps < N;
-        const int4 si = act ? gld(S.sinfo + (ps)) : make_int4(-1, 0, 0, 0);
-        const double4 bi = act ? gld(S.spos + (ps)) : make_double4(0.0, 0.0, 0.0, 0.0);
-        const int i = si.x;  // -1 on an idle lane
-        const int fi = si.z;
-        const int ix = fi & 1023, iy = (fi >> 10) & 1023, iz = fi >> 20;
-        // the coarse cell, as the binning step derived it from the fine one
-        const int qx = min(ix / cq, Mq - 1), qy = min(iy / cq, Mq - 1), qz = min(iz / cq, Mq - 1);
-        const int4 oi = gld(S.ovr + (act ? i : 0));
-        int nr = 0;
-#pragma unroll
-        for (int t = 0; t < 27; ++t) {
-            const int a = t / 9, bb = (t / 3) % 3, cc = t % 3;
-            if (act && a < noff && bb < noff && cc < noff) {
-                const int oa = a == 2 ? -1 : a, ob = bb == 2 ? -1 : bb, oc = cc == 2 ? -1 : cc;
-                // periodic neighbour of a coarse cell in [0, Mq) by one step
-                const int nx = wrap1(qx + oa, Mq), ny = wrap1(qy + ob, Mq), nz = wrap1(qz + oc, Mq);
-                const int cell = nx + Mq * (ny + Mq * nz);
-                const int c0 = gl1(S.cstart + (cell)), c1 = gl1(S.cstart + (cell + 1));
-                if (c1 > c0) {
-                    rng[nr * kW + lane] = make_int2(c0, c1);
-                    ++nr;
-                }
-            }
-        }
-        wave_sync();
-        // candidates in (cell, index) order, four in flight per lane
-        int ri = 0, p = 0, pe = 0;
-        if (nr > 0) {
-            const int2 r0 = rng[lane];
-            p = r0.x;
-            pe = r0.y;
-        }
-        int nu = 0, nd = 0;
-        while (__ballot(ri < nr)) {
-            int pu[4];
-            bool vu[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                vu[u] = ri < nr;
-                pu[u] = p;
-                if (vu[u]) {
-                    ++p;
-                    if (p >= pe) {
-                        ++ri;
-                        if (ri < nr) {
-                            const int2 r1 = rng[ri * kW + lane];
-                            p = r1.x;
-                            pe = r1.y;
-                        }
-                    }
-                }
-            }
-            int4 inf[4];
-            double4 pj[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                if (vu[u]) {
-                    inf[u] = gld(S.sinfo + (pu[u]));
-                    pj[u] = gld(S.spos + (pu[u]));
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                if (!vu[u]) continue;
-                const int jb = inf[u].x;
-                if (jb == i) continue;
-                const int fj = inf[u].z;
-                // fine cells lie in [0, M): differences in (-M, M), taken mod M
-                int dx = (fj & 1023) - ix, dy = ((fj >> 10) & 1023) - iy, dz = (fj >> 20) - iz;
-                dx += dx < 0 ? M : 0;
-                dy += dy < 0 ? M : 0;
-                dz += dz < 0 ? M : 0;
-                if ((dx > 2 && dx < M - 2) || (dy > 2 && dy < M - 2) || (dz > 2 && dz < M - 2)) continue;
-                const int stat = static_t(inf[u].y, si.y);
-                // ev_code(j,i), nbor.f:63: j's overrides exist only towards i's
-                int code = stat;
-                if ((oi.x >= 0 && (oi.x >> 8) == jb) || (oi.y >= 0 && (oi.y >> 8) == jb) ||
-                    (oi.z >= 0 && (oi.z >> 8) == jb) || (oi.w >= 0 && (oi.w >> 8) == jb))
-                    code = dyn_code(gld(S.ovr + (jb)), i, stat);
-                bool take;
-                if ((code >= 4 && code <= 12) || (code >= 17 && code < 27)) {
-                    take = true;
-                } else {
-                    double rx = bi.x - pj[u].x, ry = bi.y - pj[u].y, rz = bi.z - pj[u].z;
-                    rx = rx - round(rx);
-                    ry = ry - round(ry);
-                    rz = rz - round(rz);
-                    const double r2 = rx * rx + ry * ry + rz * rz;
-                    take = code >= 1 && code <= 50 && r2 <= T.rlsq[code];
-                }
-                if (!take) continue;
-                if (jb > i) {
-                    if (nu < cap) gs1(S.nb_up + ((size_t)i * cap + nu), jb | (stat << 24));
-                    ++nu;
-                } else {
-                    if (nd < cap) gs1(S.nb_dn + ((size_t)i * cap + nd), jb | (stat << 24));
-                    ++nd;
-                }
-            }
-        }
-        if (act) {
-            if (nu > cap || nd > cap) status = kErrListCapacity;
-            mx = max(mx, max(nu, nd));
-            gs1(S.nup + (i), min(nu, cap));
-            gs1(S.ndn + (i), min(nd, cap));
-            // the up-row length rides with the bead's list place, for the
-            // down rows that name the bead (sort_rows)
-            const int2 fp = gl2(S.cfp + (i));
-            gs2(S.cfp + (i), make_int2(fp.x, fp.y | (min(nu, cap) << 16)));
-        }
-        wave_sync();
-    }
+    for (int i0 = wave * kW; i0 < S.N; i0 += nw * kW) list_search(S, T, i0, mx, status);
     PH_END(S, kPhLSearch, trl);
     status = wave_status(status);
     if (status && !c.status) c.status = status;
@@ -3785,7 +3767,6 @@ __device__ void rebuild_lists_dense(const SysDev&, const Lds&, Sc& c) {
             for (int m = 0; m < kW; ++m) pos += (__builtin_amdgcn_readlane(v, m) == f && q0 + m > k) ? 1 : 0;
         }
         if (k < N) {
-            gs1(S.cfine + (k), f);
             gs2(S.cfp + (k), make_int2(f, pos));
         }
     }
@@ -3803,7 +3784,7 @@ __device__ void rebuild_lists_dense(const SysDev&, const Lds&, Sc& c) {
         if (v) {
             const Stage si = stg[i], sj = stg[jb];
             const int4 oi = sovr[i];
-            stat = static_t(sj.topo, si.topo);
+            stat = static_t(T, sj.topo, si.topo);
             // ev_code(j,i), nbor.f:63: j's overrides exist only towards i's
             int code = stat;
             if ((oi.x >= 0 && (oi.x >> 8) == jb) || (oi.y >= 0 && (oi.y >> 8) == jb) ||
@@ -3905,12 +3886,27 @@ __device__ void events_all(const SysDev&, const DevTables&, const Lds&, Sc&) {
         const double2 bwi = gld(S.bw + (i));
         double ti = c.interval_max + kLt;
         int pi = -1, ci = -1;
+        // the next partner's loads are in flight while one is predicted
         const int n = gl1(S.nup + (i));
+        const int* const row = S.nb_up + (size_t)i * cap;
+        int ent = n > 0 ? gl1(row) : 0, ent1 = n > 1 ? gl1(row + 1) : 0;
+        Rec bm1 = bi;
+        int4 om1 = make_int4(-1, -1, -1, -1);
+        if (n > 0) {
+            bm1 = gld(S.rec + (ent & 0xFFFF));
+            om1 = gld(S.ovr + (ent & 0xFFFF));
+        }
         for (int k = 0; k < n; ++k) {
-            const int ent = gl1(S.nb_up + ((size_t)i * cap + k));
-            const int m = ent & 0xFFFFFF;
-            const Rec bm = gld(S.rec + (m));
-            const int code = dyn_code(gld(S.ovr + (m)), i, ent >> 24);
+            const Rec bm = bm1;
+            const int4 om = om1;
+            const int m = ent & 0xFFFF, stat = ent >> 24;
+            ent = ent1;
+            if (k + 1 < n) {
+                bm1 = gld(S.rec + (ent & 0xFFFF));
+                om1 = gld(S.ovr + (ent & 0xFFFF));
+            }
+            if (k + 2 < n) ent1 = gl1(row + (k + 2));
+            const int code = dyn_code(om, i, stat);
             double tij = 1000000000.0;
             int ty = 0;
             predict(T, code, bi, bm, dyn_bptnr(bi.dyn) == m, bwi, 0.0, tij, ty);
@@ -3927,7 +3923,7 @@ __device__ void events_all(const SysDev&, const DevTables&, const Lds&, Sc&) {
             const int m = k == 0 ? e.x : (k == 1 ? e.y : e.z);
             if (m > i) {
                 const Rec bm = gld(S.rec + (m));
-                const int code = dyn_code(gld(S.ovr + (m)), i, static_t(bm.topo, bi.topo));
+                const int code = dyn_code(gld(S.ovr + (m)), i, static_t(T, bm.topo, bi.topo));
                 double tij = 1000000000.0;
                 int ty = 0;
                 // events.f:79-83: code 1 -> core, anything else -> shoulder
@@ -3962,93 +3958,99 @@ __device__ void events_all(const SysDev&, const DevTables&, const Lds&, Sc&) {
 // nbor_key, so that the lowest list position among partners tied in time
 // is the one eventredo_up.f's strict < takes in nbor.f's row, and down
 // rows are walked in partial_events.f's order.  One lane per row (row r:
-// bead r / 2, its up row for even r, its down row for odd r): the row's
-// entries and keys in the wavefront's scratch (kSortMax each per lane,
-// [slot][lane]), the row in up to five 16-byte loads and all its partner
-// loads in flight, then every entry written at its rank; a longer row is
-// sorted by the whole wavefront, one lane per entry.
+// bead r / 2, its up row for even r, its down row for odd r): the row in
+// registers (up to five 16-byte loads), its partners' cells and places in one
+// round of loads, every entry written at its rank, the count of lower keys.
+// The loops run to the longest row of the wavefront's 64.  A row of more than
+// kSortMax entries is sorted by the whole wavefront, one lane per entry.
+// Down-row entries take their bead's up-row length on the way (bits 16-22).
 constexpr int kSortMax = 20;
-static_assert(12 * kSortMax * kW <= kScratch, "row sort staging exceeds the rebuild scratch");
-__device__ void sort_rows(const SysDev&, const DevTables&, const Lds&) {
-    const Lds& L = ldsv();
-    const SysDev& S = sdev();
-    const DevTables& T = tabs();
-    const int lane = lane_id(), wave = wave_id(), nw = L.nw, N = S.N, cap = S.cap, M = S.M;
-    unsigned long long* const keys = reinterpret_cast<unsigned long long*>(smem + L.o_pool + wave * kScratch);  // [kSortMax][kW]
-    int* const ents = reinterpret_cast<int*>(keys + kSortMax * kW);                        // [kSortMax][kW]
+__device__ inline void sort_rows(const SysDev& S, const DevTables& T, int r0) {
+    const int lane = lane_id(), N = S.N, cap = S.cap, M = S.M;
     const bool vec = (cap & 3) == 0;  // rows of whole int4s (row bases are 16-byte aligned)
-    for (int r0 = wave * kW; wave < L.nwr && r0 < 2 * N; r0 += L.nwr * kW) {
-        const int r = r0 + lane;
-        const bool act = r < 2 * N;
-        const int x = act ? r >> 1 : 0;
-        int* const row = ((r & 1) == 0 ? S.nb_up : S.nb_dn) + (size_t)x * cap;
-        const int n = act ? min(gl1(((r & 1) == 0 ? S.nup : S.ndn) + (x)), cap) : 0;
-        const int2 cx = gl2(S.cfp + (x));
-        const bool dnr = (r & 1) != 0;  // a down row's entries carry their bead's up-row length in bits 16 to 22
-        if ((n >= 2 || (dnr && n == 1)) && n <= kSortMax) {
+    const int r = r0 + lane;
+    const bool act = r < 2 * N;
+    const int x = act ? r >> 1 : 0;
+    const bool dnr = (r & 1) != 0;
+    int* const row = (dnr ? S.nb_dn : S.nb_up) + (size_t)x * cap;
+    const int n = act ? min(gl1((dnr ? S.ndn : S.nup) + (x)), cap) : 0;
+    const int2 cx = gl2(S.cfp + (x));
+    const unsigned lx = fine_lin(cx.x, M + 4);
+    const int ns = n <= kSortMax ? n : 0;
+    const int nmax = wave_imax(ns);
+    int e[kSortMax];
+#pragma unroll
+    for (int u = 0; u < kSortMax / 4; ++u) {
+        e[4 * u] = e[4 * u + 1] = e[4 * u + 2] = e[4 * u + 3] = 0;
+        if (4 * u < ns) {
             if (vec) {
                 // reads up to the next multiple of 4 (<= kSortMax, <= cap)
-                int4 v[kSortMax / 4];
-#pragma unroll
-                for (int u = 0; u < kSortMax / 4; ++u)
-                    if (4 * u < n) v[u] = gld(reinterpret_cast<const int4*>(row) + u);
-#pragma unroll
-                for (int u = 0; u < kSortMax / 4; ++u)
-                    if (4 * u < n) {
-                        ents[(4 * u) * kW + lane] = v[u].x;
-                        ents[(4 * u + 1) * kW + lane] = v[u].y;
-                        ents[(4 * u + 2) * kW + lane] = v[u].z;
-                        ents[(4 * u + 3) * kW + lane] = v[u].w;
-                    }
+                const int4 v = gld(reinterpret_cast<const int4*>(row) + u);
+                e[4 * u] = v.x;
+                e[4 * u + 1] = v.y;
+                e[4 * u + 2] = v.z;
+                e[4 * u + 3] = v.w;
             } else {
-                for (int k = 0; k < n; ++k) ents[k * kW + lane] = gl1(row + (k));
-            }
-            {
-                int e[kSortMax];
-                int2 cb[kSortMax];
 #pragma unroll
-                for (int u = 0; u < kSortMax; ++u) e[u] = u < n ? ents[u * kW + lane] & 0xFFFFFF : x;
-#pragma unroll
-                for (int u = 0; u < kSortMax; ++u)
-                    if (u < n) cb[u] = gl2(S.cfp + (e[u]));
-#pragma unroll
-                for (int u = 0; u < kSortMax; ++u)
-                    if (u < n) {
-                        keys[u * kW + lane] = nbor_key(M, T, cx, cb[u]);
-                        if (dnr) ents[u * kW + lane] |= (cb[u].y >> 16) << 16;
-                    }
+                for (int w = 0; w < 4; ++w)
+                    if (4 * u + w < ns) e[4 * u + w] = gl1(row + (4 * u + w));
             }
-            for (int k = 0; k < n; ++k) {
-                const unsigned long long kk = keys[k * kW + lane];
-                int rk = 0;
-#pragma unroll
-                for (int m = 0; m < kSortMax; ++m) rk += m < n && keys[m * kW + lane] < kk ? 1 : 0;
-                gs1(row + (rk), ents[k * kW + lane]);
-            }
-        }
-        // rows longer than the staging: the wavefront sorts each in turn
-        unsigned long long big = __ballot(n > kSortMax);
-        while (big) {
-            const int src = __ffsll((long long)big) - 1;
-            big &= big - 1;
-            const int rb_ = r0 + src, xb = rb_ >> 1, nbig = __shfl(n, src, kW);
-            int* const rb = ((rb_ & 1) == 0 ? S.nb_up : S.nb_dn) + (size_t)xb * cap;
-            const int2 cxb = gl2(S.cfp + (xb));
-            int e = lane < nbig ? gl1(rb + (lane)) : 0;
-            const int2 ce = gl2(S.cfp + (e & 0xFFFF));
-            const unsigned long long kk = lane < nbig ? nbor_key(M, T, cxb, ce) : ~0ull;
-            if ((rb_ & 1) != 0) e |= (ce.y >> 16) << 16;
-            int rk = 0;
-            for (int m = 0; m < nbig; ++m) {
-                const unsigned long long km = (unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)kk, m) |
-                                              ((unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(kk >> 32), m) << 32);
-                rk += km < kk ? 1 : 0;
-            }
-            wave_sync_mem();  // every lane has read its entry before any is written
-            if (lane < nbig) gs1(rb + (rk), e);
-            wave_sync_mem();
         }
     }
+    int2 cb[kSortMax];
+#pragma unroll
+    for (int u = 0; u < kSortMax; ++u) {
+        cb[u] = make_int2(0, 0);
+        if (u < ns) cb[u] = gl2(S.cfp + (e[u] & 0xFFFF));
+    }
+    unsigned long long key[kSortMax];
+#pragma unroll
+    for (int u = 0; u < kSortMax; ++u) {
+        key[u] = ~0ull;
+        if (u < nmax) {
+            const unsigned long long k = nbor_key(M, T, cx, lx, cb[u]);
+            key[u] = u < ns ? k : ~0ull;
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < kSortMax; ++u) {
+        if (u < nmax) {
+            int rk = 0;
+#pragma unroll
+            for (int m = 0; m < 8; ++m) rk += key[m] < key[u] ? 1 : 0;
+            if (nmax > 8) {
+#pragma unroll
+                for (int m = 8; m < 12; ++m) rk += key[m] < key[u] ? 1 : 0;
+            }
+            if (nmax > 12) {
+#pragma unroll
+                for (int m = 12; m < kSortMax; ++m) rk += key[m] < key[u] ? 1 : 0;
+            }
+            const int len = dnr ? cb[u].y >> 16 << 16 : 0;
+            if (u < ns) gs1(row + (rk), (int)((unsigned)e[u] & 0xFF00FFFFu) | len);
+        }
+    }
+    // rows longer than that: the wavefront sorts each in turn
+    unsigned long long big = __ballot(n > kSortMax);
+    while (big) {
+        const int src = __ffsll((long long)big) - 1;
+        big &= big - 1;
+        const int rb_ = r0 + src, xb = rb_ >> 1, nbig = __shfl(n, src, kW);
+        int* const rb = ((rb_ & 1) == 0 ? S.nb_up : S.nb_dn) + (size_t)xb * cap;
+        const int2 cxb = gl2(S.cfp + (xb));
+        int e1 = lane < nbig ? gl1(rb + (lane)) : 0;
+        const int2 ce = gl2(S.cfp + (e1 & 0xFFFF));
+        const unsigned long long kk = lane < nbig ? nbor_key(M, T, cxb, fine_lin(cxb.x, M + 4), ce) : ~0ull;
+        if ((rb_ & 1) != 0) e1 |= (ce.y >> 16) << 16;
+        int rk = 0;
+        for (int m = 0; m < nbig; ++m) rk += readlane_u64(kk, m) < kk ? 1 : 0;
+        wave_sync_mem();  // every lane has read its entry before any is written
+        if (lane < nbig) gs1(rb + (rk), e1);
+        wave_sync_mem();
+    }
+}
+__device__ inline void sort_all_rows(const SysDev& S, const DevTables& T, int wave, int nw) {
+    for (int r0 = wave * kW; r0 < 2 * S.N; r0 += nw * kW) sort_rows(S, T, r0);
     wg_sync(nw);
 }
 
@@ -4076,7 +4078,7 @@ __device__ void wrap_and_lists(const SysDev&, const Lds&, Sc&) {
         rebuild_lists_dense(S, L, c);
     else
         rebuild_lists(S, L, c);
-    sort_rows(S, tabs(), L);
+    sort_all_rows(S, tabs(), wave_id(), L.nw);
 }
 
 // Wrap, lists and full reschedule; all wavefronts of the system take part.
@@ -4836,7 +4838,7 @@ __global__ void k_check(const SysDev* sys, int id, const Rec* alt, unsigned long
     for (int j = i + 1; j < N; ++j) {
         const Rec rj = rec[j];
         const int idj = dyn_ident(rj.dyn);
-        const int code = dyn_code(S.ovr[j], i, static_t(rj.topo, ri.topo));  // ev_code(j, i)
+        const int code = dyn_code(S.ovr[j], i, static_t(T, rj.topo, ri.topo));  // ev_code(j, i)
         if (code == 1 || code >= 15) {
             const double pe = T.ev_param[1][code];
             double sigsq = T.sigma_sq[idi][idj] * (pe * pe);
@@ -5061,7 +5063,7 @@ __global__ void k_predict(const SysDev* sys, int id, int n, const int* pi, const
         return;
     }
     const Rec ri = gld(S.rec + (i)), rj = gld(S.rec + (j));
-    const int code = dyn_code(gld(S.ovr + (j)), i, static_t(rj.topo, ri.topo));
+    const int code = dyn_code(gld(S.ovr + (j)), i, static_t(*S.tab, rj.topo, ri.topo));
     double t = 1000000000.0;
     int ty = 0;
     predict(*S.tab, code, ri, rj, dyn_bptnr(ri.dyn) == j, gld(S.bw + (i)), S.st->tfalse, t, ty);
