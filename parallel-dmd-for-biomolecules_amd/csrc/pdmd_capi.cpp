@@ -645,7 +645,7 @@ int prepared_add(pdmd_ctx* ctx, PreparedSystem* ps, int32_t* sys_id) {
     if (ctx->d_ids.n < 1) HIPCHK(ctx->d_ids.alloc(4096));
     if (ctx->d_inc.n < 1) HIPCHK(ctx->d_inc.alloc(4096));
     HIPCHK(hipMemcpy(ctx->d_ids.p, &id, sizeof(int), hipMemcpyHostToDevice));
-    HIPCHK(engine_setup(ctx->d_sys.p, ctx->d_ids.p, 1, N, engine_maxw(H.cap), ctx->lds_limit, ctx->stream));
+    HIPCHK(engine_setup(ctx->d_sys.p, ctx->d_ids.p, 1, N, ctx->stream));
     HIPCHK(hipStreamSynchronize(ctx->stream));
     SysState chk;
     HIPCHK(hipMemcpy(&chk, H.st.p, sizeof chk, hipMemcpyDeviceToHost));
@@ -773,7 +773,7 @@ int pdmd_rebuild(pdmd_ctx* ctx, int32_t nsys, const int32_t* ids) {
     if (!ctx || nsys <= 0 || !ids) return fail("pdmd_rebuild: bad arguments");
     if (nsys > 4096) return fail("pdmd_rebuild: at most 4096 systems per call");
     std::vector<int> dids(nsys);
-    int max_n = 0, max_cap = 0;
+    int max_n = 0;
     for (int k = 0; k < nsys; ++k) {
         HostSys* H = get_sys(ctx, ids[k]);
         if (!H) return -1;
@@ -781,10 +781,9 @@ int pdmd_rebuild(pdmd_ctx* ctx, int32_t nsys, const int32_t* ids) {
             if (ids[q] == ids[k]) return fail("pdmd_rebuild: duplicate system id");
         dids[k] = ids[k] - 1;
         max_n = std::max(max_n, H->N);
-        max_cap = std::max(max_cap, H->cap);
     }
     HIPCHK(hipMemcpyAsync(ctx->d_ids.p, dids.data(), sizeof(int) * nsys, hipMemcpyHostToDevice, ctx->stream));
-    HIPCHK(engine_rebuild(ctx->d_sys.p, ctx->d_ids.p, nsys, max_n, engine_maxw(max_cap), ctx->lds_limit, ctx->stream));
+    HIPCHK(engine_rebuild(ctx->d_sys.p, ctx->d_ids.p, nsys, max_n, ctx->stream));
     HIPCHK(hipStreamSynchronize(ctx->stream));
     for (int k = 0; k < nsys; ++k) {
         SysState chk;

@@ -3867,6 +3867,66 @@ __device__ void rebuild_lists_dense(const SysDev&, const Lds&, Sc& c) {
     wg_sync(nw);
 }
 
+// events.f:19-103 for bead i at false time 0: its first event before `limit`
+// over its up row and upper shoulder partners
+__device__ inline void bead_event(const SysDev& S, const DevTables& T, int i, double limit, double& ti, int& pi, int& ci,
+                                  int& status) {
+    const int cap = S.cap;
+    const Rec bi = gld(S.rec + (i));
+    const double2 bwi = gld(S.bw + (i));
+    ti = limit;
+    pi = ci = -1;
+    // the next partner's loads are in flight while one is predicted
+    const int n = gl1(S.nup + (i));
+    const int* const row = S.nb_up + (size_t)i * cap;
+    int ent = n > 0 ? gl1(row) : 0, ent1 = n > 1 ? gl1(row + 1) : 0;
+    Rec bm1 = bi;
+    int4 om1 = make_int4(-1, -1, -1, -1);
+    if (n > 0) {
+        bm1 = gld(S.rec + (ent & 0xFFFF));
+        om1 = gld(S.ovr + (ent & 0xFFFF));
+    }
+    for (int k = 0; k < n; ++k) {
+        const Rec bm = bm1;
+        const int4 om = om1;
+        const int m = ent & 0xFFFF, stat = ent >> 24;
+        ent = ent1;
+        if (k + 1 < n) {
+            bm1 = gld(S.rec + (ent & 0xFFFF));
+            om1 = gld(S.ovr + (ent & 0xFFFF));
+        }
+        if (k + 2 < n) ent1 = gl1(row + (k + 2));
+        const int code = dyn_code(om, i, stat);
+        double tij = 1000000000.0;
+        int ty = 0;
+        predict(T, code, bi, bm, dyn_bptnr(bi.dyn) == m, bwi, 0.0, tij, ty);
+        if (ty == -99) status = kErrBadCode;
+        if (tij < ti) {
+            ti = tij;
+            pi = m;
+            ci = ty;
+        }
+        if (tij < 0.0 && fabs(tij) > 1.0e-10) status = kErrNegativeTime;
+    }
+    const int4 e = gld(S.extra + (i));
+    for (int k = 0; k < 3; ++k) {
+        const int m = k == 0 ? e.x : (k == 1 ? e.y : e.z);
+        if (m > i) {
+            const Rec bm = gld(S.rec + (m));
+            const int code = dyn_code(gld(S.ovr + (m)), i, static_t(T, bm.topo, bi.topo));
+            double tij = 1000000000.0;
+            int ty = 0;
+            // events.f:79-83: code 1 -> core, anything else -> shoulder
+            predict(T, code == 1 ? 1 : 40, bi, bm, dyn_bptnr(bi.dyn) == m, bwi, 0.0, tij, ty);
+            if (tij < 0.0 && fabs(tij) > 1.0e-10) status = kErrNegativeTime;
+            if (tij < ti) {
+                pi = m;
+                ci = ty;
+                ti = tij;
+            }
+        }
+    }
+}
 // events.f:11-127 with tfalse = 0: every bead's next event, then the
 // calendar (the pseudo-events' entries from Batch::pseudo); all wavefronts of the system take part (the master scalars'
 // scan position is at bin 1 already)
@@ -3879,63 +3939,12 @@ __device__ void events_all(const SysDev&, const DevTables&, const Lds&, Sc&) {
     Sc& c = *L.msc();
 
     const int tid = (int)threadIdx.x, nthr = kW * L.nw;
-    const int N = S.N, cap = S.cap;
+    const int N = S.N;
     int status = 0;
     for (int i = tid; i < N; i += nthr) {
-        const Rec bi = gld(S.rec + (i));
-        const double2 bwi = gld(S.bw + (i));
-        double ti = c.interval_max + kLt;
-        int pi = -1, ci = -1;
-        // the next partner's loads are in flight while one is predicted
-        const int n = gl1(S.nup + (i));
-        const int* const row = S.nb_up + (size_t)i * cap;
-        int ent = n > 0 ? gl1(row) : 0, ent1 = n > 1 ? gl1(row + 1) : 0;
-        Rec bm1 = bi;
-        int4 om1 = make_int4(-1, -1, -1, -1);
-        if (n > 0) {
-            bm1 = gld(S.rec + (ent & 0xFFFF));
-            om1 = gld(S.ovr + (ent & 0xFFFF));
-        }
-        for (int k = 0; k < n; ++k) {
-            const Rec bm = bm1;
-            const int4 om = om1;
-            const int m = ent & 0xFFFF, stat = ent >> 24;
-            ent = ent1;
-            if (k + 1 < n) {
-                bm1 = gld(S.rec + (ent & 0xFFFF));
-                om1 = gld(S.ovr + (ent & 0xFFFF));
-            }
-            if (k + 2 < n) ent1 = gl1(row + (k + 2));
-            const int code = dyn_code(om, i, stat);
-            double tij = 1000000000.0;
-            int ty = 0;
-            predict(T, code, bi, bm, dyn_bptnr(bi.dyn) == m, bwi, 0.0, tij, ty);
-            if (ty == -99) status = kErrBadCode;
-            if (tij < ti) {
-                ti = tij;
-                pi = m;
-                ci = ty;
-            }
-            if (tij < 0.0 && fabs(tij) > 1.0e-10) status = kErrNegativeTime;
-        }
-        const int4 e = gld(S.extra + (i));
-        for (int k = 0; k < 3; ++k) {
-            const int m = k == 0 ? e.x : (k == 1 ? e.y : e.z);
-            if (m > i) {
-                const Rec bm = gld(S.rec + (m));
-                const int code = dyn_code(gld(S.ovr + (m)), i, static_t(T, bm.topo, bi.topo));
-                double tij = 1000000000.0;
-                int ty = 0;
-                // events.f:79-83: code 1 -> core, anything else -> shoulder
-                predict(T, code == 1 ? 1 : 40, bi, bm, dyn_bptnr(bi.dyn) == m, bwi, 0.0, tij, ty);
-                if (tij < 0.0 && fabs(tij) > 1.0e-10) status = kErrNegativeTime;
-                if (tij < ti) {
-                    pi = m;
-                    ci = ty;
-                    ti = tij;
-                }
-            }
-        }
+        double ti;
+        int pi, ci;
+        bead_event(S, T, i, c.interval_max + kLt, ti, pi, ci, status);
         Leaf lf;
         lf.tim = ti;
         lf.nptnr = pi;
@@ -4092,10 +4101,8 @@ __device__ void rebuild(const SysDev&, const DevTables&, const Lds&, Sc&) {
     PH_END(S, kPhLists, trb);
     events_all(S, T, L, c);
     // the scratch lay over the round's footprint marks too
-    if (L.o_mark >= 0) {
-        const int nm = (int)min((unsigned)S.N, L.mark_mask) + 1;
-        for (int b = (int)threadIdx.x; b < nm; b += kW * L.nw) lds_words(L.o_mark)[b] = 0u;
-    }
+    const int nm = (int)min((unsigned)S.N, L.mark_mask) + 1;
+    for (int b = (int)threadIdx.x; b < nm; b += kW * L.nw) lds_words(L.o_mark)[b] = 0u;
     PH_END(S, kPhEvents, trb);
     PH_COUNT(S, kPhNRebuild);
 }
@@ -4255,23 +4262,19 @@ __device__ Lds make_lds(const SysDev&, int maxw, int lds_bytes, int nw, int wave
     L.o_sc = kMscOff;
     L.o_blk = take((int)sizeof(unsigned) * L.nblk);
     // a footprint mark per bead, or as large a power of two as fits
-    L.o_mark = -1;
     L.mark_mask = ~0u;
-    if (lds_bytes > 0) {
-        const int words = (lds_bytes - p) / (int)sizeof(unsigned);
-        int n = S.N + 1;
-        if (n > words) {
-            n = 1024;
-            while (2 * n <= words) n *= 2;
-            L.mark_mask = (unsigned)n - 1u;
-        }
-        L.o_mark = take((int)sizeof(unsigned) * n);
+    const int words = (lds_bytes - p) / (int)sizeof(unsigned);
+    int nm = S.N + 1;
+    if (nm > words) {
+        nm = 1024;
+        while (2 * nm <= words) nm *= 2;
+        L.mark_mask = (unsigned)nm - 1u;
     }
+    L.o_mark = take((int)sizeof(unsigned) * nm);
     L.o_leaf = p;
     L.leaf_lds = N3 <= (lds_bytes - p) / (int)sizeof(Leaf);
     L.gleaf = S.leaf;
-    // the rebuild kernels' launches (lds_bytes 0) hold every wavefront's scratch
-    const int room = lds_bytes > 0 ? (lds_bytes - kPoolOff) / kScratch : nw;
+    const int room = (lds_bytes - kPoolOff) / kScratch;
     L.nwr = room < nw ? room : nw;
     return L;
 }
@@ -4330,125 +4333,138 @@ __device__ void copy_tables(const DevTables* src, DevTables* dst) {
 // ------------------------------------------------------------------------
 // kernels
 // ------------------------------------------------------------------------
-// Start-up of one system per wavefront: wrap, lists, pseudo-event seeds and
-// events() (main.F90:205-424 after the host-side H-bond restore).
-// One workgroup of up to kSetupWaves wavefronts per system: the list
-// rebuild and events() run on all of them, the rest on the first lane.
-constexpr int kSetupWaves = 4;
-__global__ __launch_bounds__(64 * kSetupWaves) void k_setup(const SysDev* __restrict__ sys, const int* ids, int maxw) {
-    const int nw = (int)(blockDim.x >> 6), wave = wave_id();
-    if (threadIdx.x == 0) *reinterpret_cast<SysDev*>(smem + kSdOff) = sys[ids[blockIdx.x]];
-    __syncthreads();
-    const SysDev& S = sdev();
-    if (lane_id() == 0)
-        *reinterpret_cast<Lds*>(smem + kLdOff + wave * kLdStride) = make_lds(S, maxw, 0, nw, wave);
-    __syncthreads();
-    const Lds& L = ldsv();
-    copy_tables(S.tab, const_cast<DevTables*>(&tabs()));
-    __syncthreads();
-    const DevTables& T = tabs();
-    Sc& c = *L.sc();
-    if (threadIdx.x == 0) load_sc(S.st, c);
-    __syncthreads();
-    const int N = S.N;
+// ---- start-up (main.F90:205-424 after the host-side H-bond restore) and a
+// list update forced at the current time (pdmd_rebuild: the sync
+// pseudo-event's shift of the time origin and its update branch,
+// main.F90:1126-1187, without displacement test, rate adaptation or new sync
+// entry): each step is one launch over the whole GPU, blockIdx.y the system.
+// As a single workgroup per system the steps of 23 424 beads took 8.6 ms on
+// one of 256 compute units, at 512 beads 205 us; the launches cost a few
+// microseconds each, so small systems gain too.
+constexpr int kGridT = 256;
+__device__ inline void report(const SysDev& S, int status) {
+    status = wave_status(status);
+    if (status && lane_id() == 0) atomicCAS(&S.st->status, 0, status);  // the first error stays
+}
+// Beads to the new time origin (forced: advanced by the free flight) and
+// into the box; the pseudo-events' entries seeded, or shifted; empty cells.
+__global__ __launch_bounds__(kGridT) void k_list_beads(const SysDev* __restrict__ sys, const int* ids, int forced) {
+    const SysDev& S = sys[ids[blockIdx.y]];
+    const int gid = (int)(blockIdx.x * kGridT + threadIdx.x), N = S.N;
+    const double tf = forced ? S.st->tfalse : 0.0;
+    if (gid < N) {
+        Rec b = gld(S.rec + (gid));
+        if (forced) {
+            b.x = b.x + b.vx * tf;
+            b.y = b.y + b.vy * tf;
+            b.z = b.z + b.vz * tf;
+        }
+        b.x = b.x - round(b.x);
+        b.y = b.y - round(b.y);
+        b.z = b.z - round(b.z);
+        gst(S.rec + (gid), b);
+        gst(S.old_r + (gid), make_double4(b.x, b.y, b.z, 0.0));
+    } else if (gid < N + 3) {
+        Leaf g;
+        if (forced) {
+            g = gld(S.leaf + (gid));
+            g.tim = g.tim - tf;
+        } else {
+            if (gid == N) {
+                g.tim = 1000000000.0;
+                if (S.canon) {
+                    double tgho = 0.0;
+                    int guard = 0;
+                    unsigned long long rc = S.st->rng_ctr[0];
+                    do {
+                        tgho = rng_u01(S.seed, 0, rc++);
+                    } while ((tgho < 1.e-18 || tgho == 1.0) && ++guard < 1000);
+                    S.st->rng_ctr[0] = rc;
+                    g.tim = -1.0 * dlog(tgho) * S.avegtime * .0000001;
+                }
+            } else
+                g.tim = gid == N + 1 ? S.st->interval : 3.3 / (sqrt(S.setemp)) + 5;
+            g.nptnr = -2;
+            g.meta = make_meta(-1, -2);
+        }
+        gst(S.leaf + (gid), g);
+    }
+    const int Mq = S.M / S.cq, NC = Mq * Mq * Mq;
+    for (int q = gid; q < NC; q += (int)(gridDim.x * kGridT)) gs1(S.cstart + (q), 0);
+}
+__global__ __launch_bounds__(kGridT) void k_list_cells(const SysDev* __restrict__ sys, const int* ids) {
+    list_cells(sys[ids[blockIdx.y]], (int)(blockIdx.x * kGridT + threadIdx.x), (int)(gridDim.x * kGridT));
+}
+// the cells' starts (one workgroup per system); the scalars of a forced update
+constexpr int kScanT = 1024;
+__global__ __launch_bounds__(kScanT) void k_list_scan(const SysDev* __restrict__ sys, const int* ids, int forced) {
+    __shared__ int part[kScanT / kW];
+    const SysDev& S = sys[ids[blockIdx.y]];
     if (threadIdx.x == 0) {
-        Leaf g, s2, s3;
-        if (S.canon) {
-            double tgho = 0.0;
-            int guard = 0;
-            do {
-                tgho = rng_u01(S.seed, 0, c.rc0++);
-            } while ((tgho < 1.e-18 || tgho == 1.0) && ++guard < 1000);
-            g.tim = -1.0 * dlog(tgho) * S.avegtime * .0000001;
-        } else
-            g.tim = 1000000000.0;
-        s2.tim = c.interval;
-        s3.tim = 3.3 / (sqrt(S.setemp)) + 5;
-        g.nptnr = s2.nptnr = s3.nptnr = -2;
-        g.meta = s2.meta = s3.meta = make_meta(-1, -2);
-        gst(S.leaf + (N), g);
-        gst(S.leaf + (N + 1), s2);
-        gst(S.leaf + (N + 2), s3);
+        SysState& st = *S.st;
+        st.nbin = 1;
+        if (forced) {
+            st.t = st.t + st.tfalse;
+            st.tfalse = 0.0;
+            st.interval_max = st.interval * st.n_forced;
+            st.sortsize = st.interval_max / (double)kNumbin;
+            st.tbin_off = 0.0;
+            st.nupdates++;
+        }
     }
-    __threadfence_block();
-    __syncthreads();
-    rebuild(S, T, L, c);
-    __syncthreads();
-    if (threadIdx.x == 0) store_sc(S.st, c);
+    const int Mq = S.M / S.cq;
+    list_scan(S.cstart, Mq * Mq * Mq, part, wave_id(), kScanT / kW);
 }
-
-// Workgroup entry of the rebuild kernels: the system's descriptor, the work
-// areas and the tables into LDS; the first lane loads the master scalars
-// (each wavefront's own copy is not loaded here).
-__device__ void enter_system(const SysDev* __restrict__ sys, const int* ids, int maxw) {
-    const int nw = (int)(blockDim.x >> 6), wave = wave_id();
-    if (threadIdx.x == 0) *reinterpret_cast<SysDev*>(smem + kSdOff) = sys[ids[blockIdx.x]];
-    __syncthreads();
-    const SysDev& S = sdev();
-    if (lane_id() == 0)
-        *reinterpret_cast<Lds*>(smem + kLdOff + wave * kLdStride) = make_lds(S, maxw, 0, nw, wave);
-    __syncthreads();
-    copy_tables(S.tab, const_cast<DevTables*>(&tabs()));
-    if (threadIdx.x == 0) load_sc(S.st, *ldsv().msc());
-    __syncthreads();
+__global__ __launch_bounds__(kGridT) void k_list_copy(const SysDev* __restrict__ sys, const int* ids) {
+    list_copy(sys[ids[blockIdx.y]], (int)(blockIdx.x * kGridT + threadIdx.x), (int)(gridDim.x * kGridT));
 }
-
-// A list update forced at the current time (pdmd_rebuild), in two
-// dispatches so that the list build and the full reschedule are timed and
-// counted apart.  This first one runs the sync pseudo-event's shift of the
-// time origin and its update branch (main.F90:1126-1187) up to the new
-// lists, on every wavefront of the system's workgroup.  No displacement
-// test, no rate adaptation and no new sync entry: the pending one keeps its
-// shifted time.
-__global__ __launch_bounds__(64 * kSetupWaves) void k_rebuild_lists(const SysDev* __restrict__ sys, const int* ids,
-                                                                    int maxw) {
-    enter_system(sys, ids, maxw);
-    const SysDev& S = sdev();
-    const Lds& L = ldsv();
-    Sc& c = *L.msc();
-    const int N = S.N;
-    const double tf = c.tfalse;
-    __syncthreads();  // every wavefront holds tf before the first lane moves the origin
-    for (int e = (int)threadIdx.x; e < N + 3; e += (int)blockDim.x) {
-        Leaf lf = gld(S.leaf + (e));
-        lf.tim = lf.tim - tf;
-        gst(S.leaf + (e), lf);
-    }
-    for (int k = (int)threadIdx.x; k < N; k += (int)blockDim.x) {
-        Rec b = gld(S.rec + (k));
-        b.x = b.x + b.vx * tf;
-        b.y = b.y + b.vy * tf;
-        b.z = b.z + b.vz * tf;
-        gst(S.rec + (k), b);
-    }
-    if (threadIdx.x == 0) {
-        c.t = c.t + tf;
-        c.tfalse = 0.0;
-        c.interval_max = c.interval * c.n_forced;
-        c.sortsize = c.interval_max / (double)kNumbin;
-        c.tbin_off = 0.0;
-        c.nupdates++;
-    }
-    __threadfence_block();
+// the tables in LDS
+__device__ inline const DevTables& block_tables(const SysDev& S) {
+    __shared__ __attribute__((aligned(16))) unsigned char mem[sizeof(DevTables)];
+    DevTables& T = *reinterpret_cast<DevTables*>(mem);
+    copy_tables(S.tab, &T);
     __syncthreads();
-    wrap_and_lists(S, L, c);
-    __syncthreads();
-    if (threadIdx.x == 0) store_sc(S.st, c);
+    return T;
 }
-
-// The second dispatch of a forced list update: events() over the new lists
-// (events.f), every bead's next event and the pseudo-events' bins.
-__global__ __launch_bounds__(64 * kSetupWaves) void k_rebuild_events(const SysDev* __restrict__ sys, const int* ids,
-                                                                     int maxw) {
-    enter_system(sys, ids, maxw);
-    const SysDev& S = sdev();
-    const Lds& L = ldsv();
-    Sc& c = *L.msc();
-    if (threadIdx.x < 3) L.batch()->pseudo[threadIdx.x] = gld(S.leaf + (S.N + (int)threadIdx.x));
-    __syncthreads();
-    events_all(S, tabs(), L, c);
-    __syncthreads();
-    if (threadIdx.x == 0) store_sc(S.st, c);
+__global__ __launch_bounds__(kGridT) void k_list_search(const SysDev* __restrict__ sys, const int* ids) {
+    const SysDev& S = sys[ids[blockIdx.y]];
+    if ((int)(blockIdx.x * kGridT) >= S.N) return;
+    const DevTables& T = block_tables(S);
+    const int i0 = (int)(blockIdx.x * kGridT) + wave_id() * kW;
+    int mx = 0, status = 0;
+    if (i0 < S.N) list_search(S, T, i0, mx, status);
+    report(S, status);
+    mx = wave_imax(mx);
+    if (lane_id() == 0) atomicMax(&S.st->max_nb_seen, (long long)mx);
+}
+__global__ __launch_bounds__(kGridT) void k_list_sort(const SysDev* __restrict__ sys, const int* ids) {
+    const SysDev& S = sys[ids[blockIdx.y]];
+    if ((int)(blockIdx.x * kGridT) >= 2 * S.N) return;
+    const DevTables& T = block_tables(S);
+    const int r0 = (int)(blockIdx.x * kGridT) + wave_id() * kW;
+    if (r0 < 2 * S.N) sort_rows(S, T, r0);
+}
+// events() over the new lists (events.f), and the pseudo-events' bins
+__global__ __launch_bounds__(kGridT) void k_list_events(const SysDev* __restrict__ sys, const int* ids) {
+    const SysDev& S = sys[ids[blockIdx.y]];
+    if ((int)(blockIdx.x * kGridT) >= S.N + 3) return;
+    const DevTables& T = block_tables(S);
+    const int i = (int)(blockIdx.x * kGridT + threadIdx.x), N = S.N;
+    const SysState& st = *S.st;
+    const double imax = st.interval_max;
+    int status = 0;
+    if (i < N + 3) {
+        Leaf lf;
+        int ci = -2;
+        if (i < N)
+            bead_event(S, T, i, imax + kLt, lf.tim, lf.nptnr, ci, status);
+        else
+            lf = gld(S.leaf + (i));
+        lf.meta = make_meta(bin_of(imax, st.tbin_off, st.sortsize, 1, lf.tim, status), ci);
+        gst(S.leaf + (i), lf);
+        gs1(S.stamp + (i), mk_stamp(st.coll, i + 1));  // events.f:111-122 adds in index order
+    }
+    report(S, status);
 }
 
 // Takes up to kmax entries from the pool in key order (wavefront 0): the
@@ -5086,30 +5102,25 @@ static size_t lds_fixed(int nblk_max, int maxw, int nw) {
 size_t engine_lds_bytes(int nblk_max, int maxw, int leaf_cap, int nw) {
     return lds_fixed(nblk_max, maxw, nw) + sizeof(Leaf) * (size_t)leaf_cap;
 }
-// the rebuild kernels: scratch for every wavefront, no leaves
-static size_t lds_rebuild(int nblk_max, int maxw, int nw) {
-    return std::max(lds_fixed(nblk_max, maxw, nw), (size_t)kPoolOff + (size_t)nw * kScratch);
-}
 static int nblk_for(int n) { return (n + 3 + kBlk - 1) / kBlk; }
 
-hipError_t engine_setup(const SysDev* d_sys, const int* d_ids, int n, int max_n, int maxw, size_t lds_limit,
-                        hipStream_t s) {
-    int nw = kSetupWaves;
-    while (nw > 1 && lds_rebuild(nblk_for(max_n), maxw, nw) > lds_limit) --nw;
-    const size_t lds = lds_rebuild(nblk_for(max_n), maxw, nw);
-    hipLaunchKernelGGL(k_setup, dim3(n), dim3(kW * nw), lds, s, d_sys, d_ids, maxw);
+static hipError_t list_launches(const SysDev* d_sys, const int* d_ids, int n, int max_n, int forced, hipStream_t s) {
+    const unsigned beads = (unsigned)(max_n + 3 + kGridT - 1) / kGridT, rows = (unsigned)(2 * max_n + kGridT - 1) / kGridT;
+    const dim3 t(kGridT), g(beads, (unsigned)n);
+    hipLaunchKernelGGL(k_list_beads, g, t, 0, s, d_sys, d_ids, forced);
+    hipLaunchKernelGGL(k_list_cells, g, t, 0, s, d_sys, d_ids);
+    hipLaunchKernelGGL(k_list_scan, dim3(1, (unsigned)n), dim3(kScanT), 0, s, d_sys, d_ids, forced);
+    hipLaunchKernelGGL(k_list_copy, g, t, 0, s, d_sys, d_ids);
+    hipLaunchKernelGGL(k_list_search, g, t, 0, s, d_sys, d_ids);
+    hipLaunchKernelGGL(k_list_sort, dim3(rows, (unsigned)n), t, 0, s, d_sys, d_ids);
+    hipLaunchKernelGGL(k_list_events, g, t, 0, s, d_sys, d_ids);
     return hipGetLastError();
 }
-hipError_t engine_rebuild(const SysDev* d_sys, const int* d_ids, int n, int max_n, int maxw, size_t lds_limit,
-                          hipStream_t s) {
-    int nw = kSetupWaves;
-    while (nw > 1 && lds_rebuild(nblk_for(max_n), maxw, nw) > lds_limit) --nw;
-    const size_t lds = lds_rebuild(nblk_for(max_n), maxw, nw);
-    hipLaunchKernelGGL(k_rebuild_lists, dim3(n), dim3(kW * nw), lds, s, d_sys, d_ids, maxw);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_rebuild_events, dim3(n), dim3(kW * nw), lds, s, d_sys, d_ids, maxw);
-    return hipGetLastError();
+hipError_t engine_setup(const SysDev* d_sys, const int* d_ids, int n, int max_n, hipStream_t s) {
+    return list_launches(d_sys, d_ids, n, max_n, 0, s);
+}
+hipError_t engine_rebuild(const SysDev* d_sys, const int* d_ids, int n, int max_n, hipStream_t s) {
+    return list_launches(d_sys, d_ids, n, max_n, 1, s);
 }
 // clears the start word of a budgeted launch (a kernel rather than a memset,
 // so that a captured graph replays it faithfully)
@@ -5230,14 +5241,7 @@ hipError_t engine_observables_noalloc(const SysDev* d_sys, int id, int device, c
 }
 
 hipError_t engine_prepare(size_t lds_limit) {
-    hipError_t e = hipFuncSetAttribute((const void*)k_run, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_limit);
-    if (e != hipSuccess) return e;
-    e = hipFuncSetAttribute((const void*)k_setup, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_limit);
-    if (e != hipSuccess) return e;
-    e = hipFuncSetAttribute((const void*)k_rebuild_lists, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_limit);
-    if (e != hipSuccess) return e;
-    return hipFuncSetAttribute((const void*)k_rebuild_events, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              (int)lds_limit);
+    return hipFuncSetAttribute((const void*)k_run, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_limit);
 }
 
 }  // namespace pdmd
