@@ -65,7 +65,7 @@ struct HostSys {
     DevBuf<DevTables> tab;
     DevBuf<Rec> rec;
     DevBuf<double2> bw;
-    DevBuf<int> nb_up, nup, nb_dn, ndn, ckey, cstart, crank;
+    DevBuf<int> nb_up, nup, nb_dn, ndn, ckey, cstart, ccnt, crank;
     DevBuf<int4> extra, ovr;
     DevBuf<int2> cfp;
     DevBuf<Leaf> leaf;
@@ -408,7 +408,7 @@ int64_t device_bytes(const Prep& pp) {
                              N * 16 /*ovr*/, N * 32 /*old_r*/, N * cap * 4 /*nb_up*/, N * cap * 4 /*nb_dn*/,
                              (N + 1) * 4 /*nup*/, (N + 1) * 4 /*ndn*/, (N + 3) * (int64_t)sizeof(Leaf),
                              N * 4 /*ckey*/, N * 8 /*cfp*/, N * 4 /*crank*/, N * 32 /*spos*/, N * 16 /*sinfo*/,
-                             (nc + 1) * 4 /*cstart*/, (N + 3) * 8 /*stamp*/,
+                             (nc + 1) * 4 /*cstart*/, nc * 4 /*ccnt*/, (N + 3) * 8 /*stamp*/,
                              (int64_t)sizeof(SysState)};
     int64_t b = 0;
     for (int64_t x : sizes) b += (x + 4095) / 4096 * 4096;
@@ -579,6 +579,8 @@ int prepared_add(pdmd_ctx* ctx, PreparedSystem* ps, int32_t* sys_id) {
     HIPCHK(H.stamp.alloc(N + 3));
     HIPCHK(hipMemsetAsync(H.stamp.p, 0, sizeof(unsigned long long) * (size_t)(N + 3), ctx->stream));
     HIPCHK(H.cstart.alloc((size_t)Mq * Mq * Mq + 1));
+    HIPCHK(H.ccnt.alloc((size_t)Mq * Mq * Mq));
+    HIPCHK(hipMemsetAsync(H.ccnt.p, 0, sizeof(int) * (size_t)Mq * Mq * Mq, ctx->stream));
     {
         std::vector<SysState> sv(1, st);
         HIPCHK(upload(H.st, sv));
@@ -615,6 +617,7 @@ int prepared_add(pdmd_ctx* ctx, PreparedSystem* ps, int32_t* sys_id) {
     D.ckey = H.ckey.p;
     D.cfp = H.cfp.p;
     D.cstart = H.cstart.p;
+    D.ccnt = H.ccnt.p;
     D.crank = H.crank.p;
     D.spos = H.spos.p;
     D.sinfo = H.sinfo.p;

@@ -151,6 +151,7 @@ struct SysDev {
     int* ckey;     // coarse cell per bead
     int2* cfp;     // [N] fine cell; the place in its list as cell_add.f builds it (1 = highest index) | up-row length << 16
     int* cstart;   // [ncoarse+1]
+    int* ccnt;     // [ncoarse] beads per cell while they are counted, zero between list rebuilds
     int* crank;    // [N] the bead's place among its coarse cell's beads
     double4* spos; // [N] positions in coarse-cell order (list rebuild)
     int4* sinfo;   // [N] bead, topo word, fine cell, 0 in coarse-cell order

@@ -3500,7 +3500,7 @@ __device__ inline void list_cells(const SysDev& S, int tid, int nthr) {
         const int key = qx + Mq * (qy + Mq * qz);
         gs1(&S.cfp[k].x, f);
         gs1(S.ckey + (k), key);
-        gs1(S.crank + (k), atomicAdd(&S.cstart[key], 1));
+        gs1(S.crank + (k), atomicAdd(&S.ccnt[key], 1));
     }
 }
 // wave-inclusive sum
@@ -3513,10 +3513,11 @@ __device__ inline int wave_scan(int v) {
     v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
     return v;
 }
-// Exclusive scan of the NC cell counts on the workgroup's nw wavefronts, a
-// contiguous part each: its sum, then (after the others' sums) its starts.
-// part: nw words of LDS.  The counts were made by atomics: read at the L2.
-__device__ inline void list_scan(int* cnt, int NC, int* part, int wave, int nw) {
+// Exclusive scan of the NC cell counts into the cells' starts on the
+// workgroup's nw wavefronts, a contiguous part each: its sum, then (after the
+// others' sums) its starts.  The counts, made by atomics and read at the L2,
+// are zero again afterwards.  part: nw words of LDS.
+__device__ inline void list_scan(int* cnt, int* start, int NC, int* part, int wave, int nw) {
     const int lane = lane_id();
     const int seg = ((NC + nw - 1) / nw + 255) / 256 * 256, lo = min(wave * seg, NC), hi = min(lo + seg, NC);
     auto at = [&](int q) { return q < hi ? __hip_atomic_load((GLB int*)cnt + q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0; };
@@ -3538,11 +3539,14 @@ __device__ inline void list_scan(int* cnt, int NC, int* part, int wave, int nw) 
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             const int q = base + u * kW + lane, incl = wave_scan(v[u]);
-            if (q < hi) gs1(cnt + q, carry + incl - v[u]);
+            if (q < hi) {
+                gs1(start + q, carry + incl - v[u]);
+                gs1(cnt + q, 0);
+            }
             carry += __builtin_amdgcn_readlane(incl, kW - 1);
         }
     }
-    if (wave == 0 && lane == 0) gs1(cnt + NC, all);
+    if (wave == 0 && lane == 0) gs1(start + NC, all);
 }
 // beads [tid, N) by nthr to their sorted places
 __device__ inline void list_copy(const SysDev& S, int tid, int nthr) {
@@ -3679,12 +3683,10 @@ __device__ void rebuild_lists(const SysDev&, const Lds&, Sc& c) {
     const int tid = (int)threadIdx.x, nthr = kW * nw;
     const int Mq = S.M / S.cq, NC = Mq * Mq * Mq;
     PH_BEGIN(trl);
-    for (int q = tid; q < NC; q += nthr) gs1(S.cstart + (q), 0);
-    wg_sync(nw);
     list_cells(S, tid, nthr);
     wg_sync(nw);
     PH_END(S, kPhLCells, trl);
-    list_scan(S.cstart, NC, reinterpret_cast<int*>(smem + L.o_pool), wave, nw);
+    list_scan(S.ccnt, S.cstart, NC, reinterpret_cast<int*>(smem + L.o_pool), wave, nw);
     wg_sync(nw);
     PH_END(S, kPhLScan, trl);
     list_copy(S, tid, nthr);
@@ -4347,7 +4349,7 @@ __device__ inline void report(const SysDev& S, int status) {
     if (status && lane_id() == 0) atomicCAS(&S.st->status, 0, status);  // the first error stays
 }
 // Beads to the new time origin (forced: advanced by the free flight) and
-// into the box; the pseudo-events' entries seeded, or shifted; empty cells.
+// into the box; the pseudo-events' entries seeded, or shifted.
 __global__ __launch_bounds__(kGridT) void k_list_beads(const SysDev* __restrict__ sys, const int* ids, int forced) {
     const SysDev& S = sys[ids[blockIdx.y]];
     const int gid = (int)(blockIdx.x * kGridT + threadIdx.x), N = S.N;
@@ -4389,8 +4391,6 @@ __global__ __launch_bounds__(kGridT) void k_list_beads(const SysDev* __restrict_
         }
         gst(S.leaf + (gid), g);
     }
-    const int Mq = S.M / S.cq, NC = Mq * Mq * Mq;
-    for (int q = gid; q < NC; q += (int)(gridDim.x * kGridT)) gs1(S.cstart + (q), 0);
 }
 __global__ __launch_bounds__(kGridT) void k_list_cells(const SysDev* __restrict__ sys, const int* ids) {
     list_cells(sys[ids[blockIdx.y]], (int)(blockIdx.x * kGridT + threadIdx.x), (int)(gridDim.x * kGridT));
@@ -4413,7 +4413,7 @@ __global__ __launch_bounds__(kScanT) void k_list_scan(const SysDev* __restrict__
         }
     }
     const int Mq = S.M / S.cq;
-    list_scan(S.cstart, Mq * Mq * Mq, part, wave_id(), kScanT / kW);
+    list_scan(S.ccnt, S.cstart, Mq * Mq * Mq, part, wave_id(), kScanT / kW);
 }
 __global__ __launch_bounds__(kGridT) void k_list_copy(const SysDev* __restrict__ sys, const int* ids) {
     list_copy(sys[ids[blockIdx.y]], (int)(blockIdx.x * kGridT + threadIdx.x), (int)(gridDim.x * kGridT));
