@@ -60,30 +60,6 @@ __host__ __device__ inline int leaf_bin(int meta) { return (meta & 0xFFFF) - 1; 
 __host__ __device__ inline int leaf_ct(int meta) { return meta >> 16; }
 __host__ __device__ inline int make_meta(int bin, int ct) { return ((bin + 1) & 0xFFFF) | (ct << 16); }
 
-// Pair code of two beads of one chain (make_code.f), kinds ka <= kb (0
-// Calpha, 1 N, 2 C, 3 R) and residue distance d = rb - ra (d >= 0 for equal
-// kinds); 16 holds for two hydrophobic side chains only.  Constant beyond
-// |d| = 4.
-inline int chain_code(int ka, int kb, int d) {
-    switch (ka * 4 + kb) {
-        case 0: return d == 1 ? 9 : 1;
-        case 1: return d == 0 ? 4 : (d == 1 ? 7 : (d == -1 ? 18 : 1));
-        case 2: return d == 0 ? 5 : (d == -1 ? 8 : (d == 1 ? 17 : 1));
-        case 3: return d == 0 ? 10 : (d == 1 ? 24 : (d == -1 ? 25 : 1));
-        case 5: return d == 1 ? 20 : 1;
-        case 6:
-            if (d == -1) return 6;
-            if (d == 0) return 8;
-            if (d == -2) return 19;
-            return (d >= -3 && d <= 3) ? 1 : 15;
-        case 7: return d == 0 ? 11 : (d == -1 ? 23 : 1);
-        case 10: return d == 1 ? 21 : 1;
-        case 11: return d == 0 ? 12 : (d == 1 ? 22 : (d == 2 ? 26 : 1));
-        case 15: return d >= 4 ? 16 : 1;
-        default: return 1;
-    }
-}
-
 // Scaled parameter tables of one system (box units), from
 // scale_down.f / make_code.f / nbor_setup.f.
 struct DevTables {

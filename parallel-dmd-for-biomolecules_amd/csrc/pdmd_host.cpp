@@ -246,24 +246,10 @@ int static_code(const Topology& t, int a, int b) {
             std::swap(ra, rb);
         }
         const int d = rb - ra;  // residue offset of the second kind relative to the first
-        switch (ka * 4 + kb) {
-            case 0 * 4 + 0: return (d == 1) ? 9 : 1;                                     // Ca-Ca
-            case 0 * 4 + 1: return d == 0 ? 4 : (d == 1 ? 7 : (d == -1 ? 18 : 1));       // Ca-N
-            case 0 * 4 + 2: return d == 0 ? 5 : (d == -1 ? 8 : (d == 1 ? 17 : 1));       // Ca-C
-            case 0 * 4 + 3: return d == 0 ? 10 : (d == 1 ? 24 : (d == -1 ? 25 : 1));     // Ca-R
-            case 1 * 4 + 1: return (d == 1) ? 20 : 1;                                    // N-N
-            case 1 * 4 + 2:                                                              // N-C
-                if (d == -1) return 6;
-                if (d == 0) return 8;
-                if (d == -2) return 19;
-                return (d >= -3 && d <= 3) || t.no_hbs ? 1 : 15;
-            case 1 * 4 + 3: return d == 0 ? 11 : (d == -1 ? 23 : 1);                    // N-R
-            case 2 * 4 + 2: return (d == 1) ? 21 : 1;                                    // C-C
-            case 2 * 4 + 3: return d == 0 ? 12 : (d == 1 ? 22 : (d == 2 ? 26 : 1));     // C-R
-            case 3 * 4 + 3:                                                              // R-R
-                return (d >= 4 && t.hp[t.res[a]] == 1 && t.hp[t.res[b]] == 1) ? 16 : 1;
-            default: return 1;
-        }
+        const int code = chain_code(ka, kb, d);
+        if (code == 15 && t.no_hbs) return 1;
+        if (code == 16 && !(t.hp[t.res[a]] == 1 && t.hp[t.res[b]] == 1)) return 1;
+        return code;
     }
     // different chains
     // -Dno_h zeroes hp for make_code.f:80-104 only (inputinfo.f:270-280);
@@ -329,50 +315,93 @@ void nbor_setup(const Params& p, const Topology& t, const std::vector<int>& iden
         for (int ch = 0; ch < (int)t.chain_len.size(); ++ch)
             if (seen.emplace(t.species[ch], ch).second) firsts.push_back(ch);
     }
+    // Pairs of one chain.  Beyond a residue distance of 4 the code depends on
+    // the kinds and hp flags only, so those pairs are taken once per pair of
+    // distinct (identity, kind, hp) combinations that lie that far apart
+    // somewhere in the chain; nearer ones pair by pair.
+    auto code_of = [&](int ka, int hpa, int kb, int hpb, int d) {  // static_code of two beads of a chain
+        const int code = chain_code(ka, kb, d);
+        return (code == 16 && !(hpa == 1 && hpb == 1)) || (code == 15 && t.no_hbs) ? 1 : code;
+    };
     for (int ch : firsts) {
-        const int s = t.chain_start[ch], n = 4 * t.chain_len[ch];
-        for (int i = s; i < s + n - 1; ++i)
-            for (int j = i + 1; j < s + n; ++j) consider(i, j, static_code(t, j, i));
+        const int s = t.chain_start[ch], L = t.chain_len[ch], n = 4 * L;
+        if (t.free_bead(s)) {
+            for (int i = s; i < s + n - 1; ++i)
+                for (int j = i + 1; j < s + n; ++j) consider(i, j, static_code(t, j, i));
+            continue;
+        }
+        struct Far { int ident, kind, hp, lo, hi, bead; };
+        std::vector<Far> far;
+        for (int i = s; i < s + n; ++i) {
+            const int kind = (i - s) / L, r = (i - s) % L, hp = kind == 3 ? t.hp[t.res[i]] : 0;
+            bool known = false;
+            for (Far& y : far)
+                if (y.ident == ident[i] && y.kind == kind && y.hp == hp) {
+                    y.hi = r;
+                    known = true;
+                    break;
+                }
+            if (!known) far.push_back({ident[i], kind, hp, r, r, i});
+            // the later beads (in index order) within 4 residues
+            for (int k2 = kind; k2 < 4; ++k2)
+                for (int r2 = k2 == kind ? r + 1 : std::max(0, r - 4); r2 <= std::min(L - 1, r + 4); ++r2) {
+                    const int j = s + k2 * L + r2;
+                    consider(i, j, code_of(kind, hp, k2, k2 == 3 ? t.hp[t.res[j]] : 0, r2 - r));
+                }
+        }
+        for (const Far& x : far)
+            for (const Far& y : far) {
+                // x before y in index order: a lower kind, or the same kind and a lower residue
+                if (x.kind > y.kind) continue;
+                const bool apart = y.hi - x.lo >= 4 || (x.kind < y.kind && x.hi - y.lo >= 4);
+                if (!apart) continue;
+                consider(x.bead, y.bead, code_of(x.kind, x.hp, y.kind, y.hp, 4));
+            }
     }
     // Cross pairs between species: the code of an inter-chain pair depends
     // on the two bead kinds, side-chain hp flags and the proline rule only,
     // so the max over all pairs equals the max over the distinct
-    // (identity, hp/proline class) combinations present in each first chain.
-    struct Cls { int ident, kind, hp, pro; };
-    std::vector<std::vector<Cls>> cls(firsts.size());
+    // (identity, hp/proline class) combinations of a first chain and a later
+    // one.  A combination occurs if the first class's first chain lies before
+    // the second one's last: one pass over the distinct classes of all first
+    // chains (some forty) instead of one per pair of chains (10 ms at 183
+    // chains of their own species).
+    struct Cls { int ident, kind, hp, pro, first, last; };
+    std::vector<Cls> cls;
     for (size_t q = 0; q < firsts.size(); ++q) {
         const int ch = firsts[q], s = t.chain_start[ch], n = 4 * t.chain_len[ch];
-        std::vector<Cls>& v = cls[q];
         for (int i = s; i < s + n; ++i) {
             int kind, r;
             kind_of(t, i, kind, r);
-            Cls x{ident[i], kind, kind == 3 ? t.hp[t.res[i]] : 0,
-                  kind == 1 ? (t.restype[t.res[i]] == 17 ? 1 : 0) : 0};
-            bool dup = false;
-            for (const Cls& y : v)
-                if (y.ident == x.ident && y.kind == x.kind && y.hp == x.hp && y.pro == x.pro) dup = true;
-            if (!dup) v.push_back(x);
+            const Cls x{ident[i], kind, kind == 3 ? t.hp[t.res[i]] : 0, kind == 1 ? (t.restype[t.res[i]] == 17 ? 1 : 0) : 0,
+                        (int)q, (int)q};
+            bool known = false;
+            for (Cls& y : cls)
+                if (y.ident == x.ident && y.kind == x.kind && y.hp == x.hp && y.pro == x.pro) {
+                    y.last = (int)q;
+                    known = true;
+                    break;
+                }
+            if (!known) cls.push_back(x);
         }
     }
-    for (size_t qa = 0; qa < firsts.size(); ++qa)
-        for (size_t qb = qa + 1; qb < firsts.size(); ++qb)
-            for (const Cls& x : cls[qa])
-                for (const Cls& y : cls[qb]) {
-                    int code = 1;
-                    if (x.kind == 3 && y.kind == 3) code = (!t.no_h && x.hp == 1 && y.hp == 1) ? 16 : 1;
-                    else if (x.kind == 1 && y.kind == 2) code = x.pro || t.no_hbs ? 1 : 15;  // N in the earlier chain
-                    else if (x.kind == 2 && y.kind == 1) code = t.no_hbs ? 1 : 15;
-                    const int a = x.ident, b = y.ident;
-                    if (code > 26) continue;
-                    double s;
-                    if (code <= 3) s = p.sigma_2b[b][a];
-                    else if (code == 15) s = 0.5 * (p.welldia[a] + p.welldia[b]);
-                    else s = p.wel[a][b] / p.boxl_orig;
-                    if (s > sig_max[code]) {
-                        sig_max[code] = s;
-                        if (sig_max[code] > c.sig_max_all) c.sig_max_all = sig_max[code];
-                    }
-                }
+    for (const Cls& x : cls)
+        for (const Cls& y : cls) {
+            if (x.first >= y.last) continue;
+            int code = 1;
+            if (x.kind == 3 && y.kind == 3) code = (!t.no_h && x.hp == 1 && y.hp == 1) ? 16 : 1;
+            else if (x.kind == 1 && y.kind == 2) code = x.pro || t.no_hbs ? 1 : 15;  // N in the earlier chain
+            else if (x.kind == 2 && y.kind == 1) code = t.no_hbs ? 1 : 15;
+            const int a = x.ident, b = y.ident;
+            double s;
+            if (code <= 3) s = p.sigma_2b[b][a];
+            else if (code == 15) s = 0.5 * (p.welldia[a] + p.welldia[b]);
+            else s = p.wel[a][b] / p.boxl_orig;
+            if (s > sig_max[code]) {
+                sig_max[code] = s;
+                if (sig_max[code] > c.sig_max_all) c.sig_max_all = sig_max[code];
+            }
+        }
     double sigij = 0.0, sig = 0.0;
     for (int i = 1; i <= 4; ++i)
         for (int j = 1; j <= 4; ++j) {

@@ -52,6 +52,30 @@ struct Topology {
                const std::vector<int>& restype, const std::vector<int>& hp);
 };
 
+// Pair code of two beads of one chain (make_code.f), kinds ka <= kb (0
+// Calpha, 1 N, 2 C, 3 R) and residue distance d = rb - ra (d >= 0 for equal
+// kinds); 16 holds for two hydrophobic side chains only.  Constant beyond
+// |d| = 4.
+inline int chain_code(int ka, int kb, int d) {
+    switch (ka * 4 + kb) {
+        case 0: return d == 1 ? 9 : 1;
+        case 1: return d == 0 ? 4 : (d == 1 ? 7 : (d == -1 ? 18 : 1));
+        case 2: return d == 0 ? 5 : (d == -1 ? 8 : (d == 1 ? 17 : 1));
+        case 3: return d == 0 ? 10 : (d == 1 ? 24 : (d == -1 ? 25 : 1));
+        case 5: return d == 1 ? 20 : 1;
+        case 6:
+            if (d == -1) return 6;
+            if (d == 0) return 8;
+            if (d == -2) return 19;
+            return (d >= -3 && d <= 3) ? 1 : 15;
+        case 7: return d == 0 ? 11 : (d == -1 ? 23 : 1);
+        case 10: return d == 1 ? 21 : 1;
+        case 11: return d == 0 ? 12 : (d == 1 ? 22 : (d == 2 ? 26 : 1));
+        case 15: return d >= 4 ? 16 : 1;
+        default: return 1;
+    }
+}
+
 // Static pair code ev_code(a,b) as left by make_code.f (symmetric, a != b,
 // 0-based bead indices).  Closed form of make_code.f:72-563.
 int static_code(const Topology& t, int a, int b);
