@@ -54,6 +54,33 @@ struct DevBuf {
     }
 };
 
+// Page-locked host memory that kernels of one context write for the host to
+// read after the stream's next synchronisation (a context has one host
+// thread).  It grows to the largest request: a state of 65 533 beads, the
+// most a system may have, takes 6 MB, 4096 systems' counters 7 MB.
+struct HostStage {
+    void* p = nullptr;
+    size_t n = 0;
+    ~HostStage() {
+        if (p) (void)hipHostFree(p);
+    }
+    hipError_t reserve(size_t bytes) {
+        if (bytes <= n) return hipSuccess;
+        size_t want = n ? n : (size_t)1 << 20;
+        while (want < bytes) want *= 2;
+        if (p) (void)hipHostFree(p);
+        p = nullptr;
+        n = 0;
+        const hipError_t e = hipHostMalloc(&p, want, hipHostMallocDefault);
+        if (e == hipSuccess) n = want;
+        return e;
+    }
+    template <class T>
+    T* at(size_t byte) const {
+        return reinterpret_cast<T*>(static_cast<char*>(p) + byte);
+    }
+};
+
 struct HostSys {
     Topology topo;
     Params p;  // scaled to this box
@@ -89,6 +116,7 @@ struct pdmd_ctx {
     pdmd::DevBuf<int> d_ids;
     pdmd::DevBuf<long long> d_inc;
     pdmd::DevBuf<unsigned long long> d_clock;  // start of a budgeted launch
+    pdmd::HostStage stage;
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     bool timed = false;
@@ -474,8 +502,7 @@ int pdmd_ctx_create(const char* param_dir, pdmd_ctx** out) {
             ctx->lds_limit = (size_t)std::max(lds, 32768);
         }
     }
-    // the fixed staging array of pdmd_observables_noalloc on this device
-    HIPCHK(engine_scratch_init(ctx->device));
+    HIPCHK(ctx->stage.reserve(1));
     HIPCHK(ctx->d_clock.alloc(1));
     {
         int khz = 0;
@@ -770,6 +797,71 @@ int advance_launch(pdmd_ctx* ctx, int32_t nsys, const int32_t* ids, const int64_
 }  // namespace
 }  // namespace pdmd
 
+namespace pdmd {
+namespace {
+void fill_stats(const HostSys& H, const SysStats& r, long long wall_khz, pdmd_stats_t& out) {
+    const SysState& st = r.st;
+    std::memset(&out, 0, sizeof out);
+    out.coll = st.coll;
+    long long pe = 0;
+    for (int k = 1; k <= 30; ++k) {
+        out.nevents[k] = st.nevents[k];
+        pe += st.nevents[k];
+    }
+    out.pair_events = pe;
+    out.numghosts = st.numghosts;
+    out.nupdates = st.nupdates;
+    out.nforced = st.nforced;
+    out.t = st.t;
+    out.tfalse = st.tfalse;
+    out.interval = st.interval;
+    out.interval_max = st.interval_max;
+    out.status = st.status;
+    out.max_list = (int32_t)st.max_nb_seen;
+    out.nbeads = H.N;
+    out.avg_up = (double)r.up / H.N;
+    out.avg_dn = (double)r.dn / H.N;
+    for (int k = 0; k < kPhaseSlots; ++k) out.phase_cycles[k] = st.phase[k];
+    out.device_ms = (double)st.run_ticks / (double)wall_khz;
+    out.rebuild_ms = (double)st.rebuild_ticks / (double)wall_khz;
+    out.rebuilds = st.rebuilds;
+    out.waves = H.dev.waves_cap;
+    out.cell_factor = H.dev.cq;
+    out.cells_axis = H.dev.M;
+}
+}  // namespace
+
+int stats_of(pdmd_ctx* ctx, int32_t nsys, const int32_t* ids, pdmd_stats_t* out) {
+    if (nsys <= 0) return 0;
+    const size_t data = (sizeof(int) * (size_t)nsys + 255) / 256 * 256;  // after the list of systems
+    // the stage may be written only when no launch of the stream reads it:
+    // every use of it ends with a synchronisation
+    HIPCHK(ctx->stage.reserve(data + sizeof(SysStats) * (size_t)nsys));
+    for (int k = 0; k < nsys; ++k) {
+        if (!get_sys(ctx, ids[k])) return -1;
+        ctx->stage.at<int>(0)[k] = ids[k] - 1;
+    }
+    SysStats* r = ctx->stage.at<SysStats>(data);
+    HIPCHK(engine_stats(ctx->d_sys.p, ctx->stage.at<int>(0), nsys, r, ctx->stream));
+    HIPCHK(hipStreamSynchronize(ctx->stream));
+    for (int k = 0; k < nsys; ++k) fill_stats(*get_sys(ctx, ids[k]), r[k], ctx->wall_khz, out[k]);
+    return 0;
+}
+}  // namespace pdmd
+
+namespace pdmd {
+namespace {
+// waits for the stream; the statuses of the nsys systems listed in d_ids are
+// then at the start of the stage
+int read_status(pdmd_ctx* ctx, int nsys) {
+    HIPCHK(ctx->stage.reserve(sizeof(int) * (size_t)nsys));
+    HIPCHK(engine_status(ctx->d_sys.p, ctx->d_ids.p, nsys, ctx->stage.at<int>(0), ctx->stream));
+    HIPCHK(hipStreamSynchronize(ctx->stream));
+    return 0;
+}
+}  // namespace
+}  // namespace pdmd
+
 extern "C" {
 
 int pdmd_rebuild(pdmd_ctx* ctx, int32_t nsys, const int32_t* ids) {
@@ -787,13 +879,10 @@ int pdmd_rebuild(pdmd_ctx* ctx, int32_t nsys, const int32_t* ids) {
     }
     HIPCHK(hipMemcpyAsync(ctx->d_ids.p, dids.data(), sizeof(int) * nsys, hipMemcpyHostToDevice, ctx->stream));
     HIPCHK(engine_rebuild(ctx->d_sys.p, ctx->d_ids.p, nsys, max_n, ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
-    for (int k = 0; k < nsys; ++k) {
-        SysState chk;
-        HIPCHK(hipMemcpy(&chk, get_sys(ctx, ids[k])->st.p, sizeof chk, hipMemcpyDeviceToHost));
-        if (chk.status) return fail("pdmd_rebuild: system " + std::to_string(ids[k]) + " status " +
-                                    std::to_string(chk.status), -3);
-    }
+    if (int rc = read_status(ctx, nsys)) return rc;
+    for (int k = 0; k < nsys; ++k)
+        if (const int st = ctx->stage.at<int>(0)[k])
+            return fail("pdmd_rebuild: system " + std::to_string(ids[k]) + " status " + std::to_string(st), -3);
     return 0;
 }
 
@@ -819,14 +908,11 @@ int pdmd_wait(pdmd_ctx* ctx) {
 int pdmd_advance(pdmd_ctx* ctx, int32_t nsys, const int32_t* ids, const int64_t* nev) {
     int e = pdmd_advance_async(ctx, nsys, ids, nev);
     if (e) return e;
-    e = pdmd_wait(ctx);
+    e = read_status(ctx, nsys);
     if (e) return e;
-    for (int k = 0; k < nsys; ++k) {
-        HostSys* H = get_sys(ctx, ids[k]);
-        int status = 0;
-        HIPCHK(hipMemcpy(&status, &H->st.p->status, sizeof(int), hipMemcpyDeviceToHost));
-        if (status) return fail("system " + std::to_string(ids[k]) + " stopped with device status " + std::to_string(status), -10 - status);
-    }
+    for (int k = 0; k < nsys; ++k)
+        if (const int status = ctx->stage.at<int>(0)[k])
+            return fail("system " + std::to_string(ids[k]) + " stopped with device status " + std::to_string(status), -10 - status);
     return 0;
 }
 
@@ -967,86 +1053,32 @@ int pdmd_download(pdmd_ctx* ctx, int32_t id, double* sv, int32_t* identity, int3
                   double* tim, int32_t* nptnr, int32_t* coltype) {
     HostSys* H = get_sys(ctx, id);
     if (!H) return -1;
-    HIPCHK(hipStreamSynchronize(ctx->stream));
     const int N = H->N;
-    std::vector<Rec> b(N);
-    HIPCHK(hipMemcpy(b.data(), H->rec.p, sizeof(Rec) * N, hipMemcpyDeviceToHost));
-    for (int k = 0; k < N; ++k) {
-        if (sv) {
-            sv[6 * k] = b[k].x;
-            sv[6 * k + 1] = b[k].y;
-            sv[6 * k + 2] = b[k].z;
-            sv[6 * k + 3] = b[k].vx;
-            sv[6 * k + 4] = b[k].vy;
-            sv[6 * k + 5] = b[k].vz;
-        }
-        if (identity) identity[k] = dyn_ident(b[k].dyn);
-        if (bptnr) bptnr[k] = dyn_bptnr(b[k].dyn) + 1;
-    }
-    if (extra_repuls) {
-        std::vector<int4> e(N);
-        HIPCHK(hipMemcpy(e.data(), H->extra.p, sizeof(int4) * N, hipMemcpyDeviceToHost));
-        for (int k = 0; k < N; ++k) {
-            extra_repuls[4 * k] = e[k].x + 1;
-            extra_repuls[4 * k + 1] = e[k].y + 1;
-            extra_repuls[4 * k + 2] = e[k].z + 1;
-            extra_repuls[4 * k + 3] = e[k].w + 1;
-        }
-    }
-    if (tim || nptnr || coltype) {
-        std::vector<Leaf> lf(N + 3);
-        HIPCHK(hipMemcpy(lf.data(), H->leaf.p, sizeof(Leaf) * (N + 3), hipMemcpyDeviceToHost));
-        for (int k = 0; k < N + 3; ++k) {
-            if (tim) tim[k] = lf[k].tim;
-            if (nptnr) nptnr[k] = lf[k].nptnr >= 0 ? lf[k].nptnr + 1 : lf[k].nptnr;
-            if (coltype) coltype[k] = leaf_ct(lf[k].meta);
-        }
-    }
+    const StateLayout at(N);
+    struct {
+        int flag;
+        void* dst;
+        size_t from, bytes;
+    } const part[] = {{kStateSv, sv, 0, 48 * (size_t)N},
+                      {kStateTim, tim, 8 * at.tim, 8 * (size_t)(N + 3)},
+                      {kStateIdent, identity, 4 * at.ident, 4 * (size_t)N},
+                      {kStateBptnr, bptnr, 4 * at.bptnr, 4 * (size_t)N},
+                      {kStateExtra, extra_repuls, 4 * at.extra, 16 * (size_t)N},
+                      {kStateNptnr, nptnr, 4 * at.nptnr, 4 * (size_t)(N + 3)},
+                      {kStateColtype, coltype, 4 * at.coltype, 4 * (size_t)(N + 3)}};
+    int want = 0;
+    for (const auto& q : part) want |= q.dst ? q.flag : 0;
+    HIPCHK(ctx->stage.reserve(at.bytes));
+    HIPCHK(engine_state(ctx->d_sys.p, id - 1, N, want, ctx->stage.at<double>(0), ctx->stream));
+    HIPCHK(hipStreamSynchronize(ctx->stream));
+    for (const auto& q : part)
+        if (q.dst) std::memcpy(q.dst, ctx->stage.at<char>(q.from), q.bytes);
     return 0;
 }
 
 int pdmd_stats(pdmd_ctx* ctx, int32_t id, pdmd_stats_t* out) {
-    HostSys* H = get_sys(ctx, id);
-    if (!H || !out) return -1;
-    HIPCHK(hipStreamSynchronize(ctx->stream));
-    SysState st;
-    HIPCHK(hipMemcpy(&st, H->st.p, sizeof st, hipMemcpyDeviceToHost));
-    std::memset(out, 0, sizeof *out);
-    out->coll = st.coll;
-    long long pe = 0;
-    for (int k = 1; k <= 30; ++k) {
-        out->nevents[k] = st.nevents[k];
-        pe += st.nevents[k];
-    }
-    out->pair_events = pe;
-    out->numghosts = st.numghosts;
-    out->nupdates = st.nupdates;
-    out->nforced = st.nforced;
-    out->t = st.t;
-    out->tfalse = st.tfalse;
-    out->interval = st.interval;
-    out->interval_max = st.interval_max;
-    out->status = st.status;
-    out->max_list = (int32_t)st.max_nb_seen;
-    out->nbeads = H->N;
-    std::vector<int> nu(H->N), nd(H->N);
-    HIPCHK(hipMemcpy(nu.data(), H->nup.p, sizeof(int) * H->N, hipMemcpyDeviceToHost));
-    HIPCHK(hipMemcpy(nd.data(), H->ndn.p, sizeof(int) * H->N, hipMemcpyDeviceToHost));
-    long long su = 0, sd = 0;
-    for (int k = 0; k < H->N; ++k) {
-        su += nu[k];
-        sd += nd[k];
-    }
-    out->avg_up = (double)su / H->N;
-    out->avg_dn = (double)sd / H->N;
-    for (int k = 0; k < kPhaseSlots; ++k) out->phase_cycles[k] = st.phase[k];
-    out->device_ms = (double)st.run_ticks / (double)ctx->wall_khz;
-    out->rebuild_ms = (double)st.rebuild_ticks / (double)ctx->wall_khz;
-    out->rebuilds = st.rebuilds;
-    out->waves = H->dev.waves_cap;
-    out->cell_factor = H->dev.cq;
-    out->cells_axis = H->dev.M;
-    return 0;
+    if (!get_sys(ctx, id) || !out) return -1;
+    return stats_of(ctx, 1, &id, out);
 }
 
 int pdmd_log_enable(pdmd_ctx* ctx, int32_t id, int32_t capacity) {
@@ -1184,27 +1216,22 @@ int pdmd_check(pdmd_ctx* ctx, int32_t id, const double* sv, pdmd_check_t* out) {
     return 0;
 }
 
-int pdmd_observables(pdmd_ctx* ctx, int32_t id, pdmd_obs_t* o) {
-    HostSys* H = get_sys(ctx, id);
-    if (!H || !o) return fail("pdmd_observables: bad arguments");
-    const Topology& t = H->topo;
+static int observe(pdmd_ctx* ctx, const HostSys& H, int32_t id, pdmd_obs_t* o) {
+    const Topology& t = H.topo;
     const int nch = (int)t.chain_len.size();
     int nfirst = 0;  // chains of the leading species block: the reference's species 1
     while (nfirst < nch && t.species[nfirst] == t.species[0]) nfirst++;
-    DevBuf<int> cs, cl, oi;
-    DevBuf<double> od;
-    HIPCHK(cs.alloc(nch));
-    HIPCHK(cl.alloc(nch));
-    HIPCHK(od.alloc(7));
-    HIPCHK(oi.alloc(3));
-    HIPCHK(hipMemcpyAsync(cs.p, t.chain_start.data(), sizeof(int) * nch, hipMemcpyHostToDevice, ctx->stream));
-    HIPCHK(hipMemcpyAsync(cl.p, t.chain_len.data(), sizeof(int) * nch, hipMemcpyHostToDevice, ctx->stream));
-    HIPCHK(engine_observables(ctx->d_sys.p, id - 1, cs.p, cl.p, nch, nfirst, H->p.boxl_orig, od.p, oi.p, ctx->stream));
+    // the results, then the chain tables
+    constexpr size_t kInts = 64, kChains = 256;
+    const size_t row = sizeof(int) * (size_t)nch;
+    HIPCHK(ctx->stage.reserve(kChains + 2 * row));
+    double* d = ctx->stage.at<double>(0);
+    int* n = ctx->stage.at<int>(kInts);
+    int *cs = ctx->stage.at<int>(kChains), *cl = cs + nch;
+    std::memcpy(cs, t.chain_start.data(), row);
+    std::memcpy(cl, t.chain_len.data(), row);
+    HIPCHK(engine_observables(ctx->d_sys.p, id - 1, H.N, cs, cl, nch, nfirst, H.p.boxl_orig, d, n, ctx->stream));
     HIPCHK(hipStreamSynchronize(ctx->stream));
-    double d[7];
-    int n[3];
-    HIPCHK(hipMemcpy(d, od.p, sizeof d, hipMemcpyDeviceToHost));
-    HIPCHK(hipMemcpy(n, oi.p, sizeof n, hipMemcpyDeviceToHost));
     std::memset(o, 0, sizeof *o);
     o->ered = d[0];
     o->tred = d[1];
@@ -1219,30 +1246,16 @@ int pdmd_observables(pdmd_ctx* ctx, int32_t id, pdmd_obs_t* o) {
     return 0;
 }
 
+int pdmd_observables(pdmd_ctx* ctx, int32_t id, pdmd_obs_t* o) {
+    HostSys* H = get_sys(ctx, id);
+    if (!H || !o) return fail("pdmd_observables: bad arguments");
+    return observe(ctx, *H, id, o);
+}
+
 int pdmd_observables_noalloc(pdmd_ctx* ctx, int32_t id, pdmd_obs_t* o) {
     HostSys* H = get_sys(ctx, id);
     if (!H || !o) return fail("pdmd_observables_noalloc: bad arguments");
-    const Topology& t = H->topo;
-    const int nch = (int)t.chain_len.size();
-    if (nch > 4096) return fail("pdmd_observables_noalloc: at most 4096 chains (the staging array's size)");
-    int nfirst = 0;  // chains of the leading species block: the reference's species 1
-    while (nfirst < nch && t.species[nfirst] == t.species[0]) nfirst++;
-    double d[7];
-    int n[3];
-    HIPCHK(engine_observables_noalloc(ctx->d_sys.p, id - 1, ctx->device, t.chain_start.data(), t.chain_len.data(), nch,
-                                      nfirst, H->p.boxl_orig, d, n, ctx->stream));
-    std::memset(o, 0, sizeof *o);
-    o->ered = d[0];
-    o->tred = d[1];
-    o->sumvel = d[2];
-    o->ehh_ii = d[3];
-    o->ehh_ij = d[4];
-    o->rg_avg = d[5];
-    o->e2e_avg = d[6];
-    o->hb_alpha = n[0];
-    o->hb_ii = n[1];
-    o->hb_ij = n[2];
-    return 0;
+    return observe(ctx, *H, id, o);
 }
 
 int pdmd_pair_codes(const pdmd_system_desc* d, int32_t n, const int32_t* a, const int32_t* b, int32_t* code) {

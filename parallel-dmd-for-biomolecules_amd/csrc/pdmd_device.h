@@ -99,6 +99,30 @@ struct SysState {
     long long rebuilds;       // list rebuilds those ticks cover
 };
 
+// what k_stats writes for a system
+struct SysStats {
+    SysState st;
+    long long up, dn;  // row lengths summed over the beads
+};
+
+// Layout of a downloaded state of N beads, in the C ABI's arrays: sv[6N] and
+// tim[N+3] from the start, in doubles; then the 32-bit arrays, their places
+// in 32-bit words from the start.
+enum { kStateSv = 1, kStateTim = 2, kStateIdent = 4, kStateBptnr = 8, kStateExtra = 16, kStateNptnr = 32, kStateColtype = 64 };
+struct StateLayout {
+    size_t tim, ident, bptnr, extra, nptnr, coltype, bytes;
+    __host__ __device__ explicit StateLayout(int n) {
+        const size_t N = (size_t)n;
+        tim = 6 * N;
+        ident = 2 * (7 * N + 3);
+        bptnr = ident + N;
+        extra = bptnr + N;
+        nptnr = extra + 4 * N;
+        coltype = nptnr + N + 3;
+        bytes = 4 * (coltype + N + 3);
+    }
+};
+
 struct LogRec {
     long long coll;
     int i, j, type, pad;

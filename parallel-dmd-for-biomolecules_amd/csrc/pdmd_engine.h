@@ -35,21 +35,18 @@ hipError_t engine_run(const SysDev* d_sys, const int* d_ids, const long long* d_
 // counters (zeroed by the caller, out[3] preset to all ones); alt replaces
 // the resident state records when not null.
 hipError_t engine_check(const SysDev* d_sys, int id, int n, const Rec* alt, unsigned long long* out, hipStream_t s);
-// Observables of system id (energy.f, radgyr.f, end2end.f) on one
-// workgroup: outd[7] ered, tred, sumvel, ehh_ii, ehh_ij, rg_avg, e2e_avg;
-// outi[3] hb_alpha, hb_ii, hb_ij.  cstart/clen: nch chains (device arrays);
-// nfirst: chains of the leading species block; boxl in Angstrom.
-hipError_t engine_observables(const SysDev* d_sys, int id, const int* cstart, const int* clen, int nch, int nfirst,
+// Observables of system id of n beads (energy.f, radgyr.f, end2end.f):
+// outd[7] ered, tred, sumvel, ehh_ii, ehh_ij, rg_avg, e2e_avg; outi[3]
+// hb_alpha, hb_ii, hb_ij.  cstart/clen: nch chains (addresses the device can
+// read); nfirst: chains of the leading species block; boxl in Angstrom.
+hipError_t engine_observables(const SysDev* d_sys, int id, int n, const int* cstart, const int* clen, int nch, int nfirst,
                               double boxl, double* outd, int* outi, hipStream_t s);
-// The same without device allocation (pdmd_observables_noalloc): the chain
-// tables (host arrays, nch <= 4096) and the results pass through a fixed
-// 33 KB device array per GPU; returns after the results reached h_outd[7]
-// and h_outi[3].  Calls that overlap on one GPU race on that array.
-hipError_t engine_observables_noalloc(const SysDev* d_sys, int id, int device, const int* h_cstart, const int* h_clen,
-                                      int nch, int nfirst, double boxl, double* h_outd, int* h_outi, hipStream_t s);
-// Looks up this GPU's copy of that array (device must be current); done
-// once per device at context creation.
-hipError_t engine_scratch_init(int device);
+// State arrays of system id of n beads into out (StateLayout), those in
+// `want` (kStateSv ...).
+hipError_t engine_state(const SysDev* d_sys, int id, int n, int want, double* out, hipStream_t s);
+// SysState::status, and all counters, of n systems.
+hipError_t engine_status(const SysDev* d_sys, const int* d_ids, int n, int* out, hipStream_t s);
+hipError_t engine_stats(const SysDev* d_sys, const int* ids, int n, SysStats* out, hipStream_t s);
 // Test hook: collision times of (i, j) pairs (1-based) of system id.
 hipError_t engine_predict(const SysDev* d_sys, int id, int n, const int* pi, const int* pj, double* tij, int* type,
                           hipStream_t s);

@@ -4344,6 +4344,7 @@ __device__ void copy_tables(const DevTables* src, DevTables* dst) {
 // one of 256 compute units, at 512 beads 205 us; the launches cost a few
 // microseconds each, so small systems gain too.
 constexpr int kGridT = 256;
+constexpr int kStatsT = 1024;
 __device__ inline void report(const SysDev& S, int status) {
     status = wave_status(status);
     if (status && lane_id() == 0) atomicCAS(&S.st->status, 0, status);  // the first error stays
@@ -4920,139 +4921,185 @@ __global__ void k_check(const SysDev* sys, int id, const Rec* alt, unsigned long
 
 // ------------------------------------------------------------------------
 // observables of one system: energy.f:25-101, radgyr.f:18-135,
-// end2end.f:14-44, on one workgroup of kObsT lanes
+// end2end.f:14-44
 // ------------------------------------------------------------------------
+// Latency: three launches, sums in a fixed order, k_obs_parts (bead sums, and
+// every chain unwrapped), k_obs_chains (chain sums), k_obs_sum.  One workgroup
+// per system with a lane per chain walked 128 beads serially through memory:
+// 95 us at 6144 beads on one compute unit.  List update, calendars and
+// observables of 16 systems of up to 23 424 beads with either (and with the
+// reads below): 4.51 ms, 1.49 ms.
 constexpr int kObsT = 256;
-// sum over the workgroup in a fixed tree (the same result on every call)
-__device__ inline double obs_sum(double v, double* red) {
-    const int t = (int)threadIdx.x;
-    red[t] = v;
-    __syncthreads();
-    for (int w = kObsT / 2; w > 0; w >>= 1) {
-        if (t < w) red[t] = red[t] + red[t + w];
-        __syncthreads();
-    }
-    const double r = red[0];
-    __syncthreads();
-    return r;
+constexpr int kObsBeads = 64;  // beads per workgroup: a 16-lane row takes a side chain's pairs
+constexpr int kObsSums = 6;    // sumvel, ehh_ii, ehh_ij, hb_ii, hb_ij, hb_alpha
+// partial sums in the list rebuild's scratch: 48 bytes per 64 beads, then 16
+// per chain of at least 16 beads; sinfo has 16 per bead
+__device__ inline double* obs_bead_sums(const SysDev& S) { return reinterpret_cast<double*>(S.sinfo); }
+__device__ inline double* obs_chain_sums(const SysDev& S) {
+    return obs_bead_sums(S) + kObsSums * ((S.N + kObsBeads - 1) / kObsBeads);
 }
-// Bead sums in a fixed order per lane (kinetic energy, H-bond counts,
-// side-chain well energies over the up lists: every side-chain pair inside
-// a well is listed, wells lie inside the list cutoff); chain walks one lane
-// per chain (backbone unwrapping into q, then radius of gyration and
-// end-to-end distance).  nfirst: chains of the leading species block.
-// outd: ered, tred, sumvel, ehh_ii, ehh_ij, rg_avg, e2e_avg; outi: hb_alpha,
-// hb_ii, hb_ij.
-__global__ __launch_bounds__(kObsT) void k_obs(const SysDev* sys, int id, const int* cstart, const int* clen, int nch,
-                                              int nfirst, double boxl, double* outd, int* outi) {
-    __shared__ double red[kObsT];
+// sum over the wavefront in a fixed tree, in every lane
+__device__ inline double wave_sum(double v) {
+    for (int w = kW / 2; w > 0; w >>= 1) v = v + __shfl_xor(v, w);
+    return v;
+}
+// one coordinate's image next to the unwrapped neighbour's (radgyr.f:48-104)
+__device__ inline double unwrap(double a, double b) {
+    const double dd = a - b;
+    return dd > 0.5 ? a - 1.0 : (dd < -0.5 ? a + 1.0 : a);
+}
+// Workgroups [0, nb): bead sums (kinetic energy, H-bond counts, side-chain
+// well energies over the up lists: every side-chain pair inside a well is
+// listed, wells lie inside the list cutoff).  The others: a wavefront per
+// chain, backbone unwrapped into spos.
+__global__ __launch_bounds__(kObsT) void k_obs_parts(const SysDev* __restrict__ sys, int id, int nb, const int* cstart,
+                                                     const int* clen, int nch) {
     const SysDev& S = sys[id];
-    const DevTables& T = *S.tab;
-    const int N = S.N, cap = S.cap, t = (int)threadIdx.x;
+    const int N = S.N, wave = wave_id(), lane = lane_id();
     const double tf = S.st->tfalse;
-    double sumvel = 0.0, eii = 0.0, eij = 0.0;
-    double hii = 0.0, hij = 0.0, halpha = 0.0;
-    for (int i = t; i < N; i += kObsT) {
+    if ((int)blockIdx.x >= nb) {
+        const int c = ((int)blockIdx.x - nb) * (kObsT / kW) + wave;
+        if (c >= nch) return;
+        const int s = cstart[c], L = clen[c];
+        double4* q = S.spos;
+        auto at = [&](int k) {
+            const Rec b = S.rec[k];
+            return make_double4(b.x + b.vx * tf, b.y + b.vy * tf, b.z + b.vz * tf, 0.0);
+        };
+        double4 prev = make_double4(0.0, 0.0, 0.0, 0.0);  // the residue before the chunk's
+        for (int base = 0; base < L; base += kW) {
+            const int r = base + lane, n = min(kW, L - base);
+            const double4 zero = make_double4(0.0, 0.0, 0.0, 0.0);
+            double4 ca = r < L ? at(s + r) : zero;
+            // each Calpha next to the one before it, in order
+            for (int u = 0; u < n; ++u) {
+                double4 v = make_double4(readlane_d(ca.x, u), readlane_d(ca.y, u), readlane_d(ca.z, u), 0.0);
+                if (base + u > 0) v = make_double4(unwrap(v.x, prev.x), unwrap(v.y, prev.y), unwrap(v.z, prev.z), 0.0);
+                if (lane == u) ca = v;
+                prev = v;
+            }
+            if (r < L) {
+                q[s + r] = ca;
+                // N and C next to their Calpha; the side chain as it is: the
+                // second species' sums can reach an earlier chain's
+                for (int kind = 1; kind < 3; ++kind) {
+                    const double4 v = at(s + kind * L + r);
+                    q[s + kind * L + r] =
+                        make_double4(unwrap(v.x, ca.x), unwrap(v.y, ca.y), unwrap(v.z, ca.z), 0.0);
+                }
+                q[s + 3 * L + r] = at(s + 3 * L + r);
+            }
+        }
+        return;
+    }
+    __shared__ double red[kObsT / kW][kObsSums];
+    const DevTables& T = *S.tab;
+    double sum[kObsSums] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    const int first = (int)blockIdx.x * kObsBeads;
+    if ((int)threadIdx.x < kObsBeads && first + (int)threadIdx.x < N) {
+        const int i = first + (int)threadIdx.x;
         const Rec r = S.rec[i];
-        sumvel = sumvel + r.bm * (r.vx * r.vx + r.vy * r.vy + r.vz * r.vz);
+        sum[0] = r.bm * (r.vx * r.vx + r.vy * r.vy + r.vz * r.vz);
         const int j = dyn_bptnr(r.dyn);
         if (j > i) {
-            if (topo_chain(r.topo) == topo_chain(S.rec[j].topo))
-                hii = hii + 1.0;
-            else
-                hij = hij + 1.0;
+            const bool same = topo_chain(r.topo) == topo_chain(S.rec[j].topo);
+            sum[3] = same ? 1.0 : 0.0;
+            sum[4] = same ? 0.0 : 1.0;
         }
-        const int kind = topo_kind(r.topo), res = topo_res(r.topo), L = topo_len(r.topo);
-        if (kind == 1 && res >= 5 && j == i + L - 4) halpha = halpha + 1.0;
-        if (kind == 3) {
-            const int nu = min(S.nup[i], cap), idi = dyn_ident(r.dyn);
-            for (int k = 0; k < nu; ++k) {
-                const int ent = S.nb_up[(size_t)i * cap + k];
-                const int m = ent & 0xFFFFFF;
-                if ((ent >> 24) != 16 || m == j) continue;
-                const Rec rm = S.rec[m];
-                Geo g;
-                geo(r, rm, tf, g);
-                const int idm = dyn_ident(rm.dyn);
-                if (g.r2 <= T.welldia_sq[idi][idm]) {
-                    if (topo_chain(r.topo) == topo_chain(rm.topo))
-                        eii = eii + T.ep_sqrt[idi][idm];
-                    else
-                        eij = eij + T.ep_sqrt[idi][idm];
-                }
+        if (topo_kind(r.topo) == 1 && topo_res(r.topo) >= 5 && j == i + topo_len(r.topo) - 4) sum[5] = 1.0;
+    }
+    constexpr int kRows = kObsT / 16;
+    for (int u = 0; u < kObsBeads / kRows; ++u) {
+        const int i = first + u * kRows + (int)threadIdx.x / 16;
+        if (i >= N) break;
+        const Rec r = S.rec[i];
+        if (topo_kind(r.topo) != 3) continue;
+        const int nu = min(S.nup[i], S.cap), idi = dyn_ident(r.dyn), j = dyn_bptnr(r.dyn);
+        for (int k = lane & 15; k < nu; k += 16) {
+            const int ent = S.nb_up[(size_t)i * S.cap + k], m = ent & 0xFFFFFF;
+            if ((ent >> 24) != 16 || m == j) continue;
+            const Rec rm = S.rec[m];
+            Geo g;
+            geo(r, rm, tf, g);
+            const int idm = dyn_ident(rm.dyn);
+            if (g.r2 <= T.welldia_sq[idi][idm]) {
+                const double e = T.ep_sqrt[idi][idm];
+                if (topo_chain(r.topo) == topo_chain(rm.topo))
+                    sum[1] = sum[1] + e;
+                else
+                    sum[2] = sum[2] + e;
             }
         }
     }
-    // backbone unwrapping along each chain (radgyr.f:48-104) into q
-    double4* q = S.spos;
-    for (int c = t; c < nch; c += kObsT) {
-        const int s = cstart[c], L = clen[c];
-        // every bead of the chain: the second species' sums below can reach
-        // into an earlier chain's side-chain beads
-        for (int k = s; k < s + 4 * L; ++k) {
-            const Rec b = S.rec[k];
-            q[k] = make_double4(b.x + b.vx * tf, b.y + b.vy * tf, b.z + b.vz * tf, 0.0);
-        }
-        auto unwrap = [&](int a, int b) {
-            double4 qa = q[a];
-            const double4 qb = q[b];
-            double dd = qa.x - qb.x;
-            if (dd > 0.5) qa.x = qa.x - 1.0;
-            else if (dd < -1.0 * 0.5) qa.x = qa.x + 1.0;
-            dd = qa.y - qb.y;
-            if (dd > 0.5) qa.y = qa.y - 1.0;
-            else if (dd < -1.0 * 0.5) qa.y = qa.y + 1.0;
-            dd = qa.z - qb.z;
-            if (dd > 0.5) qa.z = qa.z - 1.0;
-            else if (dd < -1.0 * 0.5) qa.z = qa.z + 1.0;
-            q[a] = qa;
-        };
-        for (int k = s + 1; k < s + L; ++k) unwrap(k, k - 1);
-        for (int k = s; k < s + L; ++k) unwrap(L + k, k);
-        for (int k = s; k < s + L; ++k) unwrap(2 * L + k, k);
+    for (int k = 0; k < kObsSums; ++k) {
+        const double v = wave_sum(sum[k]);
+        if (lane == 0) red[wave][k] = v;
     }
-    __threadfence_block();
     __syncthreads();
-    double rg = 0.0, e2e = 0.0, nbb = 0.0;
-    for (int c = t; c < nch; c += kObsT) {
-        const int s = cstart[c], L = clen[c];
-        // radgyr.f:117-125 sums a chain of the second species block over
-        // beads (c-1)*numbeads2+1 .. +3*chnln2 without the first block's
-        // offset its unwrapping uses (:78), while those beads exist
-        int rb = s;
-        if (c >= nfirst && c * 4 * L + 3 * L <= s + 4 * L) rb = c * 4 * L;
-        double cx = 0, cy = 0, cz = 0, rgs = 0;
-        for (int k = rb; k < rb + 3 * L; ++k) {
-            const double4 v = q[k];
-            cx = cx + v.x;
-            cy = cy + v.y;
-            cz = cz + v.z;
-        }
-        cx = cx / (double)(3 * L);
-        cy = cy / (double)(3 * L);
-        cz = cz / (double)(3 * L);
-        for (int k = rb; k < rb + 3 * L; ++k) {
-            const double4 v = q[k];
-            const double rx = (v.x - cx) * (v.x - cx), ry = (v.y - cy) * (v.y - cy), rz = (v.z - cz) * (v.z - cz);
-            rgs = rgs + rx + ry + rz;
-        }
-        rg = rg + rgs;
-        nbb = nbb + (double)(3 * L);
-        e2e = e2e + dist_rec(S.rec[s + L], S.rec[s + 3 * L - 1], tf);  // end2end.f: N of residue 1 to C of residue L
+    if ((int)threadIdx.x < kObsSums) {
+        double v = red[0][threadIdx.x];
+        for (int w = 1; w < kObsT / kW; ++w) v = v + red[w][threadIdx.x];
+        obs_bead_sums(S)[kObsSums * (size_t)blockIdx.x + threadIdx.x] = v;
     }
-    sumvel = obs_sum(sumvel, red);
-    eii = obs_sum(eii, red);
-    eij = obs_sum(eij, red);
-    hii = obs_sum(hii, red);
-    hij = obs_sum(hij, red);
-    halpha = obs_sum(halpha, red);
-    rg = obs_sum(rg, red);
-    e2e = obs_sum(e2e, red);
-    nbb = obs_sum(nbb, red);
-    if (t == 0) {
-        const double eps_hb = T.ep_sqrt[5][8];
-        const int sum_hb = (int)hii + (int)hij;
-        const double sumeps = -(sum_hb * eps_hb + (eii + eij));
+}
+// A wavefront per chain: squared radius of gyration, summed over the
+// backbone, and end-to-end distance.  nfirst: chains of the leading species
+// block.
+__global__ __launch_bounds__(kObsT) void k_obs_chains(const SysDev* __restrict__ sys, int id, const int* cstart,
+                                                      const int* clen, int nch, int nfirst) {
+    const SysDev& S = sys[id];
+    const int c = (int)blockIdx.x * (kObsT / kW) + wave_id(), lane = lane_id();
+    if (c >= nch) return;
+    const int s = cstart[c], L = clen[c], n = 3 * L;
+    // radgyr.f:117-125 sums a chain of the second species block over
+    // beads (c-1)*numbeads2+1 .. +3*chnln2 without the first block's
+    // offset its unwrapping uses (:78), while those beads exist
+    int rb = s;
+    if (c >= nfirst && c * 4 * L + 3 * L <= s + 4 * L) rb = c * 4 * L;
+    const double4* q = S.spos + rb;
+    double cx = 0.0, cy = 0.0, cz = 0.0, rg = 0.0;
+    for (int k = lane; k < n; k += kW) {
+        const double4 v = q[k];
+        cx = cx + v.x;
+        cy = cy + v.y;
+        cz = cz + v.z;
+    }
+    cx = wave_sum(cx) / (double)n;
+    cy = wave_sum(cy) / (double)n;
+    cz = wave_sum(cz) / (double)n;
+    for (int k = lane; k < n; k += kW) {
+        const double4 v = q[k];
+        rg = rg + (v.x - cx) * (v.x - cx) + (v.y - cy) * (v.y - cy) + (v.z - cz) * (v.z - cz);
+    }
+    rg = wave_sum(rg);
+    if (lane == 0) {
+        obs_chain_sums(S)[2 * c] = rg;
+        // end2end.f: N of residue 1 to C of residue L
+        obs_chain_sums(S)[2 * c + 1] = dist_rec(S.rec[s + L], S.rec[s + 3 * L - 1], S.st->tfalse);
+    }
+}
+// outd: ered, tred, sumvel, ehh_ii, ehh_ij, rg_avg, e2e_avg; outi: hb_alpha,
+// hb_ii, hb_ij.
+__global__ __launch_bounds__(kW) void k_obs_sum(const SysDev* __restrict__ sys, int id, int nb, int nch, double boxl,
+                                                double* outd, int* outi) {
+    const SysDev& S = sys[id];
+    const int N = S.N, lane = lane_id();
+    double v[kObsSums] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0}, rg = 0.0, e2e = 0.0;
+    const double* pb = obs_bead_sums(S);
+    const double* pc = obs_chain_sums(S);
+    for (int b = lane; b < nb; b += kW)
+        for (int k = 0; k < kObsSums; ++k) v[k] = v[k] + pb[kObsSums * b + k];
+    for (int c = lane; c < nch; c += kW) {
+        rg = rg + pc[2 * c];
+        e2e = e2e + pc[2 * c + 1];
+    }
+    for (int k = 0; k < kObsSums; ++k) v[k] = wave_sum(v[k]);
+    rg = wave_sum(rg);
+    e2e = wave_sum(e2e);
+    if (lane == 0) {
+        const double sumvel = v[0], eii = v[1], eij = v[2], nbb = (double)(3 * (N / 4));  // backbone beads
+        const int hii = (int)v[3], hij = (int)v[4], sum_hb = hii + hij;
+        const double sumeps = -(sum_hb * S.tab->ep_sqrt[5][8] + (eii + eij));
         outd[0] = 0.5 * sumvel + sumeps;
         outd[1] = sumvel / 3.0 / (double)N;
         outd[2] = sumvel;
@@ -5060,9 +5107,73 @@ __global__ __launch_bounds__(kObsT) void k_obs(const SysDev* sys, int id, const 
         outd[4] = eij;
         outd[5] = sqrt(rg / nbb) * boxl;
         outd[6] = e2e / (double)nch * boxl;
-        outi[0] = (int)halpha;
-        outi[1] = (int)hii;
-        outi[2] = (int)hij;
+        outi[0] = (int)v[5];
+        outi[1] = hii;
+        outi[2] = hij;
+    }
+}
+
+// ------------------------------------------------------------------------
+// What the host reads, written by kernels straight into page-locked host
+// memory in the host's layout: one launch and one wait.  A state read as three
+// blocking copies to pageable memory and a pass over the records on the host
+// took 45 us more at 128 to 1536 beads (320 systems advanced by 2000 entries
+// and read: 35.1 ms, 20.5 ms).
+// ------------------------------------------------------------------------
+__global__ __launch_bounds__(kGridT) void k_state(const SysDev* __restrict__ sys, int id, int want, double* out) {
+    const SysDev& S = sys[id];
+    const int N = S.N, w = (int)(blockIdx.x * kGridT + threadIdx.x);
+    const StateLayout at(N);
+    int* iout = reinterpret_cast<int*>(out);
+    // a lane per output word, so that a wavefront writes whole lines
+    if ((want & kStateSv) && w < 6 * N) {
+        const int k = w / 6;
+        out[w] = gl1(reinterpret_cast<const double*>(S.rec + k) + (w - 6 * k));
+    }
+    if (w < N + 3) {
+        if (want & kStateTim) out[at.tim + w] = gl1(&S.leaf[w].tim);
+        if (want & kStateNptnr) {
+            const int p = gl1(&S.leaf[w].nptnr);
+            iout[at.nptnr + w] = p >= 0 ? p + 1 : p;
+        }
+        if (want & kStateColtype) iout[at.coltype + w] = leaf_ct(gl1(&S.leaf[w].meta));
+    }
+    if (w < N) {
+        const int dyn = gl1(&S.rec[w].dyn);
+        if (want & kStateIdent) iout[at.ident + w] = dyn_ident(dyn);
+        if (want & kStateBptnr) iout[at.bptnr + w] = dyn_bptnr(dyn) + 1;
+    }
+    if ((want & kStateExtra) && w < 4 * N) iout[at.extra + w] = gl1(reinterpret_cast<const int*>(S.extra) + w) + 1;
+}
+__global__ __launch_bounds__(kGridT) void k_status(const SysDev* __restrict__ sys, const int* ids, int n, int* out) {
+    const int k = (int)(blockIdx.x * kGridT + threadIdx.x);
+    if (k < n) out[k] = sys[ids[k]].st->status;
+}
+// The counters, and the row lengths summed over the beads, of system ids[blockIdx.x].
+__global__ __launch_bounds__(kStatsT) void k_stats(const SysDev* __restrict__ sys, const int* ids, SysStats* out) {
+    __shared__ unsigned long long red[2][kStatsT / kW];
+    const SysDev& S = sys[ids[blockIdx.x]];
+    const int N = S.N, t = (int)threadIdx.x, lane = lane_id(), wave = wave_id();
+    unsigned long long* o = reinterpret_cast<unsigned long long*>(out + blockIdx.x);
+    const unsigned long long* st = reinterpret_cast<const unsigned long long*>(S.st);
+    for (int k = t; k < (int)(sizeof(SysState) / 8); k += kStatsT) o[k] = st[k];
+    int up = 0, dn = 0;  // a wavefront sums at most 65 533 rows of 64 entries
+#pragma unroll 4
+    for (int k = t; k < N; k += kStatsT) {
+        up += S.nup[k];
+        dn += S.ndn[k];
+    }
+    up = __builtin_amdgcn_readlane(wave_scan(up), kW - 1);
+    dn = __builtin_amdgcn_readlane(wave_scan(dn), kW - 1);
+    if (lane == 0) {
+        red[0][wave] = (unsigned long long)up;
+        red[1][wave] = (unsigned long long)dn;
+    }
+    __syncthreads();
+    if (t < 2) {
+        unsigned long long v = 0;
+        for (int w = 0; w < kStatsT / kW; ++w) v += red[t][w];
+        o[sizeof(SysState) / 8 + t] = v;
     }
 }
 
@@ -5180,70 +5291,25 @@ hipError_t engine_check(const SysDev* d_sys, int id, int n, const Rec* alt, unsi
     hipLaunchKernelGGL(k_check, dim3((n + 255) / 256), dim3(256), 0, s, d_sys, id, alt, out);
     return hipGetLastError();
 }
-hipError_t engine_observables(const SysDev* d_sys, int id, const int* cstart, const int* clen, int nch, int nfirst,
+hipError_t engine_observables(const SysDev* d_sys, int id, int n, const int* cstart, const int* clen, int nch, int nfirst,
                               double boxl, double* outd, int* outi, hipStream_t s) {
-    hipLaunchKernelGGL(k_obs, dim3(1), dim3(kObsT), 0, s, d_sys, id, cstart, clen, nch, nfirst, boxl, outd, outi);
+    const int nb = (n + kObsBeads - 1) / kObsBeads, nc = (nch + kObsT / kW - 1) / (kObsT / kW);
+    hipLaunchKernelGGL(k_obs_parts, dim3(nb + nc), dim3(kObsT), 0, s, d_sys, id, nb, cstart, clen, nch);
+    hipLaunchKernelGGL(k_obs_chains, dim3(nc), dim3(kObsT), 0, s, d_sys, id, cstart, clen, nch, nfirst);
+    hipLaunchKernelGGL(k_obs_sum, dim3(1), dim3(kW), 0, s, d_sys, id, nb, nch, boxl, outd, outi);
     return hipGetLastError();
 }
-// ------------------------------------------------------------------------
-// observables without device allocation: the chain tables and the results
-// are staged in one fixed device array per GPU
-// ------------------------------------------------------------------------
-constexpr int kScratchChains = 4096;  // a system holds at most 2047 chains
-constexpr size_t kScratchClen = sizeof(int) * kScratchChains;
-constexpr size_t kScratchOutd = 2 * kScratchClen;
-constexpr size_t kScratchOuti = kScratchOutd + 64;
-constexpr size_t kScratchBytes = kScratchOuti + 256;  // 33 024 bytes
-// Host code must not use this name as a device address: each GPU holds its
-// own copy, whose address engine_scratch_init looks up.
-static __device__ __align__(256) unsigned char scratch[kScratchBytes];
-namespace {
-constexpr int kMaxDevices = 64;
-std::mutex g_scratch_mu;
-unsigned char* g_scratch[kMaxDevices];
-}  // namespace
-
-hipError_t engine_scratch_init(int device) {
-    if (device < 0 || device >= kMaxDevices) return hipErrorInvalidDevice;
-    std::lock_guard<std::mutex> lock(g_scratch_mu);
-    if (g_scratch[device]) return hipSuccess;
-    int cur = -1;
-    hipError_t e = hipGetDevice(&cur);
-    if (e != hipSuccess) return e;
-    if (cur != device) return hipErrorInvalidDevice;
-    void* p = nullptr;
-    e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
-    if (e != hipSuccess) return e;
-    g_scratch[device] = static_cast<unsigned char*>(p);
-    return hipSuccess;
+hipError_t engine_state(const SysDev* d_sys, int id, int n, int want, double* out, hipStream_t s) {
+    hipLaunchKernelGGL(k_state, dim3((6 * n + kGridT - 1) / kGridT), dim3(kGridT), 0, s, d_sys, id, want, out);
+    return hipGetLastError();
 }
-
-hipError_t engine_observables_noalloc(const SysDev* d_sys, int id, int device, const int* h_cstart, const int* h_clen,
-                                      int nch, int nfirst, double boxl, double* h_outd, int* h_outi, hipStream_t s) {
-    if (nch < 1 || nch > kScratchChains) return hipErrorInvalidValue;
-    hipError_t e = engine_scratch_init(device);
-    if (e != hipSuccess) return e;
-    unsigned char* base;
-    {
-        std::lock_guard<std::mutex> lock(g_scratch_mu);
-        base = g_scratch[device];
-    }
-    int* cs = reinterpret_cast<int*>(base);
-    int* cl = reinterpret_cast<int*>(base + kScratchClen);
-    double* od = reinterpret_cast<double*>(base + kScratchOutd);
-    int* oi = reinterpret_cast<int*>(base + kScratchOuti);
-    e = hipMemcpyAsync(cs, h_cstart, sizeof(int) * (size_t)nch, hipMemcpyHostToDevice, s);
-    if (e != hipSuccess) return e;
-    e = hipMemcpyAsync(cl, h_clen, sizeof(int) * (size_t)nch, hipMemcpyHostToDevice, s);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_obs, dim3(1), dim3(kObsT), 0, s, d_sys, id, cs, cl, nch, nfirst, boxl, od, oi);
-    e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    e = hipMemcpyAsync(h_outd, od, sizeof(double) * 7, hipMemcpyDeviceToHost, s);
-    if (e != hipSuccess) return e;
-    e = hipMemcpyAsync(h_outi, oi, sizeof(int) * 3, hipMemcpyDeviceToHost, s);
-    if (e != hipSuccess) return e;
-    return hipStreamSynchronize(s);
+hipError_t engine_status(const SysDev* d_sys, const int* d_ids, int n, int* out, hipStream_t s) {
+    hipLaunchKernelGGL(k_status, dim3((n + kGridT - 1) / kGridT), dim3(kGridT), 0, s, d_sys, d_ids, n, out);
+    return hipGetLastError();
+}
+hipError_t engine_stats(const SysDev* d_sys, const int* ids, int n, SysStats* out, hipStream_t s) {
+    hipLaunchKernelGGL(k_stats, dim3(n), dim3(kStatsT), 0, s, d_sys, ids, out);
+    return hipGetLastError();
 }
 
 hipError_t engine_prepare(size_t lds_limit) {

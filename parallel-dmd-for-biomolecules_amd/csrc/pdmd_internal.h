@@ -23,4 +23,7 @@ int64_t prepared_bytes(const PreparedSystem* p);
 // system up; p is consumed (left empty) whether or not it succeeds.
 int prepared_add(pdmd_ctx* ctx, PreparedSystem* p, int32_t* sys_id);
 
+// pdmd_stats of nsys systems with one launch and one wait
+int stats_of(pdmd_ctx* ctx, int32_t nsys, const int32_t* ids, pdmd_stats_t* out);
+
 }  // namespace pdmd

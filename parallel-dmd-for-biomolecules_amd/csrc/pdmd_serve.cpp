@@ -87,11 +87,14 @@ int retire(pdmd_server* s, int32_t* ndone) {
     s->inflight = false;
     const double t = now_s() - s->t0;
     std::vector<Req*> keep;
+    std::vector<int32_t> ids;
+    for (const Req* r : s->resident) ids.push_back(r->sys);
+    std::vector<pdmd_stats_t> stats(ids.size());
+    rc = pdmd::stats_of(s->ctx, (int32_t)ids.size(), ids.data(), stats.data());
+    if (rc) return rc;
     for (size_t k = 0; k < s->resident.size(); ++k) {
         Req* r = s->resident[k];
-        pdmd_stats_t st;
-        rc = pdmd_stats(s->ctx, r->sys, &st);
-        if (rc) return rc;
+        const pdmd_stats_t& st = stats[k];
         const int64_t now_done = st.coll - r->coll0;
         s->committed += now_done - r->done;
         r->done = now_done;
