@@ -1325,9 +1325,11 @@ __device__ inline int accepted(const Batch& B) {
     const int top = uni(min(B.K, B.cut));
     const int q = lane & (kMaxWaves - 1);
     const bool in = lane < top;
+    const int st = in ? B.st[q] : 0;
+    const unsigned long long sm = __ballot(st != 0);
+    if (__ballot(in && B.knew[q].bc != kEmptyBc) == 0) return sm ? min(top, (int)__ffsll((long long)sm)) : top;
     const double pk = key_proxy(B.key[q]);
     const double pn = in ? key_proxy(B.knew[q]) : __hiloint2double(kInfHi, 0);
-    const int st = in ? B.st[q] : 0;
     auto shr = [](double v, auto ctrl) {
         constexpr int C = decltype(ctrl)::value;
         return __hiloint2double(__builtin_amdgcn_update_dpp(kInfHi, __double2hiint(v), C, 0xf, 0xf, false),
@@ -1339,7 +1341,7 @@ __device__ inline int accepted(const Batch& B) {
     lo = min_raw(lo, shr(lo, std::integral_constant<int, 0x114>{}));
     const bool live = in && lane >= 1;
     if (__ballot(live && pk == lo)) return uni(batch_accepted());
-    const unsigned long long fail = __ballot(live && pk > lo), sm = __ballot(st != 0);
+    const unsigned long long fail = __ballot(live && pk > lo);
     int A = top;
     if (fail) A = min(A, __ffsll((long long)fail) - 1);
     if (sm) A = min(A, (int)__ffsll((long long)sm));
@@ -2521,7 +2523,8 @@ constexpr int kOwners = 2 + kMaxSpec;
 struct OnePass {
     BaseRec base[kOwners];  // 0: bead i, 1: bead j, then the beads recomputed in full
     double wt[kW];
-    unsigned long long tkey[kOwners];
+    unsigned long long tkey[kOwners];  // least time
+    int win[kOwners];                  // its lane, the first of equal ones
     int wy[kW];
     int lst[kW];
 };
@@ -2641,7 +2644,7 @@ __device__ inline GhostDraw ghost_draw(unsigned long long seed, unsigned long lo
 // e: the calendar entry; jp, ct: its partner and type; tf, nbin, coll: the
 // false time, bin and number of the event; bk: its place in the round.
 // Returns the round's accepted events if this one is committed, else 0.
-// solo: the round's only event, which needs no footprint marks and no
+// K: the round's entries; a single one needs no footprint marks and no
 // acceptance.  The new calendar entries below the pool's edge go to the
 // wavefront's share of Batch::fresh and the rewritten blocks to
 // Batch::dirty[par].
@@ -2665,14 +2668,14 @@ __device__ inline GhostDraw ghost_draw(unsigned long long seed, unsigned long lo
 // is the length of its dependent chain, so the code keeps wave-uniform
 // values in scalar registers and replaces divergent branches by selects.
 __device__ __forceinline__ int run_event(const Hot& H, const Gather& G, int e, int jp, int ct, double tf, int nbin,
-                                         long long coll, int bk, bool solo, int par, int fsh) {
+                                         long long coll, int bk, int K, int par, int fsh) {
     const int lane = lane_id();
     const DevTables& T = tabs();
     Sc& mc = master();
     Batch& B = round_rec();
     OnePass& W = *reinterpret_cast<OnePass*>(smem + H.o_w);
     const double interval_max = mc.interval_max, tbin_off = mc.tbin_off, sortsize = mc.sortsize;
-    const bool batch = !solo;
+    const bool solo = K == 1, batch = !solo;
     int flags = 0, st0 = 0, nb = 0, extra_blk = -1;
     bool xdel = false;
     const int cap = H.cap, sl = min(lane, cap - 1);
@@ -3019,7 +3022,10 @@ __device__ __forceinline__ int run_event(const Hot& H, const Gather& G, int e, i
         if (lane < 16) reinterpret_cast<double*>(&W.base[jside ? 1 : 0].r)[comp] = val;
         if (lane >= 22 && lane < 26) reinterpret_cast<double*>(&W.base[(lane - 22) >> 1].bw)[lane & 1] = val;
         if (lane < 2) W.base[lane].idx = lane == 0 ? i : j;
-        if (lane < kOwners) W.tkey[lane] = ~0ull;
+        if (lane < kOwners) {
+            W.tkey[lane] = ~0ull;
+            W.win[lane] = kW;
+        }
         wave_sync();
         PH_END(sdev(), kPhRows, tph);
         // ---- every entry's bead; a down entry's own calendar entry and bond window
@@ -3037,10 +3043,20 @@ __device__ __forceinline__ int run_event(const Hot& H, const Gather& G, int e, i
         if (dn) bwm = ld_at(H.bw, m);
         // ---- down entries of one bead: its ops with i and with j, and the
         //      lane of an op of each kind (equal predictions)
-        {
-            const int key = dn ? m : -1 - lane;
+        const int rj0 = ncand + nDi, key = dn ? m : -1 - lane;
+        if (!has_x) {
+            // a row holds a bead once: only an entry of i and one of j can be
+            // of one bead.  An entry of i looks for its mate, and tells it.
+            int mate = -1;
+            for (int r = rj0; r < n0; ++r) mate = key == __builtin_amdgcn_readlane(key, r) ? r : mate;
+            const bool of_i = dn && lane < rj0, both = of_i && mate >= 0;
+            cI = of_i ? 1 : 0;
+            cJ = mate >= 0 ? 1 : 0;
+            pJ = mate >= 0 ? mate : lane;
+            const int told = __builtin_amdgcn_ds_permute((both ? mate : kLaneJ) << 2, both ? 1 : 0);
+            dups = __ballot(dn && told != 0);
+        } else {
             int r = ncand;
-            const int rj0 = ncand + nDi;
             unsigned long long above = ~((2ull << r) - 1ull);
             for (; r < rj0; ++r, above <<= 1) {
                 const bool eq = key == __builtin_amdgcn_readlane(key, r);
@@ -3084,6 +3100,9 @@ __device__ __forceinline__ int run_event(const Hot& H, const Gather& G, int e, i
             int ent2 = 0;
             if (late) ent2 = ld_at(H.nb_up, rowat);
             const unsigned long long xm = __ballot(spec && (xl.x > m || xl.y > m || xl.z > m));
+            // (a load's unused word would free its register at once, and the
+            // next value there wait for every load in flight)
+            asm volatile("" ::"v"(xl.w));
             if (xm) {
                 // shoulder partners follow their rows' order within an owner
                 // because the owner's least position wins only among equal times
@@ -3120,8 +3139,8 @@ __device__ __forceinline__ int run_event(const Hot& H, const Gather& G, int e, i
             if (late && !multi) {
                 m = ent2 & 0xFFFF;
                 stat = (ent2 >> 24) & 0x3F;
-                mine = ld_at(H.rec, m);
                 om = ld_at(H.ovr, m);
+                mine = ld_at(H.rec, m);
             }
         }
     }
@@ -3253,43 +3272,28 @@ __device__ __forceinline__ int run_event(const Hot& H, const Gather& G, int e, i
         W.wy[lane] = ty;
     }
     wave_sync();
-    const unsigned long long win = __ballot(cnd && tk == W.tkey[slot]);
+    if (cnd && tk == W.tkey[slot]) atomicMin(&W.win[slot], lane);
     PH_END(sdev(), kPhPred, tph);
-    // owner results (full recompute rule: an event only below T0)
-    double ti = T0 + tf, tj = T0 + tf;
-    int pi = -1, ci = -1, pj = -1, cj = -1;
-    auto owner_min = [&](unsigned long long seg, double& t, int& p, int& c) __attribute__((always_inline)) {
-        const unsigned long long w = win & seg;
-        if (w) {
-            const int src = __ffsll((long long)w) - 1;
-            const double bt = readlane_d(tij, src);
-            if (bt < T0) {
-                t = bt + tf;
-                p = __builtin_amdgcn_readlane(m, src);
-                c = __builtin_amdgcn_readlane(ty, src);
-            }
-        }
-    };
-    const unsigned long long tag0 = __ballot(act && tag == 0), tag1 = __ballot(act && tag == 1);
-    owner_min(tag0, ti, pi, ci);
-    owner_min(tag1, tj, pj, cj);
-    double ft = T0 + tf;  // the bead's own full recompute
+    // an owner's result, on its lane: those of i and j, and the lanes of the
+    // beads recomputed (full recompute rule: an event only below T0)
+    double ft = T0 + tf;
     int fp = -1, fc = -1;
     {
-        int q = 0;
-        for (unsigned long long sm = specm; sm; sm &= sm - 1, ++q) {
-            const int src = __ffsll((long long)sm) - 1;
-            double t = T0 + tf;
-            int p = -1, c = -1;
-            owner_min(__ballot(act && tag == 4 + q), t, p, c);
-            ft = lane == src ? t : ft;
-            fp = lane == src ? p : fp;
-            fc = lane == src ? c : fc;
+        const int rslot = lane == kLaneI || is_i ? 0 : (lane == kLaneJ ? 1 : 2 + __popcll(specm & below));
+        wave_sync();
+        const int src = own >= 0 || is_i || spec ? W.win[rslot] : kW;
+        const double bt = __shfl(tij, src & (kW - 1), kW);
+        const int bp = __shfl(m, src & (kW - 1), kW), bc = __shfl(ty, src & (kW - 1), kW);
+        if (src < kW && bt < T0) {
+            ft = bt + tf;
+            fp = bp;
+            fc = bc;
         }
     }
     // ---- each down bead's ops, those with i first
-    double st_t = is_i ? ti : lf0.tim;
-    int st_p = is_i ? pi : lf0.nptnr, st_c = is_i ? ci : leaf_ct(lf0.meta);
+    const bool whole = is_i || own >= 0;
+    double st_t = whole ? ft : lf0.tim;
+    int st_p = whole ? fp : lf0.nptnr, st_c = whole ? fc : leaf_ct(lf0.meta);
     bool modified = false;
     double sI = tij, sJ = tij;
     int yI = ty, yJ = ty;
@@ -3298,11 +3302,6 @@ __device__ __forceinline__ int run_event(const Hot& H, const Gather& G, int e, i
         yI = W.wy[pI];
         sJ = W.wt[pJ];
         yJ = W.wy[pJ];
-    }
-    if (is_i) {
-        ft = ti;
-        fp = pi;
-        fc = ci;
     }
     auto op = [&](bool on, int p, double t, int y) __attribute__((always_inline)) {
         const bool full = on && st_p == p;
@@ -3324,23 +3323,20 @@ __device__ __forceinline__ int run_event(const Hot& H, const Gather& G, int e, i
     if (has_x && __ballot(first && cJ >= 2)) {
         for (int k = 2; k <= 4; ++k) op(first && cJ >= k, j, sJ, yJ);
     }
-    // bead i's state lives in (ti, pi, ci) and is written with i's entry
+    // bead i's state, with the updates of the entry that names it among j's
+    // down set, is written by i's lane
     const unsigned long long im = __ballot(is_i);
     if (im) {
         const int src = __ffsll((long long)im) - 1;
-        ti = readlane_d(st_t, src);
-        pi = __builtin_amdgcn_readlane(st_p, src);
-        ci = __builtin_amdgcn_readlane(st_c, src);
+        const double t = readlane_d(st_t, src);
+        const int p = __builtin_amdgcn_readlane(st_p, src), y = __builtin_amdgcn_readlane(st_c, src);
+        st_t = lane == kLaneI ? t : st_t;
+        st_p = lane == kLaneI ? p : st_p;
+        st_c = lane == kLaneI ? y : st_c;
     }
     // ---- the new calendar entries, one per lane: the modified down beads',
     //      i's and j's
-    bool wr = modified && !is_i;
-    if (own >= 0) {
-        st_t = lane == kLaneI ? ti : tj;
-        st_p = lane == kLaneI ? pi : pj;
-        st_c = lane == kLaneI ? ci : cj;
-        wr = true;
-    }
+    const bool wr = (modified && !is_i) || own >= 0;
     const int rb = own >= 0 ? own : m;
     const unsigned long long stp = mk_stamp(coll, own >= 0 ? sub0 + (lane - kLaneI) : sub0 + 2 + (lane - ncand));
     Leaf lf;
@@ -3362,8 +3358,10 @@ __device__ __forceinline__ int run_event(const Hot& H, const Gather& G, int e, i
     if (batch) {
         // report the least new calendar key and the status, then commit
         // only within the round's accepted prefix
+        // (only one ahead of the round's last entry can end the prefix)
         unsigned long long kns = 0;
-        const Key kl = key_min_wave_st(kn, ks, kns);
+        Key kl = empty_key();
+        if (__ballot(key_proxy(kn) <= key_proxy(B.key[K - 1]))) kl = key_min_wave_st(kn, ks, kns);
         if (lane == 0) {
             B.knew[bk] = kl;
             B.knew_st[bk] = kns;
@@ -4760,8 +4758,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_run(const SysDev* __restrict
                 // pair events (a ghost event may lead them), one per
                 // wavefront; event k of a round is numbered and stamped as
                 // the master will count it
-                A = run_event(H, G, e, uni(key_p(k)), uni(key_ct(k)), k.t, uni(key_bin(k)), master().coll + wave, wave, K == 1,
-                              par, fsh);
+                A = run_event(H, G, e, uni(key_p(k)), uni(key_ct(k)), k.t, uni(key_bin(k)), master().coll + wave, wave, K, par, fsh);
                 if (A > 0 && lane == 0) {
                     const int ty = B.ty[wave];
                     if (ty >= 1 && ty <= 30)
