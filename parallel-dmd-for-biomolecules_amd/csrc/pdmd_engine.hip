@@ -1043,6 +1043,20 @@ template <int CTRL>
 __device__ inline unsigned ror_min(unsigned v) {
     return min(v, (unsigned)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xf, 0xf, true));
 }
+// U entries of the calendar per lane (index -1: none), all loads in flight
+// together: a branch on where the leaves are around each one waited for it
+template <int U>
+__device__ inline void leaves_ld(const Hot& H, const int (&idx)[U], Leaf (&lf)[U]) {
+    if (H.leaf_lds) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) lf[u] = reinterpret_cast<const Leaf*>(smem + H.o_leaf)[max(idx[u], 0)];
+    } else {
+#pragma unroll
+        for (int u = 0; u < U; ++u) lf[u] = ld_at(H.leaf, max(idx[u], 0));
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) lf[u].meta = idx[u] >= 0 ? lf[u].meta : 0;
+}
 // minima of the blocks in the list: one row of 16 lanes per block, 32 blocks
 // per step so that eight independent reductions overlap
 __device__ inline void rescan_listed(const Hot& H, const int* list, int nb) {
@@ -1057,13 +1071,13 @@ __device__ inline void rescan_listed(const Hot& H, const int* list, int nb) {
             bq[u] = q < nb ? list[q] : -1;
         }
         Leaf lf[8];
+        int idx[8];
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
-            const int idx = bq[u] * kBlk + (lane & 15);
-            lf[u].meta = 0;
-            lf[u].tim = 0.0;
-            if (base + 4 * u < nb && bq[u] >= 0 && idx < N3) lf[u] = leaf_ld(H, idx);
+            const int k = bq[u] * kBlk + (lane & 15);
+            idx[u] = bq[u] >= 0 && k < N3 ? k : -1;
         }
+        leaves_ld(H, idx, lf);
 #pragma unroll
         for (int u = 0; u < 8; ++u) v[u] = leaf_time(lf[u]);
 #pragma unroll
@@ -1160,22 +1174,17 @@ __device__ inline void collect_pool(const Hot& H, int K, double t0, int want, in
         wave_sync();
         // their entries below it
         count = 0;
-        for (int base = 0; base < n && !many; base += 32) {
-            Leaf lf[8];
-            int idx[8];
+        for (int base = 0; base < n && !many; base += 16) {
+            Leaf lf[4];
+            int idx[4];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const int q = base + 4 * u + (lane >> 4);
-                idx[u] = (q < n ? list[q] : H.nblk) * kBlk + (lane & 15);
-                lf[u].meta = 0;
-                lf[u].tim = 0.0;
-                lf[u].nptnr = 0;
+            for (int u = 0; u < 4; ++u) {
+                const int q = base + 4 * u + (lane >> 4), k = (q < n ? list[q] : H.nblk) * kBlk + (lane & 15);
+                idx[u] = k < N3 ? k : -1;
             }
+            leaves_ld(H, idx, lf);
 #pragma unroll
-            for (int u = 0; u < 8; ++u)
-                if (base + 4 * u < n && idx[u] < N3) lf[u] = leaf_ld(H, idx[u]);
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
+            for (int u = 0; u < 4; ++u) {
                 if (base + 4 * u >= n) continue;
                 const Key e = leaf_key(lf[u], idx[u]);
                 const double p = key_proxy(e);
