@@ -483,6 +483,11 @@ __device__ inline unsigned long long readlane_u64(unsigned long long v, int l) {
     return (unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)v, l) |
            ((unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(v >> 32), l) << 32);
 }
+// lanes of mask before this one (without a mask of the lanes below, which
+// would stay in two registers)
+__device__ inline int before_me(unsigned long long mask) {
+    return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(mask >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0u));
+}
 // first non-zero status of the wave (0 if none); wave-uniform
 __device__ inline int wave_status(int v) {
     const unsigned long long m = __ballot(v != 0);
@@ -1097,7 +1102,7 @@ constexpr int kListMax = 512;  // blocks of a work list (one wavefront's one-pas
 // Adds the blocks 64 s + bit of mask to the list.
 __device__ inline int list_blocks(int* list, int n, int s, unsigned long long mask) {
     const int lane = lane_id();
-    if ((mask >> lane) & 1ull) list[n + __popcll(mask & ((1ull << lane) - 1ull))] = s * kSup + lane;
+    if ((mask >> lane) & 1ull) list[n + before_me(mask)] = s * kSup + lane;
     return n + __popcll(mask);
 }
 // The block minima after the entries of the blocks in Batch::dirty[par]
@@ -1157,19 +1162,23 @@ __device__ inline void collect_pool(const Hot& H, int K, double t0, int want, in
         const unsigned te = (unsigned)max(__float_as_int((float)ek.t), 0) + 2u;
         int n = 0;
         bool many = false;
-        for (int s0 = 0; s0 < H.nsup && !many; s0 += 4) {
-            unsigned v[4];
+        for (int s0 = 0; s0 < H.nsup && !many; s0 += 8) {
+            unsigned v[8], least = kNoTime;
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
+            for (int u = 0; u < 8; ++u) {
                 const int b = (s0 + u) * kSup + lane;
-                v[u] = b < H.nblk ? blk[b] : kNoTime;
+                v[u] = blk[min(b, H.nblk - 1)];
+                v[u] = b < H.nblk ? v[u] : kNoTime;
+                least = min(least, v[u]);
             }
+            if (__ballot(least < te) == 0) continue;
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
+            for (int u = 0; u < 8; ++u) {
                 const unsigned long long m = __ballot(v[u] < te);
                 if (m) n = list_blocks(list, n, s0 + u, m);
+                many = many || n > kListMax - kSup;
+                if (many) break;
             }
-            many = n > kListMax - 4 * kSup;
         }
         wave_sync();
         // their entries below it
@@ -1193,7 +1202,7 @@ __device__ inline void collect_pool(const Hot& H, int K, double t0, int want, in
                     for (int q = 0; q < K; ++q) in = in && uni(key_idx(B.key[q])) != idx[u];
                 }
                 const unsigned long long m = __ballot(in);
-                const int pos = count + __popcll(m & ((1ull << lane) - 1ull));
+                const int pos = count + before_me(m);
                 if (in && pos < kCandMax) B.cand[pos] = e;
                 count += __popcll(m);
             }
@@ -1542,7 +1551,7 @@ __device__ void reschedule_generic(const SysDev&, const DevTables&, const Lds&, 
         const int l = edj & 0xFFFF;
         const bool keep = lane < ndj && l != i;
         const unsigned long long bal = __ballot(keep);
-        const int pre = __popcll(bal & ((1ull << lane) - 1ull));
+        const int pre = before_me(bal);
         if (keep) {
             L.wm()[w + pre] = l;
             L.wx()[w + pre] = 3;
@@ -1706,7 +1715,7 @@ __device__ void reschedule_generic(const SysDev&, const DevTables&, const Lds&, 
             stamp_set(l, mk_stamp(c.coll, (j >= 0 ? 3 : 4) + q));
         }
         const unsigned long long mm = __ballot(modified);
-        const int pre = __popcll(mm & ((1ull << lane) - 1ull));
+        const int pre = before_me(mm);
         if (modified && nbl + pre < kMaxBlist) L.blist()[nbl + pre] = l / kBlk;
         nbl += __popcll(mm);
         if (nbl > kMaxBlist) nbl = kMaxBlist;
@@ -1835,7 +1844,7 @@ __device__ __noinline__ void reschedule(const SysDev&, const DevTables&, const L
         const int l = edj & 0xFFFF;
         const bool keep = lane < ndj && l != i;
         const unsigned long long bal = __ballot(keep);
-        const int pre = __popcll(bal & ((1ull << lane) - 1ull));
+        const int pre = before_me(bal);
         if (keep) {
             v_wm[dbase + d + pre] = l;
             v_wx[dbase + d + pre] = 3;
@@ -1895,7 +1904,7 @@ __device__ __noinline__ void reschedule(const SysDev&, const DevTables&, const L
     if (first && !is_i) lf0 = leaf_get(L, l);
     bool spec = first && !is_i && ((lf0.nptnr == i && cI > 0) || (lf0.nptnr == j && cJ > 0));
     const unsigned long long smask = __ballot(spec);
-    const int myslot = spec ? __popcll(smask & ((1ull << lane) - 1ull)) : -1;
+    const int myslot = spec ? before_me(smask) : -1;
     if (myslot >= kMaxSpec) spec = false;
     const int nspec = min(__popcll(smask), kMaxSpec);
     if (spec) v_spec[myslot].l = l;
@@ -2010,13 +2019,12 @@ __device__ __noinline__ void reschedule(const SysDev&, const DevTables&, const L
     //      that bead, so one per (bead, partner) serves the whole op sequence
     int sqI = -1, sqJ = -1;
     if (sing_fit) {
-        const unsigned long long below = (1ull << lane) - 1ull;
         if (wantI) {
-            sqI = npairs + __popcll(mI & below);
+            sqI = npairs + before_me(mI);
             v_wm[sqI] = lane;
         }
         if (wantJ) {
-            sqJ = npairs + nI + __popcll(mJ & below);
+            sqJ = npairs + nI + before_me(mJ);
             v_wm[sqJ] = lane | 0x100;
         }
     }
@@ -2288,7 +2296,7 @@ __device__ __noinline__ void reschedule(const SysDev&, const DevTables&, const L
         L.blist()[2] = extra_blk >= 0 ? extra_blk : i / kBlk;
     }
     const unsigned long long mm = __ballot(wr);
-    const int pre = __popcll(mm & ((1ull << lane) - 1ull));
+    const int pre = before_me(mm);
     if (wr) L.blist()[3 + pre] = l / kBlk;
     const int nbl = 3 + __popcll(mm);
     PH_END(S, kPhDown, tph);
@@ -2955,7 +2963,6 @@ __device__ __forceinline__ int run_event(const Hot& H, const Gather& G, int e, i
     }
     if (lane == 0) B.ty[bk] = ct;
 
-    const unsigned long long below = (1ull << lane) - 1ull;
     // place of i's add among this event's calendar adds (a ghost event adds
     // its own entry first); j follows, then the down set in list order
     const int sub0 = j >= 0 ? 1 : 2;
@@ -2991,7 +2998,7 @@ __device__ __forceinline__ int run_event(const Hot& H, const Gather& G, int e, i
             if (lane < nui) W.lst[lane] = eui;
             if (lane < nuj) W.lst[nui + lane] = euj | kCaJ;
             if (lane < ndi) W.lst[ncand + lane] = edi | kDnI;
-            if (keep) W.lst[ncand + ndi + __popcll(bal & below)] = edj | kDnJ;
+            if (keep) W.lst[ncand + ndi + before_me(bal)] = edj | kDnJ;
         } else {
             int w = nui;
             if (lane < nui) W.lst[lane] = eui;
@@ -3021,7 +3028,7 @@ __device__ __forceinline__ int run_event(const Hot& H, const Gather& G, int e, i
             if (j >= 0) {
                 const bool keep = lane < ndj && (edj & 0xFFFF) != i;
                 const unsigned long long bal = __ballot(keep);
-                if (keep) W.lst[w + __popcll(bal & below)] = edj | kDnJ;
+                if (keep) W.lst[w + before_me(bal)] = edj | kDnJ;
                 w += __popcll(bal);
                 lowers(xj, j, kDnJ);
             }
@@ -3140,7 +3147,7 @@ __device__ __forceinline__ int run_event(const Hot& H, const Gather& G, int e, i
             // the pair's own beads take their new states
             if (act && (m == i || m == j)) mine = W.base[m == i ? 0 : 1].r;
             if (spec) {
-                BaseRec& b = W.base[2 + __popcll(specm & below)];
+                BaseRec& b = W.base[2 + before_me(specm)];
                 b.r = mine;
                 b.bw = bwm;
                 b.idx = m;
@@ -3288,7 +3295,7 @@ __device__ __forceinline__ int run_event(const Hot& H, const Gather& G, int e, i
     double ft = T0 + tf;
     int fp = -1, fc = -1;
     {
-        const int rslot = lane == kLaneI || is_i ? 0 : (lane == kLaneJ ? 1 : 2 + __popcll(specm & below));
+        const int rslot = lane == kLaneI || is_i ? 0 : (lane == kLaneJ ? 1 : 2 + before_me(specm));
         wave_sync();
         const int src = own >= 0 || is_i || spec ? W.win[rslot] : kW;
         const double bt = __shfl(tij, src & (kW - 1), kW);
@@ -3433,7 +3440,7 @@ __device__ __forceinline__ int run_event(const Hot& H, const Gather& G, int e, i
         if (wb || gl) dirty_or(par, gl ? extra_blk : rb / kBlk);
         const bool near = key_proxy(kn) < B.edge;
         const unsigned long long nm = __ballot(near);
-        const int n = __popcll(nm), cap_f = 1 << fsh, pos = __popcll(nm & below);
+        const int n = __popcll(nm), cap_f = 1 << fsh, pos = before_me(nm);
         if (near && pos < cap_f) B.fresh[(bk << fsh) + pos] = kn;
         if (lane == 0) {
             B.nfresh[bk] = min(n, cap_f);
@@ -3578,7 +3585,6 @@ __device__ inline void list_copy(const SysDev& S, int tid, int nthr) {
 __device__ inline void list_search(const SysDev& S, const DevTables& T, int i0, int& mx, int& status) {
     const int lane = lane_id();
     const int N = S.N, M = S.M, cq = S.cq, Mq = M / cq, cap = S.cap;
-    const unsigned long long below = (1ull << lane) - 1ull;
     const int ps = i0 + lane;
     int c0 = -1, c1 = -1, q = 0;
     if (ps < N) {
@@ -3664,8 +3670,8 @@ __device__ inline void list_search(const SysDev& S, const DevTables& T, int i0, 
                     const bool take = in && (local || cut), up = jb > i;
                     const unsigned long long mu = __ballot(take && up), md = __ballot(take && !up);
                     const unsigned long long mp = __ballot(cand && fj == fi && up);
-                    const int pos = up ? __builtin_amdgcn_readlane(nu, b) + __popcll(mu & below)
-                                       : __builtin_amdgcn_readlane(nd, b) + __popcll(md & below);
+                    const int pos = up ? __builtin_amdgcn_readlane(nu, b) + before_me(mu)
+                                       : __builtin_amdgcn_readlane(nd, b) + before_me(md);
                     if (take && pos < cap) gs1((up ? S.nb_up : S.nb_dn) + ((size_t)i * cap + pos), jb | (stat << 24));
                     nu += lane == b ? __popcll(mu) : 0;
                     nd += lane == b ? __popcll(md) : 0;
@@ -3851,7 +3857,7 @@ __device__ void rebuild_lists_dense(const SysDev&, const Lds&, Sc& c) {
                 pass = !((dx > 2 && dx < M - 2) || (dy > 2 && dy < M - 2) || (dz > 2 && dz < M - 2));
             }
             const unsigned long long m = __ballot(pass);
-            if (pass) q[(qh + qn + __popcll(m & below)) & (kDenseQ - 1)] = (i << 16) | jb;
+            if (pass) q[(qh + qn + before_me(m)) & (kDenseQ - 1)] = (i << 16) | jb;
             qn += __popcll(m);
             if (qn >= kW) drain();
         }
@@ -4484,7 +4490,7 @@ __global__ __launch_bounds__(kGridT) void k_list_events(const SysDev* __restrict
 // order).  Returns the number taken, 0 if the pool is empty.
 //
 // Every lane counts the proxies below its own, so one sweep over the
-// entries (about a dozen) orders all of them; popping a round's entries one
+// entries (about a dozen, four per LDS access in flight) orders all of them; popping a round's entries one
 // by one from the min tree took 2 200 cycles each.
 __device__ __forceinline__ int select_pool(const Hot& H, int kmax, int A, int Kp, int ne, int fsh) {
     Batch& B = round_rec();
@@ -4510,32 +4516,37 @@ __device__ __forceinline__ int select_pool(const Hot& H, int kmax, int A, int Kp
         const Key now = leaf_key(leaf_ld(H, idx), idx);
         have = now.t == k.t && now.bc == k.bc && now.ip == k.ip;
     }
-    // an entry rewritten with an equal key stands in fresh and elsewhere
-    const bool isf = lane >= kCandMax && lane < kCandMax + kFreshMax;
-    unsigned long long fm = __ballot(have && isf);
-    while (fm) {
-        const int s = __ffsll((long long)fm) - 1;
-        fm &= fm - 1;
-        if (idx == __builtin_amdgcn_readlane(idx, s) && lane != s) have = have && isf && lane < s;
-    }
-    const double p = have ? pk : __hiloint2double(kInfHi, 0);
-    const unsigned long long vm = __ballot(have);
-    const int n = __popcll(vm);
+    // The proxies side by side in LDS, every lane counts those below its own.
+    // (An entry rewritten with an equal key stands in fresh and elsewhere: it
+    // shows as a shared proxy.)
+    unsigned long long vm = __ballot(have);
+    int n = __popcll(vm);
     if (n == 0) return 0;
+    double* const px = reinterpret_cast<double*>(smem + H.o_w);
+    if (have) px[before_me(vm)] = pk;
+    if (lane >= n) px[lane] = __hiloint2double(kInfHi, 0);
+    wave_sync();
     int rank = 0;
-    unsigned long long sm = vm;
-    while (sm) {
-        const int s = __ffsll((long long)sm) - 1;
-        sm &= sm - 1;
-        rank += readlane_d(p, s) < p ? 1 : 0;
+    for (int q0 = 0; q0 < n; q0 += 4) {
+        const double a = px[q0], b = px[q0 + 1], c = px[q0 + 2], d = px[q0 + 3];
+        rank += (a < pk ? 1 : 0) + (b < pk ? 1 : 0) + (c < pk ? 1 : 0) + (d < pk ? 1 : 0);
     }
     const int last = kmax < kMaxWaves ? kmax : kMaxWaves - 1;
     if (have && rank <= last) B.order[rank] = lane;
     wave_sync();
     if (__ballot(have && rank <= last && B.order[rank] != lane)) {
-        // shared proxies: the exact order
+        // shared proxies: one of each entry, in the exact order
+        const bool isf = lane >= kCandMax && lane < kCandMax + kFreshMax;
+        unsigned long long fm = __ballot(have && isf);
+        while (fm) {
+            const int s = __ffsll((long long)fm) - 1;
+            fm &= fm - 1;
+            if (idx == __builtin_amdgcn_readlane(idx, s) && lane != s) have = have && isf && lane < s;
+        }
+        vm = __ballot(have);
+        n = __popcll(vm);
         rank = 0;
-        sm = vm;
+        unsigned long long sm = vm;
         while (sm) {
             const int s = __ffsll((long long)sm) - 1;
             sm &= sm - 1;
