@@ -727,6 +727,7 @@ struct Batch {
     int gbead;            // the bead of a ghost event leading the round
     long long t0;         // start of a budgeted launch (wall_clock64)
     Leaf pseudo[3];       // the ghost, sync and output entries across a list rebuild
+    int share[3];         // taken so far of a list rebuild's search, sort and events
 };
 // Order proxy of a calendar key: a positive double with the bin in its
 // exponent field (bins 1 to kNumbin = 2000 of 2046 values) and the top 52
@@ -3572,119 +3573,224 @@ __device__ inline void list_copy(const SysDev& S, int tid, int nthr) {
         gst(S.sinfo + (p), make_int4(k, b.topo, gl1(&S.cfp[k].x), 0));
     }
 }
-// The lists of the coarse cells whose first sorted bead lies in the 64 places
-// from i0 on (one wavefront): rows, their lengths, and each bead's place in
-// its fine cell's list as cell_add.f builds it (head first: the highest index
-// at 1) with the up-row length in cfp.  mx: longest row met.
-// A cell's candidates (the beads of the up to 27 cells around it) are loaded
-// once, one per lane, and tested against each of the cell's beads in turn:
-// lanes stay full, rows are written by ballot, and only the next cell's loads
-// are a dependent chain.  One lane per bead, each with its own cell ranges,
-// waited for the longest range among 64 scattered beads at every step (178 K
-// cycles per 64 beads at 6144 beads).
-__device__ inline void list_search(const SysDev& S, const DevTables& T, int i0, int& mx, int& status) {
+// The next `step` items of a list rebuild's step k for this wavefront.  Five
+// wavefronts stand on four SIMDs, where two share one: even shares let the
+// three others wait for them.
+__device__ inline int next_share(int k, int step) {
+    int v = 0;
+    if (lane_id() == 0) v = atomicAdd(&round_rec().share[k], step);
+    return uni(v);
+}
+// A wavefront's scratch of list_search: a window of candidates, the queue of
+// pairs (bead of the cell << 16 | place in the window) and, per bead of the
+// cell, its up and down entries and the later beads of its fine cell.
+constexpr int kWindow = 2 * kW;  // candidates staged at a time
+struct SearchLds {
+    double x[kWindow], y[kWindow], z[kWindow];
+    int bead[kWindow], topo[kWindow], fine[kWindow];
+    int q[2 * kW];
+    int cnt[3][kW];
+};
+constexpr int kSearchStride = kScratch / 2;
+static_assert(sizeof(SearchLds) <= kSearchStride && kSearchStride % 16 == 0, "two wavefronts search in one's rebuild scratch");
+constexpr int kCells = 16;  // sorted places whose cells a wavefront takes at a time
+// The lists of the coarse cells whose first sorted bead lies in the kCells
+// places from i0 on (one wavefront): rows, their lengths, and each bead's
+// place in its fine cell's list as cell_add.f builds it (head first: the
+// highest index at 1) with the up-row length in cfp.  mx: longest row met.
+// A cell of four beads has some 35 candidates in the 27 cells around it at
+// 6144 beads, 29 of them inside the stencil.  What bounds a cell is its chain:
+// its rows' starts and beads (loaded while the cell before is searched), its
+// candidates (staged in LDS), the pairs.  A bead is first tested against 64
+// candidates by the stencil alone, a dozen instructions on packed bytes; the
+// pairs that pass are queued, and batches of 64 of them take the exact test,
+// ninety instructions on full lanes.  Testing each of a cell's beads exactly
+// against every 64 candidates, with even shares of the cells, a list update
+// (with its sort) took 412 K cycles at 512 beads, 1 820 K with 1920 at ten
+// times the density, 3 850 K at 6144, on five wavefronts; so 317 K, 1 590 K
+// and 3 680 K.
+__device__ inline void list_search(const SysDev& S, const DevTables& T, int i0, SearchLds& W, int& mx, int& status) {
     const int lane = lane_id();
-    const int N = S.N, M = S.M, cq = S.cq, Mq = M / cq, cap = S.cap;
+    const int N = uni(S.N), M = uni(S.M), cq = uni(S.cq), Mq = M / cq, cap = uni(S.cap);
+    const int4* const sinfo = sgpr_ptr(S.sinfo);
+    const double4* const spos = sgpr_ptr(S.spos);
+    const int4* const ovr = sgpr_ptr(S.ovr);
+    const int* const cstart = sgpr_ptr(S.cstart);
+    int* const nb_up = sgpr_ptr(S.nb_up);
+    int* const nb_dn = sgpr_ptr(S.nb_dn);
     const int ps = i0 + lane;
     int c0 = -1, c1 = -1, q = 0;
-    if (ps < N) {
-        const int4 si = gld(S.sinfo + (ps));
+    if (lane < kCells && ps < N) {
+        const int4 si = ld_at(sinfo, ps);
         int qx, qy, qz;
         coarse_of(si.z, cq, Mq, qx, qy, qz);
         q = qx | (qy << 10) | (qz << 20);
         const int key = qx + Mq * (qy + Mq * qz);
-        c0 = gl1(S.cstart + (key));
-        c1 = gl1(S.cstart + (key + 1));
+        c0 = ld_at(cstart, key);
+        c1 = ld_at(cstart, key + 1);
     }
     // lane t < 9: the cells of one (y, z) neighbour row, consecutive along x;
     // lane 9 + t: the one across the box's face where there is one
     const int noff = Mq > 2 ? 3 : Mq;  // distinct offsets {0, +1, -1}
     const int t9 = lane < 9 ? lane : lane - 9, oy = t9 / 3, oz = t9 - 3 * oy;
     const bool rowl = lane < 18 && oy < noff && oz < noff;
-    for (unsigned long long heads = __ballot(c0 == ps && ps < N); heads; heads &= heads - 1) {
-        const int src = __ffsll((long long)heads) - 1;
-        const int b0 = __builtin_amdgcn_readlane(c0, src), b1 = __builtin_amdgcn_readlane(c1, src);
-        const int qq = __builtin_amdgcn_readlane(q, src);
-        const int qx = qq & 1023, qy = (qq >> 10) & 1023, qz = qq >> 20;
+    // a cell's rows and first 64 beads, loaded while the cell before is searched
+    struct Cell {
+        int b0, b1, qc, r0, len;
+        int4 sb;
+        double4 bp;
+    };
+    auto fetch = [&](int src) __attribute__((always_inline)) {
+        Cell c;
+        c.b0 = __builtin_amdgcn_readlane(c0, src);
+        c.b1 = __builtin_amdgcn_readlane(c1, src);
+        c.qc = __builtin_amdgcn_readlane(q, src);
+        const int qx = c.qc & 1023, qy = (c.qc >> 10) & 1023, qz = c.qc >> 20;
         const bool wrap = Mq > 2 && (qx == 0 || qx == Mq - 1);
-        int r0 = 0, len = 0;
-        if (rowl && (lane < 9 || wrap)) {
-            const int ny = wrap1(qy + (oy == 2 ? -1 : oy), Mq), nz = wrap1(qz + (oz == 2 ? -1 : oz), Mq);
-            const int row = Mq * (ny + Mq * nz), xw = qx == 0 ? Mq - 1 : 0;
-            r0 = gl1(S.cstart + (row + (lane < 9 ? max(qx - 1, 0) : xw)));
-            len = gl1(S.cstart + (row + (lane < 9 ? min(qx + 1, Mq - 1) : xw) + 1)) - r0;
-        }
+        const int ny = wrap1(qy + (oy == 2 ? -1 : oy), Mq), nz = wrap1(qz + (oz == 2 ? -1 : oz), Mq);
+        const int row = Mq * (ny + Mq * nz), xw = qx == 0 ? Mq - 1 : 0;
+        const bool on = rowl && (lane < 9 || wrap);
+        c.r0 = ld_at(cstart, on ? row + (lane < 9 ? max(qx - 1, 0) : xw) : 0);
+        c.len = ld_at(cstart, on ? row + (lane < 9 ? min(qx + 1, Mq - 1) : xw) + 1 : 0) - c.r0;
+        const int me = min(c.b0 + lane, N - 1);
+        c.sb = ld_at(sinfo, me);
+        c.bp = ld_at(spos, me);
+        return c;
+    };
+    unsigned long long heads = __ballot(c0 == ps);
+    if (heads == 0) return;
+    Cell next = fetch(__ffsll((long long)heads) - 1);
+    while (heads) {
+        const Cell cell = next;
+        heads &= heads - 1;
+        next = fetch(heads ? __ffsll((long long)heads) - 1 : 0);
+        const int b0 = cell.b0, b1 = cell.b1, r0 = cell.r0, len = cell.len;
+        const int qx = cell.qc & 1023, qy = (cell.qc >> 10) & 1023, qz = cell.qc >> 20;
         const int incl = wave_scan(len), excl = incl - len;
         const int C = __builtin_amdgcn_readlane(incl, kW - 1);
         const unsigned long long rows = __ballot(len > 0);
+        // A fine cell relative to the cell's first, one byte per axis: from
+        // the least of the cell before on, so the window of M cells holds
+        // each residue once (the last coarse cell takes the remainder)
+        const int last = M - (Mq - 1) * cq;
+        auto rel = [&](int f, int o, int qc) {
+            const int lo = qc > 0 ? -cq : -last;
+            int d = f - o;
+            d += d < lo ? M : 0;
+            return d >= lo + M ? d - M : d;
+        };
+        auto packed = [&](int f) {
+            return rel(f & 1023, qx * cq, qx) + (rel((f >> 10) & 1023, qy * cq, qy) << 8) +
+                   (rel(f >> 20, qz * cq, qz) << 16);
+        };
         for (int bb = b0; bb < b1; bb += kW) {
             // the cell's beads, one per lane
             const int nb = min(b1 - bb, kW);
-            int4 sb = make_int4(0, 0, 0, 0), ob = make_int4(-1, -1, -1, -1);
-            double4 bp = make_double4(0.0, 0.0, 0.0, 0.0);
-            if (lane < nb) {
-                sb = gld(S.sinfo + (bb + lane));
-                bp = gld(S.spos + (bb + lane));
-                ob = gld(S.ovr + (sb.x));
+            int4 sb = cell.sb;
+            double4 bp = cell.bp;
+            if (bb > b0) {
+                sb = ld_at(sinfo, min(bb + lane, N - 1));
+                bp = ld_at(spos, min(bb + lane, N - 1));
             }
-            const unsigned long long om = __ballot((ob.x & ob.y & ob.z & ob.w) != -1);
-            int nu = 0, nd = 0, place = 1;
-            for (int cb = 0; cb < C; cb += kW) {
-                const int cpos = cb + lane;
-                int at = 0;
+            const int4 ob = ld_at(ovr, sb.x);
+            const int brel = packed(sb.z);
+            W.cnt[0][lane] = W.cnt[1][lane] = W.cnt[2][lane] = 0;
+            int qh = 0, qn = 0;  // queue head and length
+            const unsigned long long om = __ballot(lane < nb && (ob.x & ob.y & ob.z & ob.w) != -1);
+            // the exact test of the next min(qn, 64) queued pairs
+            auto drain = [&]() {
+                wave_sync();
+                const bool v = lane < min(qn, kW);
+                const int e = v ? W.q[(qh + lane) & (2 * kW - 1)] : 0, b = e >> 16, at = e & 0xFFFF;
+                const double xj = W.x[at], yj = W.y[at], zj = W.z[at];
+                const int jb = W.bead[at], tj = W.topo[at], fj = W.fine[at];
+                const int i = __shfl(sb.x, b, kW), ti = __shfl(sb.y, b, kW), fi = __shfl(sb.z, b, kW);
+                const double xi = __shfl(bp.x, b, kW), yi = __shfl(bp.y, b, kW), zi = __shfl(bp.z, b, kW);
+                // fine cells lie in [0, M): differences in (-M, M), taken mod M
+                int dx = (fj & 1023) - (fi & 1023), dy = ((fj >> 10) & 1023) - ((fi >> 10) & 1023), dz = (fj >> 20) - (fi >> 20);
+                dx += dx < 0 ? M : 0;
+                dy += dy < 0 ? M : 0;
+                dz += dz < 0 ? M : 0;
+                const bool far = (dx > 2 && dx < M - 2) || (dy > 2 && dy < M - 2) || (dz > 2 && dz < M - 2);
+                const bool in = v && jb != i && !far;
+                const int stat = static_t(T, tj, ti);
+                // ev_code(j,i), nbor.f:63: j's overrides exist only towards i's
+                int code = stat;
+                if (om && __ballot(in && ((om >> b) & 1ull))) {
+                    const int ox = __shfl(ob.x, b, kW), oyv = __shfl(ob.y, b, kW);
+                    const int ozv = __shfl(ob.z, b, kW), ow = __shfl(ob.w, b, kW);
+                    if (in && ((ox >= 0 && (ox >> 8) == jb) || (oyv >= 0 && (oyv >> 8) == jb) ||
+                               (ozv >= 0 && (ozv >> 8) == jb) || (ow >= 0 && (ow >> 8) == jb)))
+                        code = dyn_code(ld_at(ovr, jb), i, stat);
+                }
+                const double rx = min_image(xi - xj), ry = min_image(yi - yj), rz = min_image(zi - zj);
+                const double r2 = rx * rx + ry * ry + rz * rz;
+                const bool local = (code >= 4 && code <= 12) || (code >= 17 && code < 27);
+                const bool cut = code >= 1 && code <= 50 && r2 <= T.rlsq[min((unsigned)code, 50u)];
+                const bool up = jb > i;
+                if (in && (local || cut)) {
+                    const int pos = atomicAdd(&W.cnt[up ? 0 : 1][b], 1);
+                    if (pos < cap) gs1((up ? nb_up : nb_dn) + (i * cap + pos), jb | (stat << 24));
+                }
+                if (in && up && fj == fi) atomicAdd(&W.cnt[2][b], 1);
+                qh += min(qn, kW);
+                qn -= min(qn, kW);
+            };
+            for (int w0 = 0; w0 < C; w0 += kWindow) {
+                // stage the window's candidates
+                const int wn = min(C - w0, kWindow);
+                int p0 = 0, p1 = 0;
                 for (unsigned long long rm = rows; rm; rm &= rm - 1) {
                     const int t = __ffsll((long long)rm) - 1;
-                    const int ex = __builtin_amdgcn_readlane(excl, t), st = __builtin_amdgcn_readlane(r0, t);
-                    at = cpos >= ex ? st + (cpos - ex) : at;
+                    const int ex = __builtin_amdgcn_readlane(excl, t) - w0, st = __builtin_amdgcn_readlane(r0, t) - ex;
+                    p0 = lane >= ex ? st + lane : p0;
+                    p1 = lane + kW >= ex ? st + lane + kW : p1;
                 }
-                const bool cand = cpos < C;
-                at = cand ? at : 0;
-                const int4 inf = gld(S.sinfo + (at));
-                const double4 pj = gld(S.spos + (at));
-                const int jb = inf.x, fj = inf.z;
-                for (int b = 0; b < nb; ++b) {
-                    const int i = __builtin_amdgcn_readlane(sb.x, b), fi = __builtin_amdgcn_readlane(sb.z, b);
-                    const int ti = __builtin_amdgcn_readlane(sb.y, b);
-                    // fine cells lie in [0, M): differences in (-M, M), taken mod M
-                    int dx = (fj & 1023) - (fi & 1023), dy = ((fj >> 10) & 1023) - ((fi >> 10) & 1023), dz = (fj >> 20) - (fi >> 20);
-                    dx += dx < 0 ? M : 0;
-                    dy += dy < 0 ? M : 0;
-                    dz += dz < 0 ? M : 0;
-                    const bool far = (dx > 2 && dx < M - 2) || (dy > 2 && dy < M - 2) || (dz > 2 && dz < M - 2);
-                    const bool in = cand && jb != i && !far;
-                    const int stat = static_t(T, inf.y, ti);
-                    // ev_code(j,i), nbor.f:63: j's overrides exist only towards i's
-                    int code = stat;
-                    if ((om >> b) & 1ull) {
-                        const int ox = __builtin_amdgcn_readlane(ob.x, b), oyv = __builtin_amdgcn_readlane(ob.y, b);
-                        const int ozv = __builtin_amdgcn_readlane(ob.z, b), ow = __builtin_amdgcn_readlane(ob.w, b);
-                        if (in && ((ox >= 0 && (ox >> 8) == jb) || (oyv >= 0 && (oyv >> 8) == jb) ||
-                                   (ozv >= 0 && (ozv >> 8) == jb) || (ow >= 0 && (ow >> 8) == jb)))
-                            code = dyn_code(gld(S.ovr + (jb)), i, stat);
+                p0 = lane < wn ? p0 : 0;
+                p1 = lane + kW < wn ? p1 : 0;
+                const int4 i0_ = ld_at(sinfo, p0);
+                const double4 x0 = ld_at(spos, p0);
+                const int4 i1_ = ld_at(sinfo, p1);
+                const double4 x1 = ld_at(spos, p1);
+                wave_sync();
+                W.x[lane] = x0.x;
+                W.y[lane] = x0.y;
+                W.z[lane] = x0.z;
+                W.bead[lane] = i0_.x;
+                W.topo[lane] = i0_.y;
+                W.fine[lane] = i0_.z;
+                W.x[lane + kW] = x1.x;
+                W.y[lane + kW] = x1.y;
+                W.z[lane + kW] = x1.z;
+                W.bead[lane + kW] = i1_.x;
+                W.topo[lane + kW] = i1_.y;
+                W.fine[lane + kW] = i1_.z;
+                for (int h = 0; h < wn; h += kW) {
+                    const bool cand = h + lane < wn;
+                    // per byte 64 + 2 + the difference to a bead of the cell:
+                    // 64 to 68 inside the stencil
+                    const int crel = packed(h == 0 ? i0_.z : i1_.z) + 0x424242;
+                    for (int b = 0; b < nb; ++b) {
+                        const int x = (crel - __builtin_amdgcn_readlane(brel, b)) ^ 0x404040;
+                        const bool near = Mq <= 2 || ((x | (x + 0x030303)) & 0xF8F8F8) == 0;
+                        const unsigned long long m = __ballot(cand && near);
+                        if (cand && near) W.q[(qh + qn + before_me(m)) & (2 * kW - 1)] = (b << 16) | (h + lane);
+                        qn += __popcll(m);
+                        const bool end = h + kW >= wn && b == nb - 1;
+                        while (qn >= kW || (end && qn > 0)) drain();
                     }
-                    const double rx = min_image(readlane_d(bp.x, b) - pj.x), ry = min_image(readlane_d(bp.y, b) - pj.y),
-                                 rz = min_image(readlane_d(bp.z, b) - pj.z);
-                    const double r2 = rx * rx + ry * ry + rz * rz;
-                    const bool local = (code >= 4 && code <= 12) || (code >= 17 && code < 27);
-                    const bool cut = code >= 1 && code <= 50 && r2 <= T.rlsq[min((unsigned)code, 50u)];
-                    const bool take = in && (local || cut), up = jb > i;
-                    const unsigned long long mu = __ballot(take && up), md = __ballot(take && !up);
-                    const unsigned long long mp = __ballot(cand && fj == fi && up);
-                    const int pos = up ? __builtin_amdgcn_readlane(nu, b) + before_me(mu)
-                                       : __builtin_amdgcn_readlane(nd, b) + before_me(md);
-                    if (take && pos < cap) gs1((up ? S.nb_up : S.nb_dn) + ((size_t)i * cap + pos), jb | (stat << 24));
-                    nu += lane == b ? __popcll(mu) : 0;
-                    nd += lane == b ? __popcll(md) : 0;
-                    place += lane == b ? __popcll(mp) : 0;
                 }
             }
+            wave_sync();
             if (lane < nb) {
+                const int nu = W.cnt[0][lane], nd = W.cnt[1][lane];
                 if (nu > cap || nd > cap) status = kErrListCapacity;
                 mx = max(mx, max(nu, nd));
                 gs1(S.nup + (sb.x), min(nu, cap));
                 gs1(S.ndn + (sb.x), min(nd, cap));
-                gs2(S.cfp + (sb.x), make_int2(sb.z, place | (min(nu, cap) << 16)));
+                gs2(S.cfp + (sb.x), make_int2(sb.z, (1 + W.cnt[2][lane]) | (min(nu, cap) << 16)));
             }
+            wave_sync();
         }
     }
 }
@@ -3706,7 +3812,10 @@ __device__ void rebuild_lists(const SysDev&, const Lds&, Sc& c) {
     wg_sync(nw);
     PH_END(S, kPhLCopy, trl);
     int mx = 0, status = 0;
-    for (int i0 = wave * kW; i0 < S.N; i0 += nw * kW) list_search(S, T, i0, mx, status);
+    if (wave < 2 * L.nwr) {  // wavefronts with scratch
+        SearchLds& W = *reinterpret_cast<SearchLds*>(smem + L.o_pool + wave * kSearchStride);
+        for (int i0; (i0 = next_share(0, kCells)) < S.N;) list_search(S, T, i0, W, mx, status);
+    }
     PH_END(S, kPhLSearch, trl);
     status = wave_status(status);
     if (status && !c.status) c.status = status;
@@ -3956,7 +4065,9 @@ __device__ void events_all(const SysDev&, const DevTables&, const Lds&, Sc&) {
     const int tid = (int)threadIdx.x, nthr = kW * L.nw;
     const int N = S.N;
     int status = 0;
-    for (int i = tid; i < N; i += nthr) {
+    for (int i0; (i0 = next_share(2, kW)) < N;) {
+        const int i = i0 + lane_id();
+        if (i >= N) break;
         double ti;
         int pi, ci;
         bead_event(S, T, i, c.interval_max + kLt, ti, pi, ci, status);
@@ -4073,8 +4184,8 @@ __device__ inline void sort_rows(const SysDev& S, const DevTables& T, int r0) {
         wave_sync_mem();
     }
 }
-__device__ inline void sort_all_rows(const SysDev& S, const DevTables& T, int wave, int nw) {
-    for (int r0 = wave * kW; r0 < 2 * S.N; r0 += nw * kW) sort_rows(S, T, r0);
+__device__ inline void sort_all_rows(const SysDev& S, const DevTables& T, int nw) {
+    for (int r0; (r0 = next_share(1, kW)) < 2 * S.N;) sort_rows(S, T, r0);
     wg_sync(nw);
 }
 
@@ -4088,6 +4199,7 @@ __device__ void wrap_and_lists(const SysDev&, const Lds&, Sc&) {
 
     const int tid = (int)threadIdx.x, nthr = kW * L.nw;
     if (tid == 0) c.nbin = 1;
+    if (tid < 3) L.batch()->share[tid] = 0;
     if (tid < 3) L.batch()->pseudo[tid] = leaf_get(L, S.N + tid);
     for (int k = tid; k < S.N; k += nthr) {
         Rec b = gld(S.rec + (k));
@@ -4102,7 +4214,7 @@ __device__ void wrap_and_lists(const SysDev&, const Lds&, Sc&) {
         rebuild_lists_dense(S, L, c);
     else
         rebuild_lists(S, L, c);
-    sort_all_rows(S, tabs(), wave_id(), L.nw);
+    sort_all_rows(S, tabs(), L.nw);
 }
 
 // Wrap, lists and full reschedule; all wavefronts of the system take part.
@@ -4442,11 +4554,13 @@ __device__ inline const DevTables& block_tables(const SysDev& S) {
 }
 __global__ __launch_bounds__(kGridT) void k_list_search(const SysDev* __restrict__ sys, const int* ids) {
     const SysDev& S = sys[ids[blockIdx.y]];
-    if ((int)(blockIdx.x * kGridT) >= S.N) return;
+    constexpr int kPlaces = kCells * (kGridT / kW);  // of a workgroup
+    if ((int)(blockIdx.x * kPlaces) >= S.N) return;
     const DevTables& T = block_tables(S);
-    const int i0 = (int)(blockIdx.x * kGridT) + wave_id() * kW;
+    __shared__ SearchLds W[kGridT / kW];
+    const int i0 = (int)(blockIdx.x * kPlaces) + wave_id() * kCells;
     int mx = 0, status = 0;
-    if (i0 < S.N) list_search(S, T, i0, mx, status);
+    if (i0 < S.N) list_search(S, T, i0, W[wave_id()], mx, status);
     report(S, status);
     mx = wave_imax(mx);
     if (lane_id() == 0) atomicMax(&S.st->max_nb_seen, (long long)mx);
@@ -5234,12 +5348,13 @@ static int nblk_for(int n) { return (n + 3 + kBlk - 1) / kBlk; }
 
 static hipError_t list_launches(const SysDev* d_sys, const int* d_ids, int n, int max_n, int forced, hipStream_t s) {
     const unsigned beads = (unsigned)(max_n + 3 + kGridT - 1) / kGridT, rows = (unsigned)(2 * max_n + kGridT - 1) / kGridT;
+    const unsigned places = kCells * (kGridT / kW), search = ((unsigned)max_n + places - 1) / places;
     const dim3 t(kGridT), g(beads, (unsigned)n);
     hipLaunchKernelGGL(k_list_beads, g, t, 0, s, d_sys, d_ids, forced);
     hipLaunchKernelGGL(k_list_cells, g, t, 0, s, d_sys, d_ids);
     hipLaunchKernelGGL(k_list_scan, dim3(1, (unsigned)n), dim3(kScanT), 0, s, d_sys, d_ids, forced);
     hipLaunchKernelGGL(k_list_copy, g, t, 0, s, d_sys, d_ids);
-    hipLaunchKernelGGL(k_list_search, g, t, 0, s, d_sys, d_ids);
+    hipLaunchKernelGGL(k_list_search, dim3(search, (unsigned)n), t, 0, s, d_sys, d_ids);
     hipLaunchKernelGGL(k_list_sort, dim3(rows, (unsigned)n), t, 0, s, d_sys, d_ids);
     hipLaunchKernelGGL(k_list_events, g, t, 0, s, d_sys, d_ids);
     return hipGetLastError();
