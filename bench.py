@@ -482,8 +482,8 @@ def main():
             "source": "standalone dispatches on this workload (kernel_report.py under rocprofv3), "
                       "profiles/k_rebuild_uneven64_counters.md and profiles/k_predict_uneven64_counters.md",
             "unit": "GB/s of algorithmic bytes",
-            "k_rebuild_lists": profile_figure("k_rebuild_uneven64_counters.md", "lists_algorithmic_gbps"),
-            "k_rebuild_events": profile_figure("k_rebuild_uneven64_counters.md", "events_algorithmic_gbps"),
+            "k_list_beads_to_sort": profile_figure("k_rebuild_uneven64_counters.md", "lists_algorithmic_gbps"),
+            "k_list_events": profile_figure("k_rebuild_uneven64_counters.md", "events_algorithmic_gbps"),
             "k_predict_largest": profile_figure("k_predict_uneven64_counters.md", "predict_largest_algorithmic_gbps"),
             "k_predict_largest_fp64_frac": profile_figure("k_predict_uneven64_counters.md",
                                                           "predict_largest_fp64_frac"),

@@ -145,9 +145,11 @@ int pdmd_advance_budget_async(pdmd_ctx* ctx, int32_t nsys, const int32_t* sys_id
  * entries: the points where the reference's driver writes observables
  * (energy.f, radgyr.f, end2end.f) and configurations (config.f). */
 int pdmd_advance_to_output(pdmd_ctx* ctx, int32_t nsys, const int32_t* sys_ids, const int64_t* max_nevents);
-/* Wavefronts per system for the context's later advances (1 to 8; larger
- * values are lowered to what the device's LDS holds).  With W > 1 every
- * round of a system's event loop pops up to W calendar entries and runs
+/* Event wavefronts per system for the context's later advances (1 to 8; at
+ * most seven run beside the calendar wavefront, three in a launch of more
+ * systems than compute units, and no more than the device's LDS holds).
+ * With W > 1 every
+ * round of a system's event loop takes up to W calendar entries and runs
  * the pair events among them side by side, one per wavefront; the round
  * commits the prefix that the serial order would have run identically
  * (disjoint footprints, no new calendar entry ahead of a later popped one),
@@ -243,12 +245,10 @@ int pdmd_pair_codes(const pdmd_system_desc* desc, int32_t n, const int32_t* a, c
  * neighbour lists instead of energy.f's all-pairs loop. */
 int pdmd_observables(pdmd_ctx* ctx, int32_t sys_id, pdmd_obs_t* out);
 /* The same observables, for callers that cannot allocate device memory
- * (code under HIP graph capture, tight serving loops, harnesses that forbid
- * hipMalloc): no counterpart in the reference.  Identical results; nothing
- * is allocated per call -- the chain tables and results pass through one
- * fixed 33 KB device array per GPU, located at context creation, so systems
- * of at most 4096 chains (every system pdmd_system_add accepts).  Calls
- * that overlap on one GPU, from any context, race on that array. */
+ * (tight serving loops, harnesses that forbid hipMalloc): no counterpart in
+ * the reference.  Identical results; nothing is allocated per call -- the
+ * chain tables and results pass through page-locked memory that the context
+ * allocates when it is created. */
 int pdmd_observables_noalloc(pdmd_ctx* ctx, int32_t sys_id, pdmd_obs_t* out);
 
 typedef struct {

@@ -6,10 +6,11 @@
 
 namespace pdmd {
 
-// LDS bytes of one system's workgroup of nw wavefronts for a calendar of
+// LDS bytes of one system's workgroup of nw wavefronts (the calendar
+// wavefront among them) for a calendar of
 // nblk 16-entry blocks, work lists of maxw entries and leaf_cap leaves in LDS.
 size_t engine_lds_bytes(int nblk, int maxw, int leaf_cap, int nw);
-// most wavefronts per system whose work areas fit in lds_limit
+// most event wavefronts per system whose work areas fit in lds_limit
 int engine_max_waves(int max_n, int maxw, size_t lds_limit);
 // work-list capacity of the event kernels for a list capacity
 int engine_maxw(int cap);
@@ -25,8 +26,9 @@ hipError_t engine_rebuild(const SysDev* d_sys, const int* d_ids, int n, int max_
 // budget_ticks: wall_clock64 ticks after the launch's start after which
 // each system stops between rounds (0 = run to the event targets), with
 // launch_t0 a device word that takes the start (needed with a budget);
-// waves: wavefronts per system (1 to 8, lowered to what fits in lds_limit),
-// each round runs up to that many conflict-free pair events side by side
+// waves: event wavefronts per system (1 to 8; seven run at most, three in a
+// launch of more systems than compute units, fewer where lds_limit asks for
+// it), each round runs up to that many conflict-free pair events side by side
 constexpr int kStopAtOutput = 1;  // engine_run flag: stop after the next output pseudo-event
 hipError_t engine_run(const SysDev* d_sys, const int* d_ids, const long long* d_inc, int n, int max_n, int maxw,
                       size_t lds_limit, hipStream_t s, long long budget_ticks = 0, int flags = 0, int waves = 1,

@@ -1,22 +1,24 @@
 // pdmd_engine.hip -- gfx950 kernels of the PRIME20 discontinuous-MD event
-// loop.  One workgroup of W wavefronts (64 lanes each) owns one system for a
-// whole launch and commits its events in the reference's serial order.
-//   * Each round pops up to W calendar entries; the pair events among them
+// loop.  One workgroup owns one system for a whole launch and commits its
+// events in the reference's serial order, on up to seven event wavefronts (64
+// lanes each) and one calendar wavefront.
+//   * Each round takes up to W calendar entries; the pair events among them
 //     run side by side, one per wavefront, and the round commits the prefix
-//     the serial order would have run the same way (per-bead footprint marks
-//     in HBM, no new calendar key ahead of a later popped one).
+//     the serial order would have run the same way (footprint marks per bead
+//     in LDS, no new calendar key ahead of a later one of the round).
 //   * Inside an event the wavefront issues every collision-time prediction
 //     the event triggers (full recomputes of the colliding pair and of the
 //     down beads that pointed at it, single-pair updates of the down set) as
 //     one batch of 64-byte gathers, one lane per pair, FP64 in the
 //     reference's evaluation order (no contraction).
-//   * The calendar is a three-level min tree (16-entry leaf blocks, 64-block
-//     superblocks) whose block/superblock minima carry partner and type, so
-//     the next entry comes out of one LDS min-reduction; leaves live in LDS
-//     when the system fits, else in HBM.
-//   * Neighbour-list rebuilds (coarse-cell counting sort + per-bead search),
-//     free flight and displacement checks at the sync event run on all W
-//     wavefronts.
+//   * The calendar is a leaf per bead, in LDS when the system fits, else in
+//     HBM, and a time per 16 leaves in LDS.  While events run, the calendar
+//     wavefront brings those times up to date and collects the least entries,
+//     from which and from the events' new entries the next round is taken.
+//   * Neighbour-list rebuilds (coarse-cell counting sort, a wavefront per
+//     cell), free flight and displacement checks at the sync event run on all
+//     wavefronts of the system; at start-up and where an update is forced
+//     their steps are launches over the whole GPU.
 // Many systems in one launch run concurrently, one workgroup each.
 #include <hip/hip_runtime.h>
 
@@ -47,25 +49,25 @@ __device__ inline int wave_id() { return __builtin_amdgcn_readfirstlane((int)(th
 // Phase timers (device clock cycles summed into SysState::phase[k]) when
 // built with -DPDMD_PHASE_TIMERS; no code otherwise.  Phases: 0 selection,
 // 1 pair event before rescheduling, 2 reschedule loads and work list,
-// 3 reschedule predictions, 4 down-set updates, 5 leaf writes, 6 block
-// rescans, 7 sync event without rebuild, 8 list rebuild, 9 full events(),
+// 3 reschedule predictions, 4 down-set updates, 5 leaf writes,
+// 7 sync event without rebuild, 8 list rebuild, 9 full events(),
 // 10 ghost event before rescheduling, 11 reschedule rows and work list,
 // 12 reschedule down-set scan, 13 rebuild count, 14 sync count; list
-// rebuild steps: 16 cells and histogram, 17 scan, 18 scatter, 19 sorted
+// rebuild steps: 16 cells and histogram, 17 scan, 19 sorted
 // copies, 20 neighbour search; multi-wavefront rounds: 21 rounds of two or
 // more pair events, 22 entries popped in them, 23 entries committed, 24
 // footprint marks up to the first round barrier, 25 footprint checks up to
-// the second, 26 new keys up to the third, 27 the round's rescans and merge,
+// the second, 26 new keys up to the third, 27 the wait for the other wavefronts,
 // 28 rounds cut by a footprint conflict or an event that cannot speculate,
 // 29 rounds cut by the key order; round selection: 30 the pops, 31 the
-// scalar copies after them; rescheduling batches: 32 pair predictions made
+// pool collected again for them; rescheduling batches: 32 pair predictions made
 // in them, 33 their 64-lane passes (32 / (64 * 33) is their lane occupancy);
 // down-set work outside the batches: 34 single-pair updates predicted one
 // per lane, 35 full recomputes run one bead at a time, 36 events rescheduled
 // by the generic form.
-enum { kPhSelect = 0, kPhPair = 1, kPhLoads = 2, kPhPred = 3, kPhDown = 4, kPhLeaf = 5, kPhRescan = 6,
+enum { kPhSelect = 0, kPhPair = 1, kPhLoads = 2, kPhPred = 3, kPhDown = 4, kPhLeaf = 5,
        kPhSync = 7, kPhLists = 8, kPhEvents = 9, kPhGhost = 10, kPhRows = 11, kPhScan = 12, kPhNRebuild = 13,
-       kPhNSync = 14, kPhLCells = 16, kPhLScan = 17, kPhLScatter = 18, kPhLCopy = 19, kPhLSearch = 20,
+       kPhNSync = 14, kPhLCells = 16, kPhLScan = 17, kPhLCopy = 19, kPhLSearch = 20,
        kPhNRound = 21, kPhNPopped = 22, kPhNCommit = 23, kPhBMark = 24, kPhBCheck = 25, kPhBKeys = 26,
        kPhBTail = 27, kPhNCutMark = 28, kPhNCutKey = 29, kPhSelPop = 30, kPhSelCopy = 31, kPhNPred = 32,
        kPhNPredPass = 33, kPhNSingle = 34, kPhNFull = 35, kPhNGeneric = 36 };
@@ -593,22 +595,6 @@ __device__ inline Key leaf_key(const Leaf& lf, int idx) {
     k.ip = ((unsigned)idx << 16) | (unsigned)(lf.nptnr + 2);
     return k;
 }
-template <int CTRL, int RM>
-__device__ inline void key_step(Key& k) {
-    Key o;
-    o.t = dpp_d<CTRL, RM>(k.t);
-    o.bc = dpp_i<CTRL, RM>(k.bc);
-    o.ip = (unsigned)dpp_i<CTRL, RM>((int)k.ip);
-    if (key_less(o, k)) k = o;
-}
-// exact minimum over each row of 16 lanes, in the row's last lane
-__device__ __noinline__ Key key_min_rows_exact(Key k) {
-    key_step<0x111, 0xf>(k);
-    key_step<0x112, 0xf>(k);
-    key_step<0x114, 0xf>(k);
-    key_step<0x118, 0xf>(k);
-    return k;
-}
 __device__ inline Key readlane_key(const Key& k, int l) {
     Key r;
     r.t = readlane_d(k.t, l);
@@ -690,7 +676,7 @@ __device__ inline unsigned long long t_order(double t) {
 }
 
 
-// lanes of the selection: candidates from the tree, then the committed
+// lanes of the selection: the pool's candidates, then the committed
 // events' new entries, then up to 8 popped entries that were not committed
 constexpr int kCandMax = 24, kFreshMax = 32;
 // One round of a multi-wavefront system: the popped calendar entries (in
@@ -839,20 +825,6 @@ __device__ inline Key key_min_wave_st(const Key& k, unsigned long long st, unsig
     const int src = (tie & (tie - 1)) ? uni(tie_lane_st(k, st, tie)) : __ffsll((long long)tie) - 1;
     out_st = readlane_u64(st, src);
     return readlane_key(k, src);
-}
-// Minimum over each row of 16 lanes.  Returns true on the lane that holds
-// its row's minimum in k afterwards (the row's last lane when the row is
-// empty or when shared proxies need the exact scan).
-__device__ inline bool key_min_rows(Key& k) {
-    const int lane = lane_id();
-    const double p = key_proxy(k), rm = row_min(p);
-    const unsigned long long tie = __ballot(p == rm && !proxy_none(rm));
-    const unsigned rb = (unsigned)(tie >> (lane & 48)) & 0xFFFFu;
-    if (__ballot((rb & (rb - 1u)) != 0u)) {
-        k = key_min_rows_exact(k);
-        return (lane & 15) == 15;
-    }
-    return proxy_none(rm) ? (lane & 15) == 15 : p == rm;
 }
 
 // LDS views, one set per wavefront: the calendar tree, the master scalars
@@ -4605,7 +4577,7 @@ __global__ __launch_bounds__(kGridT) void k_list_events(const SysDev* __restrict
 //
 // Every lane counts the proxies below its own, so one sweep over the
 // entries (about a dozen, four per LDS access in flight) orders all of them; popping a round's entries one
-// by one from the min tree took 2 200 cycles each.
+// by one from a tree of minima took 2 200 cycles each.
 __device__ __forceinline__ int select_pool(const Hot& H, int kmax, int A, int Kp, int ne, int fsh) {
     Batch& B = round_rec();
     const int lane = lane_id(), N = H.N;
@@ -4749,8 +4721,8 @@ __device__ inline void log_event(const SysDev& S, int& log_count, long long coll
 }
 
 // The event loop: each workgroup commits events of its system until the
-// system's coll counter has advanced by inc[k].  With one wavefront per
-// workgroup each round is one event.  With W wavefronts a round pops up to
+// system's coll counter has advanced by inc[k].  With one event wavefront
+// each round is one event.  With W of them a round takes up to
 // W entries; pair events run side by side, one per wavefront, and the
 // round commits the prefix of them that the serial order would have run
 // the same way (disjoint footprints, no new entry ahead of a later one).
@@ -4879,7 +4851,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_run(const SysDev* __restrict
         A = 0;
         Kp = K;
         if (wave == ne) {
-            // the calendar wavefront: the tree after the last round's
+            // the calendar wavefront: the minima after the last round's
             // events, then the pool the next round is taken from, while
             // this round's events run
             tree_update(H, par ^ 1, list);

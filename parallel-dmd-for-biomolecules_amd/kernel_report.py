@@ -9,10 +9,11 @@ counters give achieved GB/s and the FP64 fraction per kernel.
     python parallel-dmd-for-biomolecules_amd/kernel_report.py run --chains 4 --residues 8 [--entries 30000]
 
 rebuild: the 64 systems, each advanced by --advance committed entries, then
---reps forced list updates of all of them at once (pdmd_rebuild: one
-k_rebuild_lists dispatch, the sync pseudo-event's origin shift, wrap and
-lists of nbor.f, then one k_rebuild_events dispatch, events.f over the new
-lists; one workgroup per system in each).
+--reps forced list updates of all of them at once (pdmd_rebuild: k_list_beads,
+the sync pseudo-event's origin shift and wrap; k_list_cells, k_list_scan,
+k_list_copy, k_list_search and k_list_sort, the lists of nbor.f; then
+k_list_events, events.f over the new lists; each one dispatch over all
+systems).
 predict: every listed up-pair of every system through the predictor hook
 (pdmd_predict_pairs: one k_predict dispatch per system, one lane per pair),
 --reps times.

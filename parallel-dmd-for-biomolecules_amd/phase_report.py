@@ -22,15 +22,15 @@ import pdmd  # noqa: E402
 
 # slot: (name, parent slot or None); slots 13/14, 21-23, 28-29 and 32-36 are counts
 PHASES = {
-    0: ("select", None), 30: ("select: pops", 0), 31: ("select: scalar copies", 0),
+    0: ("select", None), 30: ("select: from the pool", 0), 31: ("select: pool collected again", 0),
     1: ("pair event before rescheduling", None), 11: ("resched: list rows + work list", None),
     12: ("resched: down-set scan", None), 2: ("resched: loads", None), 3: ("resched: predictions", None),
-    4: ("resched: down-set updates", None), 5: ("resched: leaf writes", None), 6: ("block rescans", None),
+    4: ("resched: down-set updates", None), 5: ("resched: leaf writes", None),
     24: ("round: footprint marks + barrier", None), 25: ("round: footprint checks + barrier", None),
-    26: ("round: new keys + barrier", None), 27: ("round: rescans, merge, barrier", None),
+    26: ("round: new keys + barrier", None), 27: ("round: wait for the others", None),
     7: ("sync pseudo-event (no rebuild part)", None), 10: ("ghost event before rescheduling", None),
     8: ("list rebuild", None), 16: ("list: cells + histogram", 8), 17: ("list: count scan", 8),
-    18: ("list: stable scatter", 8), 19: ("list: sorted copies", 8), 20: ("list: neighbour search", 8),
+    19: ("list: sorted copies", 8), 20: ("list: neighbour search", 8),
     9: ("events() full reschedule", None),
 }
 CASES = [  # name, chains, residues per chain, density, T*

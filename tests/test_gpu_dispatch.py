@@ -3,6 +3,7 @@ import numpy as np
 import pytest
 
 import pdmd
+from oracle import Oracle
 
 pytestmark = pytest.mark.gpu
 
@@ -91,3 +92,140 @@ def test_observables_at_the_edges(chains, length, second):
     assert o.hb_ii == sum(chain_of[i] == chain_of[j] for i, j in pairs)
     assert o.hb_ij == sum(chain_of[i] != chain_of[j] for i, j in pairs)
     assert o.tred > 0.0 and abs(o.sumvel - 3.0 * n * o.tred) <= tol * o.sumvel
+
+
+def _same_log_and_state(eng, sid, orc, n):
+    g, o = eng.log_read(sid, n), orc.run(n, log_cap=n)
+    assert eng.stats(sid).status == 0 and len(g) == n
+    for f in ("i", "j", "type"):
+        bad = np.nonzero(g[f] != o[f])[0]
+        assert bad.size == 0, f"{f} differs first at event {bad[0] + 1}: gpu {g[bad[0]]} oracle {o[bad[0]]}"
+    assert np.array_equal(g["t"].view(np.int64), o["t"].view(np.int64))
+    gs, os_ = _bits(eng.download(sid)), _bits(orc.state())
+    for f in ("sv", "identity", "bptnr", "extra", "tim", "nptnr", "coltype"):
+        assert np.array_equal(gs[f], os_[f]), f
+
+
+@pytest.mark.parametrize("waves", [1, 7])
+def test_events_near_a_pass_of_64(param_dir, waves):
+    """Rows of up to 51 entries for a colliding pair, with the candidates of
+    the beads recomputed on top: events on both sides of the 62 entries that
+    one pass takes."""
+    n = 4000
+    sysd = pdmd.generate([16] * 20, density=0.4, tstar=0.3, seed=77)
+    print(f"1280 dense beads, {waves} wavefronts", flush=True)
+    eng = pdmd.Engine(waves=waves)
+    try:
+        sid = eng.add_system(sysd, seed=9)
+        eng.log_enable(sid, n)
+        eng.advance([sid], [n])
+        _same_log_and_state(eng, sid, Oracle(sysd, seed=9, param_dir=param_dir), n)
+    finally:
+        eng.close()
+
+
+def _copies(length, per_axis, density, seed):
+    """One chain copied onto a cubic lattice: every event happens per_axis**3
+    times at (nearly) one time."""
+    s = pdmd.generate([length], density=density, tstar=0.3, seed=seed)
+    x = s["sv"].reshape(-1, 6).copy()
+    p = x[:, :3]
+    for k in range(1, length):
+        p[k] = p[k] - np.round(p[k] - p[k - 1])
+    for k in range(length, 4 * length):
+        p[k] = p[k] - np.round(p[k] - p[k % length])
+    out = []
+    for cell in np.ndindex(per_axis, per_axis, per_axis):
+        y = x / per_axis
+        y[:, :3] += (np.array(cell) - (per_axis - 1) / 2) / per_axis
+        out.append(y)
+    sv = np.concatenate(out)
+    sv[:, :3] -= np.round(sv[:, :3])
+    m = per_axis ** 3
+    return dict(s, chain_len=np.full(m, length, np.int32), restype=np.tile(s["restype"], m), hp=np.tile(s["hp"], m),
+                sv=np.ascontiguousarray(sv.ravel()), boxl=per_axis * s["boxl"])
+
+
+@pytest.mark.parametrize("waves", [1, 4, 7])
+@pytest.mark.parametrize("per_axis", [2, 3, 4])
+def test_many_entries_of_one_time(param_dir, waves, per_axis):
+    """8, 27 and 64 copies of one chain: more entries of one time than the
+    selection's pool of 24 holds, whose order is that of their insertion."""
+    n = 2500
+    sysd = _copies(8, per_axis, 0.002, 5)
+    print(f"{per_axis ** 3} copies, {waves} wavefronts", flush=True)
+    eng = pdmd.Engine(waves=waves)
+    try:
+        sid = eng.add_system(sysd, seed=3, canon=False)
+        eng.log_enable(sid, n)
+        eng.advance([sid], [n])
+        orc = Oracle(sysd, seed=3, param_dir=param_dir, canon=False)
+        _same_log_and_state(eng, sid, orc, n)
+        t = eng.log_read(sid, n)["t"][:per_axis ** 3]
+        assert t.max() - t.min() < 1e-14, "the copies' first events are not of one time"
+    finally:
+        eng.close()
+
+
+def test_footprint_marks_shared_between_beads():
+    """33 600 beads: more than the LDS holds marks for, so beads share them.
+    A round may then be cut short, never wrong: seven wavefronts end where
+    one (whose rounds need no marks) ends."""
+    sysd = pdmd.generate([120] * 70, density=0.01, tstar=0.3, seed=12)
+    out = []
+    for waves in (7, 1):
+        print(f"33600 beads, {waves} wavefronts", flush=True)
+        eng = pdmd.Engine(waves=waves)
+        try:
+            sid = eng.add_system(sysd, seed=4)
+            eng.advance([sid], [3000])
+            out.append(_bits(eng.download(sid)))
+        finally:
+            eng.close()
+    for f in out[0]:
+        assert np.array_equal(out[0][f], out[1][f]), f
+
+
+@pytest.mark.parametrize("chains", [[4], [4] * 4, [5] * 12, [7, 9] * 4, [4] * 17, [16] * 16, [13] * 20])
+def test_forced_update_at_the_edges(param_dir, chains):
+    """A forced list update, whose steps are launches of 256 items each over
+    the whole GPU, at bead counts around 64, 256 and 1024: rows, calendar
+    and the events that follow are the oracle's."""
+    n = 4 * sum(chains)
+    sysd = pdmd.generate(chains, density=0.02, tstar=0.3, seed=n)
+    print(f"forced update of {n} beads", flush=True)
+    eng = pdmd.Engine(waves=4)
+    try:
+        sid = eng.add_system(sysd, seed=8)
+        eng.advance([sid], [500])
+        eng.rebuild([sid])
+        orc = Oracle(sysd, seed=8, param_dir=param_dir)
+        orc.run(500)
+        orc.rebuild()
+        up, dn = eng.lists(sid)
+        for i in range(1, n + 1):
+            assert np.array_equal(up[i - 1], orc.nb_up(i)), f"up row of bead {i}"
+            assert np.array_equal(dn[i - 1], orc.nb_dn(i)), f"down row of bead {i}"
+        eng.log_enable(sid, 1000)
+        eng.advance([sid], [1000])
+        _same_log_and_state(eng, sid, orc, 1000)
+    finally:
+        eng.close()
+
+
+def test_counters_of_a_batch():
+    """The counters and row lengths that one launch sums for a system are
+    those of the lists it returns, at bead counts around a workgroup's 1024."""
+    eng = pdmd.Engine(waves=2)
+    try:
+        ids = [eng.add_system(pdmd.generate(c, density=0.02, tstar=0.3, seed=5), seed=6)
+               for c in ([4], [16] * 15, [16] * 16, [17] * 16)]
+        eng.advance(ids, [100, 200, 300, 400])
+        for sid, want in zip(ids, (100, 200, 300, 400)):
+            st = eng.stats(sid)
+            up, dn = eng.lists(sid)
+            n = st.nbeads
+            assert st.coll == want and st.status == 0
+            assert st.avg_up == sum(r.size for r in up) / n and st.avg_dn == sum(r.size for r in dn) / n
+    finally:
+        eng.close()
