@@ -1109,7 +1109,12 @@ __device__ inline void tree_update(const Hot& H, int par, int* list) {
 // more entries than a round takes (`want`), tried again up to `tries` times.
 // Left with too many entries for the pool, it is empty (edge 0: nothing lies
 // below it).
-__device__ inline void collect_pool(const Hot& H, int K, double t0, int want, int tries, int* list) {
+// meet: the wavefront owes the round's first barrier, where the others
+// exchange footprint marks; it meets them after its first try, which takes
+// about as long as they need to get there.  With the barrier before the first
+// try they waited for the second one's end: 2 400 cycles of each round at
+// 6144 to 10 752 beads, 4 000 at 23 424, now MEET_NOW.
+__device__ inline void collect_pool(const Hot& H, int K, double t0, int want, int tries, int* list, bool meet) {
     const int lane = lane_id(), N3 = H.N + 3;
     Batch& B = round_rec();
     const Sc& c = master();
@@ -1124,6 +1129,10 @@ __device__ inline void collect_pool(const Hot& H, int K, double t0, int want, in
     int count = 0;
     double edge = 0.0;
     for (int tr = 0; tr < tries; ++tr) {
+        if (tr == 1 && meet) {
+            __syncthreads();
+            meet = false;
+        }
         Key ek;
         ek.t = t0 + w;
         const int bin = (int)min((ek.t + off) / sortsize, (double)kNumbin) + 1;
@@ -1197,6 +1206,7 @@ __device__ inline void collect_pool(const Hot& H, int K, double t0, int want, in
         B.edge = count > kCandMax ? 0.0 : edge;
     }
     wave_sync();
+    if (meet) __syncthreads();
 }
 
 // every block minimum; all wavefronts of the system take part
@@ -4670,7 +4680,7 @@ __device__ __forceinline__ int select_round(const Hot& H, Sc& c, int kmax, int A
         PH_END(sdev(), kPhSelPop, tsp);
         int* const list = reinterpret_cast<int*>(smem + H.o_w);
         tree_update(H, par, list);
-        collect_pool(H, 0, uni(c.tfalse), want, 24, list);
+        collect_pool(H, 0, uni(c.tfalse), want, 24, list, false);
         if (lane < kMaxWaves) B.nfresh[lane] = 0;
         if (lane == 0) B.full = 0;
         wave_sync();
@@ -4855,8 +4865,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_run(const SysDev* __restrict
             // events, then the pool the next round is taken from, while
             // this round's events run
             tree_update(H, par ^ 1, list);
-            if (K > 1) __syncthreads();
-            collect_pool(H, K, uni(B.key[K - 1].t), want, 2, list);
+            collect_pool(H, K, uni(B.key[K - 1].t), want, 2, list, K > 1);
             __syncthreads();
         } else {
             if (lane == 0) B.nfresh[wave] = 0;
