@@ -1110,10 +1110,11 @@ __device__ inline void tree_update(const Hot& H, int par, int* list) {
 // Left with too many entries for the pool, it is empty (edge 0: nothing lies
 // below it).
 // meet: the wavefront owes the round's first barrier, where the others
-// exchange footprint marks; it meets them after its first try, which takes
-// about as long as they need to get there.  With the barrier before the first
-// try they waited for the second one's end: 2 400 cycles of each round at
-// 6144 to 10 752 beads, 4 000 at 23 424, now MEET_NOW.
+// exchange footprint marks; it meets them once it has looked over the block
+// minima, which with tree_update takes about as long as they need to get
+// there.  With the barrier before that they waited at their second one for
+// the collection's end: 1 700 cycles of each round at 6144 beads, 4 000 at
+// 23 424.
 __device__ inline void collect_pool(const Hot& H, int K, double t0, int want, int tries, int* list, bool meet) {
     const int lane = lane_id(), N3 = H.N + 3;
     Batch& B = round_rec();
@@ -1129,10 +1130,6 @@ __device__ inline void collect_pool(const Hot& H, int K, double t0, int want, in
     int count = 0;
     double edge = 0.0;
     for (int tr = 0; tr < tries; ++tr) {
-        if (tr == 1 && meet) {
-            __syncthreads();
-            meet = false;
-        }
         Key ek;
         ek.t = t0 + w;
         const int bin = (int)min((ek.t + off) / sortsize, (double)kNumbin) + 1;
@@ -1163,6 +1160,8 @@ __device__ inline void collect_pool(const Hot& H, int K, double t0, int want, in
             }
         }
         wave_sync();
+        if (meet) __syncthreads();
+        meet = false;
         // their entries below it
         count = 0;
         for (int base = 0; base < n && !many; base += 16) {
@@ -1206,7 +1205,6 @@ __device__ inline void collect_pool(const Hot& H, int K, double t0, int want, in
         B.edge = count > kCandMax ? 0.0 : edge;
     }
     wave_sync();
-    if (meet) __syncthreads();
 }
 
 // every block minimum; all wavefronts of the system take part
