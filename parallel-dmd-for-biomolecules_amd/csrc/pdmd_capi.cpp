@@ -56,7 +56,8 @@ struct DevBuf {
 
 // Page-locked host memory that kernels of one context write for the host to
 // read after the stream's next synchronisation (a context has one host
-// thread).  It grows to the largest request: a state of 65 533 beads, the
+// thread).  64 KB at first, which holds what the observables need of the most
+// chains a system may have; it grows to the largest request: a state of 65 533 beads, the
 // most a system may have, takes 6 MB, 4096 systems' counters 7 MB.
 struct HostStage {
     void* p = nullptr;
@@ -66,7 +67,7 @@ struct HostStage {
     }
     hipError_t reserve(size_t bytes) {
         if (bytes <= n) return hipSuccess;
-        size_t want = n ? n : (size_t)1 << 20;
+        size_t want = n ? std::max(n, (size_t)1 << 20) : (size_t)1 << 16;
         while (want < bytes) want *= 2;
         if (p) (void)hipHostFree(p);
         p = nullptr;
