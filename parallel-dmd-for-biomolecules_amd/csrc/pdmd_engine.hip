@@ -2665,6 +2665,13 @@ __device__ inline GhostDraw ghost_draw(unsigned long long seed, unsigned long lo
 // runs the multi-pass form, which holds any number.  What bounds an event
 // is the length of its dependent chain, so the code keeps wave-uniform
 // values in scalar registers and replaces divergent branches by selects.
+// Measured at four wavefronts, 5000 entries of 128 / 512 beads: 45.3 / 37.1 ms
+// with the multi-pass form for every event, 29.7 / 24.8 with one pass; 27.9 /
+// 22.0 with the pair's records as wave-uniform structs, 21.8 / 17.5 spread
+// over lanes; 20.4 / 15.5 with each owner's result taken from ballots, 19.6 /
+// 14.8 with the LDS minimum of lanes.  Listing and loading the entries before
+// the outcome, to cover the loads' latency, is 2 to 6 % slower: it takes 145
+// more instructions per entry.
 __device__ __forceinline__ int run_event(const Hot& H, const Gather& G, int e, int jp, int ct, double tf, int nbin,
                                          long long coll, int bk, int K, int par, int fsh) {
     const int lane = lane_id();
@@ -3588,7 +3595,7 @@ constexpr int kCells = 16;  // sorted places whose cells a wavefront takes at a 
 // against every 64 candidates, with even shares of the cells, a list update
 // (with its sort) took 412 K cycles at 512 beads, 1 820 K with 1920 at ten
 // times the density, 3 850 K at 6144, on five wavefronts; so 317 K, 1 590 K
-// and 3 680 K.
+// and 3 680 K, and on eight 220 K at 512 beads and 2 420 K at 6144.
 __device__ inline void list_search(const SysDev& S, const DevTables& T, int i0, SearchLds& W, int& mx, int& status) {
     const int lane = lane_id();
     const int N = uni(S.N), M = uni(S.M), cq = uni(S.cq), Mq = M / cq, cap = uni(S.cap);
@@ -4738,6 +4745,10 @@ __device__ inline void log_event(const SysDev& S, int& log_count, long long coll
 // between rounds, so that one launch over systems of uneven speed ends
 // evenly; flags & kStopAtOutput stops it right after its next output
 // pseudo-event (where the reference writes observables and configurations).
+// The registers (256 per lane) allow eight wavefronts on a compute unit.  A
+// calendar wavefront that prepares the next selection while the events run,
+// instead of wavefront 0 after them: 8000 entries of 6144 beads 33.2 -> 27.5
+// ms at the step that brought it in; the whole loop 62.3 ms then, 14.3 now.
 __global__ __launch_bounds__(64 * kMaxWaves) void k_run(const SysDev* __restrict__ sys, const int* ids, const long long* inc,
                                                        int maxw, int lds_bytes, int ne, long long budget, int flags,
                                                        unsigned long long* launch_t0) {
