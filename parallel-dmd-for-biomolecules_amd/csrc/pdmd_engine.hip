@@ -2404,11 +2404,20 @@ __device__ inline double dist_rec(const Rec& a, const Rec& b, double tf) {
     geo(a, b, tf, g);
     return sqrt(g.rx * g.rx + g.ry * g.ry + g.rz * g.rz);
 }
+// An index taken from an event's H-bond partner or identities, brought into
+// the system.  A speculative event may read those while the round's first
+// event writes them: identities of before and after an H-bond formed or broke
+// order N and C bead the wrong way round, and a cleared shoulder code points
+// at a partner of -1; shoulder_idx then gives beads up to a chain's length
+// before the first.  Such an event shares a bead with the first one and is
+// discarded at the footprint check, whatever it reads; it must only read
+// inside the system.
+__device__ inline int in_system(int m, int N) { return (unsigned)m < (unsigned)N ? m : 0; }
 // a bead's record as the event sees it: the colliding pair's own from the
 // wavefront's Pair in LDS, any other from memory
 __device__ inline Rec pair_rec(int m) {
     const Pair& P = *ldsv().pair();
-    return load_rec(sdev(), P, m);
+    return load_rec(sdev(), P, in_system(m, sdev().N));
 }
 // repuls_check.f:16-81 (n = the N bead, cb = the C bead), the colliding pair
 // read from LDS; these run in few events and stay out of line, so that the
@@ -2749,7 +2758,7 @@ __device__ __forceinline__ int run_event(const Hot& H, const Gather& G, int e, i
             g.v2 = 0.0;
         }
         bool fence = false;
-        auto dyn_of = [&](int m) __attribute__((always_inline)) { return m == i ? dyni : (m == j ? dynj : uni(gl1(&H.rec[m].dyn))); };
+        auto dyn_of = [&](int m) __attribute__((always_inline)) { return m == i ? dyni : (m == j ? dynj : uni(gl1(&H.rec[in_system(m, H.N)].dyn))); };
         if (ct == 7) {
             flags |= kPairReadsSp;
             if (xi.w < 0 && xj.w < 0) {
