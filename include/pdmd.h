@@ -177,8 +177,10 @@ int pdmd_rebuild(pdmd_ctx* ctx, int32_t nsys, const int32_t* sys_ids);
  * it on.  Default off. */
 int pdmd_set_graph_launch(pdmd_ctx* ctx, int32_t on);
 /* Autotuner of the wavefronts per system: advances the listed systems by
- * probe_events entries each at 1, 2, 4 and 8 wavefronts (those that fit in
- * LDS), one launch each, and keeps the fastest for later advances.  The
+ * probe_events entries each at settings of 1, 2, 4 and 8 (the most that a
+ * launch of these systems runs, see pdmd_set_waves; a setting that runs no
+ * wider than the one before it is skipped), one launch each, and keeps the
+ * fastest for later advances.  The
  * probe entries are committed like any others (the event sequence does not
  * depend on the setting).  waves_out gets the choice, rates_out[4] (may be
  * NULL) the committed entries per second of each trial (0 if skipped). */
@@ -192,7 +194,8 @@ int pdmd_autotune_waves(pdmd_ctx* ctx, int32_t nsys, const int32_t* sys_ids, int
  * sets how many candidates each bead scans). */
 int pdmd_set_system_tuning(pdmd_ctx* ctx, int32_t sys_id, int32_t waves, int32_t cell_factor);
 /* Autotuner of both per system: advances the listed systems by
- * probe_events entries each at 1, 2, 4 and the most wavefronts that fit
+ * probe_events entries each at 1, 2, 4 and the most wavefronts that a launch
+ * of these systems runs, those that run wider than the one before
  * (one launch each, the per-system device clock timing every system
  * separately), then at cell factors 2, 3 and 4 (systems of more than 256
  * beads; smaller ones search all pairs), and keeps for each system its

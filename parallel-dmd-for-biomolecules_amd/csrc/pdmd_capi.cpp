@@ -927,14 +927,14 @@ int pdmd_autotune_waves(pdmd_ctx* ctx, int32_t nsys, const int32_t* ids, int64_t
         max_n = std::max(max_n, H->N);
         max_cap = std::max(max_cap, H->cap);
     }
-    const int top = engine_max_waves(max_n, engine_maxw(max_cap), ctx->lds_limit);
-    const int cand[4] = {1, 2, 4, 8};
+    const int top = engine_max_waves(nsys, max_n, engine_maxw(max_cap), ctx->lds_limit);
+    const int cand[4] = {1, 2, 4, 8};  // a launch lowers them to `top`
     std::vector<int64_t> nev(nsys, probe_events);
     int best = 1;
     double best_rate = -1.0;
     for (int q = 0; q < 4; ++q) {
         if (rates_out) rates_out[q] = 0.0;
-        if (cand[q] > top) continue;
+        if (q > 0 && cand[q - 1] >= top) continue;  // no wider than the trial before
         ctx->waves = cand[q];
         int e = pdmd_advance(ctx, nsys, ids, nev.data());
         if (e) return e;
@@ -977,8 +977,8 @@ int pdmd_autotune_systems(pdmd_ctx* ctx, int32_t nsys, const int32_t* ids, int64
         max_n = std::max(max_n, H->N);
         max_cap = std::max(max_cap, H->cap);
     }
-    const int top = engine_max_waves(max_n, engine_maxw(max_cap), ctx->lds_limit);
-    int cand[4] = {1, 2, 4, top > 4 ? top : 0};
+    const int top = engine_max_waves(nsys, max_n, engine_maxw(max_cap), ctx->lds_limit);
+    const int cand[4] = {1, 2, 4, std::max(top, 5)};
     std::vector<int64_t> nev(nsys, probe_events);
     std::vector<SysState> st0(nsys), st1(nsys);
     auto snap = [&](std::vector<SysState>& v) -> int {
@@ -993,7 +993,7 @@ int pdmd_autotune_systems(pdmd_ctx* ctx, int32_t nsys, const int32_t* ids, int64
     for (int q = 0; q < 4; ++q) {
         for (int k = 0; k < nsys; ++k)
             if (rates_out) rates_out[4 * k + q] = 0.0;
-        if (cand[q] == 0 || cand[q] > top) continue;
+        if (q > 0 && cand[q - 1] >= top) continue;  // no wider than the trial before
         for (int k = 0; k < nsys; ++k)
             if (int e = pdmd_set_system_tuning(ctx, ids[k], cand[q], 0)) return e;
         ctx->waves = cand[q];

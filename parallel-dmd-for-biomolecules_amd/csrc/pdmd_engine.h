@@ -10,8 +10,8 @@ namespace pdmd {
 // wavefront among them) for a calendar of
 // nblk 16-entry blocks, work lists of maxw entries and leaf_cap leaves in LDS.
 size_t engine_lds_bytes(int nblk, int maxw, int leaf_cap, int nw);
-// most event wavefronts per system whose work areas fit in lds_limit
-int engine_max_waves(int max_n, int maxw, size_t lds_limit);
+// most event wavefronts per system in a launch of n systems of up to max_n beads
+int engine_max_waves(int n, int max_n, int maxw, size_t lds_limit);
 // work-list capacity of the event kernels for a list capacity
 int engine_maxw(int cap);
 // Opt the event-loop kernels in to lds_limit bytes of LDS per workgroup.

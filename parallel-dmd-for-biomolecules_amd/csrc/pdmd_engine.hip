@@ -5369,20 +5369,23 @@ hipError_t engine_rebuild(const SysDev* d_sys, const int* d_ids, int n, int max_
 // so that a captured graph replays it faithfully)
 __global__ void k_clock_reset(unsigned long long* w) { *w = ~0ull; }
 
-hipError_t engine_run(const SysDev* d_sys, const int* d_ids, const long long* d_inc, int n, int max_n, int maxw,
-                      size_t lds_limit, hipStream_t s, long long budget_ticks, int flags, int waves,
-                      unsigned long long* launch_t0) {
-    const int nblk = nblk_for(max_n);
-    static int ncu = 0;
-    if (ncu == 0) {
+// Shape of a launch of n systems at `waves` event wavefronts each: nw
+// wavefronts with work areas (the event wavefronts and the calendar one), all
+// that are launched, LDS bytes.
+struct RunShape {
+    int nw, total;
+    size_t lds;
+};
+static RunShape run_shape(int n, int max_n, int maxw, size_t lds_limit, int waves) {
+    static const int ncu = [] {
         int dev = 0, v = 0;
-        if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess)
-            ncu = v > 0 ? v : 1;
-        else
-            ncu = 1;
-    }
-    // the event wavefronts and the calendar wavefront
-    int nw = 1 + (waves < 1 ? 1 : (waves > kMaxWaves - 1 ? kMaxWaves - 1 : waves));
+        const bool ok = hipGetDevice(&dev) == hipSuccess &&
+                        hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess;
+        return ok && v > 0 ? v : 1;
+    }();
+    const int nblk = nblk_for(max_n);
+    RunShape r;
+    r.nw = 1 + (waves < 1 ? 1 : (waves > kMaxWaves - 1 ? kMaxWaves - 1 : waves));
     // Up to one workgroup per compute unit each takes the whole LDS budget,
     // so every system keeps as many leaves in LDS as fit beside its own block
     // minima.  Beyond that, a compute unit holds eight wavefronts of the
@@ -5391,34 +5394,38 @@ hipError_t engine_run(const SysDev* d_sys, const int* d_ids, const long long* d_
     // another one's whole launch (320 systems, 2000 entries each, and their
     // states: 39.1 ms one by one, 35.1 ms).
     size_t room = lds_limit;
-    const int nw2 = std::min(nw, kMaxWaves / 2);
+    const int nw2 = std::min(r.nw, kMaxWaves / 2);
     if (n > ncu && engine_lds_bytes(nblk, maxw, 0, nw2) <= lds_limit / 2) {
         room = lds_limit / 2;
-        nw = nw2;
+        r.nw = nw2;
     }
-    while (nw > 2 && engine_lds_bytes(nblk, maxw, 0, nw) > lds_limit) --nw;
-    const size_t base = engine_lds_bytes(nblk, maxw, 0, nw);
-    size_t lds = room;
-    if (n > ncu) lds = std::min(room, base + (sizeof(Leaf) + sizeof(unsigned)) * (size_t)(max_n + 4));
-    if (lds < base) lds = base;
+    while (r.nw > 2 && engine_lds_bytes(nblk, maxw, 0, r.nw) > lds_limit) --r.nw;
+    const size_t base = engine_lds_bytes(nblk, maxw, 0, r.nw);
+    r.lds = room;
+    if (n > ncu) r.lds = std::min(room, base + (sizeof(Leaf) + sizeof(unsigned)) * (size_t)(max_n + 4));
+    if (r.lds < base) r.lds = base;
     // A workgroup alone on its compute unit takes all the wavefronts that the
     // unit holds: those beyond nw wait at the barriers, for nothing, except
     // where the whole workgroup works, above all in list updates (512 beads at
     // one event wavefront: 18.8 ms for 2500 entries without them, 17.6 with;
     // 1920 dense beads at four: 14.8 ms, 13.7).
-    const int total = n > ncu ? nw : kMaxWaves;
+    r.total = n > ncu ? r.nw : kMaxWaves;
+    return r;
+}
+hipError_t engine_run(const SysDev* d_sys, const int* d_ids, const long long* d_inc, int n, int max_n, int maxw,
+                      size_t lds_limit, hipStream_t s, long long budget_ticks, int flags, int waves,
+                      unsigned long long* launch_t0) {
+    const RunShape r = run_shape(n, max_n, maxw, lds_limit, waves);
     if (budget_ticks > 0) {
         if (!launch_t0) return hipErrorInvalidValue;
         hipLaunchKernelGGL(k_clock_reset, dim3(1), dim3(1), 0, s, launch_t0);
     }
-    hipLaunchKernelGGL(k_run, dim3(n), dim3(kW * total), lds, s, d_sys, d_ids, d_inc, maxw, (int)lds, nw - 1, budget_ticks, flags,
-                       launch_t0);
+    hipLaunchKernelGGL(k_run, dim3(n), dim3(kW * r.total), r.lds, s, d_sys, d_ids, d_inc, maxw, (int)r.lds, r.nw - 1,
+                       budget_ticks, flags, launch_t0);
     return hipGetLastError();
 }
-int engine_max_waves(int max_n, int maxw, size_t lds_limit) {
-    int nw = kMaxWaves;
-    while (nw > 2 && engine_lds_bytes(nblk_for(max_n), maxw, 0, nw) > lds_limit) --nw;
-    return nw - 1;
+int engine_max_waves(int n, int max_n, int maxw, size_t lds_limit) {
+    return run_shape(n, max_n, maxw, lds_limit, kMaxWaves).nw - 1;
 }
 hipError_t engine_predict(const SysDev* d_sys, int id, int n, const int* pi, const int* pj, double* tij, int* type,
                           hipStream_t s) {

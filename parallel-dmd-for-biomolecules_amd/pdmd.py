@@ -303,7 +303,8 @@ class Engine:
 
     def autotune_waves(self, ids, probe_events=2000):
         """Pick the wavefronts per system by timing short advances of the
-        listed systems (pdmd_autotune_waves); returns (waves, {waves: rate})."""
+        listed systems at 1, 2, 4 and 8, the most that a launch of them runs
+        (pdmd_autotune_waves); returns (waves, {waves: rate})."""
         a = np.ascontiguousarray(ids, np.int32)
         w = ctypes.c_int32(0)
         rates = np.zeros(4, np.float64)
