@@ -312,7 +312,8 @@ int pdmd_server_create(pdmd_ctx* ctx, int64_t mem_budget_bytes, int64_t quantum,
 int pdmd_server_destroy(pdmd_server* srv);
 /* Queue a request (the description's arrays are copied). */
 int pdmd_server_submit(pdmd_server* srv, const pdmd_system_desc* desc, int64_t ncoll, int64_t* req_id);
-/* One scheduling step; *ncompleted = requests finished by the launch it retired. */
+/* One scheduling step; *ncompleted = requests finished by the launch it
+ * retired.  Returns at once on an empty server. */
 int pdmd_server_step(pdmd_server* srv, int32_t* ncompleted);
 int pdmd_server_pending(pdmd_server* srv, int32_t* queued, int32_t* resident, int64_t* committed);
 /* Record of a request; sv (6*nbeads) receives its final state once done. */

@@ -18,7 +18,6 @@
 #include <map>
 #include <memory>
 #include <string>
-#include <thread>
 #include <vector>
 
 #include "../../include/pdmd.h"
@@ -257,7 +256,6 @@ int pdmd_server_submit(pdmd_server* s, const pdmd_system_desc* d, int64_t ncoll,
 int pdmd_server_step(pdmd_server* s, int32_t* ncompleted) {
     if (!s) return -1;
     if (ncompleted) *ncompleted = 0;
-    const bool busy = s->inflight || !s->queue.empty();
     prepare_ahead(s);  // overlaps the launch in flight
     if (s->inflight) {
         int rc = retire(s, ncompleted);
@@ -265,13 +263,7 @@ int pdmd_server_step(pdmd_server* s, int32_t* ncompleted) {
     }
     int rc = admit(s);
     if (rc) return rc;
-    rc = launch(s);
-    // An empty server pauses: a caller that polls step() for its next arrival
-    // neither keeps a core busy nor runs out of a bounded number of polls (an
-    // idle call took 4 us without it).  The pause is well under the 1-2 ms of
-    // a small request's start-up and run.
-    if (!rc && !busy) std::this_thread::sleep_for(std::chrono::microseconds(20));
-    return rc;
+    return launch(s);
 }
 
 int pdmd_server_pending(pdmd_server* s, int32_t* queued, int32_t* resident, int64_t* committed) {

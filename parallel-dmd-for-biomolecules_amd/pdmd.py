@@ -8,6 +8,7 @@ Loading fails loudly when the library has not been built.
 """
 import ctypes
 import os
+import time
 
 import numpy as np
 
@@ -426,10 +427,17 @@ class Engine:
 
 
 class Server:
-    """Continuous-batching request loop on an Engine's context (pdmd_server_*)."""
+    """Continuous-batching request loop on an Engine's context (pdmd_server_*).
 
-    def __init__(self, engine, mem_budget_bytes, quantum, slice_ms=0.0, max_resident=0):
+    idle_pause: seconds that lie at least between two steps in a row that find
+    nothing to do, so that a loop which polls step() for its next arrival does
+    not spin; a step after other work waits less or not at all.  0: none (as
+    pdmd_server_step, which never waits on an empty server)."""
+
+    def __init__(self, engine, mem_budget_bytes, quantum, slice_ms=0.0, max_resident=0, idle_pause=20e-6):
         self.engine = engine
+        self.idle_pause = float(idle_pause)
+        self._idle = None  # when the last step returned, if it found nothing to do
         self._h = ctypes.c_void_p()
         _check(lib().pdmd_server_create(engine._ctx, int(mem_budget_bytes), int(quantum), float(slice_ms),
                                         int(max_resident), ctypes.byref(self._h)))
@@ -455,6 +463,13 @@ class Server:
     def step(self):
         n = ctypes.c_int32(0)
         _check(lib().pdmd_server_step(self._h, ctypes.byref(n)))
+        if self.idle_pause > 0.0:
+            idle = n.value == 0 and self.pending()[:2] == (0, 0)
+            if idle and self._idle is not None:
+                left = self._idle + self.idle_pause - time.perf_counter()
+                if left > 0.0:
+                    time.sleep(left)
+            self._idle = time.perf_counter() if idle else None
         return n.value
 
     def pending(self):
