@@ -673,26 +673,39 @@ int prepared_add(pdmd_ctx* ctx, PreparedSystem* ps, int32_t* sys_id) {
     if (ctx->d_sys.n < nslots) {
         DevBuf<SysDev> nb;
         HIPCHK(nb.alloc(nslots + 16));
-        if (ctx->d_sys.p) HIPCHK(hipMemcpy(nb.p, ctx->d_sys.p, sizeof(SysDev) * ctx->d_sys.n, hipMemcpyDeviceToDevice));
+        if (ctx->d_sys.p) {
+            HIPCHK(hipMemcpyAsync(nb.p, ctx->d_sys.p, sizeof(SysDev) * ctx->d_sys.n, hipMemcpyDeviceToDevice, ctx->stream));
+            HIPCHK(hipStreamSynchronize(ctx->stream));
+        }
         std::swap(ctx->d_sys.p, nb.p);
         std::swap(ctx->d_sys.n, nb.n);
     }
-    HIPCHK(hipMemcpy(ctx->d_sys.p + id, &H.dev, sizeof(SysDev), hipMemcpyHostToDevice));
     // device start-up: lists, pseudo-event seeds, events()
     if (ctx->d_ids.n < 1) HIPCHK(ctx->d_ids.alloc(4096));
     if (ctx->d_inc.n < 1) HIPCHK(ctx->d_inc.alloc(4096));
-    HIPCHK(hipMemcpy(ctx->d_ids.p, &id, sizeof(int), hipMemcpyHostToDevice));
+    // room for this system's state now, not in the first read (0.16 ms at
+    // 23 424 beads and 0.39 at 65 408 in a program's first read, 1.1 and 2.7 ms
+    // with the allocation in it); a failure is the read's to report
+    if (ctx->stage.reserve(StateLayout(N).bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        HIPCHK(ctx->stage.reserve(4096));
+    }
+    // Descriptor, slot and status through page-locked memory, in stream order
+    // with the launches: as three blocking copies, with one launch more, adding
+    // and removing 16 beads took 259 us, 200 so, 128 beads 266 and 221
+    constexpr size_t kDesc = 256;
+    static_assert(kDesc + sizeof(SysDev) <= 4096, "in the stage's first page");
+    int* const slot = ctx->stage.at<int>(0);
+    SysDev* const desc = ctx->stage.at<SysDev>(kDesc);
+    *slot = id;
+    *desc = H.dev;
+    HIPCHK(hipMemcpyAsync(ctx->d_sys.p + id, desc, sizeof(SysDev), hipMemcpyHostToDevice, ctx->stream));
+    HIPCHK(hipMemcpyAsync(ctx->d_ids.p, slot, sizeof(int), hipMemcpyHostToDevice, ctx->stream));
     HIPCHK(engine_setup(ctx->d_sys.p, ctx->d_ids.p, 1, N, ctx->stream));
-    // room for this system's state while the start-up runs, not in the first
-    // read (0.16 ms at 23 424 beads and 0.39 at 65 408 in a program's first
-    // read, 1.1 and 2.7 ms with the allocation in it); a failure is the
-    // read's to report
-    if (ctx->stage.reserve(StateLayout(N).bytes) != hipSuccess) (void)hipGetLastError();
+    HIPCHK(engine_status(ctx->d_sys.p, ctx->d_ids.p, 1, ctx->stage.at<int>(64), ctx->stream));
     HIPCHK(hipStreamSynchronize(ctx->stream));
-    SysState chk;
-    HIPCHK(hipMemcpy(&chk, H.st.p, sizeof chk, hipMemcpyDeviceToHost));
-    if (chk.status)
-        return fail("pdmd_system_add: device start-up failed with status " + std::to_string(chk.status), -4);
+    if (const int status = *ctx->stage.at<int>(64))
+        return fail("pdmd_system_add: device start-up failed with status " + std::to_string(status), -4);
     if ((size_t)id == ctx->sys.size()) ctx->sys.emplace_back();
     ctx->sys[id] = std::move(pp.hs);
     *sys_id = id + 1;

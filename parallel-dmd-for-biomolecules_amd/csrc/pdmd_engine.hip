@@ -3499,20 +3499,21 @@ __device__ inline void coarse_of(int f, int cq, int Mq, int& qx, int& qy, int& q
     qy = min(((f >> 10) & 1023) / cq, Mq - 1);
     qz = min((f >> 20) / cq, Mq - 1);
 }
-// beads [tid, N) by nthr: fine cell (cfp), coarse cell and place in it
+// bead k: fine cell (cfp), coarse cell and place in it
+__device__ inline void list_cell(const SysDev& S, int Mq, int k, const Rec& b) {
+    const int f = fine_cell(S, b.x, b.y, b.z);
+    int qx, qy, qz;
+    coarse_of(f, S.cq, Mq, qx, qy, qz);
+    const int key = qx + Mq * (qy + Mq * qz);
+    gs1(&S.cfp[k].x, f);
+    gs1(S.ckey + (k), key);
+    gs1(S.crank + (k), atomicAdd(&S.ccnt[key], 1));
+}
+// the same for beads [tid, N) by nthr
 __device__ inline void list_cells(const SysDev& S, int tid, int nthr) {
-    const int N = S.N, cq = S.cq, Mq = S.M / cq;
+    const int N = S.N, Mq = S.M / S.cq;
 #pragma unroll 2
-    for (int k = tid; k < N; k += nthr) {
-        const Rec b = gld(S.rec + (k));
-        const int f = fine_cell(S, b.x, b.y, b.z);
-        int qx, qy, qz;
-        coarse_of(f, cq, Mq, qx, qy, qz);
-        const int key = qx + Mq * (qy + Mq * qz);
-        gs1(&S.cfp[k].x, f);
-        gs1(S.ckey + (k), key);
-        gs1(S.crank + (k), atomicAdd(&S.ccnt[key], 1));
-    }
+    for (int k = tid; k < N; k += nthr) list_cell(S, Mq, k, gld(S.rec + (k)));
 }
 // wave-inclusive sum
 __device__ inline int wave_scan(int v) {
@@ -4471,7 +4472,7 @@ __device__ inline void report(const SysDev& S, int status) {
     if (status && lane_id() == 0) atomicCAS(&S.st->status, 0, status);  // the first error stays
 }
 // Beads to the new time origin (forced: advanced by the free flight) and
-// into the box; the pseudo-events' entries seeded, or shifted.
+// into the box, and their cells (a launch of their own is 4 us more); the pseudo-events' entries seeded, or shifted.
 __global__ __launch_bounds__(kGridT) void k_list_beads(const SysDev* __restrict__ sys, const int* ids, int forced) {
     const SysDev& S = sys[ids[blockIdx.y]];
     const int gid = (int)(blockIdx.x * kGridT + threadIdx.x), N = S.N;
@@ -4488,6 +4489,7 @@ __global__ __launch_bounds__(kGridT) void k_list_beads(const SysDev* __restrict_
         b.z = b.z - round(b.z);
         gst(S.rec + (gid), b);
         gst(S.old_r + (gid), make_double4(b.x, b.y, b.z, 0.0));
+        list_cell(S, S.M / S.cq, gid, b);
     } else if (gid < N + 3) {
         Leaf g;
         if (forced) {
@@ -4513,9 +4515,6 @@ __global__ __launch_bounds__(kGridT) void k_list_beads(const SysDev* __restrict_
         }
         gst(S.leaf + (gid), g);
     }
-}
-__global__ __launch_bounds__(kGridT) void k_list_cells(const SysDev* __restrict__ sys, const int* ids) {
-    list_cells(sys[ids[blockIdx.y]], (int)(blockIdx.x * kGridT + threadIdx.x), (int)(gridDim.x * kGridT));
 }
 // the cells' starts (one workgroup per system); the scalars of a forced update
 constexpr int kScanT = 1024;
@@ -5351,7 +5350,6 @@ static hipError_t list_launches(const SysDev* d_sys, const int* d_ids, int n, in
     const unsigned places = kCells * (kGridT / kW), search = ((unsigned)max_n + places - 1) / places;
     const dim3 t(kGridT), g(beads, (unsigned)n);
     hipLaunchKernelGGL(k_list_beads, g, t, 0, s, d_sys, d_ids, forced);
-    hipLaunchKernelGGL(k_list_cells, g, t, 0, s, d_sys, d_ids);
     hipLaunchKernelGGL(k_list_scan, dim3(1, (unsigned)n), dim3(kScanT), 0, s, d_sys, d_ids, forced);
     hipLaunchKernelGGL(k_list_copy, g, t, 0, s, d_sys, d_ids);
     hipLaunchKernelGGL(k_list_search, dim3(search, (unsigned)n), t, 0, s, d_sys, d_ids);

@@ -10,7 +10,7 @@ counters give achieved GB/s and the FP64 fraction per kernel.
 
 rebuild: the 64 systems, each advanced by --advance committed entries, then
 --reps forced list updates of all of them at once (pdmd_rebuild: k_list_beads,
-the sync pseudo-event's origin shift and wrap; k_list_cells, k_list_scan,
+the sync pseudo-event's origin shift and wrap, and the cells; k_list_scan,
 k_list_copy, k_list_search and k_list_sort, the lists of nbor.f; then
 k_list_events, events.f over the new lists; each one dispatch over all
 systems).
