@@ -54,12 +54,15 @@ struct DevBuf {
     }
 };
 
+constexpr int kMaxBeads = 65533, kMaxChains = 2047;  // of a system
+
 // Page-locked host memory that kernels of one context write for the host to
 // read after the stream's next synchronisation (a context has one host
 // thread).  64 KB at first, which holds what the observables need of the most
 // chains a system may have; it grows to the largest resident state (5.8 MB at
 // 65 533 beads, the most a system may have) when that system is added, and to
 // the largest request for counters (776 bytes per system, 3.2 MB for 4096).
+constexpr size_t kStageFirst = (size_t)1 << 16;
 struct HostStage {
     void* p = nullptr;
     size_t n = 0;
@@ -69,14 +72,15 @@ struct HostStage {
     }
     hipError_t reserve(size_t bytes) {
         if (bytes > n) {
-            size_t want = n ? std::max(n, (size_t)1 << 20) : (size_t)1 << 16;
+            size_t want = n ? std::max(n, (size_t)1 << 20) : kStageFirst;
             while (want < bytes) want *= 2;
+            void* q = nullptr;
+            const hipError_t e = hipHostMalloc(&q, want, hipHostMallocDefault);
+            if (e != hipSuccess) return e;  // what there was stays
             if (p) (void)hipHostFree(p);
-            p = nullptr;
-            n = used = 0;
-            const hipError_t e = hipHostMalloc(&p, want, hipHostMallocDefault);
-            if (e != hipSuccess) return e;
+            p = q;
             n = want;
+            used = 0;
         }
         // a page's first use from the host costs 1.5 us: here, not in a read
         for (; used < bytes; used += 4096) static_cast<volatile char*>(p)[used] = 0;
@@ -251,8 +255,8 @@ int prepare_system(const Params& raw, const pdmd_system_desc* d, Prep& out) {
     H.N = N;
     H.cap = d->list_capacity > 0 ? d->list_capacity : 64;
     if (H.cap > 64) return fail("pdmd_system_add: list_capacity above 64 (one wavefront lane per list slot)");
-    if (N > 65533) return fail("pdmd_system_add: at most 65533 beads per system");
-    if (nc > 2047) return fail("pdmd_system_add: at most 2047 chains per system");
+    if (N > kMaxBeads) return fail("pdmd_system_add: at most 65533 beads per system");
+    if (nc > kMaxChains) return fail("pdmd_system_add: at most 2047 chains per system");
     for (int c = 0; c < nc; ++c)
         if (clen[c] > 128) return fail("pdmd_system_add: at most 128 residues per chain");
     H.canon = d->canon ? 1 : 0;
@@ -509,7 +513,7 @@ int pdmd_ctx_create(const char* param_dir, pdmd_ctx** out) {
             ctx->lds_limit = (size_t)std::max(lds, 32768);
         }
     }
-    HIPCHK(ctx->stage.reserve(1));
+    HIPCHK(ctx->stage.reserve(kStageFirst));
     HIPCHK(ctx->d_clock.alloc(1));
     {
         int khz = 0;
@@ -686,15 +690,12 @@ int prepared_add(pdmd_ctx* ctx, PreparedSystem* ps, int32_t* sys_id) {
     // room for this system's state now, not in the first read (0.16 ms at
     // 23 424 beads and 0.39 at 65 408 in a program's first read, 1.1 and 2.7 ms
     // with the allocation in it); a failure is the read's to report
-    if (ctx->stage.reserve(StateLayout(N).bytes) != hipSuccess) {
-        (void)hipGetLastError();
-        HIPCHK(ctx->stage.reserve(4096));
-    }
+    if (ctx->stage.reserve(StateLayout(N).bytes) != hipSuccess) (void)hipGetLastError();
     // Descriptor, slot and status through page-locked memory, in stream order
     // with the launches: as three blocking copies, with one launch more, adding
     // and removing 16 beads took 259 us, 200 so, 128 beads 266 and 221
     constexpr size_t kDesc = 256;
-    static_assert(kDesc + sizeof(SysDev) <= 4096, "in the stage's first page");
+    static_assert(kDesc + sizeof(SysDev) <= kStageFirst, "the stage holds it from the start");
     int* const slot = ctx->stage.at<int>(0);
     SysDev* const desc = ctx->stage.at<SysDev>(kDesc);
     *slot = id;
@@ -1248,6 +1249,7 @@ static int observe(pdmd_ctx* ctx, const HostSys& H, int32_t id, pdmd_obs_t* o) {
     while (nfirst < nch && t.species[nfirst] == t.species[0]) nfirst++;
     // the results, then the chain tables
     constexpr size_t kInts = 64, kChains = 256;
+    static_assert(kChains + 2 * sizeof(int) * kMaxChains <= kStageFirst, "nothing is allocated per call");
     const size_t row = sizeof(int) * (size_t)nch;
     HIPCHK(ctx->stage.reserve(kChains + 2 * row));
     double* d = ctx->stage.at<double>(0);
