@@ -6,10 +6,11 @@
 
 namespace pdmd {
 
-// LDS bytes of one system's workgroup of nw wavefronts (the calendar
-// wavefront among them) for a calendar of
-// nblk 16-entry blocks, work lists of maxw entries and leaf_cap leaves in LDS.
-size_t engine_lds_bytes(int nblk, int maxw, int leaf_cap, int nw);
+// LDS bytes of one system's workgroup of nw wavefronts with work areas (the
+// calendar wavefront among them) for a calendar of nblk 16-entry blocks and
+// work lists of maxw entries, before its leaves; at least one wavefront's
+// list rebuild scratch.
+size_t engine_lds_bytes(int nblk, int maxw, int nw);
 // most event wavefronts per system in a launch of n systems of up to max_n beads
 int engine_max_waves(int n, int max_n, int maxw, size_t lds_limit);
 // work-list capacity of the event kernels for a list capacity

@@ -626,6 +626,8 @@ __device__ inline int calc_bin(const Sc& c, double tim, bool uncond, int& status
     return j < c.nbin ? -1 : j;
 }
 
+// the same from values (calc_bin stays apart: through this one the loop spills a
+// register more, 0.4 % of a 128-bead system's time)
 __device__ inline int bin_of(double interval_max, double tbin_off, double sortsize, int nbin, double tim, int& status) {
     if (!(tim < interval_max)) return -1;
     int j = (int)((tim + tbin_off) / sortsize) + 1;
@@ -833,13 +835,12 @@ struct Lds {
     int o_blk, o_wm, o_wx, o_blist, o_pair, o_sc, o_leaf, o_wd, o_wt, o_wy, o_slot, o_spec, o_down;
     int o_msc, o_batch, o_mark, o_one, o_pool;
     int nwr;  // wavefronts of a list rebuild that have scratch in the pool
-    Leaf* gleaf;  // calendar leaves in HBM when they do not fit in LDS
+    Leaf* leaf;  // calendar leaves in HBM when they do not fit in LDS
     unsigned mark_mask;  // footprint mark of bead b: word b & mark_mask
     int nblk, nsup, maxw, nw;
     bool leaf_lds;
     __device__ int* wm() const { return reinterpret_cast<int*>(smem + o_wm); }  // work list: partner / bead
     __device__ int* wx() const { return reinterpret_cast<int*>(smem + o_wx); }  // work list: owner / op tag
-    __device__ int* wd() const { return reinterpret_cast<int*>(smem + o_wd); }
     __device__ double* wt() const { return reinterpret_cast<double*>(smem + o_wt); }  // predicted times
     __device__ int* wy() const { return reinterpret_cast<int*>(smem + o_wy); }  // (type + 1) << 16 | partner
     __device__ int* blist() const { return reinterpret_cast<int*>(smem + o_blist); }  // blocks to rescan
@@ -892,7 +893,7 @@ __device__ inline Lds lds_regs() {
     r.o_one = __builtin_amdgcn_readfirstlane(m.o_one);
     r.o_pool = __builtin_amdgcn_readfirstlane(m.o_pool);
     r.nwr = __builtin_amdgcn_readfirstlane(m.nwr);
-    r.gleaf = sgpr_ptr(m.gleaf);
+    r.leaf = sgpr_ptr(m.leaf);
     r.nblk = __builtin_amdgcn_readfirstlane(m.nblk);
     r.nsup = __builtin_amdgcn_readfirstlane(m.nsup);
     r.maxw = __builtin_amdgcn_readfirstlane(m.maxw);
@@ -901,12 +902,11 @@ __device__ inline Lds lds_regs() {
     r.mark_mask = (unsigned)__builtin_amdgcn_readfirstlane((int)m.mark_mask);
     return r;
 }
-__device__ inline Leaf leaf_get(const Lds& L, int k) { return L.leaf_lds ? L.lleaf()[k] : gld(L.gleaf + k); }
 // a leaf another wavefront of the workgroup has just written (its HBM copy
 // read past the vector L1)
 __device__ inline Leaf leaf_get_fresh(const Lds& L, int k) {
     if (L.leaf_lds) return L.lleaf()[k];
-    unsigned long long* q = reinterpret_cast<unsigned long long*>(L.gleaf + k);
+    unsigned long long* q = reinterpret_cast<unsigned long long*>(L.leaf + k);
     const unsigned long long a = __hip_atomic_load((GLB unsigned long long*)q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const unsigned long long b = __hip_atomic_load((GLB unsigned long long*)(q + 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     Leaf r;
@@ -915,13 +915,6 @@ __device__ inline Leaf leaf_get_fresh(const Lds& L, int k) {
     r.meta = (int)(unsigned)(b >> 32);
     return r;
 }
-__device__ inline void leaf_set(const Lds& L, int k, const Leaf& v) {
-    if (L.leaf_lds)
-        L.lleaf()[k] = v;
-    else
-        gst(L.gleaf + k, v);
-}
-
 __device__ inline unsigned* lds_words(int off) { return (unsigned*)__builtin_assume_aligned(smem + off, 16); }
 // What the event loop reads of its system and of the LDS plan, as values
 // that stay in scalar registers for the whole launch.
@@ -937,7 +930,7 @@ struct Hot {
     Leaf* leaf;
     unsigned long long* stamp;
     unsigned mark_mask;
-    int N, cap, nblk, nsup, o_blk, o_leaf, o_mark, o_w, o_blist;
+    int N, cap, nblk, nsup, o_blk, o_leaf, o_mark, o_w;
     bool leaf_lds;
 };
 __device__ inline Hot load_hot(const SysDev& S, const Lds& L) {
@@ -961,7 +954,6 @@ __device__ inline Hot load_hot(const SysDev& S, const Lds& L) {
     H.o_leaf = uni(L.o_leaf);
     H.o_mark = uni(L.o_mark);
     H.o_w = uni(L.o_one);
-    H.o_blist = uni(L.o_blist);
     H.leaf_lds = uni(L.leaf_lds ? 1 : 0) != 0;
     return H;
 }
@@ -987,10 +979,13 @@ __device__ inline void st_at(T* base, int i, const T& v) {
 #pragma unroll
     for (int k = 0; k < (int)(sizeof(T) / 16); ++k) ((GLB u32x4*)q)[k] = t[k];
 }
-__device__ inline Leaf leaf_ld(const Hot& H, int k) {
+// calendar entry k, V: Lds or Hot
+template <class V>
+__device__ inline Leaf leaf_ld(const V& H, int k) {
     return H.leaf_lds ? reinterpret_cast<const Leaf*>(smem + H.o_leaf)[k] : ld_at(H.leaf, k);
 }
-__device__ inline void leaf_st(const Hot& H, int k, const Leaf& v) {
+template <class V>
+__device__ inline void leaf_st(const V& H, int k, const Leaf& v) {
     if (H.leaf_lds)
         reinterpret_cast<Leaf*>(smem + H.o_leaf)[k] = v;
     else
@@ -1071,7 +1066,7 @@ __device__ inline void rescan_listed(const Hot& H, const int* list, int nb) {
             if ((lane & 15) == 0 && bq[u] >= 0) blk[bq[u]] = v[u];
     }
 }
-constexpr int kListMax = 512;  // blocks of a work list (one wavefront's one-pass area)
+constexpr int kListMax = 512;  // blocks of a work list (one wavefront's one-pass area, OnePass)
 // Adds the blocks 64 s + bit of mask to the list.
 __device__ inline int list_blocks(int* list, int n, int s, unsigned long long mask) {
     const int lane = lane_id();
@@ -1259,14 +1254,23 @@ __device__ inline int shoulder_bead(const SysDev&, const Pair& P, int lane) {
     const int v = q == 0 ? a[0] : (q == 1 ? a[1] : (q == 2 ? a[2] : a[3]));
     return (v >= 0 && v < S.N) ? v : -1;
 }
-// Footprint marks of bead b, in LDS.  Where a word per bead does not fit, the
-// words are shared (b & mark_mask): a shared word can only end a round
-// earlier or replay an update on an entry that nobody rewrote.
-__device__ inline void mark_or(const Lds& L, int b, unsigned bits) {
-    __hip_atomic_fetch_or(lds_words(L.o_mark) + ((unsigned)b & L.mark_mask), bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+// Footprint marks of bead b, in LDS (V: Lds or Hot).  Where a word per bead
+// does not fit, the words are shared (b & mark_mask): a shared word can only
+// end a round earlier or replay an update on an entry that nobody rewrote.
+template <class V>
+__device__ inline unsigned* mark_word(const V& L, int b) {
+    return lds_words(L.o_mark) + ((unsigned)b & L.mark_mask);
 }
-__device__ inline void mark_clear(const Lds& L, int b) {
-    __hip_atomic_store(lds_words(L.o_mark) + ((unsigned)b & L.mark_mask), 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+template <class V>
+__device__ inline void mark_or(const V& L, int b, unsigned bits) {
+    __hip_atomic_fetch_or(mark_word(L, b), bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ inline unsigned mark_get(const Hot& L, int b) {
+    return __hip_atomic_load(mark_word(L, b), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+template <class V>
+__device__ inline void mark_clear(const V& L, int b) {
+    __hip_atomic_store(mark_word(L, b), 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 // A wavefront's place in a multi-wavefront round: -1 alone; 0 the round's
 // first event (always committed, writes as it goes); k >= 1 a speculative
@@ -1482,7 +1486,7 @@ __device__ void reschedule_generic(const SysDev&, const DevTables&, const Lds&, 
     Sc& c = *L.sc();
     const Pair& P = *L.pair();
 
-    const int lane = lane_id(), cap = S.cap, N3 = S.N + 3;
+    const int lane = lane_id(), cap = S.cap;
     const int i = P.i, j = P.j;
     const double tf = c.tfalse;
     const double T0 = c.interval_max + kLt - tf;
@@ -1641,7 +1645,7 @@ __device__ void reschedule_generic(const SysDev&, const DevTables&, const Lds&, 
                 st_p = pi;
                 st_c = ci;
             } else {
-                const Leaf lf = leaf_get(L, l);
+                const Leaf lf = leaf_ld(L, l);
                 st_t = lf.tim;
                 st_p = lf.nptnr;
                 st_c = leaf_ct(lf.meta);
@@ -1692,7 +1696,7 @@ __device__ void reschedule_generic(const SysDev&, const DevTables&, const Lds&, 
             lf.tim = st_t;
             lf.nptnr = st_p;
             lf.meta = make_meta(calc_bin(c, st_t, false, status), st_c);
-            leaf_set(L, l, lf);
+            leaf_st(L, l, lf);
             stamp_set(l, mk_stamp(c.coll, (j >= 0 ? 3 : 4) + q));
         }
         const unsigned long long mm = __ballot(modified);
@@ -1709,14 +1713,14 @@ __device__ void reschedule_generic(const SysDev&, const DevTables&, const Lds&, 
         a.tim = ti;
         a.nptnr = pi;
         a.meta = make_meta(calc_bin(c, ti, false, status), ci);
-        leaf_set(L, i, a);
+        leaf_st(L, i, a);
         stamp_set(i, mk_stamp(c.coll, j >= 0 ? 1 : 2));
         if (j >= 0) {
             Leaf b;
             b.tim = tj;
             b.nptnr = pj;
             b.meta = make_meta(calc_bin(c, tj, false, status), cj);
-            leaf_set(L, j, b);
+            leaf_st(L, j, b);
             stamp_set(j, mk_stamp(c.coll, 2));
         }
     }
@@ -1771,7 +1775,7 @@ __device__ __noinline__ void reschedule(const SysDev&, const DevTables&, const L
     DownInfo* const v_down = reinterpret_cast<DownInfo*>(smem + __builtin_amdgcn_readfirstlane(L.o_down));
     const int maxw = __builtin_amdgcn_readfirstlane(L.maxw);
 
-    const int lane = lane_id(), cap = S.cap, N3 = S.N + 3;
+    const int lane = lane_id(), cap = S.cap;
     const int i = P.i, j = P.j;
     const double tf = c.tfalse;
     const double T0 = c.interval_max + kLt - tf;
@@ -1882,7 +1886,7 @@ __device__ __noinline__ void reschedule(const SysDev&, const DevTables&, const L
     lf0.tim = 0.0;
     lf0.nptnr = -1;
     lf0.meta = 0;
-    if (first && !is_i) lf0 = leaf_get(L, l);
+    if (first && !is_i) lf0 = leaf_ld(L, l);
     bool spec = first && !is_i && ((lf0.nptnr == i && cI > 0) || (lf0.nptnr == j && cJ > 0));
     const unsigned long long smask = __ballot(spec);
     const int myslot = spec ? before_me(smask) : -1;
@@ -2247,7 +2251,7 @@ __device__ __noinline__ void reschedule(const SysDev&, const DevTables&, const L
                 }
             } else {
                 // a ghost event leading the round: its next ghost time
-                const Key kg = leaf_key(leaf_get(L, S.N), S.N);
+                const Key kg = leaf_key(leaf_ld(L, S.N), S.N);
                 const unsigned long long sg = mk_stamp(c.coll, 1);  // re-added by this ghost event
                 if (key_less_st(kg, sg, kn, ks)) {
                     kn = kg;
@@ -2268,7 +2272,7 @@ __device__ __noinline__ void reschedule(const SysDev&, const DevTables&, const L
         round_clear_marks(L, S, dent, i, j, sp_w ? sp : -1);
     }
     if (wr) {
-        leaf_set(L, l, lf);
+        leaf_st(L, l, lf);
         stamp_set(l, mk_stamp(c.coll, sub0 + 2 + lane));
     }
     if (lane == 0) {
@@ -2282,10 +2286,10 @@ __device__ __noinline__ void reschedule(const SysDev&, const DevTables&, const L
     const int nbl = 3 + __popcll(mm);
     PH_END(S, kPhDown, tph);
     if (lane == 0) {
-        leaf_set(L, i, la);
+        leaf_st(L, i, la);
         stamp_set(i, mk_stamp(c.coll, sub0));
         if (j >= 0) {
-            leaf_set(L, j, lb);
+            leaf_st(L, j, lb);
             stamp_set(j, mk_stamp(c.coll, sub0 + 1));
         }
     }
@@ -2535,19 +2539,10 @@ struct OnePass {
     int wy[kW];
     int lst[kW];
 };
+static_assert(sizeof(OnePass) >= sizeof(int) * kListMax, "the calendar wavefront's block list lies over its work area");
+static_assert(sizeof(OnePass) >= sizeof(double) * kW, "so do the selection's proxies over wavefront 0's");
 // result lanes of beads i and j: entries take the lanes below
 constexpr int kLaneI = kW - 2, kLaneJ = kW - 1;
-
-// footprint marks in LDS (a word per bead, or shared: mark_or)
-__device__ inline void fp_or(const Hot& H, int b, unsigned bits) {
-    __hip_atomic_fetch_or(lds_words(H.o_mark) + ((unsigned)b & H.mark_mask), bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-__device__ inline unsigned fp_get(const Hot& H, int b) {
-    return __hip_atomic_load(lds_words(H.o_mark) + ((unsigned)b & H.mark_mask), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-__device__ inline void fp_clear(const Hot& H, int b) {
-    __hip_atomic_store(lds_words(H.o_mark) + ((unsigned)b & H.mark_mask), 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
 
 // A lane's part of one gather that fetches everything an event needs of its
 // two beads, 8 bytes per lane: lanes 0-7 and 8-15 the records of i and j,
@@ -3205,9 +3200,9 @@ __device__ __forceinline__ int run_event(const Hot& H, const Gather& G, int e, i
     //      updates only, and whose own updates here are single-pair ones,
     //      replays those updates on that event's entry once it is written.
     auto clear_marks = [&]() __attribute__((always_inline)) {
-        if (dn) fp_clear(H, m);
-        if (own >= 0) fp_clear(H, own);
-        if (bk == 0 && sp_w && sp >= 0) fp_clear(H, sp);
+        if (dn) mark_clear(H, m);
+        if (own >= 0) mark_clear(H, own);
+        if (bk == 0 && sp_w && sp >= 0) mark_clear(H, sp);
     };
     if (batch) {
         const unsigned sbit = 1u << bk, lbit = 1u << (8 + bk), fbit = 1u << (16 + bk);
@@ -3216,8 +3211,8 @@ __device__ __forceinline__ int run_event(const Hot& H, const Gather& G, int e, i
             sp = shoulder_bead(sdev(), *ldsv().pair(), lane);
         }
         if (lane == 0) B.wdone[bk] = 0;
-        if (dn || own >= 0) fp_or(H, dn ? m : own, dn ? lbit | (spec ? fbit : 0u) : sbit | lbit | fbit);
-        if (bk == 0 && sp_w && sp >= 0) fp_or(H, sp, sbit);
+        if (dn || own >= 0) mark_or(H, dn ? m : own, dn ? lbit | (spec ? fbit : 0u) : sbit | lbit | fbit);
+        if (bk == 0 && sp_w && sp >= 0) mark_or(H, sp, sbit);
         bar_to(nb, 1);
         PH_END(sdev(), kPhBMark, tph);
         if (bk >= 1) {
@@ -3225,7 +3220,7 @@ __device__ __forceinline__ int run_event(const Hot& H, const Gather& G, int e, i
             const bool look = lane < ntot || own >= 0;
             bool bad = false;
             if (look) {
-                const unsigned mk = fp_get(H, own >= 0 ? own : m);
+                const unsigned mk = mark_get(H, own >= 0 ? own : m);
                 bad = (mk & lowS) != 0u;
                 if (own >= 0) bad = (mk & (lowS | lowL)) != 0u;
                 if (!bad && first && (mk & lowL)) {
@@ -3238,7 +3233,7 @@ __device__ __forceinline__ int run_event(const Hot& H, const Gather& G, int e, i
                         bad = true;
                 }
             }
-            if (sp_r && sp >= 0 && (fp_get(H, sp) & lowS)) bad = true;
+            if (sp_r && sp >= 0 && (mark_get(H, sp) & lowS)) bad = true;
             if (__ballot(bad) && lane == 0) atomicMin(&B.cut, bk);
             PH_END(sdev(), kPhBCheck, tph);
             // the cut only moves down: a wavefront already past it stops here
@@ -4072,13 +4067,13 @@ __device__ void events_all(const SysDev&, const DevTables&, const Lds&, Sc&) {
         lf.tim = ti;
         lf.nptnr = pi;
         lf.meta = make_meta(calc_bin(c, ti, false, status), ci);
-        leaf_set(L, i, lf);
+        leaf_st(L, i, lf);
         stamp_set(i, mk_stamp(c.coll, i + 1));  // events.f:111-122 adds in index order
     }
     for (int e = N + tid; e < N + 3; e += nthr) {
         Leaf lf = L.batch()->pseudo[e - N];
         lf.meta = make_meta(calc_bin(c, lf.tim, false, status), -2);
-        leaf_set(L, e, lf);
+        leaf_st(L, e, lf);
         stamp_set(e, mk_stamp(c.coll, e + 1));
     }
     status = wave_status(status);
@@ -4197,7 +4192,7 @@ __device__ void wrap_and_lists(const SysDev&, const Lds&, Sc&) {
     const int tid = (int)threadIdx.x, nthr = kW * L.nw;
     if (tid == 0) c.nbin = 1;
     if (tid < 3) L.batch()->share[tid] = 0;
-    if (tid < 3) L.batch()->pseudo[tid] = leaf_get(L, S.N + tid);
+    if (tid < 3) L.batch()->pseudo[tid] = leaf_ld(L, S.N + tid);
     for (int k = tid; k < S.N; k += nthr) {
         Rec b = gld(S.rec + (k));
         b.x = b.x - round(b.x);
@@ -4302,7 +4297,7 @@ __device__ void sync_finish(const SysDev&, const Lds&, Sc&) {
         lf.tim = t2;
         lf.nptnr = -2;
         lf.meta = make_meta(calc_bin(c, t2, true, status), -2);
-        leaf_set(L, N + 1, lf);
+        leaf_st(L, N + 1, lf);
         stamp_set(N + 1, mk_stamp(c.coll, N + 4));  // after a rebuild's events() adds
     }
     if (status && !c.status) c.status = status;
@@ -4326,7 +4321,7 @@ __device__ void output_event(const SysDev&, const Lds&, Sc&) {
         lf.tim = t3;
         lf.nptnr = -2;
         lf.meta = make_meta(calc_bin(c, t3, false, status), -2);
-        leaf_set(L, N + 2, lf);
+        leaf_st(L, N + 2, lf);
         stamp_set(N + 2, mk_stamp(c.coll, 1));
     }
     if (status && !c.status) c.status = status;
@@ -4397,7 +4392,7 @@ __device__ Lds make_lds(const SysDev&, int maxw, int lds_bytes, int ne, int nw, 
     L.o_mark = take((int)sizeof(unsigned) * nm);
     L.o_leaf = p;
     L.leaf_lds = N3 <= (lds_bytes - p) / (int)sizeof(Leaf);
-    L.gleaf = S.leaf;
+    L.leaf = S.leaf;
     const int room = (lds_bytes - kPoolOff) / kScratch;
     L.nwr = room < nw ? room : nw;
     return L;
@@ -4778,7 +4773,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_run(const SysDev* __restrict
         lds_words(L.o_mark)[b] = 0u;
     __syncthreads();
     const DevTables& T = tabs();
-    Sc& c = *L.sc();  // wavefront 0: the master scalars; others: their own copy
+    Sc& c = *L.sc();  // the master scalars
     Batch& B = *L.batch();
     if (threadIdx.x == 0) {
         load_sc(S.st, c);
@@ -5333,15 +5328,10 @@ __global__ void k_predict(const SysDev* sys, int id, int n, const int* pi, const
 int engine_maxw(int cap) { return 6 * (cap + 3); }
 
 static size_t r16(size_t b) { return (b + 15) / 16 * 16; }
-// the bytes make_lds lays out before the leaves, for nw wavefronts; at
-// least one wavefront's rebuild scratch
-static size_t lds_fixed(int nblk_max, int maxw, int nw) {
-    const size_t b = (size_t)kPoolOff + (size_t)nw * lds_wave_bytes() + lds_multi_bytes(maxw) + r16(sizeof(unsigned) * nblk_max) +
+size_t engine_lds_bytes(int nblk, int maxw, int nw) {
+    const size_t b = (size_t)kPoolOff + (size_t)nw * lds_wave_bytes() + lds_multi_bytes(maxw) + r16(sizeof(unsigned) * nblk) +
                      4096;  // the fewest footprint marks
     return std::max(b, (size_t)kPoolOff + kScratch);
-}
-size_t engine_lds_bytes(int nblk_max, int maxw, int leaf_cap, int nw) {
-    return lds_fixed(nblk_max, maxw, nw) + sizeof(Leaf) * (size_t)leaf_cap;
 }
 static int nblk_for(int n) { return (n + 3 + kBlk - 1) / kBlk; }
 
@@ -5393,12 +5383,12 @@ static RunShape run_shape(int n, int max_n, int maxw, size_t lds_limit, int wave
     // states: 39.1 ms one by one, 35.1 ms).
     size_t room = lds_limit;
     const int nw2 = std::min(r.nw, kMaxWaves / 2);
-    if (n > ncu && engine_lds_bytes(nblk, maxw, 0, nw2) <= lds_limit / 2) {
+    if (n > ncu && engine_lds_bytes(nblk, maxw, nw2) <= lds_limit / 2) {
         room = lds_limit / 2;
         r.nw = nw2;
     }
-    while (r.nw > 2 && engine_lds_bytes(nblk, maxw, 0, r.nw) > lds_limit) --r.nw;
-    const size_t base = engine_lds_bytes(nblk, maxw, 0, r.nw);
+    while (r.nw > 2 && engine_lds_bytes(nblk, maxw, r.nw) > lds_limit) --r.nw;
+    const size_t base = engine_lds_bytes(nblk, maxw, r.nw);
     r.lds = room;
     if (n > ncu) r.lds = std::min(room, base + (sizeof(Leaf) + sizeof(unsigned)) * (size_t)(max_n + 4));
     if (r.lds < base) r.lds = base;
