@@ -5379,8 +5379,10 @@ static RunShape run_shape(int n, int max_n, int maxw, size_t lds_limit, int wave
     // minima.  Beyond that, a compute unit holds eight wavefronts of the
     // registers that k_run takes, so workgroups of at most four share it two
     // by two: a wavefront less costs a system far less than waiting for
-    // another one's whole launch (320 systems, 2000 entries each, and their
-    // states: 39.1 ms one by one, 35.1 ms).
+    // another one's whole launch.  257 systems at four wavefronts asked for,
+    // two by two / one by one: 128 beads 9.5 / 15.7 ms, 1536 8.2 / 11.1, 23 424
+    // 3.8 / 5.3; at eight 9.4 / 15.9, 8.2 / 7.7, 3.8 / 3.6, where one by one would
+    // be the better form from some 1000 beads on.
     size_t room = lds_limit;
     const int nw2 = std::min(r.nw, kMaxWaves / 2);
     if (n > ncu && engine_lds_bytes(nblk, maxw, nw2) <= lds_limit / 2) {
